@@ -1166,7 +1166,7 @@ int build_horseshoes(fp_ctx *ctx, fp_body *b)
     ++b->version;
     if (b->d_hh) { (void)hipFree(b->d_hh); b->d_hh = nullptr; }
     if (b->d_hcol) { (void)hipFree(b->d_hcol); b->d_hcol = nullptr; }
-    b->nh = 0;
+    b->nh = b->nhg = 0;
     if (b->ns == 0) return FP_OK;
     std::vector<double> rows;  // per horseshoe 12 values
     std::vector<int> cols;
@@ -1194,11 +1194,23 @@ int build_horseshoes(fp_ctx *ctx, fp_body *b)
     std::vector<double> soa((size_t)12 * nh);
     for (int h = 0; h < nh; ++h)
         for (int c = 0; c < 12; ++c) soa[(size_t)c * nh + h] = rows[(size_t)h * 12 + c];
+    // columns, then the horseshoes grouped by column for the wake assembly
+    std::vector<int> tab(cols);
+    std::vector<int> ord(nh), gptr;
+    for (int h = 0; h < nh; ++h) ord[h] = h;
+    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return cols[x] < cols[y]; });
+    for (int q = 0; q < nh; ++q)
+        if (q == 0 || cols[ord[q]] != cols[ord[q - 1]]) gptr.push_back(q);
+    const int ng = (int)gptr.size();
+    gptr.push_back(nh);
+    tab.insert(tab.end(), ord.begin(), ord.end());
+    tab.insert(tab.end(), gptr.begin(), gptr.end());
     FP_HIP(ctx, hipMalloc((void **)&b->d_hh, soa.size() * sizeof(double)));
-    FP_HIP(ctx, hipMalloc((void **)&b->d_hcol, nh * sizeof(int)));
+    FP_HIP(ctx, hipMalloc((void **)&b->d_hcol, tab.size() * sizeof(int)));
     FP_HIP(ctx, hipMemcpy(b->d_hh, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice));
-    FP_HIP(ctx, hipMemcpy(b->d_hcol, cols.data(), nh * sizeof(int), hipMemcpyHostToDevice));
+    FP_HIP(ctx, hipMemcpy(b->d_hcol, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice));
     b->nh = nh;
+    b->nhg = ng;
     return FP_OK;
 }
 

@@ -284,49 +284,55 @@ __global__ __launch_bounds__(256) void k_assemble_source(PanelView pan, TargetVi
     }
 }
 
-// Wake horseshoes into their columns: one lane per target, shedding list in order.
+// Wake horseshoes into their columns: one lane per column group (the horseshoes of one
+// column in shedding order, their twelve parameters in registers; on an ordinary trailing
+// edge every group is one horseshoe), each wave walking WAKE_T targets, so that no two
+// lanes touch the same entry.  Bound by the latency of the entry's read-modify-write and of
+// the FP64 divisions of about three segments per pair, so the launch has to fill the chip:
+// with one lane per target walking every horseshoe a 4,800-panel wing had 19 workgroups.
 // dblk > 0: G is the compact diagonal-block array of block size dblk (block b at
 // G + b dblk^2, row-major with leading dimension dblk) and only the columns in
 // the target's own block are updated.
+constexpr int WAKE_T = 4;
 template <typename T, typename TO>
 __global__ __launch_bounds__(256) void k_assemble_wake(HorseView hv, double off_, double cut_, TargetView tv,
                                                        TO *__restrict__ G, int64_t ld, int64_t col0,
                                                        float *__restrict__ G2, int dblk)
 {
-    __shared__ T sh[64][12];
-    __shared__ int sc[64];
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool ok = i < tv.M;
-    const T X = ok ? T(tv.x[i]) : T(0), Y = ok ? T(tv.y[i]) : T(0), Z = ok ? T(tv.z[i]) : T(0);
-    const T nx = ok ? T(tv.nx[i]) : T(0), ny = ok ? T(tv.ny[i]) : T(0), nz = ok ? T(tv.nz[i]) : T(0);
+    const int g = blockIdx.y * 64 + (threadIdx.x & 63);
+    const int64_t i0 = ((int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * WAKE_T;
+    if (g >= hv.ng || i0 >= tv.M) return;
     const T off = T(off_), off2 = T(off_ * off_), cut2 = T(cut_ * cut_);
-    for (int h0 = 0; h0 < hv.nh; h0 += 64) {
-        const int cnt = min(64, hv.nh - h0);
-        __syncthreads();
-        for (int t = threadIdx.x; t < cnt * 12; t += blockDim.x) {
-            const int hh = t / 12, c = t % 12;
-            sh[hh][c] = T(hv.hh[(int64_t)c * hv.nh + h0 + hh]);
-        }
-        for (int t = threadIdx.x; t < cnt; t += blockDim.x) sc[t] = hv.col[h0 + t];
-        __syncthreads();
-        if (ok) {
-            for (int hh = 0; hh < cnt; ++hh) {
-                T ux = 0, uy = 0, uz = 0;
-                TO *g;
-                if (dblk > 0) {
-                    const int64_t bb = i / dblk, c = sc[hh] - bb * dblk;
-                    if (c < 0 || c >= dblk) continue;
-                    g = G + bb * dblk * dblk + (i - bb * dblk) * dblk + c;
-                } else {
-                    g = G + i * ld + col0 + sc[hh];
-                }
-                horseshoe_u<T>(sh[hh], X, Y, Z, T(1), off, off2, cut2, ux, uy, uz);
-                const TO v = TO(T(*g) + (ux * nx + uy * ny + uz * nz));
-                *g = v;
-                if (G2 && dblk == 0) G2[i * ld + col0 + sc[hh]] = float(v);
+    const int cnt = (int)min((int64_t)WAKE_T, tv.M - i0);
+    const int q0 = hv.gptr[g], q1 = hv.gptr[g + 1];
+    for (int q = q0; q < q1; ++q) {
+        const int h = hv.ord[q], col = hv.col[h];
+        T p[12];
+#pragma unroll
+        for (int c = 0; c < 12; ++c) p[c] = T(hv.hh[(int64_t)c * hv.nh + h]);
+        for (int t = 0; t < cnt; ++t) {
+            const int64_t i = i0 + t;
+            TO *dst;
+            if (dblk > 0) {
+                const int64_t bb = i / dblk, c = col - bb * dblk;
+                if (c < 0 || c >= dblk) continue;
+                dst = G + bb * dblk * dblk + (i - bb * dblk) * dblk + c;
+            } else {
+                dst = G + i * ld + col0 + col;
             }
+            const TO old = *dst;
+            T ux = 0, uy = 0, uz = 0;
+            horseshoe_u<T>(p, T(tv.x[i]), T(tv.y[i]), T(tv.z[i]), T(1), off, off2, cut2, ux, uy, uz);
+            const TO v = TO(T(old) + (ux * T(tv.nx[i]) + uy * T(tv.ny[i]) + uz * T(tv.nz[i])));
+            *dst = v;
+            if (G2 && dblk == 0) G2[i * ld + col0 + col] = float(v);
         }
     }
+}
+
+static dim3 wake_grid(const fp_body *b, int64_t M)
+{
+    return dim3((unsigned)((M + 4 * WAKE_T - 1) / (4 * WAKE_T)), (unsigned)((b->nhg + 63) / 64));
 }
 
 int fp_launch_assemble_diag(fp_ctx *ctx, const fp_body *b, const TargetView &tv, int block, float *X)
@@ -342,8 +348,7 @@ int fp_launch_assemble_diag(fp_ctx *ctx, const fp_body *b, const TargetView &tv,
         hipLaunchKernelGGL((k_assemble_diag_vr<8, TM>), grid, dim3(256), 0, ctx->stream, panel_view(b), tv, block, X);
     FP_HIP(ctx, hipGetLastError());
     if (b->nh > 0) {
-        dim3 g2((unsigned)((tv.M + 255) / 256));
-        hipLaunchKernelGGL((k_assemble_wake<double, float>), g2, dim3(256), 0, ctx->stream, horse_view(b),
+        hipLaunchKernelGGL((k_assemble_wake<double, float>), wake_grid(b, tv.M), dim3(256), 0, ctx->stream, horse_view(b),
                            b->kernel_offset, b->kernel_cutoff, tv, X, (int64_t)0, (int64_t)0, (float *)nullptr, block);
         FP_HIP(ctx, hipGetLastError());
     }
@@ -377,8 +382,7 @@ int fp_launch_assemble(fp_ctx *ctx, const fp_body *b, const TargetView &tv, T *G
         FP_HIP(ctx, hipGetLastError());
         if (b->nh > 0) {
             ProfScope pw(ctx, "assemble_wake");
-            dim3 g2((unsigned)((tv.M + 255) / 256));
-            hipLaunchKernelGGL((k_assemble_wake<double, T>), g2, dim3(256), 0, ctx->stream, horse_view(b),
+            hipLaunchKernelGGL((k_assemble_wake<double, T>), wake_grid(b, tv.M), dim3(256), 0, ctx->stream, horse_view(b),
                                b->kernel_offset, b->kernel_cutoff, tv, G, ld, col0, G32, 0);
             FP_HIP(ctx, hipGetLastError());
         }
@@ -402,8 +406,7 @@ int fp_launch_assemble_wake(fp_ctx *ctx, const fp_body *b, const TargetView &tv,
 {
     if (b->element != FP_ELEM_VORTEXRING || b->nh == 0 || tv.M == 0) return FP_OK;
     ProfScope pw(ctx, "assemble_wake");
-    dim3 g2((unsigned)((tv.M + 255) / 256));
-    hipLaunchKernelGGL((k_assemble_wake<double, T>), g2, dim3(256), 0, ctx->stream, horse_view(b), b->kernel_offset,
+    hipLaunchKernelGGL((k_assemble_wake<double, T>), wake_grid(b, tv.M), dim3(256), 0, ctx->stream, horse_view(b), b->kernel_offset,
                        b->kernel_cutoff, tv, G, ld, col0, (float *)nullptr, 0);
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;

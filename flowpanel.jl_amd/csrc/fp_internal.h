@@ -125,8 +125,8 @@ struct fp_body {
     double *d_geo = nullptr;
     double *d_uinf = nullptr;       // 3 x N SoA
     double *d_hh = nullptr;         // horseshoes
-    int *d_hcol = nullptr;
-    int nh = 0;
+    int *d_hcol = nullptr;          // nh columns, then the horseshoes grouped by column: nh indices, nhg + 1 offsets
+    int nh = 0, nhg = 0;
     double *d_strength = nullptr;
     bool has_uinf = false, has_wake = false, solved = false;
     uint64_t version = 0;  // bumped whenever device geometry or wake buffers change
@@ -185,6 +185,10 @@ struct HorseView {
     const double *hh;
     const int *col;
     int nh;
+    // the horseshoes grouped by column (shedding order within a group): group g holds
+    // ord[gptr[g]] .. ord[gptr[g + 1] - 1]
+    const int *ord, *gptr;
+    int ng;
 };
 
 static inline PanelView panel_view(const fp_body *b)
@@ -197,6 +201,7 @@ static inline PanelView panel_view(const fp_body *b)
 static inline HorseView horse_view(const fp_body *b)
 {
     HorseView h; h.hh = b->d_hh; h.col = b->d_hcol; h.nh = b->nh;
+    h.ord = b->d_hcol + b->nh; h.gptr = b->d_hcol + 2 * b->nh; h.ng = b->nhg;
     return h;
 }
 
