@@ -12,11 +12,30 @@
 
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
+#include "fp_elements.h"
 #define FPA_HD __host__ __device__ __forceinline__
 #else
 #define FPA_HD inline
 #endif
 #include <math.h>
+
+// 1/x and 1/sqrt(x): on the device the refined hardware seeds of fp_elements.h
+FPA_HD double fpa_recip(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return fp_recip(x);
+#else
+    return 1.0 / x;
+#endif
+}
+FPA_HD double fpa_rsqrt(double x)   // x > 0
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return x >= 0x1p-1000 && x < 0x1p1000 ? fp_rsqrt_nb(x) : 1.0 / sqrt(x);
+#else
+    return 1.0 / sqrt(x);
+#endif
+}
 
 #define FPA_4PI 12.566370614359172953850573533118
 
@@ -171,9 +190,10 @@ FPA_HD void fpa_ring_rev(const double (&p)[NVP][3], double X, double Y, double Z
 #pragma unroll
     for (int k = 0; k < NVP; ++k) {
         r[k][0] = X - p[k][0]; r[k][1] = Y - p[k][1]; r[k][2] = Z - p[k][2];
-        const double l = sqrt(r[k][0] * r[k][0] + r[k][1] * r[k][1] + r[k][2] * r[k][2]);
-        iv[k] = 1.0 / (l + off);
-        sk[k] = l > 0 ? iv[k] * iv[k] / l : 0.0;
+        const double l2 = r[k][0] * r[k][0] + r[k][1] * r[k][1] + r[k][2] * r[k][2];
+        const double y = l2 > 0 ? fpa_rsqrt(l2) : 0.0;   // 1/|r|
+        iv[k] = fpa_recip(l2 * y + off);
+        sk[k] = l2 > 0 ? iv[k] * iv[k] * y : 0.0;
     }
     const double off2 = off * off, cut2 = cut * cut;
 #pragma unroll
@@ -190,8 +210,9 @@ FPA_HD void fpa_ring_rev(const double (&p)[NVP][3], double X, double Y, double Z
         const double dvz = r[k][2] * iv[k] - r[q][2] * iv[q];
         const double proj = ex * dvx + ey * dvy + ez * dvz;
         const double den = c2 + off2;
-        const double Kf = 1.0 / (FPA_4PI * den);
+        const double Kf = fpa_recip(FPA_4PI * den);
         const double A = proj * Kf;
+        const double A2 = -2.0 * FPA_4PI * A * Kf;   // -2 A / den
         const double rke = (r[k][0] * ex + r[k][1] * ey + r[k][2] * ez) * sk[k];
         const double rqe = (r[q][0] * ex + r[q][1] * ey + r[q][2] * ez) * sk[q];
         // T_k(e) - T_q(e), T_k(e), T_q(e)
@@ -202,7 +223,7 @@ FPA_HD void fpa_ring_rev(const double (&p)[NVP][3], double X, double Y, double Z
             const double sb = w[m][0] * cx + w[m][1] * cy + w[m][2] * cz;
             g[m] += A * sb;
             const double projb = sb * Kf;
-            const double c2b2 = -2.0 * sb * A / den;
+            const double c2b2 = sb * A2;
             const double cbx = A * w[m][0] + c2b2 * cx;
             const double cby = A * w[m][1] + c2b2 * cy;
             const double cbz = A * w[m][2] + c2b2 * cz;

@@ -484,7 +484,7 @@ __global__ __launch_bounds__(256) void k_assemble_vre(const int32_t *__restrict_
     const int tid = threadIdx.x;
     const int32_t *T = tab + (int64_t)blockIdx.x * VRE_BLOCK_INTS;
     const int64_t i0 = (int64_t)blockIdx.y * TM;
-    for (int t = tid; t < TM; t += blockDim.x) {
+    for (int t = threadIdx.x; t < TM; t += blockDim.x) {
         const int64_t i = i0 + t;
         const bool ok = i < tv.M;
         st[0][t] = ok ? tv.x[i] : 0.0;
@@ -503,24 +503,27 @@ __global__ __launch_bounds__(256) void k_assemble_vre(const int32_t *__restrict_
     };
     // node slots of this lane (slot s = node s * 256 + tid of the block)
     double px[VRE_NS], py[VRE_NS], pz[VRE_NS];
-    bool nok[VRE_NS];
+    bool nok[VRE_NS], nrun[VRE_NS];
 #pragma unroll
     for (int s = 0; s < VRE_NS; ++s) {
         const int n = s * VRE_P + tid;
         const int32_t ref = n < VRE_NPACK ? T[VRE_OFF_NODE + n] : -1;
         nok[s] = ref >= 0;
+        nrun[s] = __ballot(nok[s]) != 0;
         px[s] = py[s] = pz[s] = 0.0;
         if (nok[s]) node_xyz(ref, px[s], py[s], pz[s]);
     }
     // edge slots: local end nodes and the edge vector b - a in FP64 coordinates
+    const int te = tid;
     int ea[VRE_ES], eb[VRE_ES];
     double ex[VRE_ES], ey[VRE_ES], ez[VRE_ES];
-    bool eok[VRE_ES];
+    bool eok[VRE_ES], erun[VRE_ES];
 #pragma unroll
     for (int s = 0; s < VRE_ES; ++s) {
-        const int e = s * VRE_P + tid;
+        const int e = s * VRE_P + te;
         const int32_t ab = e < VRE_EPACK ? T[VRE_OFF_EDGE + e] : -1;
         eok[s] = ab >= 0;
+        erun[s] = __ballot(eok[s]) != 0;
         ea[s] = eok[s] ? (ab & 0xFFFF) : 0;
         eb[s] = eok[s] ? ((ab >> 16) & 0xFFFF) : 0;
         ex[s] = ey[s] = ez[s] = 0.0;
@@ -560,7 +563,7 @@ __global__ __launch_bounds__(256) void k_assemble_vre(const int32_t *__restrict_
                 const int t = min(t0 + tt, iend - 1);
                 const double rx = st[0][t] - px[s], ry = st[1][t] - py[s], rz = st[2][t] - pz[s];
                 q[tt].x = rx; q[tt].y = ry; q[tt].z = rz;
-                q[tt].iv = fp_recip(fp_sqrt_nb(rx * rx + ry * ry + rz * rz) + off);
+                q[tt].iv = fp_recip_nb(fp_sqrt_nb(rx * rx + ry * ry + rz * rz) + off);
             }
             if (nok[s]) {
 #pragma unroll
@@ -568,8 +571,8 @@ __global__ __launch_bounds__(256) void k_assemble_vre(const int32_t *__restrict_
             }
         }
         __syncthreads();
-        // edge terms, branch-free (the regularised factor is finite for c2 = 0 when off > 0;
-        // the select drops it below the cutoff either way)
+        // edge terms, branch-free (the select drops c2 below the cutoff, where the regularised factor
+        // need not be finite)
 #pragma unroll
         for (int s = 0; s < VRE_ES; ++s) {
             double v[TT];
@@ -583,12 +586,12 @@ __global__ __launch_bounds__(256) void k_assemble_vre(const int32_t *__restrict_
                 const double c2 = cx * cx + cy * cy + cz * cz;
                 const double proj = ex[s] * (A.x * A.iv - B.x * B.iv) + ey[s] * (A.y * A.iv - B.y * B.iv) +
                                     ez[s] * (A.z * A.iv - B.z * B.iv);
-                const double w = proj * fp_recip(k4 * (c2 + off2)) * (cx * st[3][t] + cy * st[4][t] + cz * st[5][t]);
+                const double w = proj * fp_recip_nb(fmin(k4 * (c2 + off2), 0x1p1000)) * (cx * st[3][t] + cy * st[4][t] + cz * st[5][t]);
                 v[tt] = c2 > cut2 ? w : 0.0;
             }
             if (eok[s]) {
 #pragma unroll
-                for (int tt = 0; tt < TT; ++tt) se[tt][s * VRE_P + tid] = v[tt];
+                for (int tt = 0; tt < TT; ++tt) se[tt][s * VRE_P + te] = v[tt];
             }
         }
         __syncthreads();

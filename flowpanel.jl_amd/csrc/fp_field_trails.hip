@@ -224,29 +224,33 @@ __global__ __launch_bounds__(256) void k_field_trail(const double *__restrict__ 
         }
         __syncthreads();
         // straight-line body (a select instead of branches, so that the unrolled entries
-        // interleave): a trail start (gamma = 0) and a segment below the cutoff add zero
+        // interleave): a trail start (gamma = 0) adds zero, and the select drops a segment below
+        // the cutoff (a zero c2, whose reciprocals need not be finite, among them)
 #pragma unroll 2
         for (int q = 0; q < cnt; ++q) {
             const double rx = X - st[0][q], ry = Y - st[1][q], rz = Z - st[2][q];
-            const double iv = fp_recip(fp_sqrt_nb(rx * rx + ry * ry + rz * rz) + off);
-            const double g = st[6][q];
+            const double iv = fp_recip_nb(fp_sqrt_nb(rx * rx + ry * ry + rz * rz) + off);
             const double cx = rpy * rz - rpz * ry;
             const double cy = rpz * rx - rpx * rz;
             const double cz = rpx * ry - rpy * rx;
             const double c2 = cx * cx + cy * cy + cz * cz;
             const double proj = st[3][q] * (rpx * ivp - rx * iv) + st[4][q] * (rpy * ivp - ry * iv) +
                                 st[5][q] * (rpz * ivp - rz * iv);
-            const double a = g * proj * fp_recip(4.0 * FP_PI * (c2 + off2));
-            const double aux = (g != 0.0 && c2 > cut2) ? a : 0.0;
+            // the denominator capped at 2^1000: beyond it the velocity is zero to FP64 anyway
+            const double a = st[6][q] * proj * fp_recip_nb(fmin(4.0 * FP_PI * (c2 + off2), 0x1p1000));
+            const double aux = c2 > cut2 ? a : 0.0;
             ux += aux * cx; uy += aux * cy; uz += aux * cz;
             rpx = rx; rpy = ry; rpz = rz; ivp = iv;
         }
     }
-    // wake horseshoes (split 0 only), strengths of their panels
-    if (blockIdx.y == 0 && hv.nh > 0) {
+    // wake horseshoes, strengths of their panels: split y of the launch takes the y-th part of them
+    // (all of them in one split made its workgroups the last to finish: with 10,000 targets and
+    // 51 splits, 200 horseshoes are 1.5 times a split's share of the stream)
+    const int w0 = (int)((int64_t)hv.nh * blockIdx.y / gridDim.y), w1 = (int)((int64_t)hv.nh * (blockIdx.y + 1) / gridDim.y);
+    if (w1 > w0) {
         __shared__ double sh[32][13];
-        for (int h0 = 0; h0 < hv.nh; h0 += 32) {
-            const int cnt = min(32, hv.nh - h0);
+        for (int h0 = w0; h0 < w1; h0 += 32) {
+            const int cnt = min(32, w1 - h0);
             __syncthreads();
             for (int t = threadIdx.x; t < cnt * 12; t += blockDim.x) {
                 const int hh = t / 12, c = t % 12;

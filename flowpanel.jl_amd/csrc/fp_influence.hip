@@ -546,11 +546,12 @@ __global__ __launch_bounds__(256) void k_field(PanelView pan, const double *__re
             }
         }
     }
-    // wake horseshoes (split 0 only), strengths of their panels
-    if (ELEM == FP_ELEM_VORTEXRING && blockIdx.y == 0 && hv.nh > 0) {
+    // wake horseshoes, strengths of their panels: split y of the launch takes the y-th part of them
+    const int w0 = (int)((int64_t)hv.nh * blockIdx.y / gridDim.y), w1 = (int)((int64_t)hv.nh * (blockIdx.y + 1) / gridDim.y);
+    if (ELEM == FP_ELEM_VORTEXRING && w1 > w0) {
         __shared__ double sh[32][13];
-        for (int h0 = 0; h0 < hv.nh; h0 += 32) {
-            const int cnt = min(32, hv.nh - h0);
+        for (int h0 = w0; h0 < w1; h0 += 32) {
+            const int cnt = min(32, w1 - h0);
             __syncthreads();
             for (int t = threadIdx.x; t < cnt * 12; t += blockDim.x) {
                 const int hh = t / 12, c = t % 12;
@@ -596,10 +597,15 @@ __global__ void k_field_reduce(const double *__restrict__ partial, int splits, i
     }
 }
 
+// Splits of the panel range over grid.y.  Up to 512 workgroups of targets: 2,048 workgroups, one
+// round of the chip.  Above that the last, partly filled round costs (2,344 workgroups of 600,000
+// targets are 9.2 a compute unit, of which the last 1.2 run nearly alone), so the work is cut to
+// 8,192 and more; the partial sums are 24 bytes a target and split.
 static int field_splits(int64_t M, int64_t N)
 {
     const int64_t bx = (M + 255) / 256;
-    int64_t s = (2048 + bx - 1) / bx;
+    const int64_t want = bx > 512 ? 8192 : 2048;
+    int64_t s = (want + bx - 1) / bx;
     s = std::min<int64_t>(s, (N + FIELD_TILE - 1) / FIELD_TILE);
     return (int)std::max<int64_t>(1, std::min<int64_t>(s, 256));
 }
@@ -642,8 +648,9 @@ int fp_launch_field(fp_ctx *ctx, const fp_body *b, const double *strength, const
     if (tv.M == 0 || b->N == 0) return FP_OK;
     int splits = field_splits(tv.M, b->N);
     const int comps = mode == 0 ? 3 : 1;
-    if (splits > 1 && (partial == nullptr || partial_bytes < (size_t)splits * comps * tv.M * sizeof(double)))
-        splits = 1;
+    // as many splits as the caller's scratch holds
+    const int64_t fit = partial ? (int64_t)(partial_bytes / ((size_t)comps * tv.M * sizeof(double))) : 1;
+    splits = (int)std::max<int64_t>(1, std::min<int64_t>(splits, fit));
     int64_t pchunk = (b->N + splits - 1) / splits;
     pchunk = (pchunk + FIELD_TILE - 1) / FIELD_TILE * FIELD_TILE;
     splits = (int)((b->N + pchunk - 1) / pchunk);
