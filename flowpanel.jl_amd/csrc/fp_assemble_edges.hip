@@ -481,7 +481,12 @@ __global__ __launch_bounds__(256) void k_assemble_vre(const int32_t *__restrict_
     __shared__ double st[6][TM];
     __shared__ NodeTerm sn[TT][VRE_NPACK];
     __shared__ double se[TT][VRE_EPACK];
-    const int tid = threadIdx.x;
+    // A block of 254 panels has about 292 nodes and 546 edges: slots past the first (nodes) and the
+    // second (edges) fill one wave of the four.  The waves whose slot is empty skip it, the edges'
+    // remainder goes to another wave than the nodes', and the waves are renumbered from block to
+    // block, so that the SIMDs share the remainders: 14 wave-slots per pair of targets instead of
+    // 20 (the kernel is bound by FP64 issue and by its LDS traffic, not by the stores).
+    const int tid = (threadIdx.x + 64 * ((blockIdx.x + blockIdx.y) & 3)) & (VRE_P - 1);
     const int32_t *T = tab + (int64_t)blockIdx.x * VRE_BLOCK_INTS;
     const int64_t i0 = (int64_t)blockIdx.y * TM;
     for (int t = threadIdx.x; t < TM; t += blockDim.x) {
@@ -514,7 +519,7 @@ __global__ __launch_bounds__(256) void k_assemble_vre(const int32_t *__restrict_
         if (nok[s]) node_xyz(ref, px[s], py[s], pz[s]);
     }
     // edge slots: local end nodes and the edge vector b - a in FP64 coordinates
-    const int te = tid;
+    const int te = (tid - 64) & (VRE_P - 1);
     int ea[VRE_ES], eb[VRE_ES];
     double ex[VRE_ES], ey[VRE_ES], ez[VRE_ES];
     bool eok[VRE_ES], erun[VRE_ES];
@@ -557,6 +562,7 @@ __global__ __launch_bounds__(256) void k_assemble_vre(const int32_t *__restrict_
         // per slot, the TT targets are independent chains and are stored together
 #pragma unroll
         for (int s = 0; s < VRE_NS; ++s) {
+            if (!nrun[s]) continue;
             NodeTerm q[TT];
 #pragma unroll
             for (int tt = 0; tt < TT; ++tt) {
@@ -575,6 +581,7 @@ __global__ __launch_bounds__(256) void k_assemble_vre(const int32_t *__restrict_
         // need not be finite)
 #pragma unroll
         for (int s = 0; s < VRE_ES; ++s) {
+            if (!erun[s]) continue;
             double v[TT];
 #pragma unroll
             for (int tt = 0; tt < TT; ++tt) {
