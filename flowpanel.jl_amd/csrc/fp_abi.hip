@@ -776,7 +776,7 @@ struct Solver {
         if ((st = dalloc(ctx, Ar, (size_t)n4 * ld4 * sizeof(float))) ||
             (st = dalloc(ctx, Wrbt, fp_rbt_weights_bytes(n))) || (st = dalloc(ctx, perm4, n4 * sizeof(int))) ||
             (st = dalloc(ctx, work4, fp_getrs_work_bytes(n4, 1))) || (st = dalloc(ctx, t4, n4 * sizeof(double))) ||
-            (st = dalloc(ctx, nw, fp_getrf_nopiv_work_bytes())) || (st = dalloc(ctx, info, sizeof(int))))
+            (st = dalloc(ctx, nw, fp_getrf_nopiv_work_bytes(sizeof(float)))) || (st = dalloc(ctx, info, sizeof(int))))
             return st;
         if ((st = fp_rbt_weights(ctx, n, RBT_SEED, Wrbt.as<double>()))) return st;
         st = a.R64 ? fp_rbt_matrix<double>(ctx, a.R64, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>())
@@ -793,7 +793,7 @@ struct Solver {
                 (st = fp_fill_f32(ctx, YU.as<float>(), n4 * ld4, 0.f)))
                 return st;
         }
-        if ((st = fp_getrf_nopiv_f32(ctx, Ar.as<float>(), n4, ld4, info.as<int>(), nw.p,
+        if ((st = fp_getrf_nopiv<float>(ctx, Ar.as<float>(), n4, ld4, info.as<int>(), nw.p,
                                      inv ? YL.as<float>() : nullptr, inv ? YU.as<float>() : nullptr)))
             return st;
         std::vector<int> id(n4);
@@ -1028,9 +1028,11 @@ struct Solver {
         FP_HIP(ctx, hipMemsetAsync(x, 0, n * sizeof(double), ctx->stream));
         FP_HIP(ctx, hipMemcpyAsync(rp, b, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
         double rel = bn > 0 ? 1.0 : (bn == 0 ? 0.0 : NAN), rnorm = bn;   // ||r|| of the current residual (r = b at first)
-        int k = 0, its_total = 0;
+        int k = 0, its_total = 0, k0 = 0;   // k0: refinements spent on factors given up
+        bool stalled = false;
         for (;;) {
-        while (!converged(rel, o.tol) && std::isfinite(rel) && k < o.max_refine) {
+        while (!converged(rel, o.tol) && std::isfinite(rel) && k - k0 < o.max_refine && !stalled) {
+            const double before = rel;
             // correction d ~ A^-1 r in the low-precision solver
             if (a.solver == FP_SOLVER_LU32_IR) {
                 void *wk = rbt ? work4.p : work.p;
@@ -1054,10 +1056,14 @@ struct Solver {
             rel = rn / bn;
             rnorm = rn;
             ++k;
+            // a correction by good factors gains several digits: less than one bit is a failed factorisation
+            stalled = rbt && !(rel < 0.5 * before);
         }
         // the randomized no-pivot factors failed to converge: start over with the pivoted LU
         if (rbt && !converged(rel, o.tol) && std::isfinite(bn)) {
             if ((st = lu32_pivoted(stats))) return st;
+            k0 = k;
+            stalled = false;
             FP_HIP(ctx, hipMemsetAsync(x, 0, n * sizeof(double), ctx->stream));
             FP_HIP(ctx, hipMemcpyAsync(rp, b, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
             rel = bn > 0 ? 1.0 : 0.0;
@@ -1112,13 +1118,15 @@ struct Solver {
         double rel = 1.0;
         for (int64_t c = 0; c < k; ++c)
             if (!std::isfinite(bn[c])) rel = NAN;
-        int it = 0;
+        int it = 0, it0 = 0;
+        bool stalled = false;
         DBuf wk4;
         const size_t wbytes4 = rbt ? fp_getrs_work_bytes(n4, k) : 0;
         if (rbt && (st = dalloc(ctx, wk4, wbytes4))) return st;
         const double rel0 = rel;
         for (;;) {
-        while (!converged(rel, o.tol) && std::isfinite(rel) && it < o.max_refine) {
+        while (!converged(rel, o.tol) && std::isfinite(rel) && it - it0 < o.max_refine && !stalled) {
+            const double before = rel;
             if ((st = lu32_correct(R.as<double>(), D.as<double>(), k, rbt ? wk4.p : wk.p, rbt ? wbytes4 : wbytes)))
                 return st;
             if ((st = fp_axpby(ctx, 1.0, D.as<double>(), 1.0, X, n * k))) return st;
@@ -1131,10 +1139,13 @@ struct Solver {
             for (int64_t c = 0; c < k; ++c)
                 rel = worst_residual(rel, bn[c] > 0 ? std::sqrt(rn[c] / bn[c]) : (rn[c] == 0 ? 0.0 : NAN));
             ++it;
+            stalled = rbt && !(rel < 0.5 * before);
         }
         // the randomized no-pivot factors failed to converge: start over with the pivoted LU
         if (rbt && !converged(rel, o.tol) && std::isfinite(rel0)) {
             if ((st = lu32_pivoted(stats))) return st;
+            it0 = it;
+            stalled = false;
             FP_HIP(ctx, hipMemsetAsync(X, 0, (size_t)n * k * sizeof(double), ctx->stream));
             FP_HIP(ctx, hipMemcpyAsync(R.p, B, (size_t)n * k * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
             rel = rel0;
@@ -1354,7 +1365,7 @@ struct BatchImpl {
                 if ((st = dalloc(ctx, bb->Ar, (size_t)bb->n4 * bb->ld4 * sizeof(float))) ||
                     (st = dalloc(ctx, bb->W, fp_rbt_weights_bytes(n))) || (st = dalloc(ctx, bb->perm4, bb->n4 * sizeof(int))) ||
                     (st = dalloc(ctx, bb->work4, fp_getrs_work_bytes(bb->n4, 1))) ||
-                    (st = dalloc(ctx, bb->nwork, fp_getrf_nopiv_work_bytes())) ||
+                    (st = dalloc(ctx, bb->nwork, fp_getrf_nopiv_work_bytes(sizeof(float)))) ||
                     (st = dalloc(ctx, bb->t4, bb->n4 * sizeof(double))))
                     return st;
                 if ((st = fp_rbt_weights(ctx, n, RBT_SEED, bb->W.as<double>()))) return st;
@@ -1518,7 +1529,7 @@ struct BatchImpl {
     {
         int st = rbt_matrix(bb);
         if (st) return st;
-        return fp_getrf_nopiv_f32(ctx, bb.Ar.as<float>(), bb.n4, bb.ld4, bb.info.as<int>(), bb.nwork.p);
+        return fp_getrf_nopiv<float>(ctx, bb.Ar.as<float>(), bb.n4, bb.ld4, bb.info.as<int>(), bb.nwork.p);
     }
 
     // the device table of the batched LU: every randomized (not pivoted) body's U^T A V

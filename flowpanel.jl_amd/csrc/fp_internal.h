@@ -264,9 +264,10 @@ template <typename Tin>
 int fp_rbt_matrix(fp_ctx *ctx, const Tin *A, int64_t n, int64_t lda, float *Ar, int64_t ldr, const double *d_W);
 int fp_rbt_vec(fp_ctx *ctx, const double *in, int64_t ldin, double *out, int64_t ldout, int64_t n, int64_t k,
                const double *d_W, int transpose_u);
-size_t fp_getrf_nopiv_work_bytes();
-int fp_getrf_nopiv_f32(fp_ctx *ctx, float *A, int64_t n, int64_t ld, int *info_dev, void *work, float *YL = nullptr,
-                       float *YU = nullptr);
+size_t fp_getrf_nopiv_work_bytes(int elem_bytes);
+template <typename T>
+int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void *work, T *YL = nullptr,
+                   T *YU = nullptr);
 int fp_trtri_nopiv_f32(fp_ctx *ctx, const float *A, int64_t n, int64_t ld, float *YL, float *YU, float *T);
 // One body of the batched FP32 no-pivot LU (a device array of these, one per body):
 // A (n x n, ld, row-major), the LU's work (fp_getrf_nopiv_work_bytes), its info word.

@@ -10,18 +10,14 @@
 // unnecessary with probability close to one, and the LU of A_r is then a
 // plain blocked right-looking factorisation:
 //
-//   per 64-column step:  k_nopiv_diag   the 64 x 64 diagonal block factored in
-//                                       registers (one row per lane, row k
-//                                       broadcast by v_readlane), then the
-//                                       explicit inverses of L11 and U11 (two
-//                                       waves, one each);
-//                        k_nopiv_panel  L21 = A21 U11^-1 and U12 = L11^-1 A12 as
-//                                       64 x 64 x 64 products on MFMA, in place
-//                                       (U12 within the 256-column outer block);
-//                        fp_gemm_sub    the update of the outer block's columns;
-//   per 256-column outer block: the U rows right of it (blocked forward
-//   substitution: MFMA products and k_nopiv_panel), then the rank-256 MFMA
-//   trailing update.
+//   per 256-column outer block:
+//     k_lu_first   its first 64 x 64 diagonal block, with the explicit inverses of
+//                  L11 and U11, and the U tiles of that block row;
+//     k_lu_step    (four times) L21 = A21 U11^-1 and the update of the outer
+//                  block's columns, one workgroup per 64 rows; the first of them
+//                  factors the next diagonal block;
+//     k_lu_urow    the U rows right of the outer block (blocked substitution);
+//     fp_gemm_sub  the rank-256 trailing update.
 //
 // A x = b becomes  A_r y = U^T b,  x = V y.  A depth-2 butterfly couples only
 // the four indices {p, p + m, p + 2m, p + 3m} (m = n4 / 4, n4 = n rounded up
@@ -30,348 +26,503 @@
 // transforms are 4 x 4 products per orbit.  A zero or non-finite pivot is
 // reported through `info` and the caller falls back to the pivoted LU.
 #include "fp_internal.h"
+#include "fp_elements.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 
 namespace {
 
-constexpr int NPB = 64;   // block of the no-pivot LU
-
-typedef float nf4 __attribute__((ext_vector_type(4)));
+constexpr int NPB = 64;          // block of the no-pivot LU
+constexpr int NIN = 4;           // blocks per outer block
+constexpr int NOB = NIN * NPB;   // outer block: columns per trailing update
+constexpr int UW = 32;           // columns per workgroup of the U rows
 
 __device__ __forceinline__ float bcast(float v, int lane)
 {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
+__device__ __forceinline__ double bcast(double v, int lane)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
 
-// Compile-time loop: f(cint<I>{}) for I = B, B + S, ... while I < E (S > 0)
-// or I > E (S < 0), so every register-array index below is a constant.
+// Compile-time loop: f(cint<I>{}) for I = B, ..., E - 1, so that every register-array index is a constant.
 template <int V> struct cint {
     static constexpr int v = V;
 };
-template <int B, int E, int S, typename F> __device__ __forceinline__ void static_for(F &&f)
+template <int B, int E, typename F> __device__ __forceinline__ void static_for(F &&f)
 {
-    if constexpr (S > 0 ? B < E : B > E) {
+    if constexpr (B < E) {
         f(cint<B>{});
-        static_for<B + S, E, S>(f);
+        static_for<B + 1, E>(f);
     }
 }
 
-// v[q] -= f * (v[q] of lane j) for q in [LO, HI): the broadcasts go out in
-// groups of four before their FMAs, so that no v_readlane's result is
-// consumed by the very next instruction (a readlane followed at once by its
-// use costs two wait states, which doubled the length of these loops).
-template <int LO, int HI, int G = 4>
-__device__ __forceinline__ void bcast_axpy(float (&v)[NPB], float f, int j)
-{
-#pragma unroll
-    for (int q0 = LO; q0 < HI; q0 += G) {
-        float t[G];
-#pragma unroll
-        for (int u = 0; u < G; ++u)
-            if (q0 + u < HI) t[u] = bcast(v[q0 + u], j);
-#pragma unroll
-        for (int u = 0; u < G; ++u)
-            if (q0 + u < HI) v[q0 + u] = fmaf(-f, t[u], v[q0 + u]);
+// Per type: LDS row strides of left (LDA) and right (LDB, LDX) operands of the products, chosen so
+// that the 64 lanes of a fragment read fall on different banks (left: 16 rows x 4 columns; right:
+// 4 rows x 16 columns in FP32, 4 x 4 in FP64).
+template <typename T> struct Lu;
+template <> struct Lu<float> {
+    static constexpr int LDA = 68, LDB = 80, LDX = 48, V = 4;
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    typedef float vec __attribute__((ext_vector_type(4)));
+    // accumulator element e of a 16 x 16 tile
+    static __device__ __forceinline__ int row(int lane, int e) { return 4 * (lane >> 4) + e; }
+    static __device__ __forceinline__ int col(int lane, int) { return lane & 15; }
+    static __device__ __forceinline__ float div(float a, float b) { return a / b; }
+    static __device__ __forceinline__ bool bad(float p) { return !(fabsf(p) > 0.f) || !(fabsf(p) <= 3.4e38f); }
+};
+template <> struct Lu<double> {
+    static constexpr int LDA = 68, LDB = 68, LDX = 36, V = 2;
+    typedef double v4 __attribute__((ext_vector_type(4)));
+    typedef double vec __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ int row(int lane, int) { return 4 * ((lane >> 2) & 3) + (lane >> 4); }
+    static __device__ __forceinline__ int col(int lane, int e) { return 4 * e + (lane & 3); }
+    // quotient with one residual correction (rounding to within an ulp)
+    static __device__ __forceinline__ double div(double a, double b)
+    {
+        const double r = fp_recip_nb(b), q = a * r;
+        return fma(fma(-b, q, a), r, q);
     }
-}
+    static __device__ __forceinline__ bool bad(double p) { return !(fabs(p) > 1e-290) || !(fabs(p) <= 1e290); }
+};
 
-// Columns [Q0, Q1) of X = U11^-1 for row `lane`, from row `lane` of U in u[]:
-// rows bottom-up, Y_i -= (u_ic / u_cc) Y_c for i < c, then X_i = Y_i / u_ii.
-// Column q takes the steps c <= q, so a column range is independent of the rest.
-template <int Q0, int Q1>
-__device__ __forceinline__ void nopiv_uinv_cols(const float (&u)[NPB], const float (*lu)[NPB + 1], int lane, int bs,
-                                                int64_t k0, int64_t ld, float *__restrict__ Uinv,
-                                                float *__restrict__ YU)
+// acc += P Q for 16 rows of P (16 x K) and NT 16-column tiles of Q (K x 16 NT), both in LDS.
+// FP32: v_mfma_f32_16x16x4.  FP64: v_mfma_f64_4x4x4_4b, whose four blocks take 16 rows of P and
+// the same four columns of Q (the 16x16x4 form issues at half its rate).
+template <typename T, int NT>
+__device__ __forceinline__ void mma(const T *P, int ldp, const T *Q, int ldq, int K, int lane,
+                                    typename Lu<T>::v4 (&acc)[NT])
 {
-    float x[NPB];
+    const T *pp = P + (lane & 15) * ldp + (lane >> 4);
+#pragma unroll 4
+    for (int ks = 0; ks < K; ks += 4) {
+        const T pa = pp[ks];
+        if constexpr (sizeof(T) == 4) {
+            const T *q = Q + (ks + (lane >> 4)) * ldq + (lane & 15);
 #pragma unroll
-    for (int q = Q0; q < Q1; ++q) x[q] = q == lane ? 1.f : 0.f;
-    float dii = 1.f;
-    static_for<NPB - 1, -1, -1>([&](auto C) {
-        constexpr int c = decltype(C)::v;
-        dii = lane == c ? u[c] : dii;
-        if constexpr (c < Q1) {   // else no column of the range at or right of c
-            const float coef = lane < c ? u[c] * (1.f / lu[c][c]) : 0.f;
-            bcast_axpy<(c > Q0 ? c : Q0), Q1>(x, coef, c);
-        }
-    });
-    const float rd = 1.f / dii;
-#pragma unroll
-    for (int c = Q0; c < Q1; c += 4)
-        *reinterpret_cast<float4 *>(Uinv + lane * NPB + c) =
-            make_float4(x[c] * rd, x[c + 1] * rd, x[c + 2] * rd, x[c + 3] * rd);
-    if (YU && lane < bs) {   // -U11^-1 into the diagonal block of the full inverse (ld as A)
-#pragma unroll
-        for (int c = Q0; c < Q1; ++c)
-            if (c < bs) YU[(k0 + lane) * ld + k0 + c] = -(x[c] * rd);
-    }
-}
-
-// Columns [Q0, Q1) of X = L11^-1 (unit lower) for row `lane`, the row's
-// multipliers l_lane,c in l[] (zero at and right of the diagonal): rows
-// top-down, X_i -= l_ic X_c for i > c; column q takes the steps c >= q.
-template <int Q0, int Q1>
-__device__ __forceinline__ void nopiv_linv_cols(const float (&l)[NPB], int lane, int bs, int64_t k0, int64_t ld,
-                                                float *__restrict__ Linv, float *__restrict__ YL)
-{
-    float x[NPB];
-#pragma unroll
-    for (int q = Q0; q < Q1; ++q) x[q] = q == lane ? 1.f : 0.f;
-    static_for<Q0, NPB, 1>([&](auto C) {
-        constexpr int c = decltype(C)::v;
-        bcast_axpy<Q0, (c + 1 < Q1 ? c + 1 : Q1)>(x, l[c], c);
-    });
-#pragma unroll
-    for (int c = Q0; c < Q1; c += 4)
-        *reinterpret_cast<float4 *>(Linv + lane * NPB + c) = make_float4(x[c], x[c + 1], x[c + 2], x[c + 3]);
-    if (YL && lane < bs) {   // -L11^-1 likewise
-#pragma unroll
-        for (int c = Q0; c < Q1; ++c)
-            if (c < bs) YL[(k0 + lane) * ld + k0 + c] = -x[c];
-    }
-}
-
-// Diagonal block at (k0, k0): LU without pivoting in place (rows beyond n are
-// the identity), then Linv = L11^-1 (unit lower) and Uinv = U11^-1, 64 x 64
-// row-major; 512 threads.  Wave 0 holds row `lane` of the block in registers
-// and factors it; the broadcast of row j is one v_readlane per entry (j is a
-// compile-time index, every loop is unrolled), and every row takes the update,
-// rows at and above the pivot with a zero multiplier, so no update hides
-// behind a branch (the branchy form cost 37 us per block, a broadcast through
-// LDS 46 us).  Then the eight waves invert: waves 0-3 four column ranges of
-// U^-1, waves 4-7 four of L^-1, the ranges cut so that each wave takes about
-// an eighth of the 2 x 2,080 broadcast-and-FMA steps (U column q costs q + 1,
-// L column q costs 64 - q).
-__device__ __forceinline__ void nopiv_diag_dev(float *__restrict__ A, int64_t ld, int64_t n, int64_t k0,
-                                               float *__restrict__ Linv, float *__restrict__ Uinv,
-                                               int *__restrict__ info, float *__restrict__ YL, float *__restrict__ YU)
-{
-    __shared__ float lu[NPB][NPB + 1];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int bs = (int)min((int64_t)NPB, n - k0);
-    float a[NPB];
-    if (wave == 0) {
-        float *row = A + (k0 + lane) * ld + k0;
-        if (bs == NPB) {
-#pragma unroll
-            for (int c = 0; c < NPB; c += 4) {
-                const float4 v = *reinterpret_cast<const float4 *>(row + c);
-                a[c] = v.x; a[c + 1] = v.y; a[c + 2] = v.z; a[c + 3] = v.w;
-            }
+            for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, q[16 * t], acc[t], 0, 0, 0);
         } else {
+            const T *q = Q + (ks + (lane >> 4)) * ldq + (lane & 3);
 #pragma unroll
-            for (int c = 0; c < NPB; ++c) a[c] = (lane < bs && c < bs) ? row[c] : (lane == c ? 1.f : 0.f);
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    acc[t][b] = __builtin_amdgcn_mfma_f64_4x4x4f64(pa, q[16 * t + 4 * b], acc[t][b], 0, 0, 0);
         }
-        bool bad = false;
-        static_for<0, NPB, 1>([&](auto J) {
-            constexpr int j = decltype(J)::v;
-            const float piv = bcast(a[j], j);
-            bad = bad || !(fabsf(piv) > 0.f) || !(fabsf(piv) <= 3.4e38f);
-            // rows at and above j take a zero multiplier (unconditional updates, no branches)
-            const float l = lane > j ? a[j] / piv : 0.f;
-            a[j] = lane > j ? l : a[j];
-            bcast_axpy<j + 1, NPB>(a, l, j);
-        });
-        if (bad && lane == 0) atomicCAS(info, 0, (int)(k0 + 1));
-        if (lane < bs) {
-            if (bs == NPB) {
+    }
+}
+
+template <typename T, int NT> __device__ __forceinline__ void zero(typename Lu<T>::v4 (&acc)[NT])
+{
 #pragma unroll
-                for (int c = 0; c < NPB; c += 4)
-                    *reinterpret_cast<float4 *>(row + c) = make_float4(a[c], a[c + 1], a[c + 2], a[c + 3]);
+    for (int t = 0; t < NT; ++t) acc[t] = typename Lu<T>::v4{0, 0, 0, 0};
+}
+
+// A 64 x W tile through registers: thread tid holds W / 4 values, 16 bytes of a row at a time.
+// Entries outside rows < tr, cols < tc are zero; 16-byte accesses where the row piece is inside.
+template <typename T, int W> struct Tile {
+    static constexpr int V = Lu<T>::V, PER_ROW = W / V, STEP = 256 / PER_ROW, N = NPB / STEP;
+    typedef typename Lu<T>::vec vec;
+    vec v[N];
+    __device__ __forceinline__ void load(const T *p, int64_t ld, int tr, int tc, int tid)
+    {
+        const int c = (tid % PER_ROW) * V, r0 = tid / PER_ROW;
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const int r = r0 + q * STEP;
+            if (r < tr && c + V <= tc) {
+                v[q] = *reinterpret_cast<const vec *>(p + (int64_t)r * ld + c);
             } else {
 #pragma unroll
-                for (int c = 0; c < NPB; ++c)
-                    if (c < bs) row[c] = a[c];
+                for (int e = 0; e < V; ++e) v[q][e] = r < tr && c + e < tc ? p[(int64_t)r * ld + c + e] : T(0);
             }
         }
+    }
+    __device__ __forceinline__ void put(T *s, int lds, int tid) const
+    {
+        const int c = (tid % PER_ROW) * V, r0 = tid / PER_ROW;
 #pragma unroll
-        for (int c = 0; c < NPB; ++c) lu[lane][c] = a[c];
+        for (int q = 0; q < N; ++q) *reinterpret_cast<vec *>(s + (r0 + q * STEP) * lds + c) = v[q];
+    }
+};
+
+// LDS of the step kernels: three 64 x 64 tiles and two 32 x 32 staging tiles
+template <typename T> struct StepLds {
+    T P[NPB * Lu<T>::LDA];   // left operand, then L11^-1
+    T Q[NPB * Lu<T>::LDB];   // right operand, then U11^-1
+    T D[NPB * Lu<T>::LDA];   // the diagonal block
+    T tmp[2 * 32 * 36];
+};
+
+// LU without pivoting of the 64 x 64 block D in LDS, in place, and the explicit inverses Li = L11^-1
+// (unit lower) and Ui = U11^-1, by 256 threads.  Four sub-panels of 16 columns: wave 0 factors the
+// sub-panel with one row per lane in registers (row j broadcast by v_readlane, 120 broadcast-and-FMA
+// steps instead of the 2,016 of the whole block at once), a lane per column substitutes the 16 rows
+// right of it, and the waves update the rest with 16 x 16 MFMA tiles.  The inverses grow the same
+// way, 16 -> 32 -> 64: X21 = -X22 (L21 X11), X12 = -X11 (U12 X22).  The chain of 64 pivots with
+// their divisions bounds it.  Returns (wave 0) whether a pivot was zero or not finite.
+template <typename T>
+__device__ __forceinline__ bool lu_diag64(StepLds<T> &s, int tid)
+{
+    constexpr int LDA = Lu<T>::LDA, LDB = Lu<T>::LDB, LDT = 36;
+    typedef typename Lu<T>::v4 v4;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    T *D = s.D, *Li = s.P, *Ui = s.Q;
+    for (int e = tid; e < NPB * NPB; e += 256) {
+        Li[(e >> 6) * LDA + (e & 63)] = T(0);
+        Ui[(e >> 6) * LDB + (e & 63)] = T(0);
+    }
+    bool bad = false;
+#pragma unroll 1
+    for (int p = 0; p < 4; ++p) {
+        const int c0 = 16 * p;
+        if (wave == 0) {
+            T a[16];
+            T *row = D + lane * LDA + c0;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) a[c] = row[c];
+            static_for<0, 16>([&](auto J) {
+                constexpr int j = decltype(J)::v;
+                const T piv = bcast(a[j], c0 + j);
+                bad = bad || Lu<T>::bad(piv);
+                const bool below = lane > c0 + j;
+                const T l = below ? Lu<T>::div(a[j], piv) : T(0);   // zero multiplier at and above the pivot
+                a[j] = below ? l : a[j];
+#pragma unroll
+                for (int q0 = j + 1; q0 < 16; q0 += 4) {   // broadcasts ahead of their FMAs
+                    T t[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (q0 + u < 16) t[u] = bcast(a[q0 + u], c0 + j);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (q0 + u < 16) a[q0 + u] = fma(-l, t[u], a[q0 + u]);
+                }
+            });
+#pragma unroll
+            for (int c = 0; c < 16; ++c) row[c] = a[c];
+        }
+        __syncthreads();
+        if (p == 3) break;
+        if (wave == 0 && lane < 48 - c0) {
+            T x[16];
+            T *col = D + c0 * LDA + c0 + 16 + lane;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[i] = col[i * LDA];
+#pragma unroll
+            for (int i = 1; i < 16; ++i)
+#pragma unroll
+                for (int q = 0; q < i; ++q) x[i] = fma(-D[(c0 + i) * LDA + c0 + q], x[q], x[i]);
+#pragma unroll
+            for (int i = 1; i < 16; ++i) col[i * LDA] = x[i];
+        }
+        __syncthreads();
+        const int m = 3 - p;
+        for (int q = wave; q < m * m; q += 4) {
+            const int r0 = c0 + 16 + 16 * (q / m), k0 = c0 + 16 + 16 * (q % m);
+            v4 acc[1];
+            zero<T, 1>(acc);
+            mma<T, 1>(D + r0 * LDA + c0, LDA, D + c0 * LDA + k0, LDA, 16, lane, acc);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) D[(r0 + Lu<T>::row(lane, e)) * LDA + k0 + Lu<T>::col(lane, e)] -= acc[0][e];
+        }
+        __syncthreads();
+    }
+    {
+        // 16 x 16 diagonal inverses, wave = block: lanes 0-15 the columns of L^-1, lanes 16-31 those of
+        // U^-1 with rows and columns reversed, which makes it the same forward substitution
+        const int c0 = 16 * wave, up = (lane >> 4) & 1, col = lane & 15;
+        const T rd = Lu<T>::div(T(1), D[(c0 + col) * (LDA + 1)]);
+        const T *base = up ? D + (c0 + 15) * (LDA + 1) : D + c0 * (LDA + 1);
+        const int sg = up ? -1 : 1;
+        T y[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            T v = i == col ? T(1) : T(0);
+#pragma unroll
+            for (int q = 0; q < i; ++q) v = fma(-base[sg * (i * LDA + q)], y[q], v);
+            const T d = bcast(rd, 15 - i);
+            y[i] = up ? v * d : v;
+        }
+        if (lane < 32) {
+            T *dst = up ? Ui + (c0 + 15) * LDB + c0 + 15 - col : Li + c0 * LDA + c0 + col;
+            const int st = up ? -LDB : LDA;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dst[i * st] = y[i];
+        }
     }
     __syncthreads();
-    if (wave == 0) {
-        nopiv_uinv_cols<0, 32>(a, lu, lane, bs, k0, ld, Uinv, YU);
-        return;
-    }
-    if (wave < 4) {   // U part of row `lane` (the strictly lower entries are never read)
+    const int isu = wave >> 1, h = wave & 1;
+    T *tw = s.tmp + isu * 32 * LDT;
+    {
+        // 16 -> 32: wave = (L or U, pair h)
+        const int b0 = 32 * h, b1 = b0 + 16;
+        v4 acc[1];
+        zero<T, 1>(acc);
+        if (!isu) mma<T, 1>(D + b1 * LDA + b0, LDA, Li + b0 * (LDA + 1), LDA, 16, lane, acc);
+        else mma<T, 1>(D + b0 * LDA + b1, LDA, Ui + b1 * (LDB + 1), LDB, 16, lane, acc);
+        T *th = tw + 16 * h * LDT;
 #pragma unroll
-        for (int c = 0; c < NPB; ++c) a[c] = lu[lane][c];
-        if (wave == 1) nopiv_uinv_cols<32, 44>(a, lu, lane, bs, k0, ld, Uinv, YU);
-        else if (wave == 2) nopiv_uinv_cols<44, 56>(a, lu, lane, bs, k0, ld, Uinv, YU);
-        else nopiv_uinv_cols<56, 64>(a, lu, lane, bs, k0, ld, Uinv, YU);
-        return;
-    }
+        for (int e = 0; e < 4; ++e) th[Lu<T>::row(lane, e) * LDT + Lu<T>::col(lane, e)] = acc[0][e];
+        __syncthreads();
+        zero<T, 1>(acc);
+        if (!isu) mma<T, 1>(Li + b1 * (LDA + 1), LDA, th, LDT, 16, lane, acc);
+        else mma<T, 1>(Ui + b0 * (LDB + 1), LDB, th, LDT, 16, lane, acc);
 #pragma unroll
-    for (int c = 0; c < NPB; ++c) a[c] = c < lane ? lu[lane][c] : 0.f;
-    if (wave == 4) nopiv_linv_cols<0, 8>(a, lane, bs, k0, ld, Linv, YL);
-    else if (wave == 5) nopiv_linv_cols<8, 20>(a, lane, bs, k0, ld, Linv, YL);
-    else if (wave == 6) nopiv_linv_cols<20, 32>(a, lane, bs, k0, ld, Linv, YL);
-    else nopiv_linv_cols<32, 64>(a, lane, bs, k0, ld, Linv, YL);
+        for (int e = 0; e < 4; ++e) {
+            const int r = Lu<T>::row(lane, e), c = Lu<T>::col(lane, e);
+            if (!isu) Li[(b1 + r) * LDA + b0 + c] = -acc[0][e];
+            else Ui[(b0 + r) * LDB + b1 + c] = -acc[0][e];
+        }
+        __syncthreads();
+    }
+    {
+        // 32 -> 64: wave = (L or U, 16 rows of the 32 x 32 block)
+        v4 acc[2];
+        zero<T, 2>(acc);
+        if (!isu) mma<T, 2>(D + (32 + 16 * h) * LDA, LDA, Li, LDA, 32, lane, acc);
+        else mma<T, 2>(D + 16 * h * LDA + 32, LDA, Ui + 32 * (LDB + 1), LDB, 32, lane, acc);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tw[(16 * h + Lu<T>::row(lane, e)) * LDT + 16 * t + Lu<T>::col(lane, e)] = acc[t][e];
+        __syncthreads();
+        zero<T, 2>(acc);
+        if (!isu) mma<T, 2>(Li + (32 + 16 * h) * LDA + 32, LDA, tw, LDT, 32, lane, acc);
+        else mma<T, 2>(Ui + 16 * h * LDB, LDB, tw, LDT, 32, lane, acc);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 16 * h + Lu<T>::row(lane, e), c = 16 * t + Lu<T>::col(lane, e);
+                if (!isu) Li[(32 + r) * LDA + c] = -acc[t][e];
+                else Ui[r * LDB + 32 + c] = -acc[t][e];
+            }
+    }
+    __syncthreads();
+    return bad;
 }
 
-__global__ __launch_bounds__(512) void k_nopiv_diag(float *__restrict__ A, int64_t ld, int64_t n, int64_t k0,
-                                                   float *__restrict__ Linv, float *__restrict__ Uinv,
-                                                   int *__restrict__ info, float *__restrict__ YL,
-                                                   float *__restrict__ YU)
+// One matrix of the factorisation (a batch holds one per body).  work: L11^-1 and U11^-1 of the
+// outer block's NIN diagonal blocks, 64 x 64 each; YL, YU: -L11^-1, -U11^-1 into the diagonal blocks
+// of the full inverses (may be null).
+template <typename T> struct LuMat {
+    T *A;
+    int64_t ld, n;
+    T *work;
+    int *info;
+    T *YL, *YU;
+};
+
+// The diagonal block at (c, c), held in s.D (identity outside its bs rows), inner block t of the outer
+// block that ends at kend: factor, store the factors and inverses, then the U tiles of its block row
+// inside the outer block, U = L11^-1 A.
+template <typename T>
+__device__ __forceinline__ void lu_diag_row(const LuMat<T> &m, int64_t c, int t, int64_t kend, StepLds<T> &s, int tid)
 {
-    nopiv_diag_dev(A, ld, n, k0, Linv, Uinv, info, YL, YU);
+    constexpr int LDA = Lu<T>::LDA, LDB = Lu<T>::LDB;
+    const int lane = tid & 63, wave = tid >> 6;
+    const int bs = (int)min((int64_t)NPB, m.n - c);
+    const bool bad = lu_diag64<T>(s, tid);
+    if (bad && tid == 0) atomicCAS(m.info, 0, (int)(c + 1));
+    T *Linv = m.work + (int64_t)2 * t * NPB * NPB, *Uinv = Linv + NPB * NPB;
+    for (int e = tid; e < NPB * NPB; e += 256) {
+        const int r = e >> 6, q = e & 63;
+        const T li = s.P[r * LDA + q], ui = s.Q[r * LDB + q];
+        Linv[e] = li;
+        Uinv[e] = ui;
+        if (r < bs && q < bs) {
+            m.A[(c + r) * m.ld + c + q] = s.D[r * LDA + q];
+            if (m.YL) m.YL[(c + r) * m.ld + c + q] = -li;
+            if (m.YU) m.YU[(c + r) * m.ld + c + q] = -ui;
+        }
+    }
+    for (int64_t j0 = c + NPB; j0 < kend; j0 += NPB) {
+        const int tc = (int)min((int64_t)NPB, kend - j0);
+        Tile<T, NPB> rq;
+        rq.load(m.A + c * m.ld + j0, m.ld, bs, tc, tid);
+        __syncthreads();
+        rq.put(s.Q, LDB, tid);
+        __syncthreads();
+        typename Lu<T>::v4 acc[4];
+        zero<T, 4>(acc);
+        mma<T, 4>(s.P + 16 * wave * LDA, LDA, s.Q, LDB, NPB, lane, acc);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
+                if (r < bs && cc < tc) m.A[(c + r) * m.ld + j0 + cc] = acc[q][e];
+            }
+    }
+}
+
+// First diagonal block of the outer block [k, kend) and its U tiles; one workgroup.
+template <typename T> __device__ __forceinline__ void lu_first_dev(const LuMat<T> &m, int64_t k, int64_t kend, StepLds<T> &s)
+{
+    const int tid = threadIdx.x;
+    const int bs = (int)min((int64_t)NPB, m.n - k);
+    Tile<T, NPB> rd;
+    rd.load(m.A + k * m.ld + k, m.ld, bs, bs, tid);
+    rd.put(s.D, Lu<T>::LDA, tid);
+    __syncthreads();
+    if (tid < NPB && tid >= bs) s.D[tid * (Lu<T>::LDA + 1)] = T(1);
+    __syncthreads();
+    lu_diag_row<T>(m, k, 0, kend, s, tid);
+}
+
+// Inner step t of the outer block [k, kend), c = k + 64 t, on the 64 rows below number b: the strip's
+// L tile A21 := A21 U11^-1, then A22 -= L21 U12 for the outer block's columns right of it, the U12
+// tiles being final already.  Workgroup 0 owns the next diagonal block: it goes on to factor it, so
+// that a step is one launch and the other strips run beside the next block's pivot chain.  All
+// products are 64 x 64 x 64 from LDS, the next tile loaded into registers meanwhile.
+template <typename T>
+__device__ __forceinline__ void lu_step_dev(const LuMat<T> &m, int64_t k, int t, int64_t kend, int b, StepLds<T> &s)
+{
+    constexpr int LDA = Lu<T>::LDA, LDB = Lu<T>::LDB;
+    typedef typename Lu<T>::v4 v4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t c = k + (int64_t)NPB * t, ld = m.ld, off = c + NPB + (int64_t)NPB * b;
+    const int tr = (int)min((int64_t)NPB, m.n - off);
+    T *A = m.A;
+    Tile<T, NPB> ra, rq;
+    ra.load(A + off * ld + c, ld, tr, NPB, tid);
+    rq.load(m.work + (int64_t)(2 * t + 1) * NPB * NPB, NPB, NPB, NPB, tid);
+    ra.put(s.P, LDA, tid);
+    rq.put(s.Q, LDB, tid);
+    __syncthreads();
+    int64_t j0 = c + NPB;
+    if (j0 < kend) rq.load(A + c * ld + j0, ld, NPB, (int)min((int64_t)NPB, kend - j0), tid);
+    v4 acc[4];
+    zero<T, 4>(acc);
+    mma<T, 4>(s.P + 16 * wave * LDA, LDA, s.Q, LDB, NPB, lane, acc);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
+            s.P[r * LDA + cc] = acc[q][e];
+            if (r < tr) A[(off + r) * ld + c + cc] = acc[q][e];
+        }
+    for (; j0 < kend; j0 += NPB) {
+        const int tc = (int)min((int64_t)NPB, kend - j0);
+        T cv[4][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
+                cv[q][e] = A[(off + min(r, tr - 1)) * ld + j0 + min(cc, tc - 1)];
+            }
+        rq.put(s.Q, LDB, tid);
+        __syncthreads();
+        if (j0 + NPB < kend) rq.load(A + c * ld + j0 + NPB, ld, NPB, (int)min((int64_t)NPB, kend - j0 - NPB), tid);
+        zero<T, 4>(acc);
+        mma<T, 4>(s.P + 16 * wave * LDA, LDA, s.Q, LDB, NPB, lane, acc);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
+                const bool in = r < tr && cc < tc;
+                const T v = cv[q][e] - acc[q][e];
+                if (in) A[(off + r) * ld + j0 + cc] = v;
+                if (b == 0 && j0 == c + NPB) s.D[r * LDA + cc] = in ? v : (r == cc ? T(1) : T(0));
+            }
+        __syncthreads();
+    }
+    if (b == 0 && c + NPB < kend) lu_diag_row<T>(m, c + NPB, t + 1, kend, s, tid);
+}
+
+// U rows of the outer block [k, k + NOB) in the UW columns from kend + UW b on: blocked forward
+// substitution U_t = L_tt^-1 (A_t - sum_{s<t} L_ts U_s) with the solved rows kept in LDS, one launch
+// for the four block rows (ten 64 x 64 x 32 products; four pairs of launches before).
+template <typename T> struct UrowLds {
+    T P[NPB * Lu<T>::LDA];
+    T X[NIN][NPB * Lu<T>::LDX];
+    T R[NPB * Lu<T>::LDX];
+};
+template <typename T>
+__device__ __forceinline__ void lu_urow_dev(const LuMat<T> &m, int64_t k, int64_t kend, int b, UrowLds<T> &s)
+{
+    constexpr int LDA = Lu<T>::LDA, LDX = Lu<T>::LDX, NT = UW / 16;
+    typedef typename Lu<T>::v4 v4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t ld = m.ld, j0 = kend + (int64_t)UW * b;
+    const int tc = (int)min((int64_t)UW, m.n - j0);
+    T *A = m.A;
+    // left operands in order: L_t0 .. L_t,t-1, then L_tt^-1
+    Tile<T, NPB> rp;
+    rp.load(m.work, NPB, NPB, NPB, tid);
+    for (int t = 0; t < NIN; ++t) {
+        const int64_t c = k + (int64_t)NPB * t;
+        T cv[NT][4];
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
+                cv[q][e] = A[(c + r) * ld + j0 + min(cc, tc - 1)];
+            }
+        v4 acc[NT];
+        zero<T, NT>(acc);
+        for (int q = 0; q < t; ++q) {
+            __syncthreads();
+            rp.put(s.P, LDA, tid);
+            __syncthreads();
+            if (q + 1 < t) rp.load(A + c * ld + k + NPB * (q + 1), ld, NPB, NPB, tid);
+            else rp.load(m.work + (int64_t)2 * t * NPB * NPB, NPB, NPB, NPB, tid);
+            mma<T, NT>(s.P + 16 * wave * LDA, LDA, s.X[q], LDX, NPB, lane, acc);
+        }
+        __syncthreads();
+        rp.put(s.P, LDA, tid);
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                s.R[(16 * wave + Lu<T>::row(lane, e)) * LDX + 16 * q + Lu<T>::col(lane, e)] = cv[q][e] - acc[q][e];
+        __syncthreads();
+        if (t + 1 < NIN) rp.load(A + (c + NPB) * ld + k, ld, NPB, NPB, tid);
+        zero<T, NT>(acc);
+        mma<T, NT>(s.P + 16 * wave * LDA, LDA, s.R, LDX, NPB, lane, acc);
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
+                s.X[t][r * LDX + cc] = acc[q][e];
+                if (cc < tc) A[(c + r) * ld + j0 + cc] = acc[q][e];
+            }
+    }
+}
+
+template <typename T> __global__ __launch_bounds__(256) void k_lu_first(LuMat<T> m, int64_t k, int64_t kend)
+{
+    __shared__ StepLds<T> s;
+    lu_first_dev<T>(m, k, kend, s);
+}
+
+template <typename T> __global__ __launch_bounds__(256) void k_lu_step(LuMat<T> m, int64_t k, int t, int64_t kend)
+{
+    __shared__ StepLds<T> s;
+    lu_step_dev<T>(m, k, t, kend, blockIdx.x, s);
+}
+
+template <typename T> __global__ __launch_bounds__(256) void k_lu_urow(LuMat<T> m, int64_t k, int64_t kend)
+{
+    __shared__ UrowLds<T> s;
+    lu_urow_dev<T>(m, k, kend, blockIdx.x, s);
 }
 
 __global__ void k_fill_info(int *p, int v)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
-}
-
-// One 64 x 64 tile of the block row / column of step k0, in place:
-// blocks [0, nl): L21 tile rows off = k0 + 64 (1 + b) .. off+63 := A21 U11^-1;
-// blocks [nl, nl + nu): U12 tile columns off = u_off + 64 (b - nl) .. off+63 := L11^-1 A12.
-// Both operands in LDS; wave w computes output rows 16w..16w+15 with
-// v_mfma_f32_16x16x4 (lane l supplies P(l%16, k + l/16) and Q(k + l/16, l%16);
-// accumulator element r holds C(4 (l/16) + r, l%16)).
-__device__ __forceinline__ void nopiv_panel_dev(float *__restrict__ A, int64_t ld, int64_t n, int64_t k0,
-                                                const float *__restrict__ Linv, const float *__restrict__ Uinv, int nl,
-                                                int64_t u_off, int b)
-{
-    __shared__ float P[NPB][NPB + 4];
-    __shared__ float Q[NPB][NPB + 4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const bool lpanel = b < nl;
-    const int64_t off = lpanel ? k0 + NPB + (int64_t)NPB * b : u_off + (int64_t)NPB * (b - nl);
-    float *tile = lpanel ? A + off * ld + k0 : A + k0 * ld + off;
-    const int tr = (int)min((int64_t)NPB, lpanel ? n - off : n - k0);
-    const int tc = (int)min((int64_t)NPB, lpanel ? n - k0 : n - off);
-    // the tile is the left operand of L21 (times U11^-1), the right one of U12 (L11^-1 times it)
-    const float *inv = lpanel ? Uinv : Linv;
-    const int r = tid >> 2, c0 = (tid & 3) * 16;
-    const bool full = tr == NPB && tc == NPB;
-#pragma unroll
-    for (int e = 0; e < 16; e += 4) {
-        float4 v;
-        if (full) {
-            v = *reinterpret_cast<const float4 *>(tile + r * ld + c0 + e);
-        } else {
-            v.x = (r < tr && c0 + e < tc) ? tile[r * ld + c0 + e] : 0.f;
-            v.y = (r < tr && c0 + e + 1 < tc) ? tile[r * ld + c0 + e + 1] : 0.f;
-            v.z = (r < tr && c0 + e + 2 < tc) ? tile[r * ld + c0 + e + 2] : 0.f;
-            v.w = (r < tr && c0 + e + 3 < tc) ? tile[r * ld + c0 + e + 3] : 0.f;
-        }
-        const float4 w = *reinterpret_cast<const float4 *>(inv + r * NPB + c0 + e);
-        if (lpanel) {
-            P[r][c0 + e] = v.x; P[r][c0 + e + 1] = v.y; P[r][c0 + e + 2] = v.z; P[r][c0 + e + 3] = v.w;
-            Q[r][c0 + e] = w.x; Q[r][c0 + e + 1] = w.y; Q[r][c0 + e + 2] = w.z; Q[r][c0 + e + 3] = w.w;
-        } else {
-            Q[r][c0 + e] = v.x; Q[r][c0 + e + 1] = v.y; Q[r][c0 + e + 2] = v.z; Q[r][c0 + e + 3] = v.w;
-            P[r][c0 + e] = w.x; P[r][c0 + e + 1] = w.y; P[r][c0 + e + 2] = w.z; P[r][c0 + e + 3] = w.w;
-        }
-    }
-    __syncthreads();
-    nf4 acc[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) acc[q] = nf4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < NPB; ks += 4) {
-        const float pa = P[16 * wave + (lane & 15)][ks + (lane >> 4)];
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, Q[ks + (lane >> 4)][16 * q + (lane & 15)], acc[q], 0, 0,
-                                                          0);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int col = 16 * q + (lane & 15);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = 16 * wave + 4 * (lane >> 4) + e;
-            if (row < tr && col < tc) tile[row * ld + col] = acc[q][e];
-        }
-    }
-}
-
-// C -= A B on 64 x 64 output tiles (FP32, row-major), for the small products of
-// the outer blocks (the in-block trailing updates, the U rows' substitution),
-// where the 128 x 128 tiles of fp_gemm_sub leave most of the chip idle: blockIdx.x
-// = tile (row-tile major), K in chunks of 64 through LDS, v_mfma_f32_16x16x4 as in
-// k_nopiv_panel (wave w: output rows 16w..16w+15).  Loads of partial tiles use
-// clamped addresses and a 0/1 factor (every load in bounds and unconditional).
-__device__ __forceinline__ void gemm64_dev(int64_t m, int64_t n, int64_t kk, const float *__restrict__ A, int64_t lda,
-                                           const float *__restrict__ B, int64_t ldb, float *__restrict__ C, int64_t ldc,
-                                           int64_t tile)
-{
-    __shared__ float P[NPB][NPB + 4];
-    __shared__ float Q[NPB][NPB + 4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t tn_count = (n + NPB - 1) / NPB;
-    const int64_t i0 = (tile / tn_count) * NPB, j0 = (tile % tn_count) * NPB;
-    const int tr = (int)min((int64_t)NPB, m - i0), tc = (int)min((int64_t)NPB, n - j0);
-    const int r = tid >> 2, c0 = (tid & 3) * 16;
-    nf4 acc[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) acc[q] = nf4{0.f, 0.f, 0.f, 0.f};
-    for (int64_t k0 = 0; k0 < kk; k0 += NPB) {
-        const int kc = (int)min((int64_t)NPB, kk - k0);
-        const float *ar = A + (i0 + min(r, tr - 1)) * lda + k0;
-        const float *br = B + (k0 + min(r, kc - 1)) * ldb + j0;
-        const float am = r < tr ? 1.f : 0.f, bm = r < kc ? 1.f : 0.f;
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int c = c0 + e;
-            P[r][c] = ar[min(c, kc - 1)] * (c < kc ? am : 0.f);
-            Q[r][c] = br[min(c, tc - 1)] * (c < tc ? bm : 0.f);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < NPB; ks += 4) {
-            const float pa = P[16 * wave + (lane & 15)][ks + (lane >> 4)];
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, Q[ks + (lane >> 4)][16 * q + (lane & 15)], acc[q], 0,
-                                                              0, 0);
-        }
-    }
-    // every load of C is issued before the first store (clamped addresses), then the stores
-    float cv[4][4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            cv[q][e] = C[(i0 + min(16 * wave + 4 * (lane >> 4) + e, tr - 1)) * ldc + j0 + min(16 * q + (lane & 15), tc - 1)];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int col = 16 * q + (lane & 15);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = 16 * wave + 4 * (lane >> 4) + e;
-            if (row < tr && col < tc) C[(i0 + row) * ldc + j0 + col] = cv[q][e] - acc[q][e];
-        }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_gemm64_sub(int64_t m, int64_t n, int64_t kk, const float *__restrict__ A,
-                                                   int64_t lda, const float *__restrict__ B, int64_t ldb,
-                                                   float *__restrict__ C, int64_t ldc)
-{
-    gemm64_dev(m, n, kk, A, lda, B, ldb, C, ldc, blockIdx.x);
-}
-
-static int gemm64_sub(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const float *A, int64_t lda, const float *B,
-                      int64_t ldb, float *C, int64_t ldc)
-{
-    if (m <= 0 || n <= 0 || k <= 0) return FP_OK;
-    const int64_t tiles = ((m + NPB - 1) / NPB) * ((n + NPB - 1) / NPB);
-    ProfScope ps(ctx, "gemm_f32");
-    hipLaunchKernelGGL(k_gemm64_sub, dim3((unsigned)tiles), dim3(256), 0, ctx->stream, m, n, k, A, lda, B, ldb, C, ldc);
-    FP_HIP(ctx, hipGetLastError());
-    return FP_OK;
-}
-
-__global__ __launch_bounds__(256) void k_nopiv_panel(float *__restrict__ A, int64_t ld, int64_t n, int64_t k0,
-                                                    const float *__restrict__ Linv, const float *__restrict__ Uinv,
-                                                    int nl, int64_t u_off)
-{
-    nopiv_panel_dev(A, ld, n, k0, Linv, Uinv, nl, u_off, blockIdx.x);
 }
 
 // U^T A V over the orbit blocks: thread (p, q) reads the 4 x 4 block of A at rows
@@ -591,93 +742,55 @@ int fp_rbt_vec(fp_ctx *ctx, const double *in, int64_t ldin, double *out, int64_t
     return FP_OK;
 }
 
-// Inner blocks of 64 columns per outer block of 256: the inner steps factor the
-// outer block's columns only (their trailing updates stop at its last column),
-// then the outer block's U rows right of it come from one blocked forward
-// substitution with the four inner L11^-1, and the trailing matrix takes one
-// rank-256 update: a rank-64 update per 64 columns reads and writes the whole
-// trailing matrix four times as often (at 4,800 unknowns it bound the
-// factorisation: 41 us per step against 32 us for the diagonal block).
-constexpr int NOB = 4 * NPB, NOB_MAX = 8 * NPB;
+// L11^-1 and U11^-1 of an outer block's diagonal blocks
+size_t fp_getrf_nopiv_work_bytes(int elem_bytes) { return (size_t)2 * NIN * NPB * NPB * elem_bytes; }
 
-// outer block: NOB columns, or FLOWPANEL_LU32_OUTER (a multiple of 64 up to NOB_MAX)
-static int outer_block()
-{
-    static const int v = [] {
-        const char *e = getenv("FLOWPANEL_LU32_OUTER");
-        const int o = e ? atoi(e) : NOB;
-        return (o >= NPB && o <= NOB_MAX && o % NPB == 0) ? o : NOB;
-    }();
-    return v;
-}
+static int64_t lu_tiles(int64_t x, int64_t w) { return x > 0 ? (x + w - 1) / w : (int64_t)0; }
 
-// Linv and Uinv of up to NOB_MAX / NPB inner diagonal blocks
-size_t fp_getrf_nopiv_work_bytes() { return (size_t)2 * (NOB_MAX / NPB) * NPB * NPB * sizeof(float); }
-
-// LU without pivoting of the n x n FP32 matrix A (row-major, ld a multiple of 4);
-// info_dev receives 1 + the first row of the diagonal block whose pivot was zero
-// or not finite (0 if none).
-int fp_getrf_nopiv_f32(fp_ctx *ctx, float *A, int64_t n, int64_t ld, int *info_dev, void *work, float *YL,
-                       float *YU)
+// LU without pivoting of the n x n matrix A (row-major, 16-byte aligned, ld a multiple of 4), outer
+// blocks of 256 columns: per inner block of 64 one launch (lu_step_dev), then the U rows right of the
+// outer block and one rank-256 trailing update (a rank-64 update per inner block would read and write
+// the whole trailing matrix four times as often).  info_dev receives 1 + the first row of the diagonal
+// block whose pivot was zero or not finite (0 if none).
+template <typename T>
+int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void *work, T *YL, T *YU)
 {
     if (n <= 0) return FP_OK;
     if (ld % 4) return fp_fail(ctx, FP_ERR_ARG, "internal: no-pivot LU needs a leading dimension divisible by 4");
     hipLaunchKernelGGL(k_fill_info, dim3(1), dim3(64), 0, ctx->stream, info_dev, 0);
+    const LuMat<T> m{A, ld, n, (T *)work, info_dev, YL, YU};
     int st;
-    const int nob = outer_block();
-    for (int64_t k = 0; k < n; k += nob) {
-        const int64_t ob = std::min<int64_t>(nob, n - k), kend = k + ob;
-        const int T = (int)((ob + NPB - 1) / NPB);
-        for (int t = 0; t < T; ++t) {
-            const int64_t c = k + (int64_t)NPB * t;
-            float *Linv = (float *)work + (int64_t)2 * t * NPB * NPB, *Uinv = Linv + NPB * NPB;
-            {
-                ProfScope ps(ctx, "lu_nopiv_diag");
-                hipLaunchKernelGGL(k_nopiv_diag, dim3(1), dim3(512), 0, ctx->stream, A, ld, n, c, Linv, Uinv, info_dev,
-                                   YL, YU);
-            }
-            const int64_t below = n - c - NPB, inpanel = kend - c - NPB;
-            if (below <= 0) break;
-            const int nl = (int)((below + NPB - 1) / NPB), nu = inpanel > 0 ? (int)((inpanel + NPB - 1) / NPB) : 0;
-            {
-                ProfScope ps(ctx, "lu_nopiv_panel");
-                hipLaunchKernelGGL(k_nopiv_panel, dim3((unsigned)(nl + nu)), dim3(256), 0, ctx->stream, A, ld, n, c,
-                                   (const float *)Linv, (const float *)Uinv, nl, c + NPB);
-            }
-            FP_HIP(ctx, hipGetLastError());
-            if (inpanel > 0 &&
-                (st = gemm64_sub(ctx, below, inpanel, NPB, A + (c + NPB) * ld + c, ld, A + c * ld + c + NPB, ld,
-                                 A + (c + NPB) * ld + c + NPB, ld)))
-                return st;
+    for (int64_t k = 0; k < n; k += NOB) {
+        const int64_t kend = std::min<int64_t>(k + NOB, n);
+        {
+            ProfScope ps(ctx, "lu_nopiv_diag");
+            hipLaunchKernelGGL(k_lu_first<T>, dim3(1), dim3(256), 0, ctx->stream, m, k, kend);
+        }
+        for (int t = 0; t < NIN; ++t) {
+            const int64_t strips = lu_tiles(n - k - (int64_t)NPB * (t + 1), NPB);
+            if (strips <= 0) break;
+            ProfScope ps(ctx, "lu_nopiv_step");
+            hipLaunchKernelGGL(k_lu_step<T>, dim3((unsigned)strips), dim3(256), 0, ctx->stream, m, k, t, kend);
         }
         const int64_t right = n - kend;
-        if (right <= 0) continue;
-        // U12 = L11^-1 A12 for the columns right of the outer block: U_t = L_tt^-1 (A_t - sum_{s<t} L_ts U_s)
-        const int nu = (int)((right + NPB - 1) / NPB);
-        for (int t = 0; t < T; ++t) {
-            const int64_t c = k + (int64_t)NPB * t;
-            const float *Linv = (const float *)work + (int64_t)2 * t * NPB * NPB, *Uinv = Linv + NPB * NPB;
-            if (t > 0 && (st = gemm64_sub(ctx, NPB, right, c - k, A + c * ld + k, ld, A + k * ld + kend, ld,
-                                          A + c * ld + kend, ld)))
-                return st;
-            ProfScope ps(ctx, "lu_nopiv_panel");
-            hipLaunchKernelGGL(k_nopiv_panel, dim3((unsigned)nu), dim3(256), 0, ctx->stream, A, ld, n, c, Linv, Uinv, 0,
-                               kend);
-            FP_HIP(ctx, hipGetLastError());
+        if (right > 0) {
+            ProfScope ps(ctx, "lu_nopiv_urow");
+            hipLaunchKernelGGL(k_lu_urow<T>, dim3((unsigned)lu_tiles(right, UW)), dim3(256), 0, ctx->stream, m, k, kend);
         }
-        // the rank-ob trailing update
-        if ((st = fp_gemm_sub<float>(ctx, right, right, ob, A + kend * ld + k, ld, A + k * ld + kend, ld,
-                                     A + kend * ld + kend, ld)))
+        FP_HIP(ctx, hipGetLastError());
+        if (right > 0 && (st = fp_gemm_sub<T>(ctx, right, right, NOB, A + kend * ld + k, ld, A + k * ld + kend, ld,
+                                              A + kend * ld + kend, ld)))
             return st;
     }
     return FP_OK;
 }
+template int fp_getrf_nopiv<float>(fp_ctx *, float *, int64_t, int64_t, int *, void *, float *, float *);
+template int fp_getrf_nopiv<double>(fp_ctx *, double *, int64_t, int64_t, int *, void *, double *, double *);
 
 // ---- the same factorisation for many bodies at once --------------------------
-// One launch per step covers every body (blockIdx.y or blockIdx.x = body): the bodies'
-// serial chains of 64-column diagonal blocks run side by side, and the small products
-// of different bodies fill the chip together.  Global outer blocks [kk, kk + NOB);
-// a body takes part in the steps inside its order.
+// One launch per step covers every body (blockIdx.y = body): the bodies' serial chains of
+// diagonal blocks run side by side, and the small products of different bodies fill the chip
+// together.  Global outer blocks [kk, kk + NOB); a body takes part in the steps inside its order.
 
 __global__ void k_fill_info_lub(const fp_lu_desc *__restrict__ desc, int nb)
 {
@@ -685,53 +798,34 @@ __global__ void k_fill_info_lub(const fp_lu_desc *__restrict__ desc, int nb)
     if (b < nb) *desc[b].info = 0;
 }
 
-// inner step t (column c = kk + 64 t) of body blockIdx.x
-__global__ __launch_bounds__(512) void k_nopiv_diag_lub(const fp_lu_desc *__restrict__ desc, int64_t c, int t)
+static __device__ __forceinline__ LuMat<float> lub_mat(const fp_lu_desc &d)
 {
-    const fp_lu_desc d = desc[blockIdx.x];
-    if (c >= d.n) return;   // uniform per workgroup
-    float *Linv = d.work + (int64_t)2 * t * NPB * NPB;
-    nopiv_diag_dev(d.A, d.ld, d.n, c, Linv, Linv + NPB * NPB, d.info, nullptr, nullptr);
+    return LuMat<float>{d.A, d.ld, d.n, d.work, d.info, nullptr, nullptr};
 }
 
-// mode 0: the panel tiles of inner step t (L tiles below, U tiles inside the outer block);
-// mode 1: the U-row tiles of inner block t right of the outer block
-__global__ __launch_bounds__(256) void k_nopiv_panel_lub(const fp_lu_desc *__restrict__ desc, int64_t kk, int t, int mode)
+__global__ __launch_bounds__(256) void k_lu_first_lub(const fp_lu_desc *__restrict__ desc, int64_t kk)
 {
-    const fp_lu_desc d = desc[blockIdx.y];
-    const int64_t c = kk + (int64_t)NPB * t;
-    const float *Linv = d.work + (int64_t)2 * t * NPB * NPB, *Uinv = Linv + NPB * NPB;
-    if (mode == 0) {
-        const int64_t below = d.n - c - NPB;
-        if (c >= d.n || below <= 0) return;
-        const int64_t kend = min(kk + (int64_t)NOB, d.n), inpanel = kend - c - NPB;
-        const int nl = (int)((below + NPB - 1) / NPB), nu = inpanel > 0 ? (int)((inpanel + NPB - 1) / NPB) : 0;
-        if ((int)blockIdx.x >= nl + nu) return;
-        nopiv_panel_dev(d.A, d.ld, d.n, c, Linv, Uinv, nl, c + NPB, blockIdx.x);
-    } else {
-        const int64_t kend = kk + NOB, right = d.n - kend;
-        if (right <= 0 || (int64_t)blockIdx.x >= (right + NPB - 1) / NPB) return;
-        nopiv_panel_dev(d.A, d.ld, d.n, c, Linv, Uinv, 0, kend, blockIdx.x);
-    }
+    __shared__ StepLds<float> s;
+    const LuMat<float> m = lub_mat(desc[blockIdx.y]);
+    if (kk >= m.n) return;   // uniform per workgroup
+    lu_first_dev<float>(m, kk, min(kk + (int64_t)NOB, m.n), s);
 }
 
-// mode 0: the in-block update after inner step t; mode 1: the U rows' update before inner block t
-__global__ __launch_bounds__(256) void k_gemm64_lub(const fp_lu_desc *__restrict__ desc, int64_t kk, int t, int mode)
+__global__ __launch_bounds__(256) void k_lu_step_lub(const fp_lu_desc *__restrict__ desc, int64_t kk, int t)
 {
-    const fp_lu_desc d = desc[blockIdx.y];
-    const int64_t c = kk + (int64_t)NPB * t, ld = d.ld;
-    float *A = d.A;
-    if (mode == 0) {
-        const int64_t below = d.n - c - NPB, kend = min(kk + (int64_t)NOB, d.n), inpanel = kend - c - NPB;
-        if (c >= d.n || below <= 0 || inpanel <= 0) return;
-        if ((int64_t)blockIdx.x >= ((below + NPB - 1) / NPB) * ((inpanel + NPB - 1) / NPB)) return;
-        gemm64_dev(below, inpanel, NPB, A + (c + NPB) * ld + c, ld, A + c * ld + c + NPB, ld,
-                   A + (c + NPB) * ld + c + NPB, ld, blockIdx.x);
-    } else {
-        const int64_t kend = kk + NOB, right = d.n - kend;
-        if (right <= 0 || (int64_t)blockIdx.x >= (right + NPB - 1) / NPB) return;
-        gemm64_dev(NPB, right, c - kk, A + c * ld + kk, ld, A + kk * ld + kend, ld, A + c * ld + kend, ld, blockIdx.x);
-    }
+    __shared__ StepLds<float> s;
+    const LuMat<float> m = lub_mat(desc[blockIdx.y]);
+    const int64_t below = m.n - kk - (int64_t)NPB * (t + 1);
+    if ((int64_t)blockIdx.x * NPB >= below) return;
+    lu_step_dev<float>(m, kk, t, min(kk + (int64_t)NOB, m.n), blockIdx.x, s);
+}
+
+__global__ __launch_bounds__(256) void k_lu_urow_lub(const fp_lu_desc *__restrict__ desc, int64_t kk)
+{
+    __shared__ UrowLds<float> s;
+    const LuMat<float> m = lub_mat(desc[blockIdx.y]);
+    if ((int64_t)blockIdx.x * UW >= m.n - kk - NOB) return;
+    lu_urow_dev<float>(m, kk, kk + NOB, blockIdx.x, s);
 }
 
 int fp_getrf_nopiv_f32_batched(fp_ctx *ctx, const fp_lu_desc *d_desc, const int64_t *n_host, int nb)
@@ -741,51 +835,27 @@ int fp_getrf_nopiv_f32_batched(fp_ctx *ctx, const fp_lu_desc *d_desc, const int6
     int64_t nmax = 0;
     for (int b = 0; b < nb; ++b) nmax = std::max(nmax, n_host[b]);
     hipLaunchKernelGGL(k_fill_info_lub, dim3((unsigned)((nb + 63) / 64)), dim3(64), 0, ctx->stream, d_desc, nb);
-    auto tiles = [](int64_t x) { return x > 0 ? (x + NPB - 1) / NPB : (int64_t)0; };
     int st;
     for (int64_t kk = 0; kk < nmax; kk += NOB) {
-        for (int t = 0; t < NOB / NPB; ++t) {
-            const int64_t c = kk + (int64_t)NPB * t;
-            if (c >= nmax) break;
-            int64_t gp = 0, gg = 0;   // the largest grids over the bodies
-            for (int b = 0; b < nb; ++b) {
-                const int64_t n = n_host[b];
-                if (c >= n) continue;
-                const int64_t below = n - c - NPB, inpanel = std::min(kk + (int64_t)NOB, n) - c - NPB;
-                gp = std::max(gp, tiles(below) + (below > 0 ? tiles(inpanel) : 0));
-                if (below > 0 && inpanel > 0) gg = std::max(gg, tiles(below) * tiles(inpanel));
-            }
-            {
-                ProfScope ps(ctx, "lu_nopiv_diag");
-                hipLaunchKernelGGL(k_nopiv_diag_lub, dim3((unsigned)nb), dim3(512), 0, ctx->stream, d_desc, c, t);
-            }
-            if (gp > 0) {
-                ProfScope ps(ctx, "lu_nopiv_panel");
-                hipLaunchKernelGGL(k_nopiv_panel_lub, dim3((unsigned)gp, (unsigned)nb), dim3(256), 0, ctx->stream,
-                                   d_desc, kk, t, 0);
-            }
-            if (gg > 0) {
-                ProfScope ps(ctx, "gemm_f32");
-                hipLaunchKernelGGL(k_gemm64_lub, dim3((unsigned)gg, (unsigned)nb), dim3(256), 0, ctx->stream, d_desc, kk,
-                                   t, 0);
-            }
-            FP_HIP(ctx, hipGetLastError());
+        {
+            ProfScope ps(ctx, "lu_nopiv_diag");
+            hipLaunchKernelGGL(k_lu_first_lub, dim3(1, (unsigned)nb), dim3(256), 0, ctx->stream, d_desc, kk);
         }
-        int64_t right = 0;
-        for (int b = 0; b < nb; ++b) right = std::max(right, n_host[b] - kk - NOB);
-        if (right <= 0) continue;
-        for (int t = 0; t < NOB / NPB; ++t) {
-            if (t > 0) {
-                ProfScope ps(ctx, "gemm_f32");
-                hipLaunchKernelGGL(k_gemm64_lub, dim3((unsigned)tiles(right), (unsigned)nb), dim3(256), 0, ctx->stream,
-                                   d_desc, kk, t, 1);
-            }
-            ProfScope ps(ctx, "lu_nopiv_panel");
-            hipLaunchKernelGGL(k_nopiv_panel_lub, dim3((unsigned)tiles(right), (unsigned)nb), dim3(256), 0, ctx->stream,
-                               d_desc, kk, t, 1);
-            FP_HIP(ctx, hipGetLastError());
+        for (int t = 0; t < NIN; ++t) {
+            const int64_t strips = lu_tiles(nmax - kk - (int64_t)NPB * (t + 1), NPB);
+            if (strips <= 0) break;
+            ProfScope ps(ctx, "lu_nopiv_step");
+            hipLaunchKernelGGL(k_lu_step_lub, dim3((unsigned)strips, (unsigned)nb), dim3(256), 0, ctx->stream, d_desc,
+                               kk, t);
         }
-        if ((st = fp_gemm_sub_lub(ctx, d_desc, nb, kk, NOB, right))) return st;
+        const int64_t right = nmax - kk - NOB;
+        if (right > 0) {
+            ProfScope ps(ctx, "lu_nopiv_urow");
+            hipLaunchKernelGGL(k_lu_urow_lub, dim3((unsigned)lu_tiles(right, UW), (unsigned)nb), dim3(256), 0,
+                               ctx->stream, d_desc, kk);
+        }
+        FP_HIP(ctx, hipGetLastError());
+        if (right > 0 && (st = fp_gemm_sub_lub(ctx, d_desc, nb, kk, NOB, right))) return st;
     }
     return FP_OK;
 }
@@ -793,7 +863,7 @@ int fp_getrf_nopiv_f32_batched(fp_ctx *ctx, const fp_lu_desc *d_desc, const int6
 // Explicit inverses of the no-pivot factors, for refinement sweeps that then cost
 // two GEMVs instead of two blocked triangular solves.  YL = -L^-1 and YU = -U^-1
 // (row-major, ld as A; zero outside their triangles on entry, the diagonal 64 x 64
-// blocks written by fp_getrf_nopiv_f32).  With Y = -X the block recurrences
+// blocks written by fp_getrf_nopiv).  With Y = -X the block recurrences
 //   lower:  Y_JI = Y_JJ L_JI Y_II,   upper:  Y_IJ = Y_II U_IJ Y_JJ   (I before J)
 // are two "C -= A B" products each through T = -L_JI Y_II (resp. -U_IJ Y_JJ);
 // blocks merge pairwise, 64 -> 128 -> ..., one batched launch per product and
@@ -849,14 +919,14 @@ static int64_t inv_ld(int64_t n4) { return std::max<int64_t>(64, (n4 + 63) / 64 
 size_t fp_inverse_rbt_work_bytes(int64_t n)
 {
     const int64_t n4 = fp_rbt_size(n), ld4 = inv_ld(n4);
-    return (size_t)4 * n4 * ld4 * sizeof(float) + fp_rbt_weights_bytes(n) + fp_getrf_nopiv_work_bytes() + 1024;
+    return (size_t)4 * n4 * ld4 * sizeof(float) + fp_rbt_weights_bytes(n) + fp_getrf_nopiv_work_bytes(sizeof(float)) + 1024;
 }
 
 // E^-1 in place (n x n, FP64, lde) by the LU without pivoting of the randomized
 // FP32 matrix U^T E V, the explicit inverses of its factors and one product:
 // E^-1 = V (U_r^-1 L_r^-1) U^T.  No chain of n / 64 Gauss-Jordan passes with
 // their products: the factorisation's own chain is a few launches per 64
-// columns and the rest are large MFMA products.  info_dev as fp_getrf_nopiv_f32.
+// columns and the rest are large MFMA products.  info_dev as fp_getrf_nopiv.
 // Nothing is allocated and the host is not synchronised (a side stream may run it).
 int fp_inverse_rbt_f32(fp_ctx *ctx, double *E, int64_t n, int64_t lde, void *work, size_t work_bytes, int *info_dev,
                        uint64_t seed)
@@ -872,7 +942,7 @@ int fp_inverse_rbt_f32(fp_ctx *ctx, double *E, int64_t n, int64_t lde, void *wor
     int st;
     if ((st = fp_rbt_matrix<double>(ctx, E, n, lde, Ar, ld4, W))) return st;
     if ((st = fp_fill_f32(ctx, YL, sz, 0.f)) || (st = fp_fill_f32(ctx, YU, sz, 0.f))) return st;
-    if ((st = fp_getrf_nopiv_f32(ctx, Ar, n4, ld4, info_dev, nwork, YL, YU))) return st;
+    if ((st = fp_getrf_nopiv<float>(ctx, Ar, n4, ld4, info_dev, nwork, YL, YU))) return st;
     if ((st = fp_trtri_nopiv_f32(ctx, Ar, n4, ld4, YL, YU, T))) return st;
     // Ar <- -(YU YL) = -U^-1 L^-1 (the factors are no longer needed)
     if ((st = fp_fill_f32(ctx, Ar, sz, 0.f))) return st;
