@@ -753,6 +753,9 @@ struct Solver {
     // FP32 LU of the randomized matrix U^T A V without pivoting (FP_SOLVER_LU32_IR):
     // Ar (n4 x ld4), the butterflies, identity row order for getrs, an n4 x k work vector
     bool rbt = false;
+    // the same in FP64 for FP_SOLVER_LU (rbt64_setup); |A|_F
+    bool rbt64 = false;
+    double anorm = 0;
     int64_t n4 = 0, ld4 = 0;
     DBuf Ar, Wrbt, perm4, work4, t4;
     // explicit inverses of the no-pivot factors (-L^-1, -U^-1): a correction is two GEMVs
@@ -779,8 +782,8 @@ struct Solver {
             (st = dalloc(ctx, nw, fp_getrf_nopiv_work_bytes(sizeof(float)))) || (st = dalloc(ctx, info, sizeof(int))))
             return st;
         if ((st = fp_rbt_weights(ctx, n, RBT_SEED, Wrbt.as<double>()))) return st;
-        st = a.R64 ? fp_rbt_matrix<double>(ctx, a.R64, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>())
-                   : fp_rbt_matrix<float>(ctx, a.A32, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>());
+        st = a.R64 ? fp_rbt_matrix<double, float>(ctx, a.R64, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>())
+                   : fp_rbt_matrix<float, float>(ctx, a.A32, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>());
         if (st) return st;
         // the inverses cost about twice the factorisation ((4/3) n^3 against (2/3) n^3 on MFMA) and
         // pay off when many right-hand sides are corrected together; FLOWPANEL_LU32_INVERSE=1/0 forces them
@@ -796,10 +799,8 @@ struct Solver {
         if ((st = fp_getrf_nopiv<float>(ctx, Ar.as<float>(), n4, ld4, info.as<int>(), nw.p,
                                      inv ? YL.as<float>() : nullptr, inv ? YU.as<float>() : nullptr)))
             return st;
-        std::vector<int> id(n4);
-        for (int64_t i = 0; i < n4; ++i) id[i] = (int)i;
+        if ((st = fp_iota(ctx, perm4.as<int>(), n4))) return st;
         int hinfo = 0;
-        FP_HIP(ctx, hipMemcpyAsync(perm4.p, id.data(), n4 * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
         FP_HIP(ctx, hipMemcpyAsync(&hinfo, info.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (hinfo) {
@@ -820,6 +821,130 @@ struct Solver {
         *ok = true;
         rbt = true;
         return FP_OK;
+    }
+
+    // FP64 LU of the randomized matrix without pivoting (FP_SOLVER_LU), with refinement by FP64
+    // residuals; the matrix itself stays as it is.  *ok = false, and nothing kept, where it does not
+    // serve: no room for the copy, a zero or non-finite pivot, or a pivot below 1e-11 |A|_F (a matrix
+    // singular to rounding, or near it): those take the pivoted LU in place, with its results and errors.
+    int rbt64_setup(bool *ok)
+    {
+        const int64_t n = a.n;
+        int st;
+        *ok = false;
+        diag_ready = nullptr;
+        n4 = fp_rbt_size(n);
+        ld4 = round_ld(n4);
+        DBuf nw, np, chk;
+        if ((st = dalloc(ctx, Ar, (size_t)n4 * ld4 * sizeof(double)))) {
+            if (st != FP_ERR_NOMEM) return st;
+            (void)hipGetLastError();
+            ctx->err.clear();
+            return FP_OK;
+        }
+        const int64_t parts = fp_rbt_norm_parts(n);
+        if ((st = dalloc(ctx, Wrbt, fp_rbt_weights_bytes(n))) || (st = dalloc(ctx, perm4, n4 * sizeof(int))) ||
+            (st = dalloc(ctx, work4, fp_getrs_work_bytes(n4, 1))) || (st = dalloc(ctx, t4, n4 * sizeof(double))) ||
+            (st = dalloc(ctx, nw, fp_getrf_nopiv_work_bytes(sizeof(double)))) || (st = dalloc(ctx, info, sizeof(int))) ||
+            (st = dalloc(ctx, np, parts * sizeof(double))) || (st = dalloc(ctx, chk, 2 * sizeof(double))) ||
+            (st = dalloc(ctx, r, n * sizeof(double))) || (st = dalloc(ctx, d, n * sizeof(double))))
+            return st;
+        if ((st = fp_rbt_weights(ctx, n, RBT_SEED, Wrbt.as<double>())) ||
+            (st = fp_rbt_matrix<double, double>(ctx, a.A64, n, a.ld, Ar.as<double>(), ld4, Wrbt.as<double>(),
+                                                np.as<double>())) ||
+            (st = fp_getrf_nopiv<double>(ctx, Ar.as<double>(), n4, ld4, info.as<int>(), nw.p)) ||
+            (st = fp_lu_check(ctx, np.as<double>(), n, Ar.as<double>(), ld4, chk.as<double>())) ||
+            (st = fp_iota(ctx, perm4.as<int>(), n4)))
+            return st;
+        int hinfo = 0;
+        double hc[2] = {0, 0};
+        FP_HIP(ctx, hipMemcpyAsync(&hinfo, info.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+        FP_HIP(ctx, hipMemcpyAsync(hc, chk.p, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        anorm = std::sqrt(hc[0]);
+        if (hinfo || !std::isfinite(anorm) || !(hc[1] > 1e-11 * anorm)) {
+            Ar.reset();
+            return FP_OK;
+        }
+        *ok = rbt64 = true;
+        return FP_OK;
+    }
+
+    // D (n x k, ld n) ~ A^-1 R by the FP64 factors of the randomized matrix
+    int lu64_correct(const double *R, double *D, int64_t k, double *t, void *wk, size_t wbytes)
+    {
+        int st;
+        if ((st = fp_rbt_vec(ctx, R, a.n, t, n4, a.n, k, Wrbt.as<double>(), 1))) return st;
+        const bool reuse = wk == diag_ready;
+        diag_ready = wk;
+        if ((st = fp_getrs<double>(ctx, Ar.as<double>(), n4, ld4, perm4.as<int>(), t, k, n4, wk, wbytes, reuse)))
+            return st;
+        return fp_rbt_vec(ctx, t, n4, D, a.n, a.n, k, Wrbt.as<double>(), 0);
+    }
+
+    // X = A^-1 B (n x k): the randomized factors' solution, then corrections by FP64 residuals until the
+    // worst column's |r| / (|A|_F |x| + |b|) no longer halves (or is below 4e-17, under the rounding of the
+    // residual itself: 5e-16 left 20 times the pivoted LU's residual on a system of condition 5e6).  *ok = false when
+    // that stops above 1e-14: the factors are not those of a backward stable solve.  *rel (may be
+    // null): the worst |r| / |b|.
+    int rbt64_solve(const double *B, double *X, int64_t k, bool *ok, double *rel)
+    {
+        const int64_t n = a.n;
+        int st;
+        DBuf Rk, Dk, tk, wk, nr;
+        double *R = r.as<double>(), *Dp = d.as<double>(), *t = t4.as<double>();
+        void *w = work4.p;
+        const size_t wbytes = fp_getrs_work_bytes(n4, k);
+        if ((st = dalloc(ctx, nr, 3 * k * sizeof(double)))) return st;
+        if (k > 1) {
+            if ((st = dalloc(ctx, Rk, (size_t)n * k * sizeof(double))) || (st = dalloc(ctx, Dk, (size_t)n * k * sizeof(double))) ||
+                (st = dalloc(ctx, tk, (size_t)n4 * k * sizeof(double))) || (st = dalloc(ctx, wk, wbytes)))
+                return st;
+            R = Rk.as<double>(); Dp = Dk.as<double>(); t = tk.as<double>(); w = wk.p;
+        }
+        diag_ready = k > 1 ? nullptr : diag_ready;
+        if ((st = lu64_correct(B, X, k, t, w, wbytes))) return st;
+        std::vector<double> h(3 * k);
+        double before = INFINITY;
+        for (int it = 0;; ++it) {
+            st = k > 1 ? fp_gemv_multi<double>(ctx, a.A64, n, a.ld, X, n, k, R, n)
+                       : fp_gemv<double>(ctx, a.A64, n, a.ld, X, R, 1.0, 0.0);
+            if (st || (st = fp_residual_update(ctx, B, R, n * k)) ||
+                (st = fp_colnorm2(ctx, R, n, n, k, nr.as<double>())) ||
+                (st = fp_colnorm2(ctx, X, n, n, k, nr.as<double>() + k)) ||
+                (st = fp_colnorm2(ctx, B, n, n, k, nr.as<double>() + 2 * k)))
+                return st;
+            FP_HIP(ctx, hipMemcpyAsync(h.data(), nr.p, 3 * k * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+            FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            double eta = 0, worst = 0;
+            for (int64_t c = 0; c < k; ++c) {
+                const double rn = std::sqrt(h[c]), xn = std::sqrt(h[k + c]), bn = std::sqrt(h[2 * k + c]);
+                const double den = anorm * xn + bn;
+                if (den > 0 || !(rn == 0)) eta = worst_residual(eta, rn / den);
+                worst = worst_residual(worst, bn > 0 ? rn / bn : (rn == 0 && bn == 0 ? 0.0 : NAN));
+            }
+            if (rel) *rel = worst;
+            // a right-hand side that is not finite shows in the result, whatever the factors
+            const bool last = !(eta > 4e-17) || !(eta < 0.5 * before) || it >= 6;
+            if (last) {
+                *ok = !(eta > 1e-14);
+                return FP_OK;
+            }
+            before = eta;
+            if ((st = lu64_correct(R, Dp, k, t, w, wbytes))) return st;
+            if ((st = fp_axpby(ctx, 1.0, Dp, 1.0, X, n * k))) return st;
+        }
+    }
+
+    // the pivoted FP64 LU in place of the matrix
+    int lu64_pivoted(fp_solve_stats &stats)
+    {
+        int st;
+        rbt64 = false;
+        Ar.reset();
+        if ((st = dalloc(ctx, perm, a.n * sizeof(int)))) return st;
+        if ((st = factor<double>(ctx, a.A64, a.n, a.ld, perm.as<int>(), &stats.info))) return st;
+        return dalloc(ctx, work, fp_getrs_work_bytes(a.n, 1));
     }
 
     // the pivoted FP32 LU of the refinement path
@@ -948,9 +1073,10 @@ struct Solver {
         Timer tm(ctx->stream);
         if (a.solver == FP_SOLVER_LU) {
             if (!a.A64) return fp_fail(ctx, FP_ERR_ARG, "internal: no FP64 matrix");
-            if ((st = dalloc(ctx, perm, n * sizeof(int)))) return st;
-            if ((st = factor<double>(ctx, a.A64, n, a.ld, perm.as<int>(), &stats.info))) return st;
-            if ((st = dalloc(ctx, work, fp_getrs_work_bytes(n, 1)))) return st;
+            bool ok = false;
+            const char *pv = getenv("FLOWPANEL_LU64_PIVOTED");
+            if (!(pv && pv[0] == '1') && (st = rbt64_setup(&ok))) return st;
+            if (!ok && (st = lu64_pivoted(stats))) return st;
         } else if (a.solver == FP_SOLVER_GMRES) {
             // FP64 GMRES on the FP64 operator (solve_gmres!), optional block-Jacobi
             g.reset(new Gmres());
@@ -991,6 +1117,18 @@ struct Solver {
         int st;
         Timer tm(ctx->stream);
         if (a.solver == FP_SOLVER_LU) {
+            if (rbt64) {
+                bool ok = false;
+                double rel = 0;
+                if ((st = rbt64_solve(b, x, 1, &ok, &rel))) return st;
+                if (ok) {
+                    stats.ms_solve += tm.stop();
+                    stats.residual = worst_residual(stats.residual, rel);
+                    if (!std::isfinite(rel)) return not_converged(ctx, rel, "LU solve");
+                    return FP_OK;
+                }
+                if ((st = lu64_pivoted(stats))) return st;
+            }
             FP_HIP(ctx, hipMemcpyAsync(x, b, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
             if ((st = fp_getrs<double>(ctx, a.A64, n, a.ld, perm.as<int>(), x, 1, n, work.p,
                                        fp_getrs_work_bytes(n, 1))))
@@ -1095,6 +1233,15 @@ struct Solver {
             return FP_OK;
         }
         Timer tm(ctx->stream);
+        if (a.solver == FP_SOLVER_LU && rbt64) {
+            bool ok = false;
+            if ((st = rbt64_solve(B, X, k, &ok, nullptr))) return st;
+            if (ok) {
+                stats.ms_solve += tm.stop();
+                return FP_OK;
+            }
+            if ((st = lu64_pivoted(stats))) return st;
+        }
         DBuf wk;
         const size_t wbytes = fp_getrs_work_bytes(n, k);
         if ((st = dalloc(ctx, wk, wbytes))) return st;
@@ -1369,9 +1516,7 @@ struct BatchImpl {
                     (st = dalloc(ctx, bb->t4, bb->n4 * sizeof(double))))
                     return st;
                 if ((st = fp_rbt_weights(ctx, n, RBT_SEED, bb->W.as<double>()))) return st;
-                std::vector<int> id(bb->n4);
-                for (int64_t i = 0; i < bb->n4; ++i) id[i] = (int)i;
-                FP_HIP(ctx, hipMemcpy(bb->perm4.p, id.data(), bb->n4 * sizeof(int), hipMemcpyHostToDevice));
+                if ((st = fp_iota(ctx, bb->perm4.as<int>(), bb->n4))) return st;
             }
             if ((st = dalloc(ctx, bb->rhs, n * sizeof(double))) || (st = dalloc(ctx, bb->x, n * sizeof(double))) ||
                 (st = dalloc(ctx, bb->r, n * sizeof(double))) || (st = dalloc(ctx, bb->d, n * sizeof(double))) ||
@@ -1518,9 +1663,9 @@ struct BatchImpl {
     int rbt_matrix(BatchBody &bb)
     {
         bb.diag_ready = false;
-        return stored() ? fp_rbt_matrix<double>(ctx, bb.A64.as<double>(), bb.n, bb.ld, bb.Ar.as<float>(), bb.ld4,
+        return stored() ? fp_rbt_matrix<double, float>(ctx, bb.A64.as<double>(), bb.n, bb.ld, bb.Ar.as<float>(), bb.ld4,
                                                 bb.W.as<double>())
-                        : fp_rbt_matrix<float>(ctx, bb.A32.as<float>(), bb.n, bb.ld, bb.Ar.as<float>(), bb.ld4,
+                        : fp_rbt_matrix<float, float>(ctx, bb.A32.as<float>(), bb.n, bb.ld, bb.Ar.as<float>(), bb.ld4,
                                                bb.W.as<double>());
     }
 

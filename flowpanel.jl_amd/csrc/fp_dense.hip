@@ -1635,6 +1635,14 @@ __global__ void k_fill_f32(float *__restrict__ x, int64_t n, float v)
         x[i] = v;
 }
 
+int fp_iota(fp_ctx *ctx, int *p, int64_t n)
+{
+    if (n <= 0) return FP_OK;
+    hipLaunchKernelGGL(k_iota, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, p, n);
+    FP_HIP(ctx, hipGetLastError());
+    return FP_OK;
+}
+
 int fp_fill_f32(fp_ctx *ctx, float *x, int64_t n, float v)
 {
     if (n <= 0) return FP_OK;

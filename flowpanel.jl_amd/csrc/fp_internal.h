@@ -256,12 +256,15 @@ int fp_launch_loads(fp_ctx *ctx, const fp_body *b, const double *cp, double q, c
 size_t fp_loads_partial_bytes(int64_t N);
 int fp_launch_sectional(fp_ctx *ctx, const double *F, const double *X, int64_t N, int64_t nchord, int64_t nspan,
                         const double *spandir, double *outF, double *pos);
-// FP32 LU of a randomized matrix without pivoting (fp_lu_nopiv.hip)
+// LU of a randomized matrix without pivoting, FP32 and FP64 (fp_lu_nopiv.hip)
 int64_t fp_rbt_size(int64_t n);
 size_t fp_rbt_weights_bytes(int64_t n);
 int fp_rbt_weights(fp_ctx *ctx, int64_t n, uint64_t seed, double *d_W);
-template <typename Tin>
-int fp_rbt_matrix(fp_ctx *ctx, const Tin *A, int64_t n, int64_t lda, float *Ar, int64_t ldr, const double *d_W);
+int64_t fp_rbt_norm_parts(int64_t n);   // partial sums of squares fp_rbt_matrix writes to `part` (may be null)
+template <typename Tin, typename T>
+int fp_rbt_matrix(fp_ctx *ctx, const Tin *A, int64_t n, int64_t lda, T *Ar, int64_t ldr, const double *d_W,
+                  double *part = nullptr);
+int fp_lu_check(fp_ctx *ctx, const double *part, int64_t n, const double *LU, int64_t ld, double *out);
 int fp_rbt_vec(fp_ctx *ctx, const double *in, int64_t ldin, double *out, int64_t ldout, int64_t n, int64_t k,
                const double *d_W, int transpose_u);
 size_t fp_getrf_nopiv_work_bytes(int elem_bytes);
@@ -354,6 +357,7 @@ int fp_dot(fp_ctx *ctx, const double *x, const double *y, int64_t n, double *d_o
 int fp_axpy(fp_ctx *ctx, double a, const double *x, double *y, int64_t n);
 int fp_fill(fp_ctx *ctx, double *x, int64_t n, double v);   // x[:] = v (a kernel: safe inside graphs)
 int fp_fill_f32(fp_ctx *ctx, float *x, int64_t n, float v);
+int fp_iota(fp_ctx *ctx, int *p, int64_t n);   // p[i] = i
 
 // multi-dot out[c] = sum_i V[c*ldv + i] w[i] (part: 256*nv doubles)
 int fp_mdot(fp_ctx *ctx, const double *V, int64_t ldv, int nv, const double *w, int64_t n, double *part,

@@ -527,38 +527,76 @@ __global__ void k_fill_info(int *p, int v)
 
 // U^T A V over the orbit blocks: thread (p, q) reads the 4 x 4 block of A at rows
 // p + i m, columns q + j m (the identity beyond n), forms U_p^T B V_q in FP64 and
-// stores it rounded to FP32.  W holds the 4 x 4 butterfly of every orbit,
-// row-major: U's at W[16 p], V's at W[16 (m + q)].
-template <typename Tin>
+// stores it rounded to T.  W holds the 4 x 4 butterfly of every orbit,
+// row-major: U's at W[16 p], V's at W[16 (m + q)].  With part set, part[workgroup]
+// receives the sum of squares of the entries of A it read.
+template <typename Tin, typename T>
 __global__ __launch_bounds__(256) void k_rbt_matrix(const Tin *__restrict__ A, int64_t n, int64_t lda,
-                                                   float *__restrict__ Ar, int64_t m, int64_t ldr,
-                                                   const double *__restrict__ W)
+                                                   T *__restrict__ Ar, int64_t m, int64_t ldr,
+                                                   const double *__restrict__ W, double *__restrict__ part)
 {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t p = blockIdx.y;
-    if (q >= m) return;
-    double B[4][4];
+    double sq = 0.0;
+    if (q < m) {
+        double B[4][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t gr = p + i * m;
+        for (int i = 0; i < 4; ++i) {
+            const int64_t gr = p + i * m;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t gc = q + j * m;
-            B[i][j] = (gr < n && gc < n) ? (double)A[gr * lda + gc] : (gr == gc ? 1.0 : 0.0);
+            for (int j = 0; j < 4; ++j) {
+                const int64_t gc = q + j * m;
+                B[i][j] = (gr < n && gc < n) ? (double)A[gr * lda + gc] : (gr == gc ? 1.0 : 0.0);
+                sq = fma(B[i][j], B[i][j], sq);
+            }
+        }
+        const double *U = W + 16 * p, *V = W + 16 * (m + q);
+        double X[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                X[i][j] = B[i][0] * V[j] + B[i][1] * V[4 + j] + B[i][2] * V[8 + j] + B[i][3] * V[12 + j];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            T *dst = Ar + (p + i * m) * ldr + q;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                dst[j * m] = (T)(U[i] * X[0][j] + U[4 + i] * X[1][j] + U[8 + i] * X[2][j] + U[12 + i] * X[3][j]);
         }
     }
-    const double *U = W + 16 * p, *V = W + 16 * (m + q);
-    double T[4][4];
+    if (!part) return;   // uniform
+    __shared__ double sw[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
+    if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = sq;
+    __syncthreads();
+    if (threadIdx.x == 0) part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = sw[0] + sw[1] + sw[2] + sw[3];
+}
+
+// out[0] = sum of part[0 .. np), out[1] = smallest |A(i, i)| (NaN when one is NaN); one workgroup
+__global__ __launch_bounds__(1024) void k_lu_check(const double *__restrict__ part, int64_t np,
+                                                   const double *__restrict__ A, int64_t n, int64_t ld,
+                                                   double *__restrict__ out)
+{
+    __shared__ double ss[16], sm[16];
+    double s = 0.0, v = INFINITY;
+    for (int64_t i = threadIdx.x; i < np; i += 1024) s += part[i];
+    for (int64_t i = threadIdx.x; i < n; i += 1024) {
+        const double d = fabs(A[i * ld + i]);
+        v = d < v ? d : (d == d ? v : 0.0);
+    }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) T[i][j] = B[i][0] * V[j] + B[i][1] * V[4 + j] + B[i][2] * V[8 + j] + B[i][3] * V[12 + j];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        float *dst = Ar + (p + i * m) * ldr + q;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            dst[j * m] = (float)(U[i] * T[0][j] + U[4 + i] * T[1][j] + U[8 + i] * T[2][j] + U[12 + i] * T[3][j]);
+    for (int o = 32; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o);
+        v = fmin(v, __shfl_xor(v, o));
+    }
+    if ((threadIdx.x & 63) == 0) { ss[threadIdx.x >> 6] = s; sm[threadIdx.x >> 6] = v; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; ++w) { s += ss[w]; v = fmin(v, sm[w]); }
+        out[0] = s;
+        out[1] = v;
     }
 }
 
@@ -589,49 +627,12 @@ __global__ void k_rbt_vec(const double *__restrict__ in, int64_t ldin, double *_
     }
 }
 
-// splitmix64: deterministic random weights
-uint64_t mix64(uint64_t &s)
-{
-    uint64_t z = (s += 0x9E3779B97F4A7C15ull);
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    return z ^ (z >> 31);
-}
-
-// One depth-2 recursive butterfly of size 4m as its m orbit blocks (row-major
+// Two depth-2 recursive butterflies of size 4m as their m orbit blocks (row-major
 // 4 x 4, acting on (x_p, x_p+m, x_p+2m, x_p+3m)): the outer butterfly pairs
 // p with p + 2m, the two inner ones pair p with p + m in each half; every
 // butterfly is (1/sqrt 2) [R S; R -S] with random diagonals exp(r / 10),
-// r uniform in [-1/2, 1/2].
-void butterfly_blocks(int64_t m, uint64_t seed, double *out)
-{
-    uint64_t s = seed;
-    auto rnd = [&]() { return std::exp((((double)(mix64(s) >> 11) * 0x1.0p-53) - 0.5) / 10.0); };
-    const double h = std::sqrt(0.5);
-    for (int64_t p = 0; p < m; ++p) {
-        const double R0 = rnd(), S0 = rnd(), R1 = rnd(), S1 = rnd();   // outer: positions p, p + m
-        const double Ra = rnd(), Sa = rnd(), Rb = rnd(), Sb = rnd();   // inner: first half, second half
-        // z = outer x: z_a = h (R0 x_a + S0 x_c), z_c = h (R0 x_a - S0 x_c),
-        //              z_b = h (R1 x_b + S1 x_d), z_d = h (R1 x_b - S1 x_d)
-        const double Z[4][4] = {{h * R0, 0, h * S0, 0}, {0, h * R1, 0, h * S1},
-                                {h * R0, 0, -h * S0, 0}, {0, h * R1, 0, -h * S1}};
-        // y = inner z: y_a = h (Ra z_a + Sa z_b), y_b = h (Ra z_a - Sa z_b),
-        //              y_c = h (Rb z_c + Sb z_d), y_d = h (Rb z_c - Sb z_d)
-        const double Y[4][4] = {{h * Ra, h * Sa, 0, 0}, {h * Ra, -h * Sa, 0, 0},
-                                {0, 0, h * Rb, h * Sb}, {0, 0, h * Rb, -h * Sb}};
-        double *o = out + 16 * p;
-        for (int i = 0; i < 4; ++i)
-            for (int j = 0; j < 4; ++j) {
-                double acc = 0;
-                for (int k = 0; k < 4; ++k) acc += Y[i][k] * Z[k][j];
-                o[4 * i + j] = acc;
-            }
-    }
-}
-
-// The butterflies' orbit blocks on the device (the same construction as
-// butterfly_blocks; the i-th draw of a splitmix64 stream is mix64 of seed +
-// (i + 1) * golden, so every orbit computes its own eight draws).
+// r uniform in [-1/2, 1/2].  The i-th draw of a splitmix64 stream is the mix of
+// seed + (i + 1) * golden, so every orbit computes its own eight draws.
 __device__ __forceinline__ uint64_t mix64_at(uint64_t seed, uint64_t i)
 {
     uint64_t z = seed + (i + 1) * 0x9E3779B97F4A7C15ull;
@@ -708,27 +709,44 @@ size_t fp_rbt_weights_bytes(int64_t n) { return (size_t)32 * (fp_rbt_size(n) / 4
 int fp_rbt_weights(fp_ctx *ctx, int64_t n, uint64_t seed, double *d_W)
 {
     const int64_t m = fp_rbt_size(n) / 4;
-    std::vector<double> W((size_t)32 * m);
-    butterfly_blocks(m, seed, W.data());
-    butterfly_blocks(m, seed ^ 0x5DEECE66Dull, W.data() + 16 * m);
-    FP_HIP(ctx, hipMemcpyAsync(d_W, W.data(), W.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (m == 0) return FP_OK;
+    hipLaunchKernelGGL(k_rbt_weights, dim3((unsigned)((2 * m + 127) / 128)), dim3(128), 0, ctx->stream, m, seed, d_W);
+    FP_HIP(ctx, hipGetLastError());
     return FP_OK;
 }
 
-template <typename Tin>
-int fp_rbt_matrix(fp_ctx *ctx, const Tin *A, int64_t n, int64_t lda, float *Ar, int64_t ldr, const double *d_W)
+int64_t fp_rbt_norm_parts(int64_t n)
+{
+    const int64_t m = fp_rbt_size(n) / 4;
+    return (m + 255) / 256 * m;
+}
+
+template <typename Tin, typename T>
+int fp_rbt_matrix(fp_ctx *ctx, const Tin *A, int64_t n, int64_t lda, T *Ar, int64_t ldr, const double *d_W, double *part)
 {
     const int64_t m = fp_rbt_size(n) / 4;
     if (m == 0) return FP_OK;
     ProfScope ps(ctx, "rbt");
-    hipLaunchKernelGGL(k_rbt_matrix<Tin>, dim3((unsigned)((m + 255) / 256), (unsigned)m), dim3(256), 0, ctx->stream,
-                       A, n, lda, Ar, m, ldr, d_W);
+    hipLaunchKernelGGL((k_rbt_matrix<Tin, T>), dim3((unsigned)((m + 255) / 256), (unsigned)m), dim3(256), 0, ctx->stream,
+                       A, n, lda, Ar, m, ldr, d_W, part);
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;
 }
-template int fp_rbt_matrix<double>(fp_ctx *, const double *, int64_t, int64_t, float *, int64_t, const double *);
-template int fp_rbt_matrix<float>(fp_ctx *, const float *, int64_t, int64_t, float *, int64_t, const double *);
+template int fp_rbt_matrix<double, float>(fp_ctx *, const double *, int64_t, int64_t, float *, int64_t, const double *,
+                                          double *);
+template int fp_rbt_matrix<float, float>(fp_ctx *, const float *, int64_t, int64_t, float *, int64_t, const double *,
+                                         double *);
+template int fp_rbt_matrix<double, double>(fp_ctx *, const double *, int64_t, int64_t, double *, int64_t,
+                                           const double *, double *);
+
+// out[0] = |A|_F^2 from fp_rbt_matrix's partial sums, out[1] = the smallest |pivot| of the factors LU (n4 x n4)
+int fp_lu_check(fp_ctx *ctx, const double *part, int64_t n, const double *LU, int64_t ld, double *out)
+{
+    hipLaunchKernelGGL(k_lu_check, dim3(1), dim3(1024), 0, ctx->stream, part, fp_rbt_norm_parts(n), LU, fp_rbt_size(n),
+                       ld, out);
+    FP_HIP(ctx, hipGetLastError());
+    return FP_OK;
+}
 
 // transpose_u: out (n4 x k, ldout) = U^T in (n x k, ldin); else out (n x k) = V in (n4 x k)
 int fp_rbt_vec(fp_ctx *ctx, const double *in, int64_t ldin, double *out, int64_t ldout, int64_t n, int64_t k,
@@ -940,7 +958,7 @@ int fp_inverse_rbt_f32(fp_ctx *ctx, double *E, int64_t n, int64_t lde, void *wor
     void *nwork = (char *)W + fp_rbt_weights_bytes(n);
     hipLaunchKernelGGL(k_rbt_weights, dim3((unsigned)((2 * m + 127) / 128)), dim3(128), 0, ctx->stream, m, seed, W);
     int st;
-    if ((st = fp_rbt_matrix<double>(ctx, E, n, lde, Ar, ld4, W))) return st;
+    if ((st = fp_rbt_matrix<double, float>(ctx, E, n, lde, Ar, ld4, W))) return st;
     if ((st = fp_fill_f32(ctx, YL, sz, 0.f)) || (st = fp_fill_f32(ctx, YU, sz, 0.f))) return st;
     if ((st = fp_getrf_nopiv<float>(ctx, Ar, n4, ld4, info_dev, nwork, YL, YU))) return st;
     if ((st = fp_trtri_nopiv_f32(ctx, Ar, n4, ld4, YL, YU, T))) return st;

@@ -1,0 +1,75 @@
+"""The FP64 LU path: randomized no-pivot factors with refinement, and what falls back to pivoting.
+
+Sizes straddle the 16-column sub-panels, the 64-row blocks, the 256-column outer blocks, the 32-column
+groups of the U rows and the pad to a multiple of 4.  The reference is LAPACK on the same matrix; the
+bound 64 n eps kappa is the usual forward bound of a backward stable solve with room for the constant.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(float).eps
+
+
+def _matrix(n, seed):
+    rng = np.random.default_rng(seed)
+    return rng.standard_normal((n, n)) + 0.5 * np.sqrt(n) * np.eye(n), rng
+
+
+@pytest.mark.parametrize("n", [1, 2, 5, 15, 17, 63, 64, 65, 129, 255, 256, 257, 288, 290, 321, 513, 771])
+@pytest.mark.parametrize("k", [1, 3])
+@pytest.mark.parametrize("pivoted", ["0", "1"])
+def test_fp64_lu_matches_lapack(fp, n, k, pivoted, monkeypatch):
+    monkeypatch.setenv("FLOWPANEL_LU64_PIVOTED", pivoted)
+    A, rng = _matrix(n, 100 + n)
+    X = rng.standard_normal((n, k))
+    B = A @ X
+    got = fp.solve_ludiv(None, A, B if k > 1 else B[:, 0]).reshape(n, k)
+    ref = np.linalg.solve(A, B)
+    bound = 64 * n * EPS * np.linalg.cond(A)
+    assert np.abs(got - ref).max() <= bound * np.abs(ref).max()
+    # and backward stable: the residual is at rounding whatever the condition
+    r = np.linalg.norm(A @ got - B) / (np.linalg.norm(A) * np.linalg.norm(got))
+    assert r < 16 * EPS * np.sqrt(n) + 4 * EPS, r
+
+
+@pytest.mark.parametrize("n", [64, 300])
+def test_permutation_needs_no_pivots(fp, n):
+    # a zero diagonal: plain elimination without pivoting stops at the first column
+    rng = np.random.default_rng(n)
+    A = np.eye(n)[rng.permutation(n)] * rng.uniform(1, 2, n)
+    b = rng.standard_normal(n)
+    x = fp.solve_ludiv(None, A, b)
+    assert np.abs(A @ x - b).max() < 1e-13
+
+
+def test_singular_matrix_is_refused_as_before(fp):
+    # exactly singular (a zero column), consistent right-hand side: the pivoted LU meets a zero pivot
+    A, rng = _matrix(200, 3)
+    A[:, 77] = 0.0
+    with pytest.raises(fp.FPError) as e:
+        fp.solve_ludiv(None, A, A @ rng.standard_normal(200))
+    assert e.value.code == 6
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_not_finite_is_an_error(fp, bad):
+    A, rng = _matrix(130, 4)
+    b = rng.standard_normal(130)
+    b[5] = bad
+    with pytest.raises(fp.FPError):
+        fp.solve_ludiv(None, A, b)
+
+
+def test_nearly_singular_matrix_matches_pivoted(fp, monkeypatch):
+    # condition 1e14: both paths give a backward stable solution of their own
+    rng = np.random.default_rng(9)
+    n = 150
+    Q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    P, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    A = Q @ np.diag(np.logspace(0, -14, n)) @ P
+    b = A @ rng.standard_normal(n)
+    for pv in ("0", "1"):
+        monkeypatch.setenv("FLOWPANEL_LU64_PIVOTED", pv)
+        x = fp.solve_ludiv(None, A, b)
+        assert np.linalg.norm(A @ x - b) < 64 * n * EPS * (np.linalg.norm(x) + np.linalg.norm(b))
