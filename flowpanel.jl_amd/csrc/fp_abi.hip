@@ -751,13 +751,13 @@ struct Solver {
     // block inverses started beside the assembly (BJPrecond::setup_early)
     void adopt(std::unique_ptr<BJPrecond> pre) { M = std::move(pre); }
     // FP32 LU of the randomized matrix U^T A V without pivoting (FP_SOLVER_LU32_IR):
-    // Ar (n4 x ld4), the butterflies, identity row order for getrs, an n4 x k work vector
+    // Ar (n4 x ld4), the butterflies, the factors' block inverses, n4 x k work vectors
     bool rbt = false;
     // the same in FP64 for FP_SOLVER_LU (rbt64_setup); |A|_F
     bool rbt64 = false;
     double anorm = 0;
     int64_t n4 = 0, ld4 = 0;
-    DBuf Ar, Wrbt, perm4, work4, t4;
+    DBuf Ar, Wrbt, fwork, t4, t4b;
     // explicit inverses of the no-pivot factors (-L^-1, -U^-1): a correction is two GEMVs
     bool inv = false;
     DBuf YL, YU, w4;
@@ -775,11 +775,10 @@ struct Solver {
         diag_ready = nullptr;
         n4 = fp_rbt_size(n);
         ld4 = round_ld(n4);
-        DBuf nw;
         if ((st = dalloc(ctx, Ar, (size_t)n4 * ld4 * sizeof(float))) ||
-            (st = dalloc(ctx, Wrbt, fp_rbt_weights_bytes(n))) || (st = dalloc(ctx, perm4, n4 * sizeof(int))) ||
-            (st = dalloc(ctx, work4, fp_getrs_work_bytes(n4, 1))) || (st = dalloc(ctx, t4, n4 * sizeof(double))) ||
-            (st = dalloc(ctx, nw, fp_getrf_nopiv_work_bytes(sizeof(float)))) || (st = dalloc(ctx, info, sizeof(int))))
+            (st = dalloc(ctx, Wrbt, fp_rbt_weights_bytes(n))) ||
+            (st = dalloc(ctx, t4, n4 * sizeof(double))) || (st = dalloc(ctx, t4b, n4 * sizeof(double))) ||
+            (st = dalloc(ctx, fwork, fp_getrf_nopiv_work_bytes(n4, sizeof(float)))) || (st = dalloc(ctx, info, sizeof(int))))
             return st;
         if ((st = fp_rbt_weights(ctx, n, RBT_SEED, Wrbt.as<double>()))) return st;
         st = a.R64 ? fp_rbt_matrix<double, float>(ctx, a.R64, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>())
@@ -796,10 +795,10 @@ struct Solver {
                 (st = fp_fill_f32(ctx, YU.as<float>(), n4 * ld4, 0.f)))
                 return st;
         }
-        if ((st = fp_getrf_nopiv<float>(ctx, Ar.as<float>(), n4, ld4, info.as<int>(), nw.p,
+        if ((st = fp_getrf_nopiv<float>(ctx, Ar.as<float>(), n4, ld4, info.as<int>(), fwork.p,
                                      inv ? YL.as<float>() : nullptr, inv ? YU.as<float>() : nullptr)))
             return st;
-        if ((st = fp_iota(ctx, perm4.as<int>(), n4))) return st;
+        if (!inv && (st = fp_tri_inverse<float>(ctx, Ar.as<float>(), n4, ld4, fwork.p))) return st;
         int hinfo = 0;
         FP_HIP(ctx, hipMemcpyAsync(&hinfo, info.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -823,19 +822,17 @@ struct Solver {
         return FP_OK;
     }
 
-    // FP64 LU of the randomized matrix without pivoting (FP_SOLVER_LU), with refinement by FP64
-    // residuals; the matrix itself stays as it is.  *ok = false, and nothing kept, where it does not
-    // serve: no room for the copy, a zero or non-finite pivot, or a pivot below 1e-11 |A|_F (a matrix
+    // FP64 LU of the randomized matrix without pivoting (FP_SOLVER_LU), with refinement; the matrix
+    // itself stays as it is.  *ok = false, and nothing kept, where it does not serve: no room for the copy, a zero or non-finite pivot, or a pivot below 1e-11 |A|_F (a matrix
     // singular to rounding, or near it): those take the pivoted LU in place, with its results and errors.
     int rbt64_setup(bool *ok)
     {
         const int64_t n = a.n;
         int st;
         *ok = false;
-        diag_ready = nullptr;
         n4 = fp_rbt_size(n);
         ld4 = round_ld(n4);
-        DBuf nw, np, chk;
+        DBuf np, chk;
         if ((st = dalloc(ctx, Ar, (size_t)n4 * ld4 * sizeof(double)))) {
             if (st != FP_ERR_NOMEM) return st;
             (void)hipGetLastError();
@@ -843,18 +840,18 @@ struct Solver {
             return FP_OK;
         }
         const int64_t parts = fp_rbt_norm_parts(n);
-        if ((st = dalloc(ctx, Wrbt, fp_rbt_weights_bytes(n))) || (st = dalloc(ctx, perm4, n4 * sizeof(int))) ||
-            (st = dalloc(ctx, work4, fp_getrs_work_bytes(n4, 1))) || (st = dalloc(ctx, t4, n4 * sizeof(double))) ||
-            (st = dalloc(ctx, nw, fp_getrf_nopiv_work_bytes(sizeof(double)))) || (st = dalloc(ctx, info, sizeof(int))) ||
+        if ((st = dalloc(ctx, Wrbt, fp_rbt_weights_bytes(n))) ||
+            (st = dalloc(ctx, t4, n4 * sizeof(double))) || (st = dalloc(ctx, t4b, n4 * sizeof(double))) ||
+            (st = dalloc(ctx, fwork, fp_getrf_nopiv_work_bytes(n4, sizeof(double)))) || (st = dalloc(ctx, info, sizeof(int))) ||
             (st = dalloc(ctx, np, parts * sizeof(double))) || (st = dalloc(ctx, chk, 2 * sizeof(double))) ||
             (st = dalloc(ctx, r, n * sizeof(double))) || (st = dalloc(ctx, d, n * sizeof(double))))
             return st;
         if ((st = fp_rbt_weights(ctx, n, RBT_SEED, Wrbt.as<double>())) ||
             (st = fp_rbt_matrix<double, double>(ctx, a.A64, n, a.ld, Ar.as<double>(), ld4, Wrbt.as<double>(),
                                                 np.as<double>())) ||
-            (st = fp_getrf_nopiv<double>(ctx, Ar.as<double>(), n4, ld4, info.as<int>(), nw.p)) ||
+            (st = fp_getrf_nopiv<double>(ctx, Ar.as<double>(), n4, ld4, info.as<int>(), fwork.p)) ||
             (st = fp_lu_check(ctx, np.as<double>(), n, Ar.as<double>(), ld4, chk.as<double>())) ||
-            (st = fp_iota(ctx, perm4.as<int>(), n4)))
+            (st = fp_tri_inverse<double>(ctx, Ar.as<double>(), n4, ld4, fwork.p)))
             return st;
         int hinfo = 0;
         double hc[2] = {0, 0};
@@ -871,69 +868,69 @@ struct Solver {
     }
 
     // D (n x k, ld n) ~ A^-1 R by the FP64 factors of the randomized matrix
-    int lu64_correct(const double *R, double *D, int64_t k, double *t, void *wk, size_t wbytes)
+    int lu64_correct(const double *R, double *D, int64_t k, double *t, double *t2)
     {
         int st;
         if ((st = fp_rbt_vec(ctx, R, a.n, t, n4, a.n, k, Wrbt.as<double>(), 1))) return st;
-        const bool reuse = wk == diag_ready;
-        diag_ready = wk;
-        if ((st = fp_getrs<double>(ctx, Ar.as<double>(), n4, ld4, perm4.as<int>(), t, k, n4, wk, wbytes, reuse)))
-            return st;
+        if ((st = fp_lu_solve_nopiv<double>(ctx, Ar.as<double>(), n4, ld4, fwork.p, t, k, n4, t2))) return st;
         return fp_rbt_vec(ctx, t, n4, D, a.n, a.n, k, Wrbt.as<double>(), 0);
     }
 
-    // X = A^-1 B (n x k): the randomized factors' solution, then corrections by FP64 residuals until the
-    // worst column's |r| / (|A|_F |x| + |b|) no longer halves (or is below 4e-17, under the rounding of the
-    // residual itself: 5e-16 left 20 times the pivoted LU's residual on a system of condition 5e6).  *ok = false when
-    // that stops above 1e-14: the factors are not those of a backward stable solve.  *rel (may be
-    // null): the worst |r| / |b|.
+    // X = A^-1 B (n x k): the randomized factors' solution, then corrections by residuals of twice FP64,
+    // at least one.  A correction of relative size d_i leaves an error of about d_i (d_i / d_{i-1}), so it
+    // goes on until that is below 1e-17 (one correction on a wing) or they no longer halve.  With
+    // residuals of plain FP64 the strengths of wings were 2 to 4 times as far from the exact ones as the
+    // pivoted LU's; with these they are nearer than those.  *ok = false when the final residual is above
+    // 1e-14 (|A|_F |x| + |b|): the factors are not those of a backward stable solve.  *rel (may be null):
+    // the worst column's |r| / |b|.
     int rbt64_solve(const double *B, double *X, int64_t k, bool *ok, double *rel)
     {
         const int64_t n = a.n;
         int st;
-        DBuf Rk, Dk, tk, wk, nr;
-        double *R = r.as<double>(), *Dp = d.as<double>(), *t = t4.as<double>();
-        void *w = work4.p;
-        const size_t wbytes = fp_getrs_work_bytes(n4, k);
+        DBuf Rk, Dk, tk, tk2, nr;
+        double *R = r.as<double>(), *Dp = d.as<double>(), *t = t4.as<double>(), *t2 = t4b.as<double>();
         if ((st = dalloc(ctx, nr, 3 * k * sizeof(double)))) return st;
         if (k > 1) {
             if ((st = dalloc(ctx, Rk, (size_t)n * k * sizeof(double))) || (st = dalloc(ctx, Dk, (size_t)n * k * sizeof(double))) ||
-                (st = dalloc(ctx, tk, (size_t)n4 * k * sizeof(double))) || (st = dalloc(ctx, wk, wbytes)))
+                (st = dalloc(ctx, tk, (size_t)n4 * k * sizeof(double))) || (st = dalloc(ctx, tk2, (size_t)n4 * k * sizeof(double))))
                 return st;
-            R = Rk.as<double>(); Dp = Dk.as<double>(); t = tk.as<double>(); w = wk.p;
+            R = Rk.as<double>(); Dp = Dk.as<double>(); t = tk.as<double>(); t2 = tk2.as<double>();
         }
-        diag_ready = k > 1 ? nullptr : diag_ready;
-        if ((st = lu64_correct(B, X, k, t, w, wbytes))) return st;
+        double *nrm = nr.as<double>();
         std::vector<double> h(3 * k);
-        double before = INFINITY;
-        for (int it = 0;; ++it) {
-            st = k > 1 ? fp_gemv_multi<double>(ctx, a.A64, n, a.ld, X, n, k, R, n)
-                       : fp_gemv<double>(ctx, a.A64, n, a.ld, X, R, 1.0, 0.0);
-            if (st || (st = fp_residual_update(ctx, B, R, n * k)) ||
-                (st = fp_colnorm2(ctx, R, n, n, k, nr.as<double>())) ||
-                (st = fp_colnorm2(ctx, X, n, n, k, nr.as<double>() + k)) ||
-                (st = fp_colnorm2(ctx, B, n, n, k, nr.as<double>() + 2 * k)))
-                return st;
-            FP_HIP(ctx, hipMemcpyAsync(h.data(), nr.p, 3 * k * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        auto norms = [&](const double *u) -> int {   // |u|, |X|, |B| of every column
+            int s2;
+            if ((s2 = fp_colnorm2(ctx, u, n, n, k, nrm)) || (s2 = fp_colnorm2(ctx, X, n, n, k, nrm + k)) ||
+                (s2 = fp_colnorm2(ctx, B, n, n, k, nrm + 2 * k)))
+                return s2;
+            FP_HIP(ctx, hipMemcpyAsync(h.data(), nrm, 3 * k * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
             FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            double eta = 0, worst = 0;
-            for (int64_t c = 0; c < k; ++c) {
-                const double rn = std::sqrt(h[c]), xn = std::sqrt(h[k + c]), bn = std::sqrt(h[2 * k + c]);
-                const double den = anorm * xn + bn;
-                if (den > 0 || !(rn == 0)) eta = worst_residual(eta, rn / den);
-                worst = worst_residual(worst, bn > 0 ? rn / bn : (rn == 0 && bn == 0 ? 0.0 : NAN));
-            }
-            if (rel) *rel = worst;
-            // a right-hand side that is not finite shows in the result, whatever the factors
-            const bool last = !(eta > 4e-17) || !(eta < 0.5 * before) || it >= 6;
-            if (last) {
-                *ok = !(eta > 1e-14);
-                return FP_OK;
-            }
-            before = eta;
-            if ((st = lu64_correct(R, Dp, k, t, w, wbytes))) return st;
-            if ((st = fp_axpby(ctx, 1.0, Dp, 1.0, X, n * k))) return st;
+            for (double &v : h) v = std::sqrt(v);
+            return FP_OK;
+        };
+        if ((st = lu64_correct(B, X, k, t, t2))) return st;
+        double before = 1.0;
+        for (int it = 0; it < 6; ++it) {
+            if ((st = fp_resid_dd(ctx, a.A64, n, a.ld, X, k, B, R)) || (st = lu64_correct(R, Dp, k, t, t2)) ||
+                (st = fp_axpby(ctx, 1.0, Dp, 1.0, X, n * k)) || (st = norms(Dp)))
+                return st;
+            double size = 0;
+            for (int64_t c = 0; c < k; ++c)
+                if (h[k + c] > 0 || h[c] > 0) size = worst_residual(size, h[c] / h[k + c]);
+            if (!(size * std::min(1.0, size / before) > 1e-17) || !(size < 0.5 * before)) break;
+            before = size;
         }
+        if ((st = fp_resid_dd(ctx, a.A64, n, a.ld, X, k, B, R)) || (st = norms(R))) return st;
+        double eta = 0, worst = 0;
+        for (int64_t c = 0; c < k; ++c) {
+            const double den = anorm * h[k + c] + h[2 * k + c];
+            if (den > 0 || !(h[c] == 0)) eta = worst_residual(eta, h[c] / den);
+            worst = worst_residual(worst, h[2 * k + c] > 0 ? h[c] / h[2 * k + c]
+                                                           : (h[c] == 0 && h[2 * k + c] == 0 ? 0.0 : NAN));
+        }
+        if (rel) *rel = worst;
+        *ok = !(eta > 1e-14);   // a right-hand side that is not finite shows in the result, whatever the factors
+        return FP_OK;
     }
 
     // the pivoted FP64 LU in place of the matrix
@@ -989,9 +986,10 @@ struct Solver {
                     if ((st = fp_gemv<float>(ctx, YU.as<float>(), n4, ld4, w, t, 1.0, 0.0))) return st;
                 }
             } else {
-                const bool reuse = wk == diag_ready;
-                diag_ready = wk;
-                if ((st = fp_getrs<float>(ctx, Ar.as<float>(), n4, ld4, perm4.as<int>(), t, k, n4, wk, wbytes, reuse)))
+                DBuf tk2;
+                if (k > 1 && (st = dalloc(ctx, tk2, (size_t)n4 * k * sizeof(double)))) return st;
+                if ((st = fp_lu_solve_nopiv<float>(ctx, Ar.as<float>(), n4, ld4, fwork.p, t, k, n4,
+                                                   k > 1 ? tk2.as<double>() : t4b.as<double>())))
                     return st;
             }
             return fp_rbt_vec(ctx, t, n4, dd, n, n, k, Wrbt.as<double>(), 0);
@@ -1173,8 +1171,7 @@ struct Solver {
             const double before = rel;
             // correction d ~ A^-1 r in the low-precision solver
             if (a.solver == FP_SOLVER_LU32_IR) {
-                void *wk = rbt ? work4.p : work.p;
-                if ((st = lu32_correct(rp, dp, 1, wk, fp_getrs_work_bytes(rbt ? n4 : n, 1)))) return st;
+                if ((st = lu32_correct(rp, dp, 1, work.p, fp_getrs_work_bytes(n, 1)))) return st;
             } else {
                 int its = 0;
                 double irel = 0;
@@ -1267,14 +1264,11 @@ struct Solver {
             if (!std::isfinite(bn[c])) rel = NAN;
         int it = 0, it0 = 0;
         bool stalled = false;
-        DBuf wk4;
-        const size_t wbytes4 = rbt ? fp_getrs_work_bytes(n4, k) : 0;
-        if (rbt && (st = dalloc(ctx, wk4, wbytes4))) return st;
         const double rel0 = rel;
         for (;;) {
         while (!converged(rel, o.tol) && std::isfinite(rel) && it - it0 < o.max_refine && !stalled) {
             const double before = rel;
-            if ((st = lu32_correct(R.as<double>(), D.as<double>(), k, rbt ? wk4.p : wk.p, rbt ? wbytes4 : wbytes)))
+            if ((st = lu32_correct(R.as<double>(), D.as<double>(), k, wk.p, wbytes)))
                 return st;
             if ((st = fp_axpby(ctx, 1.0, D.as<double>(), 1.0, X, n * k))) return st;
             if ((st = fp_gemv_multi<double>(ctx, a.R64, n, a.ld, X, n, k, R.as<double>(), n))) return st;
@@ -1441,9 +1435,8 @@ struct BatchBody {
     // met a bad pivot or did not converge: the tournament-pivoted LU of A32 from then on)
     bool pivoted = false;
     int64_t n4 = 0, ld4 = 0;
-    DBuf Ar, W, perm4, work4, nwork, t4;
-    // the getrs workspace (work4, or swork once pivoted) holds the diagonal-block
-    // inverses of the current factors
+    DBuf Ar, W, nwork, t4, t4b;
+    // pivoted: swork holds the diagonal-block inverses of the current factors
     bool diag_ready = false;
 };
 
@@ -1510,13 +1503,11 @@ struct BatchImpl {
                 bb->n4 = fp_rbt_size(n);
                 bb->ld4 = round_ld(bb->n4);
                 if ((st = dalloc(ctx, bb->Ar, (size_t)bb->n4 * bb->ld4 * sizeof(float))) ||
-                    (st = dalloc(ctx, bb->W, fp_rbt_weights_bytes(n))) || (st = dalloc(ctx, bb->perm4, bb->n4 * sizeof(int))) ||
-                    (st = dalloc(ctx, bb->work4, fp_getrs_work_bytes(bb->n4, 1))) ||
-                    (st = dalloc(ctx, bb->nwork, fp_getrf_nopiv_work_bytes(sizeof(float)))) ||
-                    (st = dalloc(ctx, bb->t4, bb->n4 * sizeof(double))))
+                    (st = dalloc(ctx, bb->W, fp_rbt_weights_bytes(n))) ||
+                    (st = dalloc(ctx, bb->nwork, fp_getrf_nopiv_work_bytes(bb->n4, sizeof(float)))) ||
+                    (st = dalloc(ctx, bb->t4, bb->n4 * sizeof(double))) || (st = dalloc(ctx, bb->t4b, bb->n4 * sizeof(double))))
                     return st;
                 if ((st = fp_rbt_weights(ctx, n, RBT_SEED, bb->W.as<double>()))) return st;
-                if ((st = fp_iota(ctx, bb->perm4.as<int>(), bb->n4))) return st;
             }
             if ((st = dalloc(ctx, bb->rhs, n * sizeof(double))) || (st = dalloc(ctx, bb->x, n * sizeof(double))) ||
                 (st = dalloc(ctx, bb->r, n * sizeof(double))) || (st = dalloc(ctx, bb->d, n * sizeof(double))) ||
@@ -1650,6 +1641,7 @@ struct BatchImpl {
         const int64_t n = bb.n;
         int st;
         double *x = bb.x.as<double>(), *r = bb.r.as<double>(), *rhs = bb.rhs.as<double>();
+        if (!bb.pivoted && (st = fp_tri_inverse<float>(ctx, bb.Ar.as<float>(), bb.n4, bb.ld4, bb.nwork.p))) return st;
         if ((st = fp_fill(ctx, x, n, 0.0))) return st;
         FP_HIP(ctx, hipMemcpyAsync(r, rhs, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
         for (int s = 0; s < sweeps; ++s)
@@ -1708,8 +1700,8 @@ struct BatchImpl {
         if (!bb.pivoted) {
             double *t = bb.t4.as<double>();
             if ((st = fp_rbt_vec(ctx, r, n, t, bb.n4, n, 1, bb.W.as<double>(), 1))) return st;
-            if ((st = fp_getrs<float>(ctx, bb.Ar.as<float>(), bb.n4, bb.ld4, bb.perm4.as<int>(), t, 1, bb.n4,
-                                      bb.work4.p, fp_getrs_work_bytes(bb.n4, 1), reuse)))
+            if ((st = fp_lu_solve_nopiv<float>(ctx, bb.Ar.as<float>(), bb.n4, bb.ld4, bb.nwork.p, t, 1, bb.n4,
+                                               bb.t4b.as<double>())))
                 return st;
             if ((st = fp_rbt_vec(ctx, t, bb.n4, dd, n, n, 1, bb.W.as<double>(), 0))) return st;
         } else {

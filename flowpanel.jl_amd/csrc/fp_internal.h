@@ -267,10 +267,16 @@ int fp_rbt_matrix(fp_ctx *ctx, const Tin *A, int64_t n, int64_t lda, T *Ar, int6
 int fp_lu_check(fp_ctx *ctx, const double *part, int64_t n, const double *LU, int64_t ld, double *out);
 int fp_rbt_vec(fp_ctx *ctx, const double *in, int64_t ldin, double *out, int64_t ldout, int64_t n, int64_t k,
                const double *d_W, int transpose_u);
-size_t fp_getrf_nopiv_work_bytes(int elem_bytes);
+size_t fp_getrf_nopiv_work_bytes(int64_t n, int elem_bytes);
 template <typename T>
 int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void *work, T *YL = nullptr,
                    T *YU = nullptr);
+// the block inverses of those factors (in the same work), and x (n x k) := U^-1 L^-1 x with them (tmp: n k doubles)
+template <typename T>
+int fp_tri_inverse(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, void *work);
+template <typename T>
+int fp_lu_solve_nopiv(fp_ctx *ctx, const T *LU, int64_t n, int64_t ld, const void *work, double *x, int64_t k, int64_t ldx,
+                      double *tmp);
 int fp_trtri_nopiv_f32(fp_ctx *ctx, const float *A, int64_t n, int64_t ld, float *YL, float *YU, float *T);
 // One body of the batched FP32 no-pivot LU (a device array of these, one per body):
 // A (n x n, ld, row-major), the LU's work (fp_getrf_nopiv_work_bytes), its info word.
@@ -355,9 +361,10 @@ int fp_rhs_from(fp_ctx *ctx, const fp_body *b, const double *uinf_soa, double *r
 int fp_residual_update(fp_ctx *ctx, const double *b, double *r, int64_t n);   // r = b - r
 int fp_dot(fp_ctx *ctx, const double *x, const double *y, int64_t n, double *d_out);
 int fp_axpy(fp_ctx *ctx, double a, const double *x, double *y, int64_t n);
+// R = B - A X (n x k, column-major, ld n), accumulated in twice FP64
+int fp_resid_dd(fp_ctx *ctx, const double *A, int64_t n, int64_t ld, const double *X, int64_t k, const double *B, double *R);
 int fp_fill(fp_ctx *ctx, double *x, int64_t n, double v);   // x[:] = v (a kernel: safe inside graphs)
 int fp_fill_f32(fp_ctx *ctx, float *x, int64_t n, float v);
-int fp_iota(fp_ctx *ctx, int *p, int64_t n);   // p[i] = i
 
 // multi-dot out[c] = sum_i V[c*ldv + i] w[i] (part: 256*nv doubles)
 int fp_mdot(fp_ctx *ctx, const double *V, int64_t ldv, int nv, const double *w, int64_t n, double *part,

@@ -39,6 +39,7 @@ constexpr int NPB = 64;          // block of the no-pivot LU
 constexpr int NIN = 4;           // blocks per outer block
 constexpr int NOB = NIN * NPB;   // outer block: columns per trailing update
 constexpr int UW = 32;           // columns per workgroup of the U rows
+constexpr int TBIG = 512;        // rows of the diagonal-block inverses the triangular solves use
 
 __device__ __forceinline__ float bcast(float v, int lane)
 {
@@ -308,34 +309,40 @@ __device__ __forceinline__ bool lu_diag64(StepLds<T> &s, int tid)
     return bad;
 }
 
-// One matrix of the factorisation (a batch holds one per body).  work: L11^-1 and U11^-1 of the
-// outer block's NIN diagonal blocks, 64 x 64 each; YL, YU: -L11^-1, -U11^-1 into the diagonal blocks
-// of the full inverses (may be null).
+// One matrix of the factorisation (a batch holds one per body).  DL, DU: the inverses of the TBIG x TBIG
+// diagonal blocks of L and U, block q row-major at q TBIG^2; the factorisation writes their 64 x 64
+// diagonal blocks, which its own products read, fp_tri_inverse grows them from there.  YL, YU:
+// -L11^-1, -U11^-1 into the diagonal blocks of the full inverses (may be null).
 template <typename T> struct LuMat {
     T *A;
     int64_t ld, n;
-    T *work;
+    T *DL, *DU;
     int *info;
     T *YL, *YU;
 };
+// entry (r, c) of the block inverses, both in the same TBIG block
+template <typename T> __device__ __forceinline__ T *dent(T *D, int64_t r, int64_t c)
+{
+    return D + (r / TBIG) * ((int64_t)TBIG * TBIG) + (r % TBIG) * TBIG + c % TBIG;
+}
 
-// The diagonal block at (c, c), held in s.D (identity outside its bs rows), inner block t of the outer
-// block that ends at kend: factor, store the factors and inverses, then the U tiles of its block row
+// The diagonal block at (c, c), held in s.D (identity outside its bs rows), of the outer block that
+// ends at kend: factor, store the factors and inverses, then the U tiles of its block row
 // inside the outer block, U = L11^-1 A.
 template <typename T>
-__device__ __forceinline__ void lu_diag_row(const LuMat<T> &m, int64_t c, int t, int64_t kend, StepLds<T> &s, int tid)
+__device__ __forceinline__ void lu_diag_row(const LuMat<T> &m, int64_t c, int64_t kend, StepLds<T> &s, int tid)
 {
     constexpr int LDA = Lu<T>::LDA, LDB = Lu<T>::LDB;
     const int lane = tid & 63, wave = tid >> 6;
     const int bs = (int)min((int64_t)NPB, m.n - c);
     const bool bad = lu_diag64<T>(s, tid);
     if (bad && tid == 0) atomicCAS(m.info, 0, (int)(c + 1));
-    T *Linv = m.work + (int64_t)2 * t * NPB * NPB, *Uinv = Linv + NPB * NPB;
+    T *Linv = dent(m.DL, c, c), *Uinv = dent(m.DU, c, c);
     for (int e = tid; e < NPB * NPB; e += 256) {
         const int r = e >> 6, q = e & 63;
         const T li = s.P[r * LDA + q], ui = s.Q[r * LDB + q];
-        Linv[e] = li;
-        Uinv[e] = ui;
+        Linv[r * TBIG + q] = li;
+        Uinv[r * TBIG + q] = ui;
         if (r < bs && q < bs) {
             m.A[(c + r) * m.ld + c + q] = s.D[r * LDA + q];
             if (m.YL) m.YL[(c + r) * m.ld + c + q] = -li;
@@ -373,7 +380,7 @@ template <typename T> __device__ __forceinline__ void lu_first_dev(const LuMat<T
     __syncthreads();
     if (tid < NPB && tid >= bs) s.D[tid * (Lu<T>::LDA + 1)] = T(1);
     __syncthreads();
-    lu_diag_row<T>(m, k, 0, kend, s, tid);
+    lu_diag_row<T>(m, k, kend, s, tid);
 }
 
 // Inner step t of the outer block [k, kend), c = k + 64 t, on the 64 rows below number b: the strip's
@@ -392,7 +399,7 @@ __device__ __forceinline__ void lu_step_dev(const LuMat<T> &m, int64_t k, int t,
     T *A = m.A;
     Tile<T, NPB> ra, rq;
     ra.load(A + off * ld + c, ld, tr, NPB, tid);
-    rq.load(m.work + (int64_t)(2 * t + 1) * NPB * NPB, NPB, NPB, NPB, tid);
+    rq.load(dent(m.DU, c, c), TBIG, NPB, NPB, tid);
     ra.put(s.P, LDA, tid);
     rq.put(s.Q, LDB, tid);
     __syncthreads();
@@ -437,7 +444,7 @@ __device__ __forceinline__ void lu_step_dev(const LuMat<T> &m, int64_t k, int t,
             }
         __syncthreads();
     }
-    if (b == 0 && c + NPB < kend) lu_diag_row<T>(m, c + NPB, t + 1, kend, s, tid);
+    if (b == 0 && c + NPB < kend) lu_diag_row<T>(m, c + NPB, kend, s, tid);
 }
 
 // U rows of the outer block [k, k + NOB) in the UW columns from kend + UW b on: blocked forward
@@ -459,7 +466,7 @@ __device__ __forceinline__ void lu_urow_dev(const LuMat<T> &m, int64_t k, int64_
     T *A = m.A;
     // left operands in order: L_t0 .. L_t,t-1, then L_tt^-1
     Tile<T, NPB> rp;
-    rp.load(m.work, NPB, NPB, NPB, tid);
+    rp.load(dent(m.DL, k, k), TBIG, NPB, NPB, tid);
     for (int t = 0; t < NIN; ++t) {
         const int64_t c = k + (int64_t)NPB * t;
         T cv[NT][4];
@@ -477,7 +484,7 @@ __device__ __forceinline__ void lu_urow_dev(const LuMat<T> &m, int64_t k, int64_
             rp.put(s.P, LDA, tid);
             __syncthreads();
             if (q + 1 < t) rp.load(A + c * ld + k + NPB * (q + 1), ld, NPB, NPB, tid);
-            else rp.load(m.work + (int64_t)2 * t * NPB * NPB, NPB, NPB, NPB, tid);
+            else rp.load(dent(m.DL, c, c), TBIG, NPB, NPB, tid);
             mma<T, NT>(s.P + 16 * wave * LDA, LDA, s.X[q], LDX, NPB, lane, acc);
         }
         __syncthreads();
@@ -518,6 +525,133 @@ template <typename T> __global__ __launch_bounds__(256) void k_lu_urow(LuMat<T> 
 {
     __shared__ UrowLds<T> s;
     lu_urow_dev<T>(m, k, kend, blockIdx.x, s);
+}
+
+// ---- diagonal-block inverses for the triangular solves -------------------------
+// One level of the pairwise merge of the block inverses, s -> 2s (s = 64, 128, 256): the pair of
+// blocks at c0 = 2 s blockIdx.y and c1 = c0 + s, blockIdx.z 0 for L, 1 for U, one 64 x 64 tile of
+// the s x s block per workgroup.  Phase 0: W = L21 X11 (U: U12 X22); phase 1: X21 = -X22 W
+// (U: X12 = -X11 W).  Tiles that are zero in the triangular factor are left out.
+template <typename T>
+__global__ __launch_bounds__(256) void k_tri_merge(LuMat<T> m, T *__restrict__ W, int s, int phase)
+{
+    constexpr int LDA = Lu<T>::LDA, LDB = Lu<T>::LDB;
+    __shared__ T P[NPB * LDA], Q[NPB * LDB];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nt = s / NPB, ti = blockIdx.x / nt, tj = blockIdx.x % nt, up = blockIdx.z;
+    const int64_t c0 = (int64_t)2 * s * blockIdx.y, c1 = c0 + s, n = m.n;
+    if (c1 >= n) return;
+    const int n1 = (int)min((int64_t)nt, (n - c1 + NPB - 1) / NPB);   // tiles of the second half that exist
+    if ((up ? tj : ti) >= n1) return;
+    W += ((int64_t)up * gridDim.y + blockIdx.y) * s * s;
+    T *D = up ? m.DU : m.DL;
+    const int64_t r0 = (up ? c0 : c1) + (int64_t)NPB * ti, q0 = (up ? c1 : c0) + (int64_t)NPB * tj;
+    // K tiles: phase 0 runs over the column block's triangle, phase 1 over the row block's
+    int k0, k1;
+    if (phase == 0) { k0 = up ? 0 : tj; k1 = up ? tj + 1 : nt; }
+    else { k0 = up ? ti : 0; k1 = up ? nt : ti + 1; }
+    Tile<T, NPB> rp, rq;
+    auto load = [&](int kk) {
+        if (phase == 0) {
+            const int64_t kc = (up ? c1 : c0) + (int64_t)NPB * kk;
+            rp.load(m.A + r0 * m.ld + kc, m.ld, (int)min((int64_t)NPB, n - r0), (int)min((int64_t)NPB, n - kc), tid);
+            rq.load(dent(D, kc, q0), TBIG, NPB, NPB, tid);
+        } else {
+            const int64_t kc = (up ? c0 : c1) + (int64_t)NPB * kk;
+            rp.load(dent(D, r0, kc), TBIG, NPB, NPB, tid);
+            rq.load(W + (int64_t)NPB * kk * s + NPB * tj, s, NPB, NPB, tid);
+        }
+    };
+    typename Lu<T>::v4 acc[4];
+    zero<T, 4>(acc);
+    load(k0);
+    for (int kk = k0; kk < k1; ++kk) {
+        __syncthreads();
+        rp.put(P, LDA, tid);
+        rq.put(Q, LDB, tid);
+        __syncthreads();
+        if (kk + 1 < k1) load(kk + 1);
+        mma<T, 4>(P + 16 * wave * LDA, LDA, Q, LDB, NPB, lane, acc);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int r = 16 * wave + Lu<T>::row(lane, e), c = 16 * q + Lu<T>::col(lane, e);
+            if (phase == 0) W[(int64_t)(NPB * ti + r) * s + NPB * tj + c] = acc[q][e];
+            else *dent(D, r0 + r, q0 + c) = -acc[q][e];
+        }
+}
+
+// Rows [r0, r1) of a matrix times vectors (FP64 accumulation), 512 columns at most, one wave per R rows:
+//   SOLVE: out[r] = sum over the row's triangle of the block inverse M (rows and columns from r0 on)
+//   else:  out[r] -= sum_c M[r][c0 + c] v[c0 + c], c < nc
+// NV vectors per grid row (ld lv and lo between vectors).  Bound by latency (a 512 x 512 inverse is
+// read by 64 workgroups in about 3 us), so every load of a row group is issued together.
+template <typename T, int R, int NV, bool SOLVE>
+__global__ __launch_bounds__(256) void k_tri_gemv(const T *__restrict__ M, int64_t ldm, int64_t r0, int64_t r1, int64_t c0,
+                                                  int nc, int upper, const double *__restrict__ v, int64_t lv,
+                                                  double *__restrict__ out, int64_t lo, int nv)
+{
+    constexpr int V = Lu<T>::V;
+    typedef typename Lu<T>::vec vec;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t rb = r0 + ((int64_t)blockIdx.x * 4 + wave) * R;
+    if (rb >= r1) return;
+    const int vb = blockIdx.y * NV, vn = min(NV, nv - vb);
+    v += (int64_t)vb * lv;
+    out += (int64_t)vb * lo;
+    double acc[R][NV];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) acc[i][j] = 0.0;
+    // the columns of this row group: all nc, or the tiles of its triangle (a group lies in one 64-row tile)
+    int lo_c = 0, hi_c = nc;
+    if (SOLVE) {
+        const int tile = (int)(rb - r0) & ~(NPB - 1);
+        if (upper) lo_c = tile;
+        else hi_c = min(nc, tile + NPB);
+    }
+    for (int cb = lo_c; cb < hi_c; cb += 64 * V) {
+        const int c = cb + lane * V;
+        if (c < hi_c) {
+            vec a[R];
+            if (c + V <= hi_c) {
+#pragma unroll
+                for (int i = 0; i < R; ++i)
+                    a[i] = *reinterpret_cast<const vec *>(M + (min(rb + i, r1 - 1) - (SOLVE ? r0 : 0)) * ldm + c);
+            } else {
+#pragma unroll
+                for (int i = 0; i < R; ++i)
+#pragma unroll
+                    for (int e = 0; e < V; ++e)
+                        a[i][e] = c + e < hi_c ? M[(min(rb + i, r1 - 1) - (SOLVE ? r0 : 0)) * ldm + c + e] : T(0);
+            }
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const double *x = v + (int64_t)min(j, vn - 1) * lv + c0 + c;
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    const double xe = c + e < hi_c ? x[e] : 0.0;
+#pragma unroll
+                    for (int i = 0; i < R; ++i) acc[i][j] = fma((double)a[i][e], xe, acc[i][j]);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            double t = acc[i][j];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
+            if (lane == 0 && rb + i < r1 && j < vn) {
+                double *o = out + (int64_t)j * lo + rb + i;
+                *o = SOLVE ? t : *o - t;
+            }
+        }
 }
 
 __global__ void k_fill_info(int *p, int v)
@@ -760,8 +894,12 @@ int fp_rbt_vec(fp_ctx *ctx, const double *in, int64_t ldin, double *out, int64_t
     return FP_OK;
 }
 
-// L11^-1 and U11^-1 of an outer block's diagonal blocks
-size_t fp_getrf_nopiv_work_bytes(int elem_bytes) { return (size_t)2 * NIN * NPB * NPB * elem_bytes; }
+// the diagonal-block inverses of L, then of U, then fp_tri_inverse's products
+static int64_t lu_dsize(int64_t n) { return (n + TBIG - 1) / TBIG * ((int64_t)TBIG * TBIG); }
+size_t fp_getrf_nopiv_work_bytes(int64_t n, int elem_bytes)
+{
+    return ((size_t)2 * lu_dsize(n) + (size_t)lu_dsize(n) / 2) * elem_bytes;
+}
 
 static int64_t lu_tiles(int64_t x, int64_t w) { return x > 0 ? (x + w - 1) / w : (int64_t)0; }
 
@@ -776,7 +914,7 @@ int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void
     if (n <= 0) return FP_OK;
     if (ld % 4) return fp_fail(ctx, FP_ERR_ARG, "internal: no-pivot LU needs a leading dimension divisible by 4");
     hipLaunchKernelGGL(k_fill_info, dim3(1), dim3(64), 0, ctx->stream, info_dev, 0);
-    const LuMat<T> m{A, ld, n, (T *)work, info_dev, YL, YU};
+    const LuMat<T> m{A, ld, n, (T *)work, (T *)work + lu_dsize(n), info_dev, YL, YU};
     int st;
     for (int64_t k = 0; k < n; k += NOB) {
         const int64_t kend = std::min<int64_t>(k + NOB, n);
@@ -805,6 +943,71 @@ int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void
 template int fp_getrf_nopiv<float>(fp_ctx *, float *, int64_t, int64_t, int *, void *, float *, float *);
 template int fp_getrf_nopiv<double>(fp_ctx *, double *, int64_t, int64_t, int *, void *, double *, double *);
 
+// The inverses of the TBIG-row diagonal blocks of fp_getrf_nopiv's factors (same work), from their
+// 64-row blocks: three levels of two launches.  About (2/3) n TBIG^2 flop.
+template <typename T>
+int fp_tri_inverse(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, void *work)
+{
+    ProfScope ps(ctx, "lu_nopiv_blockinv");
+    const LuMat<T> m{const_cast<T *>(A), ld, n, (T *)work, (T *)work + lu_dsize(n), nullptr, nullptr, nullptr};
+    T *W = (T *)work + 2 * lu_dsize(n);
+    for (int s = NPB; s < TBIG && s < n; s *= 2) {
+        const dim3 g((unsigned)((s / NPB) * (s / NPB)), (unsigned)lu_tiles(n, 2 * s), 2);
+        hipLaunchKernelGGL(k_tri_merge<T>, g, dim3(256), 0, ctx->stream, m, W, s, 0);
+        hipLaunchKernelGGL(k_tri_merge<T>, g, dim3(256), 0, ctx->stream, m, W, s, 1);
+    }
+    FP_HIP(ctx, hipGetLastError());
+    return FP_OK;
+}
+template int fp_tri_inverse<float>(fp_ctx *, const float *, int64_t, int64_t, void *);
+template int fp_tri_inverse<double>(fp_ctx *, const double *, int64_t, int64_t, void *);
+
+template <typename T, int NV>
+static void tri_gemvs(fp_ctx *ctx, const T *LU, int64_t n, int64_t ld, const T *D, bool upper, double *b, int64_t ldb,
+                      double *y, int64_t ldy, int64_t k)
+{
+    const unsigned gy = (unsigned)((k + NV - 1) / NV);
+    const int64_t nb = (n + TBIG - 1) / TBIG;
+    for (int64_t q = 0; q < nb; ++q) {
+        const int64_t j = upper ? nb - 1 - q : q, c0 = j * TBIG, c1 = std::min<int64_t>(c0 + TBIG, n);
+        hipLaunchKernelGGL((k_tri_gemv<T, 2, NV, true>), dim3((unsigned)lu_tiles(c1 - c0, 8), gy), dim3(256), 0, ctx->stream,
+                           D + j * ((int64_t)TBIG * TBIG), (int64_t)TBIG, c0, c1, c0, (int)(c1 - c0), upper ? 1 : 0,
+                           (const double *)b, ldb, y, ldy, (int)k);
+        // the rows still to be solved
+        const int64_t r0 = upper ? 0 : c1, r1 = upper ? c0 : n;
+        if (r1 > r0)
+            hipLaunchKernelGGL((k_tri_gemv<T, 4, NV, false>), dim3((unsigned)lu_tiles(r1 - r0, 16), gy), dim3(256), 0,
+                               ctx->stream, LU + c0, ld, r0, r1, c0, (int)(c1 - c0), 0, (const double *)y, ldy, b, ldb,
+                               (int)k);
+    }
+}
+
+// x (n x k, ldx, FP64) := U^-1 L^-1 x by fp_getrf_nopiv's factors and the block inverses in `work`
+// (fp_tri_inverse); tmp: n k doubles.  Two launches per 512-row block and sweep: the block's solution
+// y = D b, then its contribution to the rows still to be solved.  The chain of launches bounds it
+// (4,800 unknowns: 20 a sweep); a sweep that polls per 128-row block walked 38 hand-overs of 8-10 us.
+template <typename T>
+int fp_lu_solve_nopiv(fp_ctx *ctx, const T *LU, int64_t n, int64_t ld, const void *work, double *x, int64_t k, int64_t ldx,
+                      double *tmp)
+{
+    if (n <= 0 || k <= 0) return FP_OK;
+    ProfScope ps(ctx, "getrs");
+    const T *DL = (const T *)work, *DU = DL + lu_dsize(n);
+    if (k == 1) {
+        tri_gemvs<T, 1>(ctx, LU, n, ld, DL, false, x, ldx, tmp, n, k);
+        tri_gemvs<T, 1>(ctx, LU, n, ld, DU, true, tmp, n, x, ldx, k);
+    } else {
+        tri_gemvs<T, 4>(ctx, LU, n, ld, DL, false, x, ldx, tmp, n, k);
+        tri_gemvs<T, 4>(ctx, LU, n, ld, DU, true, tmp, n, x, ldx, k);
+    }
+    FP_HIP(ctx, hipGetLastError());
+    return FP_OK;
+}
+template int fp_lu_solve_nopiv<float>(fp_ctx *, const float *, int64_t, int64_t, const void *, double *, int64_t, int64_t,
+                                      double *);
+template int fp_lu_solve_nopiv<double>(fp_ctx *, const double *, int64_t, int64_t, const void *, double *, int64_t,
+                                       int64_t, double *);
+
 // ---- the same factorisation for many bodies at once --------------------------
 // One launch per step covers every body (blockIdx.y = body): the bodies' serial chains of
 // diagonal blocks run side by side, and the small products of different bodies fill the chip
@@ -818,7 +1021,8 @@ __global__ void k_fill_info_lub(const fp_lu_desc *__restrict__ desc, int nb)
 
 static __device__ __forceinline__ LuMat<float> lub_mat(const fp_lu_desc &d)
 {
-    return LuMat<float>{d.A, d.ld, d.n, d.work, d.info, nullptr, nullptr};
+    return LuMat<float>{d.A, d.ld, d.n, d.work, d.work + (d.n + TBIG - 1) / TBIG * ((int64_t)TBIG * TBIG), d.info,
+                        nullptr, nullptr};
 }
 
 __global__ __launch_bounds__(256) void k_lu_first_lub(const fp_lu_desc *__restrict__ desc, int64_t kk)
@@ -937,7 +1141,7 @@ static int64_t inv_ld(int64_t n4) { return std::max<int64_t>(64, (n4 + 63) / 64 
 size_t fp_inverse_rbt_work_bytes(int64_t n)
 {
     const int64_t n4 = fp_rbt_size(n), ld4 = inv_ld(n4);
-    return (size_t)4 * n4 * ld4 * sizeof(float) + fp_rbt_weights_bytes(n) + fp_getrf_nopiv_work_bytes(sizeof(float)) + 1024;
+    return (size_t)4 * n4 * ld4 * sizeof(float) + fp_rbt_weights_bytes(n) + fp_getrf_nopiv_work_bytes(n4, sizeof(float)) + 1024;
 }
 
 // E^-1 in place (n x n, FP64, lde) by the LU without pivoting of the randomized

@@ -73,3 +73,15 @@ def test_nearly_singular_matrix_matches_pivoted(fp, monkeypatch):
         monkeypatch.setenv("FLOWPANEL_LU64_PIVOTED", pv)
         x = fp.solve_ludiv(None, A, b)
         assert np.linalg.norm(A @ x - b) < 64 * n * EPS * (np.linalg.norm(x) + np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("n,k", [(37, 1), (300, 1), (300, 5), (1031, 2)])
+def test_refined_solution_is_accurate_to_the_data(fp, n, k):
+    # integer data, so that b = A x is exact: the residuals of twice FP64 take the solution to its own
+    # rounding (condition up to 1e6 here; a plain FP64 solve is left with about condition x eps)
+    rng = np.random.default_rng(n + k)
+    A = rng.integers(-50, 51, (n, n)).astype(float)
+    A[:, 0] = A[:, 1:].sum(axis=1) + rng.integers(-1, 2, n)
+    X = rng.integers(-9, 10, (n, k)).astype(float)
+    got = fp.solve_ludiv(None, A, A @ X).reshape(n, k)
+    assert np.abs(got - X).max() < 1e-14 * np.abs(X).max()
