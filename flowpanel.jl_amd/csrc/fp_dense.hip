@@ -34,65 +34,59 @@ template <> struct MfmaOp<float> {
 };
 
 // ----------------------------------------------------------------------------
-// C[m x n] -= A[m x k] * B[k x n], all row-major.  128 x 128 tile per 256-thread
-// workgroup (2 x 2 waves of 64 x 64), K step 32 through LDS with register
-// prefetch of the next step, 16-byte global loads.  FP32 runs v_mfma_f32_16x16x4;
-// FP64 runs v_mfma_f64_4x4x4_4b (k_gemm_sub_f64 below): on gfx950 the FP64
-// 16x16x4 form issues at half the FP64 matrix rate (measured 36 of 78.6 TFLOP/s
-// with every SIMD busy, register-only), the four-block 4x4x4 form at 67-73.
-// FP32 operand layout (16x16x4): lane l supplies A(l%16, l/16) and B(l/16, l%16);
-// accumulator rows as in MfmaOp<float>::row (measured on gfx950 with an
-// in-bounds lane-layout probe).
+// C[m x n] -= A[m x k] * B[k x n], all row-major, on 128 x 128 tiles: eight waves of 64 x 32 each, K
+// steps of 32 (FP32) or 16 (FP64) through two LDS buffers with one barrier a step (a step stores into
+// the buffer the previous step did not read; a wave that reaches the store after next has passed the
+// barrier every wave reaches only after its reads of that buffer).  What bounded the four-wave form
+// was occupancy: 64 accumulators plus a whole wave tile of C held one (FP64) or two (FP32) waves a
+// SIMD, so the first loads and the epilogue of a K = 256 update stood alone.  Eight waves of half the
+// tile fit 128 registers, two workgroups share a compute unit, and C goes through the registers in parts.
+// FP32: v_mfma_f32_16x16x4 (register-only 149 TFLOP/s, the 32x32x2 form 152).  FP64:
+// v_mfma_f64_4x4x4_4b, each instruction given the same B columns in all four blocks, a 16 x 4 x 4
+// product (76; the 16x16x4 form issues at half the rate, 36).
+// Operand layouts (in-bounds lane probes on gfx950): A(row l%16, k l/16) for both; FP32 B(k l/16, col
+// l%16) and D(row 4 (l/16) + e, col l%16); FP64 B(k l/16, col l%4) and D(row 4 ((l/4)%4) + l/16, col l%4).
+// K a multiple of the step and aligned rows (every update of the LU): the tiles go from memory to LDS
+// without passing through registers (global_load_lds, 16 bytes a lane), which frees the staging
+// registers (FP64 spilled 15, and a scratch access in the loop waits for the loads in flight) and the
+// LDS write slots; a 16-byte group is placed by an exclusive-or of its index with bits of its row, so
+// that the fragment reads' 64 lanes spread over all banks without padding.  Any other product stages
+// through registers (LDS rows padded instead).  FP64 lanes own eight consecutive columns of C.
+// Measured, C 7,744 x 7,744 of K = 256: FP32 292 us (105 TFLOP/s; 307
+// in the four-wave form), FP64 651 us (47 TFLOP/s; 1,018 in the four-wave form, 832 staged through
+// registers); a request of C before the last K step spilled and was slower (FP32 333 us).  What is left is
+// the traffic of C, 12 or 24 bytes for 512 operations, and the last round of 512 resident tiles.
 // Tile order: workgroup b runs on XCD b % 8; every XCD is given a contiguous
 // range of a grouped order (8 tile rows walked together), so the A rows of a
 // group stay in that XCD's L2 while it sweeps across the B columns.
-constexpr int GB_M = 128, GB_N = 128, GB_K = 32, GB_PAD = 4, GB_GROUP = 8, GB_XCD = 8;
+constexpr int GB_M = 128, GB_N = 128, GB_GROUP = 8, GB_XCD = 8, GB_THREADS = 512;
 
-template <typename T>
-__device__ __forceinline__ void ld16(const T *__restrict__ p, bool full, bool vec, int valid, T *out)
+template <typename T> struct Gm;
+template <> struct Gm<float> {
+    static constexpr int KS = 32, LDA = KS + 4, LDB = GB_N + 16, V = 4;
+    typedef float vec __attribute__((ext_vector_type(4)));
+    typedef float v4 __attribute__((ext_vector_type(4)));
+};
+template <> struct Gm<double> {
+    static constexpr int KS = 16, LDA = KS + 2, LDB = GB_N + 4, V = 2;
+    typedef double vec __attribute__((ext_vector_type(2)));
+    typedef double v4 __attribute__((ext_vector_type(4)));
+};
+
+// N consecutive entries from p, zero beyond `valid`; 16-byte loads where vec says the rows are aligned
+template <typename T, int N>
+__device__ __forceinline__ void gm_load(const T *p, bool vec, int valid, T (&out)[N])
 {
-    if (full && vec) {
-        if (sizeof(T) == 8) {
+    if (vec && valid == N) {
 #pragma unroll
-            for (int e = 0; e < 16; e += 2) {
-                const double2 v = *reinterpret_cast<const double2 *>(p + e);
-                out[e] = (T)v.x; out[e + 1] = (T)v.y;
-            }
-        } else {
+        for (int e = 0; e < N; e += Gm<T>::V) {
+            const typename Gm<T>::vec v = *reinterpret_cast<const typename Gm<T>::vec *>(p + e);
 #pragma unroll
-            for (int e = 0; e < 16; e += 4) {
-                const float4 v = *reinterpret_cast<const float4 *>(p + e);
-                out[e] = (T)v.x; out[e + 1] = (T)v.y; out[e + 2] = (T)v.z; out[e + 3] = (T)v.w;
-            }
+            for (int q = 0; q < Gm<T>::V; ++q) out[e + q] = v[q];
         }
     } else {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) out[e] = e < valid ? p[e] : T(0);
-    }
-}
-
-// FP32: K steps of GB_KF through two LDS buffers, one barrier per step (a step's
-// stores go to the buffer the previous step did not read; a wave reaching the
-// store after next has passed the barrier that every wave reaches only after
-// finishing its reads of that buffer).  Measured on 4,608^2 x k products:
-// 87 against 80 TFLOP/s at k = 256 and 107 against 94 at k = 1,024 for K steps
-// of 32 through one buffer (register-only 16x16x4 rate: 125 TFLOP/s).
-constexpr int GB_KF = 16;
-
-// n_ entries from p (16-byte aligned groups when vec and full), zero beyond `valid`
-template <int N_>
-__device__ __forceinline__ void ldf(const float *__restrict__ p, bool full, bool vec, int valid, float *out)
-{
-    if (full && vec) {
-#pragma unroll
-        for (int e = 0; e < N_; e += 4) {
-            const float4 v = *reinterpret_cast<const float4 *>(p + e);
-            out[e] = v.x; out[e + 1] = v.y; out[e + 2] = v.z; out[e + 3] = v.w;
-        }
-    } else {
-        // clamped addresses: every load in bounds and unconditional, the rest zeroed by a product
-#pragma unroll
-        for (int e = 0; e < N_; ++e) out[e] = valid > 0 ? p[min(e, valid - 1)] * (e < valid ? 1.f : 0.f) : 0.f;
+        for (int e = 0; e < N; ++e) out[e] = e < valid ? p[e] : T(0);
     }
 }
 
@@ -115,94 +109,280 @@ __device__ __forceinline__ bool gemm_tile_of(int64_t bx, int64_t m, int64_t n, i
     return true;
 }
 
-// One 128 x 128 tile (m0, n0) of C -= A B in FP32 (the body of k_gemm_sub, shared
-// with the batched LU's trailing updates).
-__device__ __forceinline__ void gemm_sub_f32_tile(int64_t m, int64_t n, int64_t k, const float *__restrict__ A,
-                                                  int64_t lda, const float *__restrict__ B, int64_t ldb,
-                                                  float *__restrict__ C, int64_t ldc, int vec, int64_t m0,
-                                                  int64_t n0)
-{
-    typedef float T;
-    typedef typename MfmaOp<T>::acc acc_t;
-    __shared__ T As[2][GB_KF][GB_M + GB_PAD];
-    __shared__ T Bs[2][GB_KF][GB_N + GB_PAD];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
+template <typename T> struct GmLds {
+    T A[2][GB_M * Gm<T>::LDA];
+    T B[2][Gm<T>::KS * Gm<T>::LDB];
+};
 
-    acc_t acc[4][4];
+template <typename T> struct GmAcc {
+    typename Gm<T>::v4 v[4][2];
+};
+
+// the four-row and two-column-group products of one k group of four: va the four row fragments, vb
+template <typename T, int NB>
+__device__ __forceinline__ void gm_mma(const T (&va)[4], const T (&vb)[NB], GmAcc<T> &acc)
+{
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
+        for (int b = 0; b < NB; ++b) {
+            if constexpr (sizeof(T) == 4)
+                acc.v[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[a], vb[b], acc.v[a][b], 0, 0, 0);
+            else
+                acc.v[a][b >> 2][b & 3] = __builtin_amdgcn_mfma_f64_4x4x4f64(va[a], vb[b], acc.v[a][b >> 2][b & 3], 0, 0, 0);
+        }
+}
 
-    // A: row tid/2, k (tid%2)*8..+8 ; B: k row tid/16, cols (tid%16)*8..+8
-    constexpr int AE = GB_M * GB_KF / 256, BE = GB_KF * GB_N / 256;
-    const int arow = tid / (GB_KF / AE), ak = (tid % (GB_KF / AE)) * AE;
-    const int bk = tid / (GB_N / BE), bc = (tid % (GB_N / BE)) * BE;
-    T ra[AE], rb[BE];
-    auto load = [&](int64_t k0) {
-        const int64_t gr = m0 + arow, gk = k0 + ak;
-        const int av = gr < m ? (int)max((int64_t)0, min((int64_t)AE, k - gk)) : 0;
-        ldf<AE>(A + min(gr, m - 1) * lda + gk, av == AE, vec, av, ra);
-        const int64_t gkb = k0 + bk, gc = n0 + bc;
-        const int bv = gkb < k ? (int)max((int64_t)0, min((int64_t)BE, n - gc)) : 0;
-        ldf<BE>(B + min(gkb, k - 1) * ldb + gc, bv == BE, vec, bv, rb);
+// C -= acc.  In parts: a part's loads of C are issued together before its first store (as far as the
+// compiler knows rows of C could alias, and a load after a store would wait for it).
+template <typename T>
+__device__ __forceinline__ void gm_store(int64_t m, int64_t n, T *__restrict__ C, int64_t ldc, int64_t m0, int64_t n0,
+                                         int lane, int wm, int wn, const GmAcc<T> &acc_)
+{
+    constexpr bool F32 = sizeof(T) == 4;
+    typedef typename Gm<T>::vec vecT;
+    const auto &acc = acc_.v;
+    if constexpr (F32) {
+        const bool interior = m0 + GB_M <= m && n0 + GB_N <= n;   // uniform
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            T cv[2][2][4];
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int64_t row = m0 + wm + 16 * (2 * h + a) + 4 * (lane >> 4) + e;
+                        const int64_t col = n0 + wn + 16 * t + (lane & 15);
+                        cv[a][t][e] = interior ? C[row * ldc + col] : C[min(row, m - 1) * ldc + min(col, n - 1)];
+                    }
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int64_t row = m0 + wm + 16 * (2 * h + a) + 4 * (lane >> 4) + e;
+                        const int64_t col = n0 + wn + 16 * t + (lane & 15);
+                        if (interior || (row < m && col < n)) C[row * ldc + col] = cv[a][t][e] - acc[2 * h + a][t][e];
+                    }
+        }
+    } else {
+        const int64_t row0 = m0 + wm + 4 * ((lane >> 2) & 3) + (lane >> 4), col = n0 + wn + 8 * (lane & 3);
+        const bool cvec = (ldc & 1) == 0 && ((uintptr_t)C & 15) == 0 && col + 8 <= n;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            T cv[2][8];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                const int64_t row = min(row0 + 16 * (2 * h + a), m - 1);
+                const T *c = C + row * ldc + col;
+                if (cvec) {
+#pragma unroll
+                    for (int b = 0; b < 8; b += 2) {
+                        const vecT v = *reinterpret_cast<const vecT *>(c + b);
+                        cv[a][b] = v[0];
+                        cv[a][b + 1] = v[1];
+                    }
+                } else {
+#pragma unroll
+                    for (int b = 0; b < 8; ++b) cv[a][b] = col + b < n ? c[b] : T(0);
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                const int64_t row = row0 + 16 * (2 * h + a);
+                if (row >= m) continue;
+                T *c = C + row * ldc + col;
+                if (cvec) {
+#pragma unroll
+                    for (int b = 0; b < 8; b += 2) {
+                        vecT v;
+                        v[0] = cv[a][b] - acc[2 * h + a][b >> 2][b & 3];
+                        v[1] = cv[a][b + 1] - acc[2 * h + a][b >> 2][(b & 3) + 1];
+                        *reinterpret_cast<vecT *>(c + b) = v;
+                    }
+                } else {
+#pragma unroll
+                    for (int b = 0; b < 8; ++b)
+                        if (col + b < n) c[b] = cv[a][b] - acc[2 * h + a][b >> 2][b & 3];
+                }
+            }
+        }
+    }
+}
+
+// direct to LDS: 16 bytes per lane from `g` to base + 16 lane (base wave-uniform)
+__device__ __forceinline__ void gm_dma(const void *g, void *base)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)g,
+                                     (__attribute__((address_space(3))) void *)base, 16, 0, 0);
+}
+
+// One 128 x 128 tile (m0, n0) of C -= A B, k a multiple of KS, rows of A and B 16-byte aligned.  The
+// 128-byte pieces of 128 rows of A (eight 16-byte groups each, group p at p ^ ((row / 2) % 8)) and the
+// KS rows of B (128 columns; FP32 group q at q ^ 4 (k % 4), FP64 at q ^ (k % 4)) lie densely in LDS.
+// Rows beyond m and columns beyond n take the last valid ones (their results are not stored).
+template <typename T>
+__device__ __forceinline__ void gemm_sub_dma(int64_t m, int64_t n, int64_t k, const T *__restrict__ A, int64_t lda,
+                                             const T *__restrict__ B, int64_t ldb, T *__restrict__ C, int64_t ldc,
+                                             int64_t m0, int64_t n0, GmLds<T> &s)
+{
+    constexpr int KS = Gm<T>::KS, V = Gm<T>::V;
+    constexpr bool F32 = sizeof(T) == 4;
+    constexpr int BG = GB_N / V, BR = 64 / BG;   // 16-byte groups per row of B, rows of B per wave instruction
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = (wave >> 2) * 64, wn = (wave & 3) * 32;
+    GmAcc<T> acc;
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc.v[a][t] = typename Gm<T>::v4{0, 0, 0, 0};
+    // 16 wave instructions bring A's 16 KiB (8 rows each), 16 bring B's: two of each per wave
+    const T *pa[2], *pb[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int r = 8 * (2 * wave + q) + (lane >> 3), g = (lane & 7) ^ ((r >> 1) & 7);
+        pa[q] = A + min(m0 + r, m - 1) * lda + g * V;
+        const int kr = BR * (2 * wave + q) + lane / BG, h = (lane % BG) ^ (F32 ? (kr & 3) << 2 : kr & 3);
+        pb[q] = B + (int64_t)kr * ldb + min(n0 + (int64_t)h * V, (n - 1) & ~(int64_t)(V - 1));
+    }
+    auto load = [&](int buf) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            gm_dma(pa[q], s.A[buf] + (2 * wave + q) * 64 * V);
+            gm_dma(pb[q], s.B[buf] + (2 * wave + q) * 64 * V);
+            pa[q] += KS;
+            pb[q] += KS * ldb;
+        }
     };
     load(0);
     int buf = 0;
-    for (int64_t k0 = 0; k0 < k; k0 += GB_KF) {
-#pragma unroll
-        for (int e = 0; e < AE; ++e) As[buf][ak + e][arow] = ra[e];
-#pragma unroll
-        for (int e = 0; e < BE; ++e) Bs[buf][bk][bc + e] = rb[e];
+    for (int64_t k0 = 0; k0 < k; k0 += KS) {
+        // this step's tiles have landed; every wave is done reading the other buffer
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (k0 + GB_KF < k) load(k0 + GB_KF);
+        if (k0 + KS < k) load(buf ^ 1);
+        const T *sa = s.A[buf], *sb = s.B[buf];
 #pragma unroll
-        for (int ks = 0; ks < GB_KF; ks += 4) {
-            T fa[4], fb[4];
+        for (int ks = 0; ks < KS; ks += 4) {
+            const int kk = ks + (lane >> 4), r = lane & 15, g = (kk / V) ^ ((r >> 1) & 7);
+            T va[4];
 #pragma unroll
-            for (int a = 0; a < 4; ++a) fa[a] = As[buf][ks + (lane >> 4)][wm * 64 + a * 16 + (lane & 15)];
+            for (int a = 0; a < 4; ++a) va[a] = sa[(wm + 16 * a + r) * KS + g * V + kk % V];
+            if constexpr (F32) {
+                T vb[2];
 #pragma unroll
-            for (int b = 0; b < 4; ++b) fb[b] = Bs[buf][ks + (lane >> 4)][wn * 64 + b * 16 + (lane & 15)];
+                for (int t = 0; t < 2; ++t) {
+                    const int c = wn + 16 * t + r;
+                    vb[t] = sb[kk * GB_N + (((c / V) ^ ((kk & 3) << 2)) * V) + c % V];
+                }
+                gm_mma<T, 2>(va, vb, acc);
+            } else {
+                T vb[8];
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) acc[a][b] = MfmaOp<T>::run(fa[a], fb[b], acc[a][b]);
+                for (int b = 0; b < 8; ++b) {
+                    const int c = wn + 8 * (lane & 3) + b;
+                    vb[b] = sb[kk * GB_N + (((c / V) ^ (kk & 3)) * V) + c % V];
+                }
+                gm_mma<T, 8>(va, vb, acc);
+            }
         }
         buf ^= 1;
     }
-    // epilogue: every load of the lane's 64 entries of C is issued before the first
-    // store (as far as the compiler knows rows of C could alias, and a load after a
-    // store would wait for it: one memory round trip per entry); edge tiles clamp
-    // their addresses and store only inside C
-    const bool interior = m0 + GB_M <= m && n0 + GB_N <= n;   // uniform
-    T cv[4][4][4];
+    gm_store<T>(m, n, C, ldc, m0, n0, lane, wm, wn, acc);
+}
+
+// The same for any k and alignment, staged through registers; vec: rows of A and B are 16-byte aligned.
+template <typename T>
+__device__ __forceinline__ void gemm_sub_reg(int64_t m, int64_t n, int64_t k, const T *__restrict__ A, int64_t lda,
+                                              const T *__restrict__ B, int64_t ldb, T *__restrict__ C, int64_t ldc,
+                                              int vec, int64_t m0, int64_t n0, GmLds<T> &s)
+{
+    constexpr int KS = Gm<T>::KS, LDA = Gm<T>::LDA, LDB = Gm<T>::LDB, V = Gm<T>::V, E = KS / 4;
+    constexpr bool F32 = sizeof(T) == 4;
+    typedef typename Gm<T>::vec vecT;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = (wave >> 2) * 64, wn = (wave & 3) * 32;
+
+    GmAcc<T> acc;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int t = 0; t < 2; ++t) acc.v[a][t] = typename Gm<T>::v4{0, 0, 0, 0};
+
+    // staging: E entries of a row of A (four threads a row), E of a k row of B
+    const int ar = tid >> 2, ak = (tid & 3) * E;
+    constexpr int TPB = GB_N / E;
+    const int bk = tid / TPB, bc = (tid % TPB) * E;
+    const int64_t gr = m0 + ar, gc = n0 + bc;
+    const T *pa = A + min(gr, m - 1) * lda + ak, *pb = B + (int64_t)bk * ldb + gc;
+    const int bcols = (int)max((int64_t)0, min((int64_t)E, n - gc));
+    T ra[E], rb[E];
+    auto load = [&](int64_t k0) {
+        const int av = gr < m ? (int)max((int64_t)0, min((int64_t)E, k - k0 - ak)) : 0;
+        gm_load<T, E>(pa + k0, vec, av, ra);
+        gm_load<T, E>(pb + k0 * ldb, vec, k0 + bk < k ? bcols : 0, rb);
+    };
+    load(0);
+    int buf = 0;
+    for (int64_t k0 = 0; k0 < k; k0 += KS) {
+        T *sa = s.A[buf], *sb = s.B[buf];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t row = m0 + wm * 64 + a * 16 + MfmaOp<T>::row(lane, r);
-                const int64_t col = n0 + wn * 64 + b * 16 + (lane & 15);
-                cv[a][b][r] = interior ? C[row * ldc + col] : C[min(row, m - 1) * ldc + min(col, n - 1)];
+        for (int e = 0; e < E; e += V) {
+            vecT v;
+#pragma unroll
+            for (int q = 0; q < V; ++q) v[q] = ra[e + q];
+            *reinterpret_cast<vecT *>(sa + ar * LDA + ak + e) = v;
+        }
+        if constexpr (F32) {
+#pragma unroll
+            for (int e = 0; e < E; e += V) {
+                vecT v;
+#pragma unroll
+                for (int q = 0; q < V; ++q) v[q] = rb[e + q];
+                *reinterpret_cast<vecT *>(sb + bk * LDB + bc + e) = v;
             }
+        } else {
+            // column c of a 32-column group goes to slot 4 (c % 8) + c / 8
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t row = m0 + wm * 64 + a * 16 + MfmaOp<T>::row(lane, r);
-                const int64_t col = n0 + wn * 64 + b * 16 + (lane & 15);
-                if (interior || (row < m && col < n)) C[row * ldc + col] = cv[a][b][r] - acc[a][b][r];
+            for (int e = 0; e < E; ++e) {
+                const int c = bc + e;
+                sb[bk * LDB + (c & ~31) + 4 * (c & 7) + ((c >> 3) & 3)] = rb[e];
             }
+        }
+        __syncthreads();
+        if (k0 + KS < k) load(k0 + KS);
+        const T *fa = sa + (wm + (lane & 15)) * LDA + (lane >> 4);
+        const T *fb = sb + (lane >> 4) * LDB + wn + (F32 ? (lane & 15) : (lane & 3));
+#pragma unroll
+        for (int ks = 0; ks < KS; ks += 4) {
+            T va[4];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) va[a] = fa[16 * a * LDA + ks];
+            if constexpr (F32) {
+                T vb[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) vb[t] = fb[ks * LDB + 16 * t];
+                gm_mma<T, 2>(va, vb, acc);
+            } else {
+                T vb[8];
+#pragma unroll
+                for (int b = 0; b < 8; ++b) vb[b] = fb[ks * LDB + 4 * b];
+                gm_mma<T, 8>(va, vb, acc);
+            }
+        }
+        buf ^= 1;
+    }
+    gm_store<T>(m, n, C, ldc, m0, n0, lane, wm, wn, acc);
 }
 
 // The batched LU's trailing update of outer block [kk, kk + ob) for body blockIdx.y:
 // C = A[kend:, kend:] -= A[kend:, kk:kend] A[kk:kend, kend:] (bodies with n <= kend idle).
-__global__ __launch_bounds__(256) void k_gemm_sub_lub(const fp_lu_desc *__restrict__ desc, int64_t kk, int ob)
+__global__ __launch_bounds__(GB_THREADS, 4) void k_gemm_sub_lub(const fp_lu_desc *__restrict__ desc, int64_t kk, int ob)
 {
+    __shared__ GmLds<float> s;
     const fp_lu_desc d = desc[blockIdx.y];
     const int64_t kend = kk + ob, right = d.n - kend;
     if (right <= 0) return;
@@ -210,8 +390,8 @@ __global__ __launch_bounds__(256) void k_gemm_sub_lub(const fp_lu_desc *__restri
     if (!gemm_tile_of(blockIdx.x, right, right, m0, n0)) return;
     const float *Ap = d.A + kend * d.ld + kk, *Bp = d.A + kk * d.ld + kend;
     float *Cp = d.A + kend * d.ld + kend;
-    const int vec = (((uintptr_t)Ap | (uintptr_t)Bp) & 15) == 0 && (d.ld * sizeof(float)) % 16 == 0;
-    gemm_sub_f32_tile(right, right, ob, Ap, d.ld, Bp, d.ld, Cp, d.ld, vec, m0, n0);
+    // outer blocks of 256 columns from a 16-byte aligned matrix, ld a multiple of 4
+    gemm_sub_dma<float>(right, right, ob, Ap, d.ld, Bp, d.ld, Cp, d.ld, m0, n0, s);
 }
 
 int fp_gemm_sub_lub(fp_ctx *ctx, const fp_lu_desc *d_desc, int nb, int64_t kk, int ob, int64_t max_right)
@@ -220,135 +400,53 @@ int fp_gemm_sub_lub(fp_ctx *ctx, const fp_lu_desc *d_desc, int nb, int64_t kk, i
     const int64_t t = (max_right + GB_M - 1) / GB_M;
     const int64_t grid = (t * t + GB_XCD - 1) / GB_XCD * GB_XCD;
     ProfScope ps(ctx, "gemm_f32");
-    hipLaunchKernelGGL(k_gemm_sub_lub, dim3((unsigned)grid, (unsigned)nb), dim3(256), 0, ctx->stream, d_desc, kk, ob);
+    hipLaunchKernelGGL(k_gemm_sub_lub, dim3((unsigned)grid, (unsigned)nb), dim3(GB_THREADS), 0, ctx->stream, d_desc, kk, ob);
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;
 }
 
+// strided batch: grid row y runs product y (all products the same shape)
 template <typename T>
-__global__ __launch_bounds__(256) void k_gemm_sub(int64_t m, int64_t n, int64_t k, const T *__restrict__ A,
-                                                  int64_t lda, const T *__restrict__ B, int64_t ldb,
-                                                  T *__restrict__ C, int64_t ldc, int vec, int64_t sA = 0,
-                                                  int64_t sB = 0, int64_t sC = 0)
+__global__ __launch_bounds__(GB_THREADS, 4) void k_gemm_sub(int64_t m, int64_t n, int64_t k, const T *__restrict__ A,
+                                                            int64_t lda, const T *__restrict__ B, int64_t ldb,
+                                                            T *__restrict__ C, int64_t ldc, int64_t sA, int64_t sB,
+                                                            int64_t sC)
 {
-    static_assert(sizeof(T) == 4, "FP64 products run k_gemm_sub_f64");
-    // strided batch: grid row y runs product y (all products the same shape)
+    __shared__ GmLds<T> s;
     int64_t m0, n0;
     if (!gemm_tile_of(blockIdx.x, m, n, m0, n0)) return;
-    gemm_sub_f32_tile(m, n, k, A + (int64_t)blockIdx.y * sA, lda, B + (int64_t)blockIdx.y * sB, ldb,
-                      C + (int64_t)blockIdx.y * sC, ldc, vec, m0, n0);
+    gemm_sub_dma<T>(m, n, k, A + (int64_t)blockIdx.y * sA, lda, B + (int64_t)blockIdx.y * sB, ldb,
+                    C + (int64_t)blockIdx.y * sC, ldc, m0, n0, s);
 }
 
-// FP64 tile kernel on v_mfma_f64_4x4x4_4b.  Operand layout of that instruction
-// (in-bounds lane probe on gfx950): lane L supplies A(4*blk + i, k) and B(k, j)
-// of block blk = (L>>2)&3 with k = L>>4, i = j = L&3, and receives
-// D(4*blk + (L>>4), L&3).  Every block is given the same B columns, so one
-// instruction is a 16 x 4 x 4 product; a wave's 64 x 64 tile is 4 row fragments
-// x 16 column fragments, 64 independent accumulators per lane.
-// LDS placement: slot a*16 + p of the wave's A rows holds tile row p*4 + a and
-// slot b*4 + j of its B columns holds tile column j*16 + b.  Fragment reads are
-// then 16 consecutive doubles (A) and 4 consecutive doubles per k row (B) --
-// no bank conflicts -- and lane L owns the 4 x 16 block of C at rows P*4..P*4+3,
-// P = 4*((L>>2)&3) + (L>>4), columns (L&3)*16..+15 of its wave tile, written
-// back with 16-byte accesses.
-__global__ __launch_bounds__(256) void k_gemm_sub_f64(int64_t m, int64_t n, int64_t k, const double *__restrict__ A,
-                                                      int64_t lda, const double *__restrict__ B, int64_t ldb,
-                                                      double *__restrict__ C, int64_t ldc, int vec)
+template <typename T>
+__global__ __launch_bounds__(GB_THREADS, 2) void k_gemm_sub_reg(int64_t m, int64_t n, int64_t k, const T *__restrict__ A,
+                                                                int64_t lda, const T *__restrict__ B, int64_t ldb,
+                                                                T *__restrict__ C, int64_t ldc, int64_t sA, int64_t sB,
+                                                                int64_t sC, int vec)
 {
-    __shared__ double As[GB_K][GB_M + GB_PAD];
-    __shared__ double Bs[GB_K][GB_N + GB_PAD];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int64_t tiles_m = (m + GB_M - 1) / GB_M, tiles_n = (n + GB_N - 1) / GB_N;
-    const int64_t ntiles = tiles_m * tiles_n;
-    const int64_t per = (ntiles + GB_XCD - 1) / GB_XCD;
-    const int64_t t = (int64_t)(blockIdx.x % GB_XCD) * per + blockIdx.x / GB_XCD;
-    if (t >= ntiles) return;
-    const int64_t in_group = (int64_t)GB_GROUP * tiles_n;
-    const int64_t first_m = (t / in_group) * GB_GROUP;
-    const int64_t gsize = min((int64_t)GB_GROUP, tiles_m - first_m);
-    const int64_t tm = first_m + (t % in_group) % gsize, tn = (t % in_group) / gsize;
-    const int64_t m0 = tm * GB_M, n0 = tn * GB_N;
+    __shared__ GmLds<T> s;
+    int64_t m0, n0;
+    if (!gemm_tile_of(blockIdx.x, m, n, m0, n0)) return;
+    gemm_sub_reg<T>(m, n, k, A + (int64_t)blockIdx.y * sA, lda, B + (int64_t)blockIdx.y * sB, ldb,
+                    C + (int64_t)blockIdx.y * sC, ldc, vec, m0, n0, s);
+}
 
-    double acc[4][16];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 16; ++b) acc[a][b] = 0.0;
-
-    // A: thread loads 16 k of tile row arow into LDS slot aslot; B: 16 columns of k row bk
-    const int aslot = tid >> 1, ak = (tid & 1) * 16;
-    const int arow = (aslot & 64) + (aslot & 15) * 4 + ((aslot & 63) >> 4);
-    const int bk = tid >> 3, bc = (tid & 7) * 16, bslot = (tid & 4) * 16 + (tid & 3);
-    double ra[16], rb[16];
-    auto load = [&](int64_t k0) {
-        const int64_t gr = m0 + arow, gk = k0 + ak;
-        const int av = gr < m ? (int)max((int64_t)0, min((int64_t)16, k - gk)) : 0;
-        ld16<double>(A + gr * lda + gk, av == 16, vec, av, ra);
-        const int64_t gkb = k0 + bk, gc = n0 + bc;
-        const int bv = gkb < k ? (int)max((int64_t)0, min((int64_t)16, n - gc)) : 0;
-        ld16<double>(B + gkb * ldb + gc, bv == 16, vec, bv, rb);
-    };
-    load(0);
-    for (int64_t k0 = 0; k0 < k; k0 += GB_K) {
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < 16; ++e) As[ak + e][aslot] = ra[e];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) Bs[bk][bslot + e * 4] = rb[e];
-        __syncthreads();
-        if (k0 + GB_K < k) load(k0 + GB_K);
-#pragma unroll
-        for (int ks = 0; ks < GB_K; ks += 4) {
-            double fa[4], fb[16];
-#pragma unroll
-            for (int a = 0; a < 4; ++a) fa[a] = As[ks + (lane >> 4)][wm * 64 + a * 16 + (lane & 15)];
-#pragma unroll
-            for (int b = 0; b < 16; ++b) fb[b] = Bs[ks + (lane >> 4)][wn * 64 + b * 4 + (lane & 3)];
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 16; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f64_4x4x4f64(fa[a], fb[b], acc[a][b], 0, 0, 0);
-        }
-    }
-    // epilogue: every load of the lane's 4 x 16 block of C is issued before the
-    // first store (rows of C could alias as far as the compiler knows, which
-    // would otherwise serialise one memory round trip per row)
-    const int P = 4 * ((lane >> 2) & 3) + (lane >> 4);
-    const int64_t col0 = n0 + wn * 64 + (lane & 3) * 16;
-    const int64_t row0 = m0 + wm * 64 + P * 4;
-    const bool cvec = vec && (ldc & 1) == 0 && ((uintptr_t)C & 15) == 0 && col0 + 16 <= n;
-    double cv[4][16];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const double *c = C + (row0 + a) * ldc + col0;
-        if (row0 + a < m && cvec) {
-#pragma unroll
-            for (int b = 0; b < 16; b += 2) {
-                const double2 v = *reinterpret_cast<const double2 *>(c + b);
-                cv[a][b] = v.x;
-                cv[a][b + 1] = v.y;
-            }
-        } else {
-#pragma unroll
-            for (int b = 0; b < 16; ++b) cv[a][b] = (row0 + a < m && col0 + b < n) ? c[b] : 0.0;
-        }
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        if (row0 + a >= m) continue;
-        double *c = C + (row0 + a) * ldc + col0;
-        if (cvec) {
-#pragma unroll
-            for (int b = 0; b < 16; b += 2)
-                *reinterpret_cast<double2 *>(c + b) = double2{cv[a][b] - acc[a][b], cv[a][b + 1] - acc[a][b + 1]};
-        } else {
-#pragma unroll
-            for (int b = 0; b < 16; ++b)
-                if (col0 + b < n) c[b] = cv[a][b] - acc[a][b];
-        }
-    }
+// 16-byte accesses need 16-byte aligned rows and offsets; the direct-to-LDS kernel also whole K steps
+template <typename T>
+static void gemm_launch(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const T *A, int64_t lda, int64_t sA, const T *B,
+                        int64_t ldb, int64_t sB, T *C, int64_t ldc, int64_t sC, int batch)
+{
+    const int64_t ntiles = ((m + GB_M - 1) / GB_M) * ((n + GB_N - 1) / GB_N);
+    const dim3 grid((unsigned)((ntiles + GB_XCD - 1) / GB_XCD * GB_XCD), (unsigned)batch);
+    const int vec = (((uintptr_t)A | (uintptr_t)B) & 15) == 0 && (lda * sizeof(T)) % 16 == 0 && (ldb * sizeof(T)) % 16 == 0 &&
+                    (sA * sizeof(T)) % 16 == 0 && (sB * sizeof(T)) % 16 == 0;
+    ProfScope ps(ctx, sizeof(T) == 8 ? "gemm_f64" : "gemm_f32");
+    if (vec && k % Gm<T>::KS == 0)
+        hipLaunchKernelGGL(k_gemm_sub<T>, grid, dim3(GB_THREADS), 0, ctx->stream, m, n, k, A, lda, B, ldb, C, ldc, sA, sB, sC);
+    else
+        hipLaunchKernelGGL(k_gemm_sub_reg<T>, grid, dim3(GB_THREADS), 0, ctx->stream, m, n, k, A, lda, B, ldb, C, ldc, sA, sB,
+                           sC, vec);
 }
 
 template <typename T>
@@ -356,18 +454,7 @@ static int gemm_sub(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const T *A, in
                     T *C, int64_t ldc)
 {
     if (m <= 0 || n <= 0 || k <= 0) return FP_OK;
-    const int64_t ntiles = ((m + GB_M - 1) / GB_M) * ((n + GB_N - 1) / GB_N);
-    const int64_t grid = (ntiles + GB_XCD - 1) / GB_XCD * GB_XCD;
-    // 16-byte loads need 16-byte aligned rows and offsets
-    const int vec = (((uintptr_t)A | (uintptr_t)B) & 15) == 0 && (lda * sizeof(T)) % 16 == 0 &&
-                    (ldb * sizeof(T)) % 16 == 0;
-    ProfScope ps(ctx, sizeof(T) == 8 ? "gemm_f64" : "gemm_f32");
-    if constexpr (sizeof(T) == 8)
-        hipLaunchKernelGGL(k_gemm_sub_f64, dim3((unsigned)grid), dim3(256), 0, ctx->stream, m, n, k,
-                           (const double *)A, lda, (const double *)B, ldb, (double *)C, ldc, vec);
-    else
-        hipLaunchKernelGGL(k_gemm_sub<T>, dim3((unsigned)grid), dim3(256), 0, ctx->stream, m, n, k, A, lda, B, ldb,
-                           C, ldc, vec);
+    gemm_launch<T>(ctx, m, n, k, A, lda, 0, B, ldb, 0, C, ldc, 0, 1);
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;
 }
@@ -386,13 +473,7 @@ int fp_gemm_sub_batched_f32(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const 
 {
     if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return FP_OK;
     if (batch > 65535) return fp_fail(ctx, FP_ERR_UNSUPPORTED, "batched gemm: too many products");
-    const int64_t ntiles = ((m + GB_M - 1) / GB_M) * ((n + GB_N - 1) / GB_N);
-    const int64_t grid = (ntiles + GB_XCD - 1) / GB_XCD * GB_XCD;
-    const int vec = (((uintptr_t)A | (uintptr_t)B) & 15) == 0 && (lda * 4) % 16 == 0 && (ldb * 4) % 16 == 0 &&
-                    (sA * 4) % 16 == 0 && (sB * 4) % 16 == 0;
-    ProfScope ps(ctx, "gemm_f32");
-    hipLaunchKernelGGL(k_gemm_sub<float>, dim3((unsigned)grid, (unsigned)batch), dim3(256), 0, ctx->stream, m, n, k,
-                       A, lda, B, ldb, C, ldc, vec, sA, sB, sC);
+    gemm_launch<float>(ctx, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, batch);
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;
 }
