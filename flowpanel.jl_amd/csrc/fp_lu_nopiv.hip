@@ -12,11 +12,11 @@
 //
 //   per 256-column outer block:
 //     k_lu_first   its first 64 x 64 diagonal block, with the explicit inverses of
-//                  L11 and U11, and the U tiles of that block row;
+//                  L11 and U11;
 //     k_lu_step    (four times) L21 = A21 U11^-1 and the update of the outer
 //                  block's columns, one workgroup per 64 rows; the first of them
 //                  factors the next diagonal block;
-//     k_lu_urow    the U rows right of the outer block (blocked substitution);
+//     k_lu_urow    the U rows, inside the outer block and right of it (blocked substitution);
 //     fp_gemm_sub  the rank-256 trailing update.
 //
 // A x = b becomes  A_r y = U^T b,  x = V y.  A depth-2 butterfly couples only
@@ -39,6 +39,7 @@ constexpr int NPB = 64;          // block of the no-pivot LU
 constexpr int NIN = 4;           // blocks per outer block
 constexpr int NOB = NIN * NPB;   // outer block: columns per trailing update
 constexpr int UW = 32;           // columns per workgroup of the U rows
+constexpr int LT = 512;          // threads: two waves a SIMD, one's LDS reads behind the other's products
 constexpr int TBIG = 512;        // rows of the diagonal-block inverses the triangular solves use
 
 __device__ __forceinline__ float bcast(float v, int lane)
@@ -74,8 +75,16 @@ template <> struct Lu<float> {
     // accumulator element e of a 16 x 16 tile
     static __device__ __forceinline__ int row(int lane, int e) { return 4 * (lane >> 4) + e; }
     static __device__ __forceinline__ int col(int lane, int) { return lane & 15; }
-    static __device__ __forceinline__ float div(float a, float b) { return a / b; }
-    static __device__ __forceinline__ bool bad(float p) { return !(fabsf(p) > 0.f) || !(fabsf(p) <= 3.4e38f); }
+    // reciprocal refined once, quotient corrected once (the IEEE sequence switches the denormal mode and
+    // is twice as long; the chain of 64 pivots waits for it)
+    static __device__ __forceinline__ float div(float a, float b)
+    {
+        float r = __builtin_amdgcn_rcpf(b);
+        r = fmaf(r, fmaf(-b, r, 1.f), r);
+        const float q = a * r;
+        return fmaf(fmaf(-b, q, a), r, q);
+    }
+    static __device__ __forceinline__ bool bad(float p) { return !(fabsf(p) > 1e-37f) || !(fabsf(p) <= 1e37f); }
 };
 template <> struct Lu<double> {
     static constexpr int LDA = 68, LDB = 68, LDX = 36, V = 2;
@@ -124,10 +133,10 @@ template <typename T, int NT> __device__ __forceinline__ void zero(typename Lu<T
     for (int t = 0; t < NT; ++t) acc[t] = typename Lu<T>::v4{0, 0, 0, 0};
 }
 
-// A 64 x W tile through registers: thread tid holds W / 4 values, 16 bytes of a row at a time.
+// A 64 x W tile through registers, 16 bytes of a row per thread at a time.
 // Entries outside rows < tr, cols < tc are zero; 16-byte accesses where the row piece is inside.
 template <typename T, int W> struct Tile {
-    static constexpr int V = Lu<T>::V, PER_ROW = W / V, STEP = 256 / PER_ROW, N = NPB / STEP;
+    static constexpr int V = Lu<T>::V, PER_ROW = W / V, STEP = LT / PER_ROW, N = NPB / STEP;
     typedef typename Lu<T>::vec vec;
     vec v[N];
     __device__ __forceinline__ void load(const T *p, int64_t ld, int tr, int tc, int tid)
@@ -150,7 +159,37 @@ template <typename T, int W> struct Tile {
 #pragma unroll
         for (int q = 0; q < N; ++q) *reinterpret_cast<vec *>(s + (r0 + q * STEP) * lds + c) = v[q];
     }
+    // an LDS tile to memory (rows < tr, cols < tc), times sign
+    static __device__ __forceinline__ void store(const T *s, int lds, T *p, int64_t ld, int tr, int tc, T sign, int tid)
+    {
+        const int c = (tid % PER_ROW) * V, r0 = tid / PER_ROW;
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const int r = r0 + q * STEP;
+            vec w = *reinterpret_cast<const vec *>(s + r * lds + c);
+            w = w * sign;
+            if (r < tr && c + V <= tc) {
+                *reinterpret_cast<vec *>(p + (int64_t)r * ld + c) = w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < V; ++e)
+                    if (r < tr && c + e < tc) p[(int64_t)r * ld + c + e] = w[e];
+            }
+        }
+    }
 };
+
+// The 64 x 64 product of a step: wave w takes rows 16 (w % 4) and columns 32 (w / 4).
+template <typename T> __device__ __forceinline__ void mma64(const T *P, const T *Q, int lane, int wave, typename Lu<T>::v4 (&acc)[2])
+{
+    zero<T, 2>(acc);
+    mma<T, 2>(P + 16 * (wave & 3) * Lu<T>::LDA, Lu<T>::LDA, Q + 32 * (wave >> 2), Lu<T>::LDB, NPB, lane, acc);
+}
+template <typename T> __device__ __forceinline__ int arow(int lane, int wave, int e) { return 16 * (wave & 3) + Lu<T>::row(lane, e); }
+template <typename T> __device__ __forceinline__ int acol(int lane, int wave, int q, int e)
+{
+    return 32 * (wave >> 2) + 16 * q + Lu<T>::col(lane, e);
+}
 
 // LDS of the step kernels: three 64 x 64 tiles and two 32 x 32 staging tiles
 template <typename T> struct StepLds {
@@ -160,8 +199,34 @@ template <typename T> struct StepLds {
     T tmp[2 * 32 * 36];
 };
 
+// Substitution of 16 values per lane with a 16 x 16 triangle in LDS (row stride LDA): forward with the unit
+// lower one, or (UP) backward with the upper one and the reciprocals rd of its diagonal, one per lane.
+// Column by column: the updates by one unknown are independent of each other, and the next column is read
+// meanwhile (all lanes the same word; the barrier keeps the compiler from reading all 120 ahead, which
+// spills in FP64).
+template <typename T, bool UP> __device__ __forceinline__ void subst16(T (&x)[16], const T *t, T rd)
+{
+    constexpr int LDA = Lu<T>::LDA;
+    T l[2][16];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) l[0][i] = UP ? t[(15 - i) * LDA + 15] : t[i * LDA];
+    static_for<0, 16>([&](auto Q) {
+        constexpr int q = decltype(Q)::v, xq = UP ? 15 - q : q;
+#pragma unroll
+        for (int i = q + 2; i < 16; ++i)
+            l[(q + 1) & 1][i] = UP ? t[(15 - i) * LDA + 14 - q] : t[i * LDA + q + 1];
+        if (UP) x[xq] *= bcast(rd, xq);
+#pragma unroll
+        for (int i = q + 1; i < 16; ++i) {
+            const int xi = UP ? 15 - i : i;
+            x[xi] = fma(-l[q & 1][i], x[xq], x[xi]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+
 // LU without pivoting of the 64 x 64 block D in LDS, in place, and the explicit inverses Li = L11^-1
-// (unit lower) and Ui = U11^-1, by 256 threads.  Four sub-panels of 16 columns: wave 0 factors the
+// (unit lower) and Ui = U11^-1, by 512 threads.  Four sub-panels of 16 columns: wave 0 factors the
 // sub-panel with one row per lane in registers (row j broadcast by v_readlane, 120 broadcast-and-FMA
 // steps instead of the 2,016 of the whole block at once), a lane per column substitutes the 16 rows
 // right of it, and the waves update the rest with 16 x 16 MFMA tiles.  The inverses grow the same
@@ -174,7 +239,7 @@ __device__ __forceinline__ bool lu_diag64(StepLds<T> &s, int tid)
     typedef typename Lu<T>::v4 v4;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     T *D = s.D, *Li = s.P, *Ui = s.Q;
-    for (int e = tid; e < NPB * NPB; e += 256) {
+    for (int e = tid; e < NPB * NPB; e += LT) {
         Li[(e >> 6) * LDA + (e & 63)] = T(0);
         Ui[(e >> 6) * LDB + (e & 63)] = T(0);
     }
@@ -215,16 +280,13 @@ __device__ __forceinline__ bool lu_diag64(StepLds<T> &s, int tid)
             T *col = D + c0 * LDA + c0 + 16 + lane;
 #pragma unroll
             for (int i = 0; i < 16; ++i) x[i] = col[i * LDA];
-#pragma unroll
-            for (int i = 1; i < 16; ++i)
-#pragma unroll
-                for (int q = 0; q < i; ++q) x[i] = fma(-D[(c0 + i) * LDA + c0 + q], x[q], x[i]);
+            subst16<T, false>(x, D + c0 * (LDA + 1), T(1));
 #pragma unroll
             for (int i = 1; i < 16; ++i) col[i * LDA] = x[i];
         }
         __syncthreads();
         const int m = 3 - p;
-        for (int q = wave; q < m * m; q += 4) {
+        for (int q = wave; q < m * m; q += LT / 64) {
             const int r0 = c0 + 16 + 16 * (q / m), k0 = c0 + 16 + 16 * (q % m);
             v4 acc[1];
             zero<T, 1>(acc);
@@ -234,76 +296,68 @@ __device__ __forceinline__ bool lu_diag64(StepLds<T> &s, int tid)
         }
         __syncthreads();
     }
+    const int isu = wave >> 2, h = wave & 1, t2 = (wave >> 1) & 1;   // waves 0-3 for L, 4-7 for U
     {
-        // 16 x 16 diagonal inverses, wave = block: lanes 0-15 the columns of L^-1, lanes 16-31 those of
-        // U^-1 with rows and columns reversed, which makes it the same forward substitution
-        const int c0 = 16 * wave, up = (lane >> 4) & 1, col = lane & 15;
-        const T rd = Lu<T>::div(T(1), D[(c0 + col) * (LDA + 1)]);
-        const T *base = up ? D + (c0 + 15) * (LDA + 1) : D + c0 * (LDA + 1);
-        const int sg = up ? -1 : 1;
+        // 16 x 16 diagonal inverses, a column per lane
+        const int c0 = 16 * (wave & 3), col = lane & 15;
+        const T *t = D + c0 * (LDA + 1);
         T y[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            T v = i == col ? T(1) : T(0);
-#pragma unroll
-            for (int q = 0; q < i; ++q) v = fma(-base[sg * (i * LDA + q)], y[q], v);
-            const T d = bcast(rd, 15 - i);
-            y[i] = up ? v * d : v;
-        }
-        if (lane < 32) {
-            T *dst = up ? Ui + (c0 + 15) * LDB + c0 + 15 - col : Li + c0 * LDA + c0 + col;
-            const int st = up ? -LDB : LDA;
+        for (int i = 0; i < 16; ++i) y[i] = i == col ? T(1) : T(0);
+        if (!isu) subst16<T, false>(y, t, T(1));
+        else subst16<T, true>(y, t, Lu<T>::div(T(1), t[col * (LDA + 1)]));
+        T *dst = isu ? Ui + c0 * (LDB + 1) + col : Li + c0 * (LDA + 1) + col;
+        const int st = isu ? LDB : LDA;
+        if (lane < 16)
 #pragma unroll
             for (int i = 0; i < 16; ++i) dst[i * st] = y[i];
-        }
     }
     __syncthreads();
-    const int isu = wave >> 1, h = wave & 1;
     T *tw = s.tmp + isu * 32 * LDT;
     {
-        // 16 -> 32: wave = (L or U, pair h)
+        // 16 -> 32: pair h (two waves of the four)
         const int b0 = 32 * h, b1 = b0 + 16;
-        v4 acc[1];
-        zero<T, 1>(acc);
-        if (!isu) mma<T, 1>(D + b1 * LDA + b0, LDA, Li + b0 * (LDA + 1), LDA, 16, lane, acc);
-        else mma<T, 1>(D + b0 * LDA + b1, LDA, Ui + b1 * (LDB + 1), LDB, 16, lane, acc);
         T *th = tw + 16 * h * LDT;
+        v4 acc[1];
+        if (t2 == 0) {
+            zero<T, 1>(acc);
+            if (!isu) mma<T, 1>(D + b1 * LDA + b0, LDA, Li + b0 * (LDA + 1), LDA, 16, lane, acc);
+            else mma<T, 1>(D + b0 * LDA + b1, LDA, Ui + b1 * (LDB + 1), LDB, 16, lane, acc);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) th[Lu<T>::row(lane, e) * LDT + Lu<T>::col(lane, e)] = acc[0][e];
+            for (int e = 0; e < 4; ++e) th[Lu<T>::row(lane, e) * LDT + Lu<T>::col(lane, e)] = acc[0][e];
+        }
         __syncthreads();
-        zero<T, 1>(acc);
-        if (!isu) mma<T, 1>(Li + b1 * (LDA + 1), LDA, th, LDT, 16, lane, acc);
-        else mma<T, 1>(Ui + b0 * (LDB + 1), LDB, th, LDT, 16, lane, acc);
+        if (t2 == 0) {
+            zero<T, 1>(acc);
+            if (!isu) mma<T, 1>(Li + b1 * (LDA + 1), LDA, th, LDT, 16, lane, acc);
+            else mma<T, 1>(Ui + b0 * (LDB + 1), LDB, th, LDT, 16, lane, acc);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int r = Lu<T>::row(lane, e), c = Lu<T>::col(lane, e);
-            if (!isu) Li[(b1 + r) * LDA + b0 + c] = -acc[0][e];
-            else Ui[(b0 + r) * LDB + b1 + c] = -acc[0][e];
+            for (int e = 0; e < 4; ++e) {
+                const int r = Lu<T>::row(lane, e), c = Lu<T>::col(lane, e);
+                if (!isu) Li[(b1 + r) * LDA + b0 + c] = -acc[0][e];
+                else Ui[(b0 + r) * LDB + b1 + c] = -acc[0][e];
+            }
         }
         __syncthreads();
     }
     {
-        // 32 -> 64: wave = (L or U, 16 rows of the 32 x 32 block)
-        v4 acc[2];
-        zero<T, 2>(acc);
-        if (!isu) mma<T, 2>(D + (32 + 16 * h) * LDA, LDA, Li, LDA, 32, lane, acc);
-        else mma<T, 2>(D + 16 * h * LDA + 32, LDA, Ui + 32 * (LDB + 1), LDB, 32, lane, acc);
+        // 32 -> 64: wave = (L or U, 16 rows, 16 columns of the 32 x 32 block)
+        v4 acc[1];
+        zero<T, 1>(acc);
+        if (!isu) mma<T, 1>(D + (32 + 16 * h) * LDA, LDA, Li + 16 * t2, LDA, 32, lane, acc);
+        else mma<T, 1>(D + 16 * h * LDA + 32, LDA, Ui + 32 * (LDB + 1) + 16 * t2, LDB, 32, lane, acc);
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) tw[(16 * h + Lu<T>::row(lane, e)) * LDT + 16 * t + Lu<T>::col(lane, e)] = acc[t][e];
+        for (int e = 0; e < 4; ++e) tw[(16 * h + Lu<T>::row(lane, e)) * LDT + 16 * t2 + Lu<T>::col(lane, e)] = acc[0][e];
         __syncthreads();
-        zero<T, 2>(acc);
-        if (!isu) mma<T, 2>(Li + (32 + 16 * h) * LDA + 32, LDA, tw, LDT, 32, lane, acc);
-        else mma<T, 2>(Ui + 16 * h * LDB, LDB, tw, LDT, 32, lane, acc);
+        zero<T, 1>(acc);
+        if (!isu) mma<T, 1>(Li + (32 + 16 * h) * LDA + 32, LDA, tw + 16 * t2, LDT, 32, lane, acc);
+        else mma<T, 1>(Ui + 16 * h * LDB, LDB, tw + 16 * t2, LDT, 32, lane, acc);
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = 16 * h + Lu<T>::row(lane, e), c = 16 * t + Lu<T>::col(lane, e);
-                if (!isu) Li[(32 + r) * LDA + c] = -acc[t][e];
-                else Ui[r * LDB + 32 + c] = -acc[t][e];
-            }
+        for (int e = 0; e < 4; ++e) {
+            const int r = 16 * h + Lu<T>::row(lane, e), c = 16 * t2 + Lu<T>::col(lane, e);
+            if (!isu) Li[(32 + r) * LDA + c] = -acc[0][e];
+            else Ui[r * LDB + 32 + c] = -acc[0][e];
+        }
     }
     __syncthreads();
     return bad;
@@ -326,51 +380,24 @@ template <typename T> __device__ __forceinline__ T *dent(T *D, int64_t r, int64_
     return D + (r / TBIG) * ((int64_t)TBIG * TBIG) + (r % TBIG) * TBIG + c % TBIG;
 }
 
-// The diagonal block at (c, c), held in s.D (identity outside its bs rows), of the outer block that
-// ends at kend: factor, store the factors and inverses, then the U tiles of its block row
-// inside the outer block, U = L11^-1 A.
-template <typename T>
-__device__ __forceinline__ void lu_diag_row(const LuMat<T> &m, int64_t c, int64_t kend, StepLds<T> &s, int tid)
+// The diagonal block at (c, c), held in s.D (identity outside its bs rows): factor, store the factors and
+// their inverses.
+template <typename T> __device__ __forceinline__ void lu_diag(const LuMat<T> &m, int64_t c, StepLds<T> &s, int tid)
 {
     constexpr int LDA = Lu<T>::LDA, LDB = Lu<T>::LDB;
-    const int lane = tid & 63, wave = tid >> 6;
+    typedef Tile<T, NPB> Tl;
     const int bs = (int)min((int64_t)NPB, m.n - c);
     const bool bad = lu_diag64<T>(s, tid);
     if (bad && tid == 0) atomicCAS(m.info, 0, (int)(c + 1));
-    T *Linv = dent(m.DL, c, c), *Uinv = dent(m.DU, c, c);
-    for (int e = tid; e < NPB * NPB; e += 256) {
-        const int r = e >> 6, q = e & 63;
-        const T li = s.P[r * LDA + q], ui = s.Q[r * LDB + q];
-        Linv[r * TBIG + q] = li;
-        Uinv[r * TBIG + q] = ui;
-        if (r < bs && q < bs) {
-            m.A[(c + r) * m.ld + c + q] = s.D[r * LDA + q];
-            if (m.YL) m.YL[(c + r) * m.ld + c + q] = -li;
-            if (m.YU) m.YU[(c + r) * m.ld + c + q] = -ui;
-        }
-    }
-    for (int64_t j0 = c + NPB; j0 < kend; j0 += NPB) {
-        const int tc = (int)min((int64_t)NPB, kend - j0);
-        Tile<T, NPB> rq;
-        rq.load(m.A + c * m.ld + j0, m.ld, bs, tc, tid);
-        __syncthreads();
-        rq.put(s.Q, LDB, tid);
-        __syncthreads();
-        typename Lu<T>::v4 acc[4];
-        zero<T, 4>(acc);
-        mma<T, 4>(s.P + 16 * wave * LDA, LDA, s.Q, LDB, NPB, lane, acc);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
-                if (r < bs && cc < tc) m.A[(c + r) * m.ld + j0 + cc] = acc[q][e];
-            }
-    }
+    Tl::store(s.D, LDA, m.A + c * m.ld + c, m.ld, bs, bs, T(1), tid);
+    Tl::store(s.P, LDA, dent(m.DL, c, c), TBIG, NPB, NPB, T(1), tid);
+    Tl::store(s.Q, LDB, dent(m.DU, c, c), TBIG, NPB, NPB, T(1), tid);
+    if (m.YL) Tl::store(s.P, LDA, m.YL + c * m.ld + c, m.ld, bs, bs, T(-1), tid);
+    if (m.YU) Tl::store(s.Q, LDB, m.YU + c * m.ld + c, m.ld, bs, bs, T(-1), tid);
 }
 
-// First diagonal block of the outer block [k, kend) and its U tiles; one workgroup.
-template <typename T> __device__ __forceinline__ void lu_first_dev(const LuMat<T> &m, int64_t k, int64_t kend, StepLds<T> &s)
+// First diagonal block of the outer block at k; one workgroup.
+template <typename T> __device__ __forceinline__ void lu_first_dev(const LuMat<T> &m, int64_t k, StepLds<T> &s)
 {
     const int tid = threadIdx.x;
     const int bs = (int)min((int64_t)NPB, m.n - k);
@@ -380,20 +407,25 @@ template <typename T> __device__ __forceinline__ void lu_first_dev(const LuMat<T
     __syncthreads();
     if (tid < NPB && tid >= bs) s.D[tid * (Lu<T>::LDA + 1)] = T(1);
     __syncthreads();
-    lu_diag_row<T>(m, k, kend, s, tid);
+    lu_diag<T>(m, k, s, tid);
 }
 
 // Inner step t of the outer block [k, kend), c = k + 64 t, on the 64 rows below number b: the strip's
-// L tile A21 := A21 U11^-1, then A22 -= L21 U12 for the outer block's columns right of it, the U12
-// tiles being final already.  Workgroup 0 owns the next diagonal block: it goes on to factor it, so
-// that a step is one launch and the other strips run beside the next block's pivot chain.  All
-// products are 64 x 64 x 64 from LDS, the next tile loaded into registers meanwhile.
+// L tile A21 := A21 U11^-1, and A22 -= W A12 for the outer block's columns right of it, W = L21 L11^-1
+// and A12 the block row as it stands (W A12 = L21 U12: the chain from one diagonal block to the next does
+// not wait for U12, which lu_urow_dev forms when the outer block is done).  Workgroup 0 owns the next
+// diagonal block: it goes on to factor it, so that a step is one launch and the other strips run beside
+// the next block's pivot chain.  All products are 64 x 64 x 64 from LDS, the next tile loaded into
+// registers meanwhile.  Workgroup 0 bounds it.  With the three U12 tiles in that workgroup and four waves
+// (cycles of the diagonal block, FP32 and FP64: pivots 14,700 and 20,700, 16-row substitutions 7,500 and
+// 8,900, inverses 8,000 and 12,500, U12 19,100 and 36,200, of 61,500 and 94,800) the first block took 26 and
+// 39 us and 4,800 unknowns 3.2 and 6.3 ms; with eight waves and U12 elsewhere 14 and 22 us, 2.8 and 5.2 ms.
 template <typename T>
 __device__ __forceinline__ void lu_step_dev(const LuMat<T> &m, int64_t k, int t, int64_t kend, int b, StepLds<T> &s)
 {
     constexpr int LDA = Lu<T>::LDA, LDB = Lu<T>::LDB;
     typedef typename Lu<T>::v4 v4;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t c = k + (int64_t)NPB * t, ld = m.ld, off = c + NPB + (int64_t)NPB * b;
     const int tr = (int)min((int64_t)NPB, m.n - off);
     T *A = m.A;
@@ -404,39 +436,54 @@ __device__ __forceinline__ void lu_step_dev(const LuMat<T> &m, int64_t k, int t,
     rq.put(s.Q, LDB, tid);
     __syncthreads();
     int64_t j0 = c + NPB;
-    if (j0 < kend) rq.load(A + c * ld + j0, ld, NPB, (int)min((int64_t)NPB, kend - j0), tid);
-    v4 acc[4];
-    zero<T, 4>(acc);
-    mma<T, 4>(s.P + 16 * wave * LDA, LDA, s.Q, LDB, NPB, lane, acc);
-    __syncthreads();
+    const bool more = j0 < kend;
+    if (more) {
+        ra.load(dent(m.DL, c, c), TBIG, NPB, NPB, tid);
+        rq.load(A + c * ld + j0, ld, NPB, (int)min((int64_t)NPB, kend - j0), tid);
+    }
+    v4 acc[2];
+    mma64<T>(s.P, s.Q, lane, wave, acc);
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
-            s.P[r * LDA + cc] = acc[q][e];
+            const int r = arow<T>(lane, wave, e), cc = acol<T>(lane, wave, q, e);
             if (r < tr) A[(off + r) * ld + c + cc] = acc[q][e];
         }
+    if (!more) return;   // the outer block's last step: no columns right of it
+    // W = L21 L11^-1
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s.P[arow<T>(lane, wave, e) * LDA + acol<T>(lane, wave, q, e)] = acc[q][e];
+    ra.put(s.Q, LDB, tid);
+    __syncthreads();
+    mma64<T>(s.P, s.Q, lane, wave, acc);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s.P[arow<T>(lane, wave, e) * LDA + acol<T>(lane, wave, q, e)] = acc[q][e];
     for (; j0 < kend; j0 += NPB) {
         const int tc = (int)min((int64_t)NPB, kend - j0);
-        T cv[4][4];
+        T cv[2][4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
+                const int r = arow<T>(lane, wave, e), cc = acol<T>(lane, wave, q, e);
                 cv[q][e] = A[(off + min(r, tr - 1)) * ld + j0 + min(cc, tc - 1)];
             }
         rq.put(s.Q, LDB, tid);
         __syncthreads();
         if (j0 + NPB < kend) rq.load(A + c * ld + j0 + NPB, ld, NPB, (int)min((int64_t)NPB, kend - j0 - NPB), tid);
-        zero<T, 4>(acc);
-        mma<T, 4>(s.P + 16 * wave * LDA, LDA, s.Q, LDB, NPB, lane, acc);
+        mma64<T>(s.P, s.Q, lane, wave, acc);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
+                const int r = arow<T>(lane, wave, e), cc = acol<T>(lane, wave, q, e);
                 const bool in = r < tr && cc < tc;
                 const T v = cv[q][e] - acc[q][e];
                 if (in) A[(off + r) * ld + j0 + cc] = v;
@@ -444,87 +491,178 @@ __device__ __forceinline__ void lu_step_dev(const LuMat<T> &m, int64_t k, int t,
             }
         __syncthreads();
     }
-    if (b == 0 && c + NPB < kend) lu_diag_row<T>(m, c + NPB, kend, s, tid);
+    if (b == 0) lu_diag<T>(m, c + NPB, s, tid);
 }
 
-// U rows of the outer block [k, k + NOB) in the UW columns from kend + UW b on: blocked forward
-// substitution U_t = L_tt^-1 (A_t - sum_{s<t} L_ts U_s) with the solved rows kept in LDS, one launch
-// for the four block rows (ten 64 x 64 x 32 products; four pairs of launches before).
+// The part of the previous outer block's trailing update that this outer block's launches carry, C -= L U in
+// 64 x 64 tiles (L in columns, U in rows [k - NOB, k)): columns from j0 on, `ntc` tile columns of them, rows
+// from k on; `tile0` is the launch's first tile.
+struct LuRest {
+    int64_t j0;
+    int ntc, tile0;
+};
+// The tile at (i0, j0).  The launches that factor the next 256 columns are a chain of single workgroups and at
+// most one workgroup per 64 rows: these tiles run on the compute units that they leave idle.  Double-buffered
+// through registers, two (FP32) or one (FP64) workgroups a compute unit.  diag: the tile is the diagonal
+// block at k, which stays in s.D for lu_diag.
+template <typename T>
+__device__ __forceinline__ void lu_rest_dev(const LuMat<T> &m, int64_t k, int64_t i0, int64_t j0, StepLds<T> &s, bool diag)
+{
+    constexpr int LDA = Lu<T>::LDA, LDB = Lu<T>::LDB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t ld = m.ld;
+    const int tr = (int)min((int64_t)NPB, m.n - i0), tc = (int)min((int64_t)NPB, m.n - j0);
+    const T *L = m.A + i0 * ld + k - NOB, *U = m.A + (k - NOB) * ld + j0;
+    T *C = m.A + i0 * ld + j0;
+    Tile<T, NPB> ra, rq;
+    ra.load(L, ld, tr, NPB, tid);
+    rq.load(U, ld, NPB, tc, tid);
+    T cv[2][4];
+    typename Lu<T>::v4 acc[2];
+    zero<T, 2>(acc);
+    for (int q = 0; q < NIN; ++q) {
+        if (q) __syncthreads();
+        ra.put(s.P, LDA, tid);
+        rq.put(s.Q, LDB, tid);
+        __syncthreads();
+        if (q + 1 < NIN) {
+            ra.load(L + NPB * (q + 1), ld, tr, NPB, tid);
+            rq.load(U + (int64_t)NPB * (q + 1) * ld, ld, NPB, tc, tid);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    cv[t][e] = C[min(arow<T>(lane, wave, e), tr - 1) * ld + min(acol<T>(lane, wave, t, e), tc - 1)];
+        }
+        mma<T, 2>(s.P + 16 * (wave & 3) * LDA, LDA, s.Q + 32 * (wave >> 2), LDB, NPB, lane, acc);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = arow<T>(lane, wave, e), j = acol<T>(lane, wave, t, e);
+            const bool in = i < tr && j < tc;
+            const T v = cv[t][e] - acc[t][e];
+            if (diag) s.D[i * LDA + j] = in ? v : (i == j ? T(1) : T(0));
+            else if (in) C[i * ld + j] = v;
+        }
+    if (diag) __syncthreads();
+}
+template <typename T> __device__ __forceinline__ void lu_rest_dev(const LuMat<T> &m, int64_t k, const LuRest &r, int x, StepLds<T> &s)
+{
+    x += r.tile0;
+    lu_rest_dev<T>(m, k, k + (int64_t)NPB * (x / r.ntc), r.j0 + (int64_t)NPB * (x % r.ntc), s, false);
+}
+
+// U rows of the outer block [k, kend).  Workgroups b < nr: the UW columns from kend + UW b on, by blocked
+// forward substitution U_t = L_tt^-1 (A_t - sum_{s<t} L_ts U_s) with the solved rows kept in LDS (ten
+// 64 x 64 x 32 products).  The others: a tile right of a diagonal block inside the outer block,
+// U = L_tt^-1 A, where A is what lu_step_dev left (UW columns each, lu_inner of them).
+__host__ __device__ inline int lu_inner(int64_t cols)   // tiles of UW columns inside an outer block of `cols` columns
+{
+    int n = 0;
+    for (int t = 0; t + 1 < NIN; ++t) {
+        const int64_t c = cols - (int64_t)NPB * (t + 1);
+        if (c > 0) n += (int)((c + UW - 1) / UW);
+    }
+    return n;
+}
 template <typename T> struct UrowLds {
     T P[NPB * Lu<T>::LDA];
     T X[NIN][NPB * Lu<T>::LDX];
     T R[NPB * Lu<T>::LDX];
 };
 template <typename T>
-__device__ __forceinline__ void lu_urow_dev(const LuMat<T> &m, int64_t k, int64_t kend, int b, UrowLds<T> &s)
+__device__ __forceinline__ void lu_urow_dev(const LuMat<T> &m, int64_t k, int64_t kend, int b, int nr, UrowLds<T> &s)
 {
-    constexpr int LDA = Lu<T>::LDA, LDX = Lu<T>::LDX, NT = UW / 16;
+    constexpr int LDA = Lu<T>::LDA, LDX = Lu<T>::LDX;
     typedef typename Lu<T>::v4 v4;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t ld = m.ld, j0 = kend + (int64_t)UW * b;
-    const int tc = (int)min((int64_t)UW, m.n - j0);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = 16 * (wave & 3), wc = 16 * (wave >> 2);   // 64 x 32: a 16 x 16 tile per wave
+    const int64_t ld = m.ld;
     T *A = m.A;
-    // left operands in order: L_t0 .. L_t,t-1, then L_tt^-1
+    int t0 = 0, t1 = NIN;
+    int64_t j0 = kend + (int64_t)UW * b, jend = m.n;
+    if (b >= nr) {
+        int x = b - nr;
+        jend = kend;
+        for (t0 = 0;; ++t0) {
+            j0 = k + (int64_t)NPB * (t0 + 1);
+            const int w = (int)((kend - j0 + UW - 1) / UW);
+            if (x < w) break;
+            x -= w;
+        }
+        j0 += (int64_t)UW * x;
+        t1 = t0 + 1;
+    }
+    const int tc = (int)min((int64_t)UW, jend - j0), first = b < nr ? 0 : t0;   // L tiles from block `first` on
+    // left operands in order: L_t,first .. L_t,t-1, then L_tt^-1
     Tile<T, NPB> rp;
-    rp.load(dent(m.DL, k, k), TBIG, NPB, NPB, tid);
-    for (int t = 0; t < NIN; ++t) {
+    rp.load(dent(m.DL, k + (int64_t)NPB * t0, k + (int64_t)NPB * t0), TBIG, NPB, NPB, tid);
+    for (int t = t0; t < t1; ++t) {
         const int64_t c = k + (int64_t)NPB * t;
-        T cv[NT][4];
+        T cv[4];
 #pragma unroll
-        for (int q = 0; q < NT; ++q)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
-                cv[q][e] = A[(c + r) * ld + j0 + min(cc, tc - 1)];
-            }
-        v4 acc[NT];
-        zero<T, NT>(acc);
-        for (int q = 0; q < t; ++q) {
+        for (int e = 0; e < 4; ++e)
+            cv[e] = A[(c + wr + Lu<T>::row(lane, e)) * ld + j0 + min(wc + Lu<T>::col(lane, e), tc - 1)];
+        v4 acc[1];
+        zero<T, 1>(acc);
+        for (int q = first; q < t; ++q) {
             __syncthreads();
             rp.put(s.P, LDA, tid);
             __syncthreads();
             if (q + 1 < t) rp.load(A + c * ld + k + NPB * (q + 1), ld, NPB, NPB, tid);
             else rp.load(dent(m.DL, c, c), TBIG, NPB, NPB, tid);
-            mma<T, NT>(s.P + 16 * wave * LDA, LDA, s.X[q], LDX, NPB, lane, acc);
+            mma<T, 1>(s.P + wr * LDA, LDA, s.X[q] + wc, LDX, NPB, lane, acc);
         }
         __syncthreads();
         rp.put(s.P, LDA, tid);
 #pragma unroll
-        for (int q = 0; q < NT; ++q)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                s.R[(16 * wave + Lu<T>::row(lane, e)) * LDX + 16 * q + Lu<T>::col(lane, e)] = cv[q][e] - acc[q][e];
+        for (int e = 0; e < 4; ++e) s.R[(wr + Lu<T>::row(lane, e)) * LDX + wc + Lu<T>::col(lane, e)] = cv[e] - acc[0][e];
         __syncthreads();
-        if (t + 1 < NIN) rp.load(A + (c + NPB) * ld + k, ld, NPB, NPB, tid);
-        zero<T, NT>(acc);
-        mma<T, NT>(s.P + 16 * wave * LDA, LDA, s.R, LDX, NPB, lane, acc);
+        if (t + 1 < t1) rp.load(A + (c + NPB) * ld + k, ld, NPB, NPB, tid);
+        zero<T, 1>(acc);
+        mma<T, 1>(s.P + wr * LDA, LDA, s.R + wc, LDX, NPB, lane, acc);
 #pragma unroll
-        for (int q = 0; q < NT; ++q)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = 16 * wave + Lu<T>::row(lane, e), cc = 16 * q + Lu<T>::col(lane, e);
-                s.X[t][r * LDX + cc] = acc[q][e];
-                if (cc < tc) A[(c + r) * ld + j0 + cc] = acc[q][e];
-            }
+        for (int e = 0; e < 4; ++e) {
+            const int r = wr + Lu<T>::row(lane, e), cc = wc + Lu<T>::col(lane, e);
+            s.X[t][r * LDX + cc] = acc[0][e];
+            if (cc < tc) A[(c + r) * ld + j0 + cc] = acc[0][e];
+        }
     }
 }
 
-template <typename T> __global__ __launch_bounds__(256) void k_lu_first(LuMat<T> m, int64_t k, int64_t kend)
+template <typename T> __global__ __launch_bounds__(LT) void k_lu_first(LuMat<T> m, int64_t k)
 {
     __shared__ StepLds<T> s;
-    lu_first_dev<T>(m, k, kend, s);
+    lu_first_dev<T>(m, k, s);
 }
-
-template <typename T> __global__ __launch_bounds__(256) void k_lu_step(LuMat<T> m, int64_t k, int t, int64_t kend)
+// The previous outer block's update of the columns [k, k + 64 pc), one 64 x 64 tile per workgroup (np of them),
+// and tiles of the rest; the first one goes on to factor the diagonal block at k.
+template <typename T> __global__ __launch_bounds__(LT) void k_lu_update(LuMat<T> m, int64_t k, int pc, int np, LuRest r)
 {
     __shared__ StepLds<T> s;
-    lu_step_dev<T>(m, k, t, kend, blockIdx.x, s);
+    const int x = blockIdx.x;
+    if (x >= np) {
+        lu_rest_dev<T>(m, k, r, x - np, s);
+        return;
+    }
+    lu_rest_dev<T>(m, k, k + (int64_t)NPB * (x / pc), k + (int64_t)NPB * (x % pc), s, x == 0);
+    if (x == 0) lu_diag<T>(m, k, s, threadIdx.x);
+}
+template <typename T>
+__global__ __launch_bounds__(LT) void k_lu_step(LuMat<T> m, int64_t k, int t, int64_t kend, int strips, LuRest r)
+{
+    __shared__ StepLds<T> s;
+    if ((int)blockIdx.x < strips) lu_step_dev<T>(m, k, t, kend, blockIdx.x, s);
+    else lu_rest_dev<T>(m, k, r, blockIdx.x - strips, s);
 }
 
-template <typename T> __global__ __launch_bounds__(256) void k_lu_urow(LuMat<T> m, int64_t k, int64_t kend)
+template <typename T> __global__ __launch_bounds__(LT) void k_lu_urow(LuMat<T> m, int64_t k, int64_t kend, int nr)
 {
     __shared__ UrowLds<T> s;
-    lu_urow_dev<T>(m, k, kend, blockIdx.x, s);
+    lu_urow_dev<T>(m, k, kend, blockIdx.x, nr, s);
 }
 
 // ---- diagonal-block inverses for the triangular solves -------------------------
@@ -533,11 +671,11 @@ template <typename T> __global__ __launch_bounds__(256) void k_lu_urow(LuMat<T> 
 // the s x s block per workgroup.  Phase 0: W = L21 X11 (U: U12 X22); phase 1: X21 = -X22 W
 // (U: X12 = -X11 W).  Tiles that are zero in the triangular factor are left out.
 template <typename T>
-__global__ __launch_bounds__(256) void k_tri_merge(LuMat<T> m, T *__restrict__ W, int s, int phase)
+__global__ __launch_bounds__(LT) void k_tri_merge(LuMat<T> m, T *__restrict__ W, int s, int phase)
 {
     constexpr int LDA = Lu<T>::LDA, LDB = Lu<T>::LDB;
     __shared__ T P[NPB * LDA], Q[NPB * LDB];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nt = s / NPB, ti = blockIdx.x / nt, tj = blockIdx.x % nt, up = blockIdx.z;
     const int64_t c0 = (int64_t)2 * s * blockIdx.y, c1 = c0 + s, n = m.n;
     if (c1 >= n) return;
@@ -562,8 +700,8 @@ __global__ __launch_bounds__(256) void k_tri_merge(LuMat<T> m, T *__restrict__ W
             rq.load(W + (int64_t)NPB * kk * s + NPB * tj, s, NPB, NPB, tid);
         }
     };
-    typename Lu<T>::v4 acc[4];
-    zero<T, 4>(acc);
+    typename Lu<T>::v4 acc[2];
+    zero<T, 2>(acc);
     load(k0);
     for (int kk = k0; kk < k1; ++kk) {
         __syncthreads();
@@ -571,13 +709,13 @@ __global__ __launch_bounds__(256) void k_tri_merge(LuMat<T> m, T *__restrict__ W
         rq.put(Q, LDB, tid);
         __syncthreads();
         if (kk + 1 < k1) load(kk + 1);
-        mma<T, 4>(P + 16 * wave * LDA, LDA, Q, LDB, NPB, lane, acc);
+        mma<T, 2>(P + 16 * (wave & 3) * LDA, LDA, Q + 32 * (wave >> 2), LDB, NPB, lane, acc);
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int r = 16 * wave + Lu<T>::row(lane, e), c = 16 * q + Lu<T>::col(lane, e);
+            const int r = arow<T>(lane, wave, e), c = acol<T>(lane, wave, q, e);
             if (phase == 0) W[(int64_t)(NPB * ti + r) * s + NPB * tj + c] = acc[q][e];
             else *dent(D, r0 + r, q0 + c) = -acc[q][e];
         }
@@ -908,6 +1046,19 @@ static int64_t lu_tiles(int64_t x, int64_t w) { return x > 0 ? (x + w - 1) / w :
 // outer block and one rank-256 trailing update (a rank-64 update per inner block would read and write
 // the whole trailing matrix four times as often).  info_dev receives 1 + the first row of the diagonal
 // block whose pivot was zero or not finite (0 if none).
+//
+// That update's columns of the next outer block are brought up to date in the launch that also factors the
+// next diagonal block (k_lu_update); as much of the rest as the chain of launches has room for goes into
+// these launches as further workgroups (lu_rest_dev), which need nothing of the chain and are not needed by
+// it before the U rows; only what is left is a launch of its own (fp_gemm_sub).  SLOTS: workgroups that the
+// chip holds (two FP32, one FP64 per compute unit); FIRST, STEP: tiles per slot that the launch of a diagonal
+// block and a step take before the chain waits for them, by measurement.  4,800 (8,000) unknowns, ms, FP32:
+// nothing carried 2.80 (6.66), 1/1 2.54 (6.18), 1/2 2.37 (5.85), 2/2 2.35 (5.79), 2/3 2.36 (5.80); FP64: nothing
+// 5.23 (13.1), 1/1 4.86 (12.5), 1/2 4.50 (11.95), 2/2 4.52 (12.06), 2/4 4.77 (12.5).
+template <typename T> struct LuRoom;
+template <> struct LuRoom<float> { static constexpr int SLOTS = 512, FIRST = 2, STEP = 2; };
+template <> struct LuRoom<double> { static constexpr int SLOTS = 256, FIRST = 1, STEP = 2; };
+
 template <typename T>
 int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void *work, T *YL, T *YU)
 {
@@ -916,26 +1067,53 @@ int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void
     hipLaunchKernelGGL(k_fill_info, dim3(1), dim3(64), 0, ctx->stream, info_dev, 0);
     const LuMat<T> m{A, ld, n, (T *)work, (T *)work + lu_dsize(n), info_dev, YL, YU};
     int st;
+    int64_t rest_j = n;   // columns from here on still miss the previous outer block's update
     for (int64_t k = 0; k < n; k += NOB) {
-        const int64_t kend = std::min<int64_t>(k + NOB, n);
-        {
+        const int64_t kend = std::min<int64_t>(k + NOB, n), rows = lu_tiles(n - k, NPB);
+        LuRest r{rest_j, (int)std::max<int64_t>(lu_tiles(n - rest_j, NPB), 1), 0};
+        int64_t left = rest_j < n ? r.ntc * rows : 0;
+        auto take = [&](int64_t room, bool last) {   // tiles of the next launch
+            const int64_t x = last ? left : std::min(left, std::max<int64_t>(room, 0));
+            left -= x;
+            return x;
+        };
+        if (k == 0) {
             ProfScope ps(ctx, "lu_nopiv_diag");
-            hipLaunchKernelGGL(k_lu_first<T>, dim3(1), dim3(256), 0, ctx->stream, m, k, kend);
+            hipLaunchKernelGGL(k_lu_first<T>, dim3(1), dim3(LT), 0, ctx->stream, m, k);
+        } else {
+            const int64_t pc = lu_tiles(kend - k, NPB), x = take(LuRoom<T>::SLOTS * LuRoom<T>::FIRST - pc * rows, rows == 1);
+            ProfScope ps(ctx, "lu_nopiv_update");
+            hipLaunchKernelGGL(k_lu_update<T>, dim3((unsigned)(pc * rows + x)), dim3(LT), 0, ctx->stream, m, k, (int)pc,
+                               (int)(pc * rows), r);
+            r.tile0 += (int)x;
         }
         for (int t = 0; t < NIN; ++t) {
-            const int64_t strips = lu_tiles(n - k - (int64_t)NPB * (t + 1), NPB);
+            const int64_t strips = rows - 1 - t;
             if (strips <= 0) break;
+            const int64_t x = take((LuRoom<T>::SLOTS - strips) * LuRoom<T>::STEP, t + 2 >= NIN || strips == 1);
             ProfScope ps(ctx, "lu_nopiv_step");
-            hipLaunchKernelGGL(k_lu_step<T>, dim3((unsigned)strips), dim3(256), 0, ctx->stream, m, k, t, kend);
+            hipLaunchKernelGGL(k_lu_step<T>, dim3((unsigned)(strips + x)), dim3(LT), 0, ctx->stream, m, k, t, kend, (int)strips,
+                               r);
+            r.tile0 += (int)x;
         }
         const int64_t right = n - kend;
-        if (right > 0) {
+        const int nr = (int)lu_tiles(right, UW), ni = lu_inner(kend - k);
+        if (nr + ni > 0) {
             ProfScope ps(ctx, "lu_nopiv_urow");
-            hipLaunchKernelGGL(k_lu_urow<T>, dim3((unsigned)lu_tiles(right, UW)), dim3(256), 0, ctx->stream, m, k, kend);
+            hipLaunchKernelGGL(k_lu_urow<T>, dim3((unsigned)(nr + ni)), dim3(LT), 0, ctx->stream, m, k, kend, nr);
         }
         FP_HIP(ctx, hipGetLastError());
-        if (right > 0 && (st = fp_gemm_sub<T>(ctx, right, right, NOB, A + kend * ld + k, ld, A + k * ld + kend, ld,
-                                              A + kend * ld + kend, ld)))
+        if (right <= 0) break;
+        // tile columns of the update right of the next outer block, as many as its launches have room for
+        const int64_t rt = lu_tiles(right, NPB), pt = std::min<int64_t>(NIN, rt);
+        int64_t room = std::max<int64_t>((int64_t)LuRoom<T>::SLOTS * LuRoom<T>::FIRST - pt * rt, 0);
+        for (int t = 0; t < std::min<int64_t>(NIN - 1, rt - 1); ++t)
+            room += std::max<int64_t>(LuRoom<T>::SLOTS - (rt - 1 - t), 0) * LuRoom<T>::STEP;
+        const int64_t now = rt - pt - std::min(room / rt, rt - pt);   // the others, at once
+        const int64_t j0 = kend + pt * NPB;
+        rest_j = std::min(j0 + now * NPB, n);
+        if (now > 0 && (st = fp_gemm_sub<T>(ctx, right, rest_j - j0, NOB, A + kend * ld + k, ld, A + k * ld + j0, ld,
+                                            A + kend * ld + j0, ld)))
             return st;
     }
     return FP_OK;
@@ -953,8 +1131,8 @@ int fp_tri_inverse(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, void *work)
     T *W = (T *)work + 2 * lu_dsize(n);
     for (int s = NPB; s < TBIG && s < n; s *= 2) {
         const dim3 g((unsigned)((s / NPB) * (s / NPB)), (unsigned)lu_tiles(n, 2 * s), 2);
-        hipLaunchKernelGGL(k_tri_merge<T>, g, dim3(256), 0, ctx->stream, m, W, s, 0);
-        hipLaunchKernelGGL(k_tri_merge<T>, g, dim3(256), 0, ctx->stream, m, W, s, 1);
+        hipLaunchKernelGGL(k_tri_merge<T>, g, dim3(LT), 0, ctx->stream, m, W, s, 0);
+        hipLaunchKernelGGL(k_tri_merge<T>, g, dim3(LT), 0, ctx->stream, m, W, s, 1);
     }
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;
@@ -1025,15 +1203,15 @@ static __device__ __forceinline__ LuMat<float> lub_mat(const fp_lu_desc &d)
                         nullptr, nullptr};
 }
 
-__global__ __launch_bounds__(256) void k_lu_first_lub(const fp_lu_desc *__restrict__ desc, int64_t kk)
+__global__ __launch_bounds__(LT) void k_lu_first_lub(const fp_lu_desc *__restrict__ desc, int64_t kk)
 {
     __shared__ StepLds<float> s;
     const LuMat<float> m = lub_mat(desc[blockIdx.y]);
     if (kk >= m.n) return;   // uniform per workgroup
-    lu_first_dev<float>(m, kk, min(kk + (int64_t)NOB, m.n), s);
+    lu_first_dev<float>(m, kk, s);
 }
 
-__global__ __launch_bounds__(256) void k_lu_step_lub(const fp_lu_desc *__restrict__ desc, int64_t kk, int t)
+__global__ __launch_bounds__(LT) void k_lu_step_lub(const fp_lu_desc *__restrict__ desc, int64_t kk, int t)
 {
     __shared__ StepLds<float> s;
     const LuMat<float> m = lub_mat(desc[blockIdx.y]);
@@ -1042,12 +1220,15 @@ __global__ __launch_bounds__(256) void k_lu_step_lub(const fp_lu_desc *__restric
     lu_step_dev<float>(m, kk, t, min(kk + (int64_t)NOB, m.n), blockIdx.x, s);
 }
 
-__global__ __launch_bounds__(256) void k_lu_urow_lub(const fp_lu_desc *__restrict__ desc, int64_t kk)
+__global__ __launch_bounds__(LT) void k_lu_urow_lub(const fp_lu_desc *__restrict__ desc, int64_t kk)
 {
     __shared__ UrowLds<float> s;
     const LuMat<float> m = lub_mat(desc[blockIdx.y]);
-    if ((int64_t)blockIdx.x * UW >= m.n - kk - NOB) return;
-    lu_urow_dev<float>(m, kk, kk + NOB, blockIdx.x, s);
+    if (kk >= m.n) return;
+    const int64_t kend = min(kk + (int64_t)NOB, m.n);
+    const int nr = (int)((m.n - kend + UW - 1) / UW);
+    if ((int)blockIdx.x >= nr + lu_inner(kend - kk)) return;
+    lu_urow_dev<float>(m, kk, kend, blockIdx.x, nr, s);
 }
 
 int fp_getrf_nopiv_f32_batched(fp_ctx *ctx, const fp_lu_desc *d_desc, const int64_t *n_host, int nb)
@@ -1061,20 +1242,24 @@ int fp_getrf_nopiv_f32_batched(fp_ctx *ctx, const fp_lu_desc *d_desc, const int6
     for (int64_t kk = 0; kk < nmax; kk += NOB) {
         {
             ProfScope ps(ctx, "lu_nopiv_diag");
-            hipLaunchKernelGGL(k_lu_first_lub, dim3(1, (unsigned)nb), dim3(256), 0, ctx->stream, d_desc, kk);
+            hipLaunchKernelGGL(k_lu_first_lub, dim3(1, (unsigned)nb), dim3(LT), 0, ctx->stream, d_desc, kk);
         }
         for (int t = 0; t < NIN; ++t) {
             const int64_t strips = lu_tiles(nmax - kk - (int64_t)NPB * (t + 1), NPB);
             if (strips <= 0) break;
             ProfScope ps(ctx, "lu_nopiv_step");
-            hipLaunchKernelGGL(k_lu_step_lub, dim3((unsigned)strips, (unsigned)nb), dim3(256), 0, ctx->stream, d_desc,
+            hipLaunchKernelGGL(k_lu_step_lub, dim3((unsigned)strips, (unsigned)nb), dim3(LT), 0, ctx->stream, d_desc,
                                kk, t);
         }
         const int64_t right = nmax - kk - NOB;
-        if (right > 0) {
+        int64_t gu = 0;
+        for (int b = 0; b < nb; ++b) {
+            const int64_t kend = std::min(kk + (int64_t)NOB, n_host[b]);
+            if (kk < n_host[b]) gu = std::max(gu, lu_tiles(n_host[b] - kend, UW) + lu_inner(kend - kk));
+        }
+        if (gu > 0) {
             ProfScope ps(ctx, "lu_nopiv_urow");
-            hipLaunchKernelGGL(k_lu_urow_lub, dim3((unsigned)lu_tiles(right, UW), (unsigned)nb), dim3(256), 0,
-                               ctx->stream, d_desc, kk);
+            hipLaunchKernelGGL(k_lu_urow_lub, dim3((unsigned)gu, (unsigned)nb), dim3(LT), 0, ctx->stream, d_desc, kk);
         }
         FP_HIP(ctx, hipGetLastError());
         if (right > 0 && (st = fp_gemm_sub_lub(ctx, d_desc, nb, kk, NOB, right))) return st;

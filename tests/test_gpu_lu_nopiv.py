@@ -33,6 +33,25 @@ def test_fp64_lu_matches_lapack(fp, n, k, pivoted, monkeypatch):
     assert r < 16 * EPS * np.sqrt(n) + 4 * EPS, r
 
 
+@pytest.mark.parametrize("n", [576, 577, 640, 835, 1029, 3303])
+def test_updates_carried_by_the_next_block(fp, n):
+    # from 513 unknowns on, part of each trailing update runs inside the launches that factor the next 256
+    # columns; at 3,303 a part does not fit and is a product of its own.  The factors have to be good enough
+    # by themselves: no pivoted panel runs.
+    A, rng = _matrix(n, 200 + n)
+    b = A @ rng.standard_normal(n)
+    ctx = fp._native.context()
+    ctx.profile(True)
+    x = fp.solve_ludiv(None, A, b)
+    counts = {name: ctx.profile_get(name)[0] for name in ("lu_nopiv_update", "panel_tslu", "gemm_f64")}
+    ctx.profile(False)
+    assert counts["lu_nopiv_update"] == (n + 3) // 4 * 4 // 256 - ((n + 3) // 4 * 4 % 256 == 0)
+    assert counts["panel_tslu"] == 0
+    assert (counts["gemm_f64"] > 0) == (n == 3303)
+    r = np.linalg.norm(A @ x - b) / (np.linalg.norm(A) * np.linalg.norm(x))
+    assert r < 16 * EPS * np.sqrt(n) + 4 * EPS, r
+
+
 @pytest.mark.parametrize("n", [64, 300])
 def test_permutation_needs_no_pivots(fp, n):
     # a zero diagonal: plain elimination without pivoting stops at the first column
