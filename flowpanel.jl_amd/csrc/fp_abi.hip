@@ -1393,12 +1393,21 @@ __global__ void k_cp(const double *__restrict__ U, int64_t n, double uref, doubl
     out[i] += 1 - u * u;
 }
 
-__global__ void k_kutta(const int64_t *__restrict__ sh, int64_t ns, int mode, double *__restrict__ out)
+__device__ __forceinline__ int64_t lane_value(int64_t v, int l)   // v of lane l (the same l in every lane)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    for (int64_t e = 0; e < ns; ++e) {
-        const int64_t pi = sh[6 * e], pj = sh[6 * e + 3];
-        if (mode == FP_KUTTA_REFERENCE) {
+    const uint32_t lo = __builtin_amdgcn_readlane((int)v, l), hi = __builtin_amdgcn_readlane((int)(v >> 32), l);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// One wave, 64 edges at a time: a lane per edge where no panel belongs to two of the 64 (compared lane by
+// lane), else in list order by one lane, which is the meaning of the list.  96 edges by one lane: 39 us
+// (the latency of dependent loads); a lane each: ~5.
+__global__ __launch_bounds__(64) void k_kutta(const int64_t *__restrict__ sh, int64_t ns, int mode, double *out)
+{
+    const int lane = threadIdx.x;
+    const bool ref = mode == FP_KUTTA_REFERENCE;
+    auto apply = [&](int64_t pi, int64_t pj) {
+        if (ref) {
             if (pj != -1) {
                 const double ave = (out[pi] + out[pi + 1] + out[pj] + out[pj - 1]) / 4;
                 out[pi] = ave; out[pi + 1] = ave; out[pj] = ave; out[pj - 1] = ave;
@@ -1410,6 +1419,29 @@ __global__ void k_kutta(const int64_t *__restrict__ sh, int64_t ns, int mode, do
             const double ave = (out[pi] + out[pj]) / 2;
             out[pi] = ave; out[pj] = ave;
         }
+    };
+    for (int64_t e0 = 0; e0 < ns; e0 += 64) {
+        const int m = (int)(ns - e0 < 64 ? ns - e0 : 64);
+        const int64_t pi = lane < m ? sh[6 * (e0 + lane)] : -1, pj = lane < m ? sh[6 * (e0 + lane) + 3] : -1;
+        bool clash = false;
+        for (int l = 0; l < m; ++l) {
+            const int64_t qi = lane_value(pi, l), qj = lane_value(pj, l);
+            if (l == lane || lane >= m) continue;
+            // an edge's panels: pi (and pi + 1), pj (and pj - 1)
+            for (int64_t di = 0; di <= ref; ++di)
+                for (int64_t dq = 0; dq <= ref; ++dq)
+                    clash = clash || pi + di == qi + dq || (qj != -1 && pi + di == qj - dq) ||
+                            (pj != -1 && pj - di == qi + dq) || (pj != -1 && qj != -1 && pj - di == qj - dq);
+        }
+        if (!__any(clash)) {
+            if (lane < m) apply(pi, pj);
+        } else {
+            for (int l = 0; l < m; ++l) {
+                const int64_t qi = lane_value(pi, l), qj = lane_value(pj, l);
+                if (lane == 0) apply(qi, qj);
+            }
+        }
+        __syncthreads();   // the next 64 may read what these wrote
     }
 }
 

@@ -61,23 +61,37 @@ __global__ __launch_bounds__(256) void k_ugradmu_cell(const double *__restrict__
 }
 
 // trailing-edge panels: their edge terms added back, once per appearance in
-// the shedding list, in list order
+// the shedding list.  A lane per appearance; the first one of a panel adds its
+// terms (they do not depend on `out`) as often as the panel appears, so that
+// the sum is the one in list order.  Latency bounds it: one lane walking the
+// 2 x 96 entries of a list took 608 us, a lane each takes ~10.
 template <int NVP>
-__global__ void k_ugradmu_te(const double *__restrict__ pv, const int *__restrict__ nvv, int64_t N,
-                             const double *__restrict__ geo, const int *__restrict__ nbr, const double *__restrict__ G,
-                             double sgn, const int64_t *__restrict__ sh, int64_t ns, double *__restrict__ out)
+__global__ __launch_bounds__(64) void k_ugradmu_te(const double *__restrict__ pv, const int *__restrict__ nvv, int64_t N,
+                                                   const double *__restrict__ geo, const int *__restrict__ nbr,
+                                                   const double *__restrict__ G, double sgn,
+                                                   const int64_t *__restrict__ sh, int64_t ns, double *__restrict__ out)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    for (int64_t e = 0; e < ns; ++e)
-        for (int side = 0; side < 2; ++side) {
-            const int64_t c = sh[6 * e + 3 * side];
-            if (c < 0) continue;
-            double acc[3];
-            ugm_cell<NVP>(pv, nvv, N, geo, nbr, G, sgn, c, acc);
-            out[3 * c] += acc[0];
-            out[3 * c + 1] += acc[1];
-            out[3 * c + 2] += acc[2];
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;   // entry: edge i / 2, side i % 2
+    const int64_t c = i < 2 * ns ? sh[3 * i] : -1;
+    int times = c >= 0, first = 1;
+    for (int64_t q0 = 0; q0 < 2 * ns; q0 += 64) {
+        const int64_t own = q0 + threadIdx.x < 2 * ns ? sh[3 * (q0 + threadIdx.x)] : -1;
+        const int m = (int)(2 * ns - q0 < 64 ? 2 * ns - q0 : 64);
+        for (int l = 0; l < m; ++l) {
+            const uint32_t lo = __builtin_amdgcn_readlane((int)own, l), hi = __builtin_amdgcn_readlane((int)(own >> 32), l);
+            const bool same = (int64_t)(((uint64_t)hi << 32) | lo) == c;
+            first = first && !(same && q0 + l < i);
+            times += same && q0 + l > i;
         }
+    }
+    if (c < 0 || !first) return;
+    double acc[3];
+    ugm_cell<NVP>(pv, nvv, N, geo, nbr, G, sgn, c, acc);
+    for (int d = 0; d < 3; ++d) {
+        double v = out[3 * c + d];
+        for (int q = 0; q < times; ++q) v += acc[d];
+        out[3 * c + d] = v;
+    }
 }
 
 // Node-based scheme (src/FLOWPanel_postprocess.jl:622-748): nodal values of
@@ -389,14 +403,14 @@ int fp_launch_ugradmu(fp_ctx *ctx, const fp_body *b, const int *d_nbr, const int
         hipLaunchKernelGGL(k_ugradmu_cell<4>, grid, dim3(256), 0, ctx->stream, b->d_pv, b->d_nv, N, b->d_geo, d_nbr,
                            b->d_strength, sgn, out);
         if (te && b->ns > 0)
-            hipLaunchKernelGGL(k_ugradmu_te<4>, dim3(1), dim3(64), 0, ctx->stream, b->d_pv, b->d_nv, N, b->d_geo,
-                               d_nbr, b->d_strength, sgn, d_sh, b->ns, out);
+            hipLaunchKernelGGL(k_ugradmu_te<4>, dim3((unsigned)((2 * b->ns + 63) / 64)), dim3(64), 0, ctx->stream,
+                               b->d_pv, b->d_nv, N, b->d_geo, d_nbr, b->d_strength, sgn, d_sh, b->ns, out);
     } else {
         hipLaunchKernelGGL(k_ugradmu_cell<8>, grid, dim3(256), 0, ctx->stream, b->d_pv, b->d_nv, N, b->d_geo, d_nbr,
                            b->d_strength, sgn, out);
         if (te && b->ns > 0)
-            hipLaunchKernelGGL(k_ugradmu_te<8>, dim3(1), dim3(64), 0, ctx->stream, b->d_pv, b->d_nv, N, b->d_geo,
-                               d_nbr, b->d_strength, sgn, d_sh, b->ns, out);
+            hipLaunchKernelGGL(k_ugradmu_te<8>, dim3((unsigned)((2 * b->ns + 63) / 64)), dim3(64), 0, ctx->stream,
+                               b->d_pv, b->d_nv, N, b->d_geo, d_nbr, b->d_strength, sgn, d_sh, b->ns, out);
     }
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;
