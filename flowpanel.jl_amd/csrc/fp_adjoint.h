@@ -192,7 +192,12 @@ FPA_HD void fpa_ring_rev(const double (&p)[NVP][3], double X, double Y, double Z
         r[k][0] = X - p[k][0]; r[k][1] = Y - p[k][1]; r[k][2] = Z - p[k][2];
         const double l2 = r[k][0] * r[k][0] + r[k][1] * r[k][1] + r[k][2] * r[k][2];
         const double y = l2 > 0 ? fpa_rsqrt(l2) : 0.0;   // 1/|r|
-        iv[k] = fpa_recip(l2 * y + off);
+        // |r| and 1/(|r| + off) with their roundings corrected (one residual each): where a target lies on the
+        // line of an edge the terms below are differences of 1e-8 of these values, and an ulp shows at 1e-8
+        double l = l2 * y;
+        l = fma(0.5 * y, fma(-l, l, l2), l);
+        const double d = l + off, u = fpa_recip(d);
+        iv[k] = d > 0 ? fma(fma(-d, u, 1.0), u, u) : u;
         sk[k] = l2 > 0 ? iv[k] * iv[k] * y : 0.0;
     }
     const double off2 = off * off, cut2 = cut * cut;
