@@ -93,26 +93,73 @@ __device__ __forceinline__ int kutta_ids(const int64_t *s, int mode, int64_t *id
     return 0;
 }
 
-// sequential Kutta averaging (forward) of c0, or its reverse on c0 and c1
-template <bool REV>
-__global__ void k_adj_kutta(const int64_t *__restrict__ sh, int64_t ns, int mode, double *c0, double *c1)
+// Sums of six values over the 64 lanes, all in vector registers (no LDS permutes): a step of the butterfly that
+// halves the lanes also halves the values a lane carries, so that six sums take 3 + 2 + 1 + 3 additions instead
+// of 36.  Swapping halves of two registers and adding leaves the first value's sums in one half and the
+// second's in the other: lanes 32.. hold values 3-5, odd rows of 16 lanes value 2 (5), and the upper eight
+// lanes of even rows value 1 (4).  Returns the sum of value SUM6_INDEX(lane), the same in its eight lanes.
+template <int CTRL> __device__ __forceinline__ double dpp_f64(double v)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    int64_t ids[4];
-    if (!REV) {
-        for (int64_t e = 0; e < ns; ++e) {
-            const int cnt = kutta_ids(sh + 6 * e, mode, ids);
-            if (!cnt) continue;
+    const int64_t b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((int64_t)hi << 32) | (uint32_t)lo);
+}
+__device__ __forceinline__ double swap32_add(double a, double b)
+{
+    const int64_t x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+    return __longlong_as_double((int64_t)(((uint64_t)hi[0] << 32) | lo[0])) +
+           __longlong_as_double((int64_t)(((uint64_t)hi[1] << 32) | lo[1]));
+}
+__device__ __forceinline__ double swap16_add(double a, double b)
+{
+    const int64_t x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+    return __longlong_as_double((int64_t)(((uint64_t)hi[0] << 32) | lo[0])) +
+           __longlong_as_double((int64_t)(((uint64_t)hi[1] << 32) | lo[1]));
+}
+__device__ __forceinline__ int sum6_index(int lane)   // value of the lane's sum, -1: a repetition
+{
+    const int c = (lane & 16) ? ((lane & 8) ? -1 : 2) : (lane & 8) ? 1 : 0;
+    return (lane & 7) || c < 0 ? -1 : (lane >> 5) * 3 + c;
+}
+__device__ __forceinline__ double wave_sum6(const double (&v)[6], int lane)
+{
+    const double w0 = swap32_add(v[0], v[3]), w1 = swap32_add(v[1], v[4]), w2 = swap32_add(v[2], v[5]);
+    const double x0 = swap16_add(w0, w2), x1 = swap16_add(w1, w2);   // (odd rows of x1 repeat value 2)
+    const bool up = lane & 8;
+    double s = (up ? x1 : x0) + dpp_f64<0x128>(up ? x0 : x1);   // row_ror:8
+    s += dpp_f64<0x141>(s);                                      // row_half_mirror
+    s += dpp_f64<0xb1>(s);                                       // quad_perm 1,0,3,2
+    s += dpp_f64<0x4e>(s);                                       // quad_perm 2,3,0,1
+    return s;
+}
+
+__device__ __forceinline__ int64_t lane_value(int64_t v, int l)   // v of lane l (the same l in every lane)
+{
+    const uint32_t lo = __builtin_amdgcn_readlane((int)v, l), hi = __builtin_amdgcn_readlane((int)(v >> 32), l);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// Kutta averaging (forward) of c0 in list order, or its reverse on c0 and c1 in reverse order.  One wave, 64
+// edges at a time: a lane per edge where no panel belongs to two of the 64, else one lane in order.  100 edges
+// by one lane: 194 us for the reverse (dependent loads).
+template <bool REV>
+__global__ __launch_bounds__(64) void k_adj_kutta(const int64_t *__restrict__ sh, int64_t ns, int mode, double *c0, double *c1)
+{
+    const int lane = threadIdx.x;
+    auto apply = [&](const int64_t *ids, int cnt) {
+        if (!cnt) return;
+        if (!REV) {
             double s = 0;
             for (int k = 0; k < cnt; ++k) s += c0[ids[k]];
             const double ave = s / cnt;
             for (int k = 0; k < cnt; ++k) c0[ids[k]] = ave;
+            return;
         }
-        return;
-    }
-    for (int64_t e = ns - 1; e >= 0; --e) {
-        const int cnt = kutta_ids(sh + 6 * e, mode, ids);
-        if (!cnt) continue;
         for (int pass = 0; pass < 2; ++pass) {
             double *c = pass == 0 ? c0 : c1;
             // adjoint of ave: the (distinct) overwritten entries
@@ -125,6 +172,29 @@ __global__ void k_adj_kutta(const int64_t *__restrict__ sh, int64_t ns, int mode
             for (int k = 0; k < cnt; ++k) c[ids[k]] = 0;
             for (int k = 0; k < cnt; ++k) c[ids[k]] += s / cnt;
         }
+    };
+    for (int64_t e0 = 0; e0 < ns; e0 += 64) {
+        const int m = (int)(ns - e0 < 64 ? ns - e0 : 64);
+        const bool ok = lane < m;
+        const int64_t e = REV ? ns - 1 - e0 - lane : e0 + lane;
+        int64_t ids[4] = {-1, -1, -1, -1};
+        const int cnt = ok ? kutta_ids(sh + 6 * e, mode, ids) : 0;
+        bool clash = false;
+        for (int l = 0; l < m; ++l)
+            for (int k = 0; k < 4; ++k) {
+                const int64_t other = lane_value(ids[k], l);
+                const bool used = __builtin_amdgcn_readlane(cnt, l) > k && l != lane;
+                for (int q = 0; q < 4; ++q) clash = clash || (used && q < cnt && ids[q] == other);
+            }
+        if (!__any(clash)) {
+            apply(ids, cnt);
+        } else if (lane == 0) {
+            for (int l = 0; l < m; ++l) {
+                int64_t id[4];
+                apply(id, kutta_ids(sh + 6 * (REV ? ns - 1 - e0 - l : e0 + l), mode, id));
+            }
+        }
+        __syncthreads();   // the next 64 may read what these wrote
     }
 }
 
@@ -195,7 +265,7 @@ __global__ __launch_bounds__(ADJ_BLOCK) void k_adj_pairs(const double *__restric
 {
     __shared__ double st[ADJ_TT][9];
     __shared__ double sx[ADJ_BLOCK / 64][ADJ_TT][6];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c6 = sum6_index(lane);
     const int64_t j = (int64_t)blockIdx.x * ADJ_BLOCK + tid;
     const bool ok = j < N;
     double p[NVP][3];
@@ -225,13 +295,10 @@ __global__ __launch_bounds__(ADJ_BLOCK) void k_adj_pairs(const double *__restric
             const double w[2][3] = {{st[t][3], st[t][4], st[t][5]}, {st[t][6], st[t][7], st[t][8]}};
             double xb[2][3] = {{0, 0, 0}, {0, 0, 0}};
             fpa_ring_rev<NVP, 2>(p, st[t][0], st[t][1], st[t][2], off, cut, w, g, xb, pb);
-#pragma unroll
-            for (int m = 0; m < 2; ++m)
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    const double v = wave_sum(gj * xb[m][d]);
-                    if (lane == 0) sx[wave][t][3 * m + d] = v;
-                }
+            const double v[6] = {gj * xb[0][0], gj * xb[0][1], gj * xb[0][2],
+                                 gj * xb[1][0], gj * xb[1][1], gj * xb[1][2]};
+            const double sum = wave_sum6(v, lane);
+            if (c6 >= 0) sx[wave][t][c6] = sum;
         }
         __syncthreads();
         for (int e = tid; e < cnt * 6; e += ADJ_BLOCK) {
@@ -275,21 +342,25 @@ __device__ __forceinline__ void load_horse(const double *hh, int nh, int h, fpa_
     db = fpa_mk(hh[9 * nh + h], hh[10 * nh + h], hh[11 * nh + h]);
 }
 
-// target adjoints of the horseshoes of one body: Xb[c][t] += G_h (du_h/dX)^T w_t
+// target adjoints of the horseshoes of one body: Xb[c][t] += G_h (du_h/dX)^T w_t.  A workgroup takes WX_T
+// targets; 256 / WX_T lanes share a target's horseshoes, and their sums meet in LDS in a fixed order.  (A lane
+// per target walking all horseshoes left 10,000 targets on 160 waves: 585 us.)
+constexpr int WX_T = 16, WX_H = 256 / WX_T;
 __global__ __launch_bounds__(256) void k_adj_wake_x(const double *__restrict__ hh, const int *__restrict__ hcol,
                                                     int nh, const double *__restrict__ gam, double off, double cut,
                                                     const double *__restrict__ tx, int64_t MT,
                                                     const double *__restrict__ W, double *__restrict__ Xb)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= MT) return;
+    __shared__ double red[WX_H][6][WX_T];
+    const int tl = threadIdx.x % WX_T, q = threadIdx.x / WX_T;
+    const int64_t t0 = (int64_t)blockIdx.x * WX_T, t = min(t0 + tl, MT - 1);
     const fpa_v3 X = fpa_mk(tx[t], tx[MT + t], tx[2 * MT + t]);
     fpa_v3 w[2], xb[2];
     for (int m = 0; m < 2; ++m) {
         w[m] = fpa_mk(W[(3 * m) * MT + t], W[(3 * m + 1) * MT + t], W[(3 * m + 2) * MT + t]);
         xb[m] = fpa_mk(0, 0, 0);
     }
-    for (int h = 0; h < nh; ++h) {
+    for (int h = q; h < nh; h += WX_H) {
         fpa_v3 pa, pb, da, db;
         load_horse(hh, nh, h, pa, pb, da, db);
         const double s = gam[hcol[h]];
@@ -299,9 +370,15 @@ __global__ __launch_bounds__(256) void k_adj_wake_x(const double *__restrict__ h
         }
     }
     for (int m = 0; m < 2; ++m) {
-        Xb[(3 * m) * MT + t] += xb[m].x;
-        Xb[(3 * m + 1) * MT + t] += xb[m].y;
-        Xb[(3 * m + 2) * MT + t] += xb[m].z;
+        red[q][3 * m][tl] = xb[m].x;
+        red[q][3 * m + 1][tl] = xb[m].y;
+        red[q][3 * m + 2][tl] = xb[m].z;
+    }
+    __syncthreads();
+    if (threadIdx.x < 6 * WX_T && t0 + tl < MT) {
+        double s = 0;
+        for (int k = 0; k < WX_H; ++k) s += red[k][q][tl];
+        Xb[q * MT + t0 + tl] += s;
     }
 }
 
@@ -342,12 +419,19 @@ __global__ __launch_bounds__(256) void k_adj_wake_p(const double *__restrict__ h
 }
 
 // g[m][col0 + hcol[h]] += strength adjoint of horseshoe h (in order: deterministic)
-__global__ void k_adj_wake_g(const double *__restrict__ hp, const int *__restrict__ hcol, int nh, int64_t col0,
-                             int64_t M, double *__restrict__ g)
+// a lane per horseshoe; the first one of a panel adds what all of them give it
+__global__ __launch_bounds__(64) void k_adj_wake_g(const double *__restrict__ hp, const int *__restrict__ hcol, int nh,
+                                                   int64_t col0, int64_t M, double *__restrict__ g)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    for (int h = 0; h < nh; ++h)
-        for (int m = 0; m < 2; ++m) g[m * M + col0 + hcol[h]] += hp[(int64_t)h * 26 + 24 + m];
+    const int h = blockIdx.x * 64 + threadIdx.x, c = h < nh ? hcol[h] : -1;
+    bool first = c >= 0;
+    for (int q = 0; q < nh; ++q) first = first && !(q < h && hcol[q] == c);
+    if (!first) return;
+    double s[2] = {g[col0 + c], g[M + col0 + c]};
+    for (int q = h; q < nh; ++q)
+        if (hcol[q] == c)
+            for (int m = 0; m < 2; ++m) s[m] += hp[(int64_t)q * 26 + 24 + m];
+    for (int m = 0; m < 2; ++m) g[m * M + col0 + c] = s[m];
 }
 
 // control-point weights W2 = -lambda n, normal adjoints of the no-flow-through
@@ -586,12 +670,12 @@ int fp_adj_wake(fp_ctx *ctx, const fp_body *b, const double *tx, int64_t MT, con
     if (b->nh == 0 || MT == 0) return FP_OK;
     ProfScope ps(ctx, "adjoint_wake_f64");
     const double off = b->kernel_offset, cut = b->kernel_cutoff;
-    hipLaunchKernelGGL(k_adj_wake_x, dim3(blocks(MT)), dim3(256), 0, ctx->stream, b->d_hh, b->d_hcol, b->nh,
+    hipLaunchKernelGGL(k_adj_wake_x, dim3((unsigned)((MT + WX_T - 1) / WX_T)), dim3(256), 0, ctx->stream, b->d_hh, b->d_hcol, b->nh,
                        b->d_strength, off, cut, tx, MT, W, Xb);
     if (gamma) {
         hipLaunchKernelGGL(k_adj_wake_p<true>, dim3(b->nh), dim3(256), 0, ctx->stream, b->d_hh, b->nh, off, cut, tx,
                            MT, W, hpart);
-        hipLaunchKernelGGL(k_adj_wake_g, dim3(1), dim3(64), 0, ctx->stream, (const double *)hpart, b->d_hcol, b->nh,
+        hipLaunchKernelGGL(k_adj_wake_g, dim3((unsigned)((b->nh + 63) / 64)), dim3(64), 0, ctx->stream, (const double *)hpart, b->d_hcol, b->nh,
                            col0, MT, g);
     } else {
         hipLaunchKernelGGL(k_adj_wake_p<false>, dim3(b->nh), dim3(256), 0, ctx->stream, b->d_hh, b->nh, off, cut, tx,
