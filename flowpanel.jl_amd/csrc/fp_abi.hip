@@ -409,6 +409,14 @@ struct BJPrecond : Precond {
         if (coarse > 0) FP_HIP(ctx, hipStreamWaitEvent(ctx->stream, join, 0));
         return FP_OK;
     }
+    // the coarse space once more, inverted by the Gauss-Jordan
+    int coarse_gj(const void *A, int prec, int64_t ld)
+    {
+        return prec == FP_F64 ? fp_coarse_setup<double>(ctx, (const double *)A, n, ld, cs, AZ.as<float>(), Einv.as<double>(),
+                                                        work.as<double>(), cinfo.as<int>(), false, false)
+                              : fp_coarse_setup<float>(ctx, (const float *)A, n, ld, cs, AZ.as<float>(), Einv.as<double>(),
+                                                       work.as<double>(), cinfo.as<int>(), false, false);
+    }
     int apply(const double *x, double *y) override
     {
         if (cs > 0) {
@@ -1005,7 +1013,7 @@ struct Solver {
         int st;
         if (M && M->early) {
             if ((st = M->finish_early(A, prec, a.ld, o.coarse_block))) return st;
-            return bj_check(M->binfo.as<int>(), blk);
+            return bj_check(M->binfo.as<int>(), blk, A, prec);
         }
         if ((st = dalloc(ctx, info, sizeof(int)))) return st;
         if (o.precond_order == FP_ORDER_SPATIAL) {
@@ -1029,11 +1037,11 @@ struct Solver {
         }
         M.reset(new BJPrecond(ctx, a.n, blk));
         if ((st = M->setup(A, prec, a.ld, o.coarse_block, info.as<int>()))) return st;
-        return bj_check(info.as<int>(), blk);
+        return bj_check(info.as<int>(), blk, A, prec);
     }
     // zero pivots of the block inverses and of the coarse Galerkin matrix (side
     // streams, joined into the main stream by the set-up)
-    int bj_check(const int *binfo_dev, int blk)
+    int bj_check(const int *binfo_dev, int blk, const void *A, int prec)
     {
         int st;
         int hinfo[2] = {0, 0};
@@ -1041,6 +1049,11 @@ struct Solver {
         if (M->cinfo.p)
             FP_HIP(ctx, hipMemcpyAsync(&hinfo[1], M->cinfo.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (hinfo[1] && fp_coarse_by_lu((a.n + M->cs - 1) / M->cs)) {   // not an inverse: Gauss-Jordan decides
+            if ((st = M->coarse_gj(A, prec, a.ld))) return st;
+            FP_HIP(ctx, hipMemcpyAsync(&hinfo[1], M->cinfo.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+            FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        }
         char buf[192];
         if (hinfo[0]) {
             const int64_t row = hinfo[0] - 1;

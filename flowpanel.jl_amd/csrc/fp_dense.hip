@@ -2536,41 +2536,47 @@ __global__ __launch_bounds__(256) void k_chunk_rowsum_lane(const T *__restrict__
 // Chunk sums of rows for chunks shorter than a wave, read coalesced:
 // out[k * nrows + r] = sum of A[r * ld + c] over the columns c of chunk k
 // (columns k cs .. k cs + cs - 1, the last chunk cut at ncols), summed in FP64 in
-// column order.  Each wave takes one row and walks it in segments of 64 chunks:
-// the segment goes into the wave's slice of LDS with 16-byte loads, then lane j
-// sums chunk j of the segment out of LDS.  The four waves of a workgroup take
-// the same number of segments (the barriers are uniform); dynamic LDS of
-// 4 * 64 * cs elements.
+// column order.  A workgroup takes SEG_ROWS rows and one segment of 64 chunks: each
+// of its waves brings a row's segment into its own slice of LDS with 16-byte loads
+// and lane j sums chunk j out of it, row after row; the sums are collected in LDS so
+// that a chunk's SEG_ROWS values leave as one line.  Memory bound: one row at a time
+// over all segments, with two barriers a segment and 4-byte stores 4 nrows bytes
+// apart, read 30,000 x 30,000 FP32 at 2.6 TB/s (1.39 ms); now 0.96 ms.  Dynamic LDS of 4 * 64 * cs
+// elements.
+constexpr int SEG_ROWS = 32;
+
 template <typename T, typename OT>
 __global__ __launch_bounds__(256) void k_chunk_rowsum_seg(const T *__restrict__ A, int64_t nrows, int64_t ncols,
                                                           int64_t ld, int cs, int vec, OT *__restrict__ out)
 {
     extern __shared__ __align__(16) unsigned char seg_raw[];
+    __shared__ OT sums[64][SEG_ROWS + 1];
     constexpr int V = 16 / sizeof(T);
     using VT = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t r = (int64_t)blockIdx.x * 4 + wave;
-    const bool live = r < nrows;
+    const int64_t r0 = (int64_t)blockIdx.y * SEG_ROWS, span = (int64_t)64 * cs, s0 = blockIdx.x * span;
+    const int L = (int)min(span, ncols - s0), rows = (int)min((int64_t)SEG_ROWS, nrows - r0);
+    const int LV = vec ? L / V * V : 0;   // 16-byte loads where the rows are 16-byte aligned
+    const int c0 = lane * cs, e = min(cs, L - c0);
     T *seg = reinterpret_cast<T *>(seg_raw) + (int64_t)wave * 64 * cs;
-    const int64_t span = (int64_t)64 * cs;
-    for (int64_t s0 = 0; s0 < ncols; s0 += span) {
-        const int L = (int)min(span, ncols - s0);
-        if (live) {
-            const T *a = A + r * ld + s0;
-            const int LV = vec ? L / V * V : 0;   // 16-byte loads where the rows are 16-byte aligned
-            for (int i = lane * V; i < LV; i += 64 * V)
-                *reinterpret_cast<VT *>(seg + i) = *reinterpret_cast<const VT *>(a + i);
-            for (int i = LV + lane; i < L; i += 64) seg[i] = a[i];
-        }
-        __syncthreads();
-        const int c0 = lane * cs;
-        if (live && c0 < L) {
-            const int e = min(cs, L - c0);
-            double acc = 0;
-            for (int c = 0; c < e; ++c) acc += (double)seg[c0 + c];
-            out[(s0 / cs + lane) * nrows + r] = (OT)acc;
-        }
-        __syncthreads();
+    for (int q = wave; q < rows; q += 4) {
+        const T *a = A + (r0 + q) * ld + s0;
+        for (int i = lane * V; i < LV; i += 64 * V)
+            *reinterpret_cast<VT *>(seg + i) = *reinterpret_cast<const VT *>(a + i);
+        for (int i = LV + lane; i < L; i += 64) seg[i] = a[i];
+        // the slice is the wave's own: its LDS operations complete in order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        double acc = 0;
+        for (int c = 0; c < e; ++c) acc += (double)seg[c0 + c];
+        sums[lane][q] = (OT)acc;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 64 * SEG_ROWS; i += 256) {
+        const int k = i / SEG_ROWS, q = i % SEG_ROWS;
+        if (q < rows && k * cs < L) out[(s0 / cs + k) * nrows + r0 + q] = sums[k][q];
     }
 }
 
@@ -2579,14 +2585,15 @@ static int chunk_rowsum_seg(fp_ctx *ctx, const T *A, int64_t nrows, int64_t ncol
 {
     const size_t lds = (size_t)4 * 64 * cs * sizeof(T);
     static bool raised = false;   // per instantiation
-    if (lds > 65536 && !raised) {
+    if (lds > 32768 && !raised) {
         FP_HIP(ctx, hipFuncSetAttribute((const void *)k_chunk_rowsum_seg<T, OT>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 64 * 63 * (int)sizeof(T)));
         raised = true;
     }
-    const int vec = ((uintptr_t)A % 16 == 0 && (ld * sizeof(T)) % 16 == 0) ? 1 : 0;
-    hipLaunchKernelGGL((k_chunk_rowsum_seg<T, OT>), dim3((unsigned)((nrows + 3) / 4)), dim3(256), lds, ctx->stream, A,
-                       nrows, ncols, ld, cs, vec, out);
+    const int vec = ((uintptr_t)A % 16 == 0 && (ld * sizeof(T)) % 16 == 0 && (64 * cs * sizeof(T)) % 16 == 0) ? 1 : 0;
+    const dim3 grid((unsigned)((ncols + 64 * (int64_t)cs - 1) / (64 * (int64_t)cs)),
+                    (unsigned)((nrows + SEG_ROWS - 1) / SEG_ROWS));
+    hipLaunchKernelGGL((k_chunk_rowsum_seg<T, OT>), grid, dim3(256), lds, ctx->stream, A, nrows, ncols, ld, cs, vec, out);
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;
 }
@@ -2698,27 +2705,49 @@ __global__ __launch_bounds__(256) void k_widen_f32(const float *__restrict__ x, 
     if (i < m) y[i] = (double)x[i];
 }
 
-// FLOWPANEL_COARSE_INV=lu: coarse spaces from this size up are inverted through the
-// randomized no-pivot LU and the inverses of its factors instead of the blocked
-// Gauss-Jordan.  Measured on the 30,000-panel BWB with 3,000 coarse vectors: 7.5 ms
-// on the side stream (about 4 nc^3 flop of FP32 MFMA products at ~50 TFLOP/s, and
-// ~280 launches whose host time delays the block inverses queued after them)
-// against 8.3 ms for the 47 Gauss-Jordan passes, and no shorter set-up; the pivoted
-// Gauss-Jordan also survives Galerkin matrices too close to singular for a
-// factorisation without pivoting, so it stays the default.
+// Coarse spaces from COARSE_INV_LU_MIN vectors up are inverted through the randomized
+// no-pivot FP32 LU and the inverses of its factors (about 4 nc^3 flop of MFMA products),
+// smaller ones by the blocked Gauss-Jordan (2 nc^3, but a chain of nc / 64 passes).  3,000
+// vectors (30,000 panels), whole preconditioner set-up: Gauss-Jordan 8.6 ms, LU 6.5 ms (6.2 with the row sums below).
+// The inverse has to return a probe vector from its product with E to COARSE_LU_TOL of the
+// vector's size; a zero pivot or a worse inverse sets info, and the caller repeats the
+// set-up with the Gauss-Jordan, whose verdict is final.  FLOWPANEL_COARSE_INV=gj: always
+// the Gauss-Jordan.
 constexpr int COARSE_INV_LU_MIN = 512;
+constexpr double COARSE_LU_TOL = 0.1;
 constexpr uint64_t COARSE_RBT_SEED = 0x434F415253455242ull;
 
 size_t fp_coarse_work_bytes(int64_t nc)
 {
-    return std::max<size_t>((size_t)2 * nc * nc * sizeof(double), fp_inverse_rbt_work_bytes(nc));
+    return std::max<size_t>((size_t)2 * nc * nc * sizeof(double), fp_inverse_rbt_work_bytes(nc)) + 3 * nc * sizeof(double);
+}
+
+__global__ void k_coarse_solve(const double *__restrict__ Einv, int nc, const double *__restrict__ t,
+                               double *__restrict__ c);
+
+bool fp_coarse_by_lu(int64_t nc)
+{
+    const char *ci = getenv("FLOWPANEL_COARSE_INV");
+    return nc >= COARSE_INV_LU_MIN && !(ci && !strcmp(ci, "gj"));
+}
+
+__global__ __launch_bounds__(256) void k_probe_fill(double *__restrict__ v, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) v[i] = (double)(((uint32_t)i * 2654435761u) >> 8) * 0x1p-24 - 0.5;
+}
+__global__ __launch_bounds__(256) void k_probe_check(const double *__restrict__ v, const double *__restrict__ z, int n,
+                                                     double tol, int *__restrict__ info)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n && !(fabs(z[i] - v[i]) <= tol)) atomicCAS(info, 0, i + 1);
 }
 
 // lookahead: each next Gauss-Jordan chunk's pass runs on ctx->side2 (with the
 // ctx->gj_fork / gj_join events) beside the current chunk's products
 template <typename T>
 int fp_coarse_setup(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, int cs, float *AZ, double *Einv, double *work,
-                    int *info_dev, bool lookahead)
+                    int *info_dev, bool lookahead, bool lu)
 {
     const int nc = (int)((n + cs - 1) / cs);
     if (nc > FP_COARSE_MAX) return fp_fail(ctx, FP_ERR_ARG, "coarse space larger than 4096 vectors");
@@ -2741,15 +2770,19 @@ int fp_coarse_setup(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, int cs, floa
         hipLaunchKernelGGL(k_coarse_galerkin, dim3(nc, nc), dim3(256), 0, ctx->stream, (const float *)AZ, n, cs, nc,
                            Einv);
     }
-    const char *ci = getenv("FLOWPANEL_COARSE_INV");
-    const bool gj = !(ci && !strcmp(ci, "lu"));
     if (nc <= SMALL_INV_LDS) {
         hipLaunchKernelGGL(k_small_inverse_lds, dim3(1), dim3(1024), 0, ctx->stream, Einv, nc, info_dev);
-    } else if (nc >= COARSE_INV_LU_MIN && !gj) {
-        // large coarse spaces: the randomized no-pivot FP32 LU and the inverses of its
-        // factors (the blocked Gauss-Jordan below is a chain of nc / 64 passes)
-        int st = fp_inverse_rbt_f32(ctx, Einv, nc, nc, work, fp_coarse_work_bytes(nc), info_dev, COARSE_RBT_SEED);
+    } else if (lu && fp_coarse_by_lu(nc)) {
+        const size_t wb = fp_coarse_work_bytes(nc) - 3 * nc * sizeof(double);
+        double *v = (double *)((char *)work + wb), *w = v + nc, *z = w + nc;
+        const dim3 gv((unsigned)((nc + 255) / 256)), gr((unsigned)((nc + 3) / 4));
+        hipLaunchKernelGGL(k_probe_fill, gv, dim3(256), 0, ctx->stream, v, nc);
+        hipLaunchKernelGGL(k_coarse_solve, gr, dim3(256), 0, ctx->stream, (const double *)Einv, nc, (const double *)v, w);
+        int st = fp_inverse_rbt_f32(ctx, Einv, nc, nc, work, wb, info_dev, COARSE_RBT_SEED);
         if (st) return st;
+        hipLaunchKernelGGL(k_coarse_solve, gr, dim3(256), 0, ctx->stream, (const double *)Einv, nc, (const double *)w, z);
+        hipLaunchKernelGGL(k_probe_check, gv, dim3(256), 0, ctx->stream, (const double *)v, (const double *)z, nc,
+                           0.5 * COARSE_LU_TOL, info_dev);
     } else {
         // larger coarse spaces: FP32 blocked Gauss-Jordan of E (it only feeds the
         // preconditioner), widened back in place; work (2 nc^2 doubles) holds the
@@ -2766,9 +2799,9 @@ int fp_coarse_setup(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, int cs, floa
     return FP_OK;
 }
 template int fp_coarse_setup<double>(fp_ctx *, const double *, int64_t, int64_t, int, float *, double *, double *, int *,
-                                     bool);
+                                     bool, bool);
 template int fp_coarse_setup<float>(fp_ctx *, const float *, int64_t, int64_t, int, float *, double *, double *, int *,
-                                    bool);
+                                    bool, bool);
 
 // t = Z^T v: one wave per chunk (chunk sums of v)
 __global__ __launch_bounds__(256) void k_coarse_restrict(const double *__restrict__ v, int64_t n, int cs, int nc,

@@ -347,7 +347,9 @@ int fp_bj_apply_inv(fp_ctx *ctx, const float *inv, int64_t n, int block, const d
 // Einv = (Z^T AZ)^-1 from that same AZ (so that Z^T (v - AZ Einv Z^T v) = 0)
 template <typename T>
 int fp_coarse_setup(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, int cs, float *AZ, double *Einv, double *work,
-                    int *info_dev, bool lookahead = false);
+                    int *info_dev, bool lookahead = false, bool lu = true);
+// whether fp_coarse_setup (lu) inverts a coarse space of nc vectors through the no-pivot LU; info set: repeat without
+bool fp_coarse_by_lu(int64_t nc);
 // y = Z Einv Z^T v and r2 = v - AZ Einv Z^T v (tc: 2*nc scratch)
 int fp_coarse_apply(fp_ctx *ctx, const double *v, int64_t n, int cs, const float *AZ, const double *Einv, double *tc,
                     double *y, double *r2);
