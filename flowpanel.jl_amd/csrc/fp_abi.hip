@@ -42,23 +42,19 @@ int fp_hip_fail(fp_ctx *ctx, hipError_t e, const char *what)
 
 namespace {
 
-// device buffer owned by a host scope; large ones go back to their context's
-// pool when released
+// device buffer owned by a host scope; goes back to its context's pool when released
 struct DBuf {
     void *p = nullptr;
-    fp_ctx *owner = nullptr;
+    std::shared_ptr<fp_pool> pool;
     size_t bytes = 0;
     DBuf() = default;
     DBuf(const DBuf &) = delete;
     DBuf &operator=(const DBuf &) = delete;
-    DBuf(DBuf &&o) noexcept : p(o.p), owner(o.owner), bytes(o.bytes) { o.p = nullptr; }
+    DBuf(DBuf &&o) noexcept : p(o.p), pool(std::move(o.pool)), bytes(o.bytes) { o.p = nullptr; }
     ~DBuf() { reset(); }
     void reset()
     {
-        if (p) {
-            if (owner && bytes >= FP_POOL_MIN) fp_pool_put(owner, p, bytes);
-            else (void)hipFree(p);
-        }
+        if (p) pool->put(p, bytes);
         p = nullptr;
     }
     template <typename T> T *as() const { return (T *)p; }
@@ -68,27 +64,17 @@ int dalloc(fp_ctx *ctx, DBuf &b, size_t bytes)
 {
     b.reset();
     if (bytes == 0) bytes = 16;
-    if (bytes >= FP_POOL_MIN) {
-        for (size_t i = 0; i < ctx->pool.size(); ++i)
-            if (ctx->pool[i].bytes == bytes) {
-                b.p = ctx->pool[i].p;
-                ctx->pool.erase(ctx->pool.begin() + (std::ptrdiff_t)i);
-                ctx->pool_bytes -= bytes;
-                b.owner = ctx;
-                b.bytes = bytes;
-                return FP_OK;
-            }
-    }
+    b.pool = ctx->pool;
+    b.bytes = bytes;
+    if ((b.p = ctx->pool->get(bytes))) return FP_OK;
     hipError_t e = hipMalloc(&b.p, bytes);
-    if (e != hipSuccess && !ctx->pool.empty()) {
-        // out of memory with buffers held for re-use: release them and try once more
+    if (e != hipSuccess) {
+        // out of memory: release what is held for re-use and try once more
+        b.p = nullptr;
         (void)hipGetLastError();
-        fp_pool_trim(ctx);
-        e = hipMalloc(&b.p, bytes);
+        if (ctx->pool->trim()) e = hipMalloc(&b.p, bytes);
     }
     if (e != hipSuccess) { b.p = nullptr; return fp_hip_fail(ctx, e, "hipMalloc"); }
-    b.owner = ctx;
-    b.bytes = bytes;
     return FP_OK;
 }
 
@@ -1870,25 +1856,84 @@ struct BatchImpl {
 }  // namespace
 
 // ============================================================================
-void fp_pool_put(fp_ctx *ctx, void *p, size_t bytes)
+void *fp_pool::get(size_t want)
 {
-    ctx->pool.push_back({p, bytes});
-    ctx->pool_bytes += bytes;
-    while (ctx->pool_bytes > FP_POOL_MAX && !ctx->pool.empty()) {
-        (void)hipFree(ctx->pool.front().p);
-        ctx->pool_bytes -= ctx->pool.front().bytes;
-        ctx->pool.erase(ctx->pool.begin());
+    std::lock_guard<std::mutex> g(mu);
+    for (size_t i = blks.size(); i-- > 0;)   // the latest first
+        if (blks[i].bytes == want) {
+            void *p = blks[i].p;
+            drop(i);
+            return p;
+        }
+    return nullptr;
+}
+
+void fp_pool::drop(size_t i)
+{
+    bytes -= blks[i].bytes;
+    small -= blks[i].bytes < FP_POOL_SMALL;
+    blks.erase(blks.begin() + (std::ptrdiff_t)i);
+}
+
+void fp_pool::put(void *p, size_t size)
+{
+    std::vector<void *> out;   // freed outside the lock
+    {
+        std::lock_guard<std::mutex> g(mu);
+        const bool sm = size < FP_POOL_SMALL;
+        bool keep = ctx != nullptr;
+        if (keep && sm)
+            for (hipStream_t s : {ctx->side, ctx->side2, ctx->side3}) {
+                if (!s) continue;
+                const hipError_t e = hipStreamQuery(s);
+                if (e == hipErrorNotReady) (void)hipGetLastError();   // no error of the next launch
+                keep = keep && e == hipSuccess;
+            }
+        if (!keep) {
+            out.push_back(p);
+        } else {
+            blks.push_back({p, size});
+            bytes += size;
+            small += sm;
+            while (!blks.empty() && bytes > FP_POOL_MAX) {
+                out.push_back(blks[0].p);
+                drop(0);
+            }
+            for (size_t i = 0; small > FP_POOL_SMALL_MAX && i < blks.size();) {
+                if (blks[i].bytes < FP_POOL_SMALL) {
+                    out.push_back(blks[i].p);
+                    drop(i);
+                } else {
+                    ++i;
+                }
+            }
+        }
     }
+    for (void *q : out) (void)hipFree(q);
 }
 
-void fp_pool_trim(fp_ctx *ctx)
+bool fp_pool::trim()
 {
-    for (auto &b : ctx->pool) (void)hipFree(b.p);
-    ctx->pool.clear();
-    ctx->pool_bytes = 0;
+    std::vector<Blk> out;
+    {
+        std::lock_guard<std::mutex> g(mu);
+        out.swap(blks);
+        bytes = small = 0;
+    }
+    for (auto &b : out) (void)hipFree(b.p);
+    return !out.empty();
 }
 
-fp_ctx::~fp_ctx() { fp_pool_trim(this); }
+void fp_pool::close()
+{
+    {
+        std::lock_guard<std::mutex> g(mu);
+        ctx = nullptr;
+    }
+    trim();
+}
+
+fp_ctx::~fp_ctx() { pool->close(); }
 
 extern "C" {
 
@@ -1938,7 +1983,7 @@ int fp_ctx_trim(fp_ctx *ctx)
     if (ctx->side) FP_HIP(ctx, hipStreamSynchronize(ctx->side));
     if (ctx->side2) FP_HIP(ctx, hipStreamSynchronize(ctx->side2));
     if (ctx->side3) FP_HIP(ctx, hipStreamSynchronize(ctx->side3));
-    fp_pool_trim(ctx);
+    ctx->pool->trim();
     return FP_OK;
 }
 
@@ -2616,33 +2661,21 @@ int fp_solve_bodies_multi(fp_ctx *ctx, fp_body *const *bodies, int nb, const dou
     fp_solve_stats s{};
     int64_t n = 0;
     for (int b = 0; b < nb; ++b) n += bodies[b]->N;
-    for (int64_t q = 0; q < 3 * n * k; ++q)
-        if (!std::isfinite(Uinfs[q])) return fp_fail(ctx, FP_ERR_ARG, "non-finite freestream");
-    DBuf rhs, x, U;
+    DBuf rhs, x, U, flag;
     if ((st = dalloc(ctx, rhs, (size_t)n * k * sizeof(double))) || (st = dalloc(ctx, x, (size_t)n * k * sizeof(double))) ||
-        (st = dalloc(ctx, U, (size_t)3 * n * k * sizeof(double))))
+        (st = dalloc(ctx, U, (size_t)3 * n * k * sizeof(double))) || (st = dalloc(ctx, flag, sizeof(int))))
         return st;
-    // freestream c of body b as SoA 3 x N_b at U + 3*(c*n + col_b)
-    std::vector<double> soa((size_t)3 * n * k);
-    for (int64_t c = 0; c < k; ++c) {
-        int64_t col = 0;
-        for (int b = 0; b < nb; ++b) {
-            const int64_t N = bodies[b]->N;
-            double *dst = &soa[(size_t)3 * (c * n + col)];
-            for (int64_t i = 0; i < N; ++i)
-                for (int d = 0; d < 3; ++d) dst[d * N + i] = Uinfs[3 * (c * n + col + i) + d];
-            col += N;
-        }
+    FP_HIP(ctx, hipMemcpyAsync(U.p, Uinfs, (size_t)3 * n * k * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    if ((st = fp_fill_f32(ctx, flag.as<float>(), 1, 0.f))) return st;   // (the bits of integer 0)
+    int64_t col = 0;
+    for (int b = 0; b < nb; ++b) {
+        if ((st = fp_rhs_multi(ctx, bodies[b], U.as<double>(), n, col, k, rhs.as<double>(), flag.as<int>()))) return st;
+        col += bodies[b]->N;
     }
-    FP_HIP(ctx, hipMemcpyAsync(U.p, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    for (int64_t c = 0; c < k; ++c) {
-        int64_t col = 0;
-        for (int b = 0; b < nb; ++b) {
-            if ((st = fp_rhs_from(ctx, bodies[b], U.as<double>() + 3 * (c * n + col), rhs.as<double>() + c * n + col)))
-                return st;
-            col += bodies[b]->N;
-        }
-    }
+    int bad = 0;
+    FP_HIP(ctx, hipMemcpyAsync(&bad, flag.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (bad) return fp_fail(ctx, FP_ERR_ARG, "non-finite freestream");
     st = solve_system(ctx, bodies, nb, o, rhs.as<double>(), k, x.as<double>(), s);
     if (stats) *stats = s;
     if (st) return st;

@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <map>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -33,16 +35,33 @@ struct fp_prof_rec {
     hipEvent_t a, b;
 };
 
-struct fp_pool_blk {
-    void *p;
-    size_t bytes;
-};
-// device buffers of at least FP_POOL_MIN bytes are kept by the context when the
-// call that used them ends, for the next request of the same size (repeated
-// solves of one body re-use their AIC storage without hipMalloc/hipFree); at
-// most FP_POOL_MAX bytes are kept, oldest released first
-constexpr size_t FP_POOL_MIN = (size_t)16 << 20;
+// Device buffers are kept when the call that used them ends, for the next request of the same size (repeated
+// solves re-use their storage without hipMalloc / hipFree, which take 5 to 700 us each and wait for the device):
+// at most FP_POOL_MAX bytes, and of buffers below FP_POOL_SMALL at most FP_POOL_SMALL_MAX, oldest released
+// first.  A buffer outlives neither its device work nor the pool: the next user is on the same stream, small
+// buffers are only kept while the context's other streams are idle, and the pool closes with the context
+// (buffers released later are freed).
+struct fp_ctx;
+constexpr size_t FP_POOL_SMALL = (size_t)16 << 20;
+constexpr size_t FP_POOL_SMALL_MAX = 256;
 constexpr size_t FP_POOL_MAX = (size_t)64 << 30;
+struct fp_pool {
+    struct Blk {
+        void *p;
+        size_t bytes;
+    };
+    std::mutex mu;
+    fp_ctx *ctx;   // null once the context is gone
+    std::vector<Blk> blks;
+    size_t bytes = 0, small = 0;
+    explicit fp_pool(fp_ctx *c) : ctx(c) {}
+    void *get(size_t want);            // null if there is none of this size
+    void put(void *p, size_t size);    // keeps it or frees it
+    bool trim();                       // frees all; whether there were any
+    void close();                      // the context ends
+private:
+    void drop(size_t i);
+};
 
 struct fp_ctx {
     int device = 0;
@@ -70,13 +89,10 @@ struct fp_ctx {
     std::vector<fp_prof_rec> prof_pending;
     std::vector<hipEvent_t> prof_pool;  // recycled events
     std::map<std::string, std::pair<int64_t, double>> prof_acc;
-    // released large device buffers (fp_pool_put / fp_pool_trim)
-    std::vector<fp_pool_blk> pool;
-    size_t pool_bytes = 0;
+    // released device buffers
+    std::shared_ptr<fp_pool> pool = std::make_shared<fp_pool>(this);
     ~fp_ctx();
 };
-void fp_pool_put(fp_ctx *ctx, void *p, size_t bytes);
-void fp_pool_trim(fp_ctx *ctx);
 
 // Brackets the launches of one kernel with events on the context stream when
 // profiling is on (fp_ctx_profile); the elapsed times are folded in on query.
@@ -359,7 +375,6 @@ int fp_mat_convert(fp_ctx *ctx, const double *src, int64_t n, int64_t lds, void 
                    int transpose);
 int fp_mat_narrow(fp_ctx *ctx, const double *src, float *dst, int64_t n, int64_t ld);
 int fp_rhs_kernel(fp_ctx *ctx, const fp_body *b, double *rhs);   // rhs_i = -Uinf_i . n_i
-int fp_rhs_from(fp_ctx *ctx, const fp_body *b, const double *uinf_soa, double *rhs);  // the same for a 3 x N SoA Uinf
 int fp_residual_update(fp_ctx *ctx, const double *b, double *r, int64_t n);   // r = b - r
 int fp_dot(fp_ctx *ctx, const double *x, const double *y, int64_t n, double *d_out);
 int fp_axpy(fp_ctx *ctx, double a, const double *x, double *y, int64_t n);
@@ -367,6 +382,8 @@ int fp_axpy(fp_ctx *ctx, double a, const double *x, double *y, int64_t n);
 int fp_resid_dd(fp_ctx *ctx, const double *A, int64_t n, int64_t ld, const double *X, int64_t k, const double *B, double *R);
 int fp_fill(fp_ctx *ctx, double *x, int64_t n, double v);   // x[:] = v (a kernel: safe inside graphs)
 int fp_fill_f32(fp_ctx *ctx, float *x, int64_t n, float v);
+// right-hand sides of k freestreams (3 x n point-major each) for the body at column `col`; bad: not finite
+int fp_rhs_multi(fp_ctx *ctx, const fp_body *b, const double *uinf, int64_t n, int64_t col, int64_t k, double *rhs, int *bad);
 
 // multi-dot out[c] = sum_i V[c*ldv + i] w[i] (part: 256*nv doubles)
 int fp_mdot(fp_ctx *ctx, const double *V, int64_t ldv, int nv, const double *w, int64_t n, double *part,

@@ -1,0 +1,45 @@
+"""Many freestreams in one call, and the context's pool of small buffers."""
+import gc
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k", [1, 3, 65])
+@pytest.mark.parametrize("nc,ns", [(4, 1), (8, 33)])
+def test_freestreams_match_single_solves(fp, geo, k, nc, ns):
+    # 4 and 264 panels: less than a workgroup of points, and one with a remainder
+    grid, sh = geo.loft_wing(n_chord=nc, n_span=ns, span=5.0, sweep_deg=10.0)
+    b = fp.RigidWakeBody(grid, sh)
+    rng = np.random.Generator(np.random.PCG64(k))
+    U = rng.uniform(0.5, 1.5, (3, b.ncells, k))
+    D = np.tile(fp.direction(2.0, 0.0)[:, None], (1, b.nsheddings))
+    many = fp.solve_freestreams(b, U, D, D, solver=fp.solve_ludiv)[0]
+    for c in {0, k // 2, k - 1}:
+        fp.solve(b, np.asfortranarray(U[:, :, c]), D, D, solver=fp.solve_ludiv)
+        # both are solutions to rounding; a wing with a sharp trailing edge: 1e-11 of the largest strength
+        assert np.abs(np.asarray(many)[:, c] - b.strength).max() < 1e-10 * np.abs(b.strength).max()
+    for bad in (np.nan, np.inf):
+        V = U.copy()
+        V[2, b.ncells - 1, k - 1] = bad
+        with pytest.raises(fp.FPError, match="finite"):
+            fp.solve_freestreams(b, V, D, D, solver=fp.solve_ludiv)
+
+
+def test_small_buffers_survive_many_sizes_and_a_closed_context(fp):
+    # more sizes than the pool keeps, then a trim, then matrices that outlive nothing of it
+    rng = np.random.Generator(np.random.PCG64(5))
+    for n in list(range(3, 90)) + [40, 40]:
+        A = rng.standard_normal((n, n)) + n * np.eye(n)
+        x = rng.standard_normal(n)
+        got = fp.solve_ludiv(None, A, A @ x)
+        assert np.abs(got - x).max() < 64 * n * np.finfo(float).eps * np.linalg.cond(A) * np.abs(x).max()
+    fp.context().trim()
+    A = rng.standard_normal((50, 50)) + 50 * np.eye(50)
+    assert np.allclose(fp.solve_ludiv(None, A, A @ np.ones(50)), 1.0)
+    other = fp._native.Context(0)
+    del other
+    gc.collect()
+    assert np.allclose(fp.solve_ludiv(None, A, A @ np.ones(50)), 1.0)
