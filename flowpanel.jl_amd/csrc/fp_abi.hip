@@ -861,6 +861,43 @@ struct Solver {
         return FP_OK;
     }
 
+    // Set-up from the factors of the transposed matrix, if `f` holds FP64 ones of the randomized kind:
+    // U^T A V = L U gives V^T A^T U = U^T L^T, so that the factors, the block inverses and the two
+    // butterflies change sides.  *ok = false, and nothing kept, if `f` pivoted or there is no room.
+    // 4,560 unknowns: 0.3 ms against 4.5 ms for a factorisation.
+    int setup_transposed(Solver &f, fp_solve_stats &stats, bool *ok)
+    {
+        int st;
+        *ok = false;
+        if (a.solver != FP_SOLVER_LU || !f.rbt64 || f.a.n != a.n) return FP_OK;
+        Timer tm(ctx->stream);
+        n4 = f.n4;
+        ld4 = f.ld4;
+        const size_t half = fp_rbt_weights_bytes(a.n) / 2;
+        if ((st = dalloc(ctx, Ar, (size_t)n4 * ld4 * sizeof(double))) ||
+            (st = dalloc(ctx, fwork, fp_getrf_nopiv_work_bytes(n4, sizeof(double)))) ||
+            (st = dalloc(ctx, part, 256 * 4 * sizeof(double))) || (st = dalloc(ctx, dout, 4 * sizeof(double))) ||
+            (st = dalloc(ctx, Wrbt, 2 * half)) || (st = dalloc(ctx, t4, n4 * sizeof(double))) ||
+            (st = dalloc(ctx, t4b, n4 * sizeof(double))) || (st = dalloc(ctx, info, sizeof(int))) ||
+            (st = dalloc(ctx, r, a.n * sizeof(double))) || (st = dalloc(ctx, d, a.n * sizeof(double)))) {
+            if (st != FP_ERR_NOMEM) return st;
+            (void)hipGetLastError();
+            ctx->err.clear();
+            Ar.reset();
+            fwork.reset();
+            return FP_OK;
+        }
+        if ((st = fp_mat_transpose(ctx, f.Ar.as<double>(), n4, ld4, Ar.p, FP_F64)) ||
+            (st = fp_tri_inverse_transposed<double>(ctx, n4, f.fwork.p, fwork.p)))
+            return st;
+        FP_HIP(ctx, hipMemcpyAsync(Wrbt.p, (char *)f.Wrbt.p + half, half, hipMemcpyDeviceToDevice, ctx->stream));
+        FP_HIP(ctx, hipMemcpyAsync((char *)Wrbt.p + half, f.Wrbt.p, half, hipMemcpyDeviceToDevice, ctx->stream));
+        anorm = f.anorm;
+        *ok = rbt64 = true;
+        stats.ms_factor += tm.stop();
+        return FP_OK;
+    }
+
     // D (n x k, ld n) ~ A^-1 R by the FP64 factors of the randomized matrix
     int lu64_correct(const double *R, double *D, int64_t k, double *t, double *t2)
     {
@@ -2467,6 +2504,7 @@ static int lsq_bordered(fp_ctx *ctx, fp_body *const *bodies, int nb, const std::
     FP_HIP(ctx, hipStreamSynchronize(ctx->stream));   // the host vectors go out of scope
     s.ms_assemble = tm.stop();
     // solve B^T Z = E_P, then B y = b_red - Z (Z^T Z)^-1 Z^T b_red, with the chosen solver
+    std::unique_ptr<Solver> first;   // of B^T: its LU serves B as well
     auto square_solve = [&](DBuf &M, const double *rhs_d, int64_t k, double *out) -> int {
         SolveArgs a;
         a.solver = o.solver;
@@ -2490,9 +2528,14 @@ static int lsq_bordered(fp_ctx *ctx, fp_body *const *bodies, int nb, const std::
             a.A32 = W32.as<float>();
         }
         a.nrhs = k;
-        Solver solver(ctx, a, o);
-        if ((s2 = solver.setup(s))) return s2;
-        return solver.solve_multi(rhs_d, out, k, s);
+        std::unique_ptr<Solver> solver(new Solver(ctx, a, o));
+        bool ok = false;
+        if (first && (s2 = solver->setup_transposed(*first, s, &ok))) return s2;
+        first.reset();
+        if (!ok && (s2 = solver->setup(s))) return s2;
+        if ((s2 = solver->solve_multi(rhs_d, out, k, s))) return s2;
+        if (&M == &Bt) first = std::move(solver);
+        return FP_OK;
     };
     if (np) {
         if ((st = square_solve(Bt, E.as<double>(), np, Z.as<double>()))) return st;

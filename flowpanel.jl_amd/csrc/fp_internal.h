@@ -290,6 +290,8 @@ int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void
 // the block inverses of those factors (in the same work), and x (n x k) := U^-1 L^-1 x with them (tmp: n k doubles)
 template <typename T>
 int fp_tri_inverse(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, void *work);
+// the block inverses (work of fp_tri_inverse) of the transposed factors
+template <typename T> int fp_tri_inverse_transposed(fp_ctx *ctx, int64_t n, const void *work, void *work_t);
 template <typename T>
 int fp_lu_solve_nopiv(fp_ctx *ctx, const T *LU, int64_t n, int64_t ld, const void *work, double *x, int64_t k, int64_t ldx,
                       double *tmp);

@@ -1160,6 +1160,32 @@ static void tri_gemvs(fp_ctx *ctx, const T *LU, int64_t n, int64_t ld, const T *
     }
 }
 
+// The block inverses of A^T's factors (L' = U^T, U' = L^T) from those of A's: DL' = DU^T and DU' = DL^T, block by
+// block.  64 x 64 tiles through LDS.
+template <typename T>
+__global__ __launch_bounds__(256) void k_tri_transpose(const T *__restrict__ D, T *__restrict__ E, int64_t half)
+{
+    __shared__ T s[64][65];
+    constexpr int NT = TBIG / 64;
+    const int ti = blockIdx.x / NT, tj = blockIdx.x % NT, x = threadIdx.x & 63, y = threadIdx.x >> 6;
+    const int64_t blk = (int64_t)blockIdx.y * TBIG * TBIG;
+    const T *src = D + (blockIdx.z ? 0 : half) + blk;   // z = 0: DL' from DU
+    T *dst = E + (blockIdx.z ? half : 0) + blk;
+    for (int r = y; r < 64; r += 4) s[r][x] = src[(64 * ti + r) * TBIG + 64 * tj + x];
+    __syncthreads();
+    for (int r = y; r < 64; r += 4) dst[(64 * tj + r) * TBIG + 64 * ti + x] = s[x][r];
+}
+template <typename T> int fp_tri_inverse_transposed(fp_ctx *ctx, int64_t n, const void *work, void *work_t)
+{
+    if (n <= 0) return FP_OK;
+    const int64_t half = lu_dsize(n), nb = (n + TBIG - 1) / TBIG;
+    hipLaunchKernelGGL(k_tri_transpose<T>, dim3((TBIG / 64) * (TBIG / 64), (unsigned)nb, 2), dim3(256), 0, ctx->stream,
+                       (const T *)work, (T *)work_t, half);
+    FP_HIP(ctx, hipGetLastError());
+    return FP_OK;
+}
+template int fp_tri_inverse_transposed<double>(fp_ctx *, int64_t, const void *, void *);
+
 // x (n x k, ldx, FP64) := U^-1 L^-1 x by fp_getrf_nopiv's factors and the block inverses in `work`
 // (fp_tri_inverse); tmp: n k doubles.  Two launches per 512-row block and sweep: the block's solution
 // y = D b, then its contribution to the rows still to be solved.  The chain of launches bounds it
