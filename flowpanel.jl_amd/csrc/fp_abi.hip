@@ -778,7 +778,7 @@ struct Solver {
         st = a.R64 ? fp_rbt_matrix<double, float>(ctx, a.R64, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>())
                    : fp_rbt_matrix<float, float>(ctx, a.A32, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>());
         if (st) return st;
-        // the inverses cost about as much as the factorisation (another (2/3) n^3 on MFMA, and a second matrix) and
+        // the inverses cost about twice the factorisation ((4/3) n^3 against (2/3) n^3 on MFMA) and
         // pay off when many right-hand sides are corrected together; FLOWPANEL_LU32_INVERSE=1/0 forces them
         const char *gi = getenv("FLOWPANEL_LU32_INVERSE");
         inv = gi && (gi[0] == '0' || gi[0] == '1') ? gi[0] == '1' : a.nrhs >= 4;

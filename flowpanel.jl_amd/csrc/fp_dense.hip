@@ -405,32 +405,17 @@ int fp_gemm_sub_lub(fp_ctx *ctx, const fp_lu_desc *d_desc, int nb, int64_t kk, i
     return FP_OK;
 }
 
-// The K range of tile (m0, n0) where one operand (or both) is triangular (FP_TRI_*): tiles of zeros are skipped, half
-// of a product's work and two thirds where both are.  Range bounds are multiples of the tile, so whole K steps.
-__device__ __forceinline__ void gemm_tri_range(int tri, int64_t m0, int64_t n0, int64_t &kb, int64_t &k)
-{
-    int64_t ke = k;
-    kb = 0;
-    if (tri & FP_TRI_A_LOW) ke = min(ke, m0 + GB_M);
-    if (tri & FP_TRI_B_UP) ke = min(ke, n0 + GB_N);
-    if (tri & FP_TRI_A_UP) kb = m0;
-    if (tri & FP_TRI_B_LOW) kb = max(kb, n0);
-    k = ke - kb;
-}
-
 // strided batch: grid row y runs product y (all products the same shape)
 template <typename T>
 __global__ __launch_bounds__(GB_THREADS, 4) void k_gemm_sub(int64_t m, int64_t n, int64_t k, const T *__restrict__ A,
                                                             int64_t lda, const T *__restrict__ B, int64_t ldb,
                                                             T *__restrict__ C, int64_t ldc, int64_t sA, int64_t sB,
-                                                            int64_t sC, int tri)
+                                                            int64_t sC)
 {
     __shared__ GmLds<T> s;
-    int64_t m0, n0, kb;
+    int64_t m0, n0;
     if (!gemm_tile_of(blockIdx.x, m, n, m0, n0)) return;
-    gemm_tri_range(tri, m0, n0, kb, k);
-    if (k <= 0) return;
-    gemm_sub_dma<T>(m, n, k, A + (int64_t)blockIdx.y * sA + kb, lda, B + (int64_t)blockIdx.y * sB + kb * ldb, ldb,
+    gemm_sub_dma<T>(m, n, k, A + (int64_t)blockIdx.y * sA, lda, B + (int64_t)blockIdx.y * sB, ldb,
                     C + (int64_t)blockIdx.y * sC, ldc, m0, n0, s);
 }
 
@@ -438,21 +423,19 @@ template <typename T>
 __global__ __launch_bounds__(GB_THREADS, 2) void k_gemm_sub_reg(int64_t m, int64_t n, int64_t k, const T *__restrict__ A,
                                                                 int64_t lda, const T *__restrict__ B, int64_t ldb,
                                                                 T *__restrict__ C, int64_t ldc, int64_t sA, int64_t sB,
-                                                                int64_t sC, int vec, int tri)
+                                                                int64_t sC, int vec)
 {
     __shared__ GmLds<T> s;
-    int64_t m0, n0, kb;
+    int64_t m0, n0;
     if (!gemm_tile_of(blockIdx.x, m, n, m0, n0)) return;
-    gemm_tri_range(tri, m0, n0, kb, k);
-    if (k <= 0) return;
-    gemm_sub_reg<T>(m, n, k, A + (int64_t)blockIdx.y * sA + kb, lda, B + (int64_t)blockIdx.y * sB + kb * ldb, ldb,
+    gemm_sub_reg<T>(m, n, k, A + (int64_t)blockIdx.y * sA, lda, B + (int64_t)blockIdx.y * sB, ldb,
                     C + (int64_t)blockIdx.y * sC, ldc, vec, m0, n0, s);
 }
 
 // 16-byte accesses need 16-byte aligned rows and offsets; the direct-to-LDS kernel also whole K steps
 template <typename T>
 static void gemm_launch(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const T *A, int64_t lda, int64_t sA, const T *B,
-                        int64_t ldb, int64_t sB, T *C, int64_t ldc, int64_t sC, int batch, int tri)
+                        int64_t ldb, int64_t sB, T *C, int64_t ldc, int64_t sC, int batch)
 {
     const int64_t ntiles = ((m + GB_M - 1) / GB_M) * ((n + GB_N - 1) / GB_N);
     const dim3 grid((unsigned)((ntiles + GB_XCD - 1) / GB_XCD * GB_XCD), (unsigned)batch);
@@ -460,45 +443,44 @@ static void gemm_launch(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const T *A
                     (sA * sizeof(T)) % 16 == 0 && (sB * sizeof(T)) % 16 == 0;
     ProfScope ps(ctx, sizeof(T) == 8 ? "gemm_f64" : "gemm_f32");
     if (vec && k % Gm<T>::KS == 0)
-        hipLaunchKernelGGL(k_gemm_sub<T>, grid, dim3(GB_THREADS), 0, ctx->stream, m, n, k, A, lda, B, ldb, C, ldc, sA, sB, sC,
-                           tri);
+        hipLaunchKernelGGL(k_gemm_sub<T>, grid, dim3(GB_THREADS), 0, ctx->stream, m, n, k, A, lda, B, ldb, C, ldc, sA, sB, sC);
     else
         hipLaunchKernelGGL(k_gemm_sub_reg<T>, grid, dim3(GB_THREADS), 0, ctx->stream, m, n, k, A, lda, B, ldb, C, ldc, sA, sB,
-                           sC, vec, tri);
+                           sC, vec);
 }
 
 template <typename T>
 static int gemm_sub(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const T *A, int64_t lda, const T *B, int64_t ldb,
-                    T *C, int64_t ldc, int tri = 0)
+                    T *C, int64_t ldc)
 {
     if (m <= 0 || n <= 0 || k <= 0) return FP_OK;
-    gemm_launch<T>(ctx, m, n, k, A, lda, 0, B, ldb, 0, C, ldc, 0, 1, tri);
+    gemm_launch<T>(ctx, m, n, k, A, lda, 0, B, ldb, 0, C, ldc, 0, 1);
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;
 }
 
 template <typename T>
 int fp_gemm_sub(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const T *A, int64_t lda, const T *B, int64_t ldb, T *C,
-                int64_t ldc, int tri)
+                int64_t ldc)
 {
-    return gemm_sub<T>(ctx, m, n, k, A, lda, B, ldb, C, ldc, tri);
+    return gemm_sub<T>(ctx, m, n, k, A, lda, B, ldb, C, ldc);
 }
 
 // C_b -= A_b B_b for b < batch, operand b at element offset b * s? from the
 // first (FP32): one launch for a level of small products.
 int fp_gemm_sub_batched_f32(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const float *A, int64_t lda, int64_t sA,
-                            const float *B, int64_t ldb, int64_t sB, float *C, int64_t ldc, int64_t sC, int batch, int tri)
+                            const float *B, int64_t ldb, int64_t sB, float *C, int64_t ldc, int64_t sC, int batch)
 {
     if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return FP_OK;
     if (batch > 65535) return fp_fail(ctx, FP_ERR_UNSUPPORTED, "batched gemm: too many products");
-    gemm_launch<float>(ctx, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, batch, tri);
+    gemm_launch<float>(ctx, m, n, k, A, lda, sA, B, ldb, sB, C, ldc, sC, batch);
     FP_HIP(ctx, hipGetLastError());
     return FP_OK;
 }
 template int fp_gemm_sub<double>(fp_ctx *, int64_t, int64_t, int64_t, const double *, int64_t, const double *, int64_t,
-                                 double *, int64_t, int);
+                                 double *, int64_t);
 template int fp_gemm_sub<float>(fp_ctx *, int64_t, int64_t, int64_t, const float *, int64_t, const float *, int64_t,
-                                float *, int64_t, int);
+                                float *, int64_t);
 
 // Least-squares system of the watertight formulation from C = -(G^T G) (as left
 // by fp_gemm_sub on a zero C): C := G^T G, then every prescribed strength p gets

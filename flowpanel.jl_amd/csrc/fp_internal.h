@@ -236,11 +236,9 @@ struct AssemblyItem {
 // geometry of one body (normals, CPs, areas, Hess-Smith frames)
 int fp_launch_geometry(fp_ctx *ctx, fp_body *b);
 // AIC column block of one body into a row-major matrix (T = float|double); with
-// operands of a product that are triangular (zero beyond their diagonal): A (m x k), B (k x n)
-enum { FP_TRI_A_LOW = 1, FP_TRI_A_UP = 2, FP_TRI_B_LOW = 4, FP_TRI_B_UP = 8 };
 // G32 set, the same entries rounded to FP32 go to G32 (same ld) as well
 int fp_gemm_sub_batched_f32(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const float *A, int64_t lda, int64_t sA,
-                            const float *B, int64_t ldb, int64_t sB, float *C, int64_t ldc, int64_t sC, int batch, int tri = 0);
+                            const float *B, int64_t ldb, int64_t sB, float *C, int64_t ldc, int64_t sC, int batch);
 int fp_body_build_edge_blocks(fp_ctx *ctx, fp_body *b);
 // The diagonal blocks (block x block, identity-padded) of a vortex-ring body's FP32 AIC with its wake
 // columns, compact (block b at X + b * block^2), for the block-Jacobi inverses.
@@ -341,7 +339,7 @@ int fp_gemv(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, const double *x, dou
 // C -= A B (row-major; MFMA tiles)
 template <typename T>
 int fp_gemm_sub(fp_ctx *ctx, int64_t m, int64_t n, int64_t k, const T *A, int64_t lda, const T *B, int64_t ldb, T *C,
-                int64_t ldc, int tri = 0);
+                int64_t ldc);
 // least squares of the watertight formulation: C (= -G^T G) -> normal matrix with the
 // prescribed rows/columns replaced by the identity, b[p] = val_p
 int fp_lsq_fix(fp_ctx *ctx, double *C, int64_t n, int64_t ld, const int64_t *pidx, int np, double *b,

@@ -1,28 +1,23 @@
-// fp_lu_nopiv.hip -- LU of a randomized matrix without pivoting: FP32 for the
-// mixed-precision refinement (FP_SOLVER_LU32_IR, the batch, the coarse space), FP64
-// for FP_SOLVER_LU.
+// fp_lu_nopiv.hip -- FP32 LU of a randomized matrix without pivoting, for the
+// mixed-precision refinement path (FP_SOLVER_LU32_IR).
 //
-// Neither solver rests on the factors alone: residuals of FP64 (of twice FP64 for
-// the FP64 factors) decide the result, and what does not converge is factored with
-// pivoting.  Partial pivoting is what makes the blocked LU latency-bound at the
-// sizes of a wing (4k-12k unknowns): every 32-column sub-panel runs a tournament of
-// pivot searches.  A random butterfly transformation (RBT, Parker 1995; Baboulin,
-// Dongarra, Herrmann, Tomov 2013) A_r = U^T A V with two depth-2 recursive
-// butterflies U, V makes pivoting unnecessary with probability close to one, and
-// the LU of A_r is then a plain blocked right-looking factorisation:
+// The refinement needs only an FP32 approximate inverse; the FP64 residual
+// r = b - A x decides the result.  Partial pivoting is what makes the blocked
+// LU latency-bound at the sizes of a wing (4k-12k unknowns): every 32-column
+// sub-panel runs a tournament of pivot searches.  A random butterfly
+// transformation (RBT, Parker 1995; Baboulin, Dongarra, Herrmann, Tomov 2013)
+// A_r = U^T A V with two depth-2 recursive butterflies U, V makes pivoting
+// unnecessary with probability close to one, and the LU of A_r is then a
+// plain blocked right-looking factorisation:
 //
 //   per 256-column outer block:
-//     k_lu_first   the first outer block's first 64 x 64 diagonal block, with the
-//                  explicit inverses of L11 and U11;
-//     k_lu_update  the other outer blocks: their columns' share of the previous
-//                  block's rank-256 update, and their first diagonal block;
+//     k_lu_first   its first 64 x 64 diagonal block, with the explicit inverses of
+//                  L11 and U11;
 //     k_lu_step    (four times) L21 = A21 U11^-1 and the update of the outer
 //                  block's columns, one workgroup per 64 rows; the first of them
-//                  factors the next diagonal block; the launch also carries tiles
-//                  of the previous block's update;
-//     k_lu_urow    the U rows, inside the outer block and right of it (blocked
-//                  substitution);
-//     fp_gemm_sub  the part of the rank-256 update that no launch carries.
+//                  factors the next diagonal block;
+//     k_lu_urow    the U rows, inside the outer block and right of it (blocked substitution);
+//     fp_gemm_sub  the rank-256 trailing update.
 //
 // A x = b becomes  A_r y = U^T b,  x = V y.  A depth-2 butterfly couples only
 // the four indices {p, p + m, p + 2m, p + 3m} (m = n4 / 4, n4 = n rounded up
@@ -1316,36 +1311,34 @@ int fp_trtri_nopiv_f32(fp_ctx *ctx, const float *A, int64_t n, int64_t ld, float
         if (P > 0) {
             if ((st = fp_fill_f32(ctx, T, P * s * ld, 0.f))) return st;
             // lower: T_p = -L_JI Y_II, Y_JI -= Y_JJ T_p
-            if ((st = fp_gemm_sub_batched_f32(ctx, s, s, s, A + s * ld, ld, step, YL, ld, step, T, ld, s * ld, (int)P,
-                                              FP_TRI_B_LOW)))
+            if ((st = fp_gemm_sub_batched_f32(ctx, s, s, s, A + s * ld, ld, step, YL, ld, step, T, ld, s * ld, (int)P)))
                 return st;
             if ((st = fp_gemm_sub_batched_f32(ctx, s, s, s, YL + s * ld + s, ld, step, T, ld, s * ld, YL + s * ld, ld,
-                                              step, (int)P, FP_TRI_A_LOW)))
+                                              step, (int)P)))
                 return st;
             if ((st = fp_fill_f32(ctx, T, P * s * ld, 0.f))) return st;
             // upper: T_p = -U_IJ Y_JJ, Y_IJ -= Y_II T_p
             if ((st = fp_gemm_sub_batched_f32(ctx, s, s, s, A + s, ld, step, YU + s * ld + s, ld, step, T, ld, s * ld,
-                                              (int)P, FP_TRI_B_UP)))
+                                              (int)P)))
                 return st;
-            if ((st = fp_gemm_sub_batched_f32(ctx, s, s, s, YU, ld, step, T, ld, s * ld, YU + s, ld, step, (int)P,
-                                              FP_TRI_A_UP)))
+            if ((st = fp_gemm_sub_batched_f32(ctx, s, s, s, YU, ld, step, T, ld, s * ld, YU + s, ld, step, (int)P)))
                 return st;
         }
         if (rem > s) {   // the last pair: I = [r, r + s), J = [r + s, n)
             const int64_t r = 2 * s * P, sj = rem - s, rj = r + s;
             if ((st = fp_fill_f32(ctx, T, s * ld, 0.f))) return st;
             if ((st = fp_gemm_sub_batched_f32(ctx, sj, s, s, A + rj * ld + r, ld, 0, YL + r * ld + r, ld, 0, T, ld, 0,
-                                              1, FP_TRI_B_LOW)))
+                                              1)))
                 return st;
             if ((st = fp_gemm_sub_batched_f32(ctx, sj, s, sj, YL + rj * ld + rj, ld, 0, T, ld, 0, YL + rj * ld + r, ld,
-                                              0, 1, FP_TRI_A_LOW)))
+                                              0, 1)))
                 return st;
             if ((st = fp_fill_f32(ctx, T, s * ld, 0.f))) return st;
             if ((st = fp_gemm_sub_batched_f32(ctx, s, sj, sj, A + r * ld + rj, ld, 0, YU + rj * ld + rj, ld, 0, T, ld,
-                                              0, 1, FP_TRI_B_UP)))
+                                              0, 1)))
                 return st;
             if ((st = fp_gemm_sub_batched_f32(ctx, s, sj, s, YU + r * ld + r, ld, 0, T, ld, 0, YU + r * ld + rj, ld, 0,
-                                              1, FP_TRI_A_UP)))
+                                              1)))
                 return st;
         }
     }
@@ -1386,7 +1379,7 @@ int fp_inverse_rbt_f32(fp_ctx *ctx, double *E, int64_t n, int64_t lde, void *wor
     if ((st = fp_trtri_nopiv_f32(ctx, Ar, n4, ld4, YL, YU, T))) return st;
     // Ar <- -(YU YL) = -U^-1 L^-1 (the factors are no longer needed)
     if ((st = fp_fill_f32(ctx, Ar, sz, 0.f))) return st;
-    if ((st = fp_gemm_sub<float>(ctx, n4, n4, n4, YU, ld4, YL, ld4, Ar, ld4, FP_TRI_A_UP | FP_TRI_B_LOW))) return st;
+    if ((st = fp_gemm_sub<float>(ctx, n4, n4, n4, YU, ld4, YL, ld4, Ar, ld4))) return st;
     hipLaunchKernelGGL(k_rbt_unmatrix, dim3((unsigned)((m + 255) / 256), (unsigned)m), dim3(256), 0, ctx->stream,
                        (const float *)Ar, ld4, m, E, n, lde, (const double *)W);
     FP_HIP(ctx, hipGetLastError());
