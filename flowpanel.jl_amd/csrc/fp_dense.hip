@@ -1679,6 +1679,78 @@ __global__ __launch_bounds__(256) void k_gemv_multi(const T *__restrict__ A, int
         }
 }
 
+// Y = A X for an FP32 matrix and 9 or more columns, FP64 products and sums on the matrix cores: a workgroup takes
+// MM_R rows and 16 NX columns, its eight waves chunks of 16 entries of the rows in turn.  v_mfma_f64_4x4x4_4b with
+// the columns of X as its 16 rows and four rows of A as its columns: a wave reads 16 bytes of A and 32 of X per
+// lane for four instructions per operand pair, straight from memory, and the waves' sums meet in LDS in order.
+// The vector form above re-reads A for every eight columns and converts it each time: 4,800^2 times 64 columns
+// 326 us, here 221 (the loads of X bound it).  For an FP64 matrix both take the same (313, 315), so that one keeps
+// the vector form.
+constexpr int MM_R = 16, MM_W = 8;
+template <int NX>
+__global__ __launch_bounds__(64 * MM_W, 4) void k_gemm_multi(const float *__restrict__ A, int64_t n, int64_t ld,
+                                                             const double *__restrict__ X, int64_t ldx, int k,
+                                                             double *__restrict__ Y, int64_t ldy)
+{
+    __shared__ double red[MM_W][16 * NX][MM_R];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t r0 = (int64_t)blockIdx.x * MM_R;
+    const int c0 = blockIdx.y * 16 * NX, kq = 4 * (lane >> 4);
+    const float *pa[4];
+    const double *px[NX];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) pa[g] = A + min(r0 + 4 * g + (lane & 3), n - 1) * ld + kq;
+#pragma unroll
+    for (int g = 0; g < NX; ++g) px[g] = X + (int64_t)min(c0 + 16 * g + (lane & 15), k - 1) * ldx + kq;
+    double acc[NX][4];
+#pragma unroll
+    for (int g = 0; g < NX; ++g)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) acc[g][h] = 0.0;
+    for (int64_t c = 16 * wave; c < n; c += 16 * MM_W) {
+        float va[4][4];
+        double vx[NX][4];
+        if (c + 16 <= n) {   // uniform
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) va[g][e] = pa[g][c + e];
+#pragma unroll
+            for (int g = 0; g < NX; ++g)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) vx[g][e] = px[g][c + e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool in = c + kq + e < n;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) va[g][e] = in ? pa[g][c + e] : 0.f;
+#pragma unroll
+                for (int g = 0; g < NX; ++g) vx[g][e] = in ? px[g][c + e] : 0.0;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int g = 0; g < NX; ++g)
+#pragma unroll
+                for (int h = 0; h < 4; ++h)
+                    acc[g][h] = __builtin_amdgcn_mfma_f64_4x4x4f64(vx[g][e], (double)va[h][e], acc[g][h], 0, 0, 0);
+    }
+#pragma unroll
+    for (int g = 0; g < NX; ++g)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) red[wave][16 * g + 4 * ((lane >> 2) & 3) + (lane >> 4)][4 * h + (lane & 3)] = acc[g][h];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 16 * NX * MM_R; i += 64 * MM_W) {
+        const int col = i / MM_R, row = i % MM_R;
+        double v = 0;
+#pragma unroll
+        for (int w = 0; w < MM_W; ++w) v += red[w][col][row];
+        if (c0 + col < k && r0 + row < n) Y[(int64_t)(c0 + col) * ldy + r0 + row] = v;
+    }
+}
+
 template <typename T>
 int fp_gemv_multi(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, const double *X, int64_t ldx, int64_t k, double *Y,
                   int64_t ldy)
@@ -1686,6 +1758,16 @@ int fp_gemv_multi(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, const double *
     if (n <= 0 || k <= 0) return FP_OK;
     if (ld % 4 || ((uintptr_t)A & 15)) return fp_fail(ctx, FP_ERR_ARG, "gemv needs an aligned matrix");
     ProfScope ps(ctx, sizeof(T) == 8 ? "gemv_multi_f64" : "gemv_multi_f32");
+    if constexpr (sizeof(T) == 4) {
+        if (k > GEMVM_NV) {   // up to one group of columns the vector form reads A once and wastes no products
+            const int nx = k > 32 ? 4 : k > 16 ? 2 : 1;
+            const dim3 g((unsigned)((n + MM_R - 1) / MM_R), (unsigned)((k + 16 * nx - 1) / (16 * nx)));
+            auto kern = nx == 4 ? k_gemm_multi<4> : nx == 2 ? k_gemm_multi<2> : k_gemm_multi<1>;
+            hipLaunchKernelGGL(kern, g, dim3(64 * MM_W), 0, ctx->stream, A, n, ld, X, ldx, (int)k, Y, ldy);
+            FP_HIP(ctx, hipGetLastError());
+            return FP_OK;
+        }
+    }
     const dim3 grid((unsigned)((n + 4 * GEMVM_R - 1) / (4 * GEMVM_R)), (unsigned)((k + GEMVM_NV - 1) / GEMVM_NV));
     hipLaunchKernelGGL(k_gemv_multi<T>, grid, dim3(256), 0, ctx->stream, A, n, ld, X, ldx, (int)k, Y, ldy);
     FP_HIP(ctx, hipGetLastError());

@@ -1,23 +1,28 @@
-// fp_lu_nopiv.hip -- FP32 LU of a randomized matrix without pivoting, for the
-// mixed-precision refinement path (FP_SOLVER_LU32_IR).
+// fp_lu_nopiv.hip -- LU of a randomized matrix without pivoting: FP32 for the
+// mixed-precision refinement (FP_SOLVER_LU32_IR, the batch, the coarse space), FP64
+// for FP_SOLVER_LU.
 //
-// The refinement needs only an FP32 approximate inverse; the FP64 residual
-// r = b - A x decides the result.  Partial pivoting is what makes the blocked
-// LU latency-bound at the sizes of a wing (4k-12k unknowns): every 32-column
-// sub-panel runs a tournament of pivot searches.  A random butterfly
-// transformation (RBT, Parker 1995; Baboulin, Dongarra, Herrmann, Tomov 2013)
-// A_r = U^T A V with two depth-2 recursive butterflies U, V makes pivoting
-// unnecessary with probability close to one, and the LU of A_r is then a
-// plain blocked right-looking factorisation:
+// Neither solver rests on the factors alone: residuals of FP64 (of twice FP64 for
+// the FP64 factors) decide the result, and what does not converge is factored with
+// pivoting.  Partial pivoting is what makes the blocked LU latency-bound at the
+// sizes of a wing (4k-12k unknowns): every 32-column sub-panel runs a tournament of
+// pivot searches.  A random butterfly transformation (RBT, Parker 1995; Baboulin,
+// Dongarra, Herrmann, Tomov 2013) A_r = U^T A V with two depth-2 recursive
+// butterflies U, V makes pivoting unnecessary with probability close to one, and
+// the LU of A_r is then a plain blocked right-looking factorisation:
 //
 //   per 256-column outer block:
-//     k_lu_first   its first 64 x 64 diagonal block, with the explicit inverses of
-//                  L11 and U11;
+//     k_lu_first   the first outer block's first 64 x 64 diagonal block, with the
+//                  explicit inverses of L11 and U11;
+//     k_lu_update  the other outer blocks: their columns' share of the previous
+//                  block's rank-256 update, and their first diagonal block;
 //     k_lu_step    (four times) L21 = A21 U11^-1 and the update of the outer
 //                  block's columns, one workgroup per 64 rows; the first of them
-//                  factors the next diagonal block;
-//     k_lu_urow    the U rows, inside the outer block and right of it (blocked substitution);
-//     fp_gemm_sub  the rank-256 trailing update.
+//                  factors the next diagonal block; the launch also carries tiles
+//                  of the previous block's update;
+//     k_lu_urow    the U rows, inside the outer block and right of it (blocked
+//                  substitution);
+//     fp_gemm_sub  the part of the rank-256 update that no launch carries.
 //
 // A x = b becomes  A_r y = U^T b,  x = V y.  A depth-2 butterfly couples only
 // the four indices {p, p + m, p + 2m, p + 3m} (m = n4 / 4, n4 = n rounded up

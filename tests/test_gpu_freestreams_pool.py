@@ -43,3 +43,22 @@ def test_small_buffers_survive_many_sizes_and_a_closed_context(fp):
     del other
     gc.collect()
     assert np.allclose(fp.solve_ludiv(None, A, A @ np.ones(50)), 1.0)
+
+
+@pytest.mark.parametrize("k", [8, 9, 16, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("nc,ns", [(6, 7), (10, 5), (8, 33)])
+def test_many_refined_freestreams_match_single_solves(fp, geo, k, nc, ns):
+    # the refinement's products with many columns: column groups of 8 (vector form), 16, 32 and 64 and one more;
+    # 42, 50 and 264 rows (tiles of 16, rows no multiple of 4 or 16).  Uniform freestreams: the
+    # ring matrix of a closed body is nearly singular for one with a net flux through it
+    grid, sh = geo.loft_wing(n_chord=nc, n_span=ns, span=5.0, sweep_deg=10.0)
+    b = fp.RigidWakeBody(grid, sh)
+    rng = np.random.Generator(np.random.PCG64(100 + k))
+    V = np.stack([fp.direction(a, s) for a, s in rng.uniform(-5, 5, (k, 2))], axis=1)
+    U = np.repeat(V[:, None, :], b.ncells, axis=1)
+    D = np.tile(fp.direction(2.0, 0.0)[:, None], (1, b.nsheddings))
+    many = np.asarray(fp.solve_freestreams(b, U, D, D, solver=fp.solve_lu32_ir)[0])
+    for c in sorted({0, 7, k // 2, k - 1}):
+        fp.solve(b, np.asfortranarray(U[:, :, c]), D, D, solver=fp.solve_ludiv)
+        # refined to a residual of 1e-12; the wing's amplification of it stays below 1e-8 of the largest strength
+        assert np.abs(many[:, c] - b.strength).max() < 1e-8 * np.abs(b.strength).max(), c
