@@ -351,9 +351,10 @@ struct BJPrecond : Precond {
         // the coarse space does not depend on the block inverses: it is built on the side
         // stream beside them.  The host spends a few microseconds per launch: a short coarse
         // chain (up to COARSE_FIRST_MAX vectors) is queued first so that it starts at once;
-        // a long one (nc / 64 Gauss-Jordan chunks of five launches and two events each) is
-        // queued after the block inverses, which would otherwise wait for the host to finish
-        // queueing it (3,000 vectors: the block inverses began 4.5 ms late)
+        // a long one (an LU of nc / 64 steps, the inverses of its factors) is queued after the
+        // block inverses, which would otherwise wait for the host to finish queueing it (3,000
+        // vectors: 31.2 ms a solve against 31.0; with the 350 calls of the Gauss-Jordan the block
+        // inverses began 4.5 ms late)
         auto queue_coarse = [&]() -> int {
             // the coarse inverse's look-ahead passes on the fourth stream, with events of their own
             // (the block inverses' look-ahead uses the third stream and gj_fork / gj_join meanwhile)
