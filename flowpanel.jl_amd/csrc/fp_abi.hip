@@ -854,7 +854,8 @@ struct Solver {
         FP_HIP(ctx, hipMemcpyAsync(hc, chk.p, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
         anorm = std::sqrt(hc[0]);
-        if (hinfo || !std::isfinite(anorm) || !(hc[1] > 1e-11 * anorm)) {
+        // (the norm's square has to be in range for the tests on it to mean anything)
+        if (hinfo || !(anorm > 1e-140 && anorm < 1e140) || !(hc[1] > 1e-11 * anorm)) {
             Ar.reset();
             return FP_OK;
         }
@@ -912,13 +913,16 @@ struct Solver {
     // at least one.  A correction of relative size d_i leaves an error of about d_i (d_i / d_{i-1}), so it
     // goes on until that is below 1e-17 (one correction on a wing) or they no longer halve.  With
     // residuals of plain FP64 the strengths of wings were 2 to 4 times as far from the exact ones as the
-    // pivoted LU's; with these they are nearer than those.  *ok = false when the final residual is above
-    // 1e-14 (|A|_F |x| + |b|): the factors are not those of a backward stable solve.  *rel (may be null):
-    // the worst column's |r| / |b|.
+    // pivoted LU's; with these they are nearer than those.  *ok = false unless the final residual of every
+    // column is within 1e-14 (|A|_F |x| + |b|): the factors are not those of a backward stable solve.  A
+    // column whose right-hand side holds a NaN has no solution to judge and does not speak for the others; one
+    // with an infinity, or whose squares leave the range of FP64, is left to the pivoted LU with the rest.
+    // *rel (may be null): the worst column's |r| / |b|.
     int rbt64_solve(const double *B, double *X, int64_t k, bool *ok, double *rel)
     {
         const int64_t n = a.n;
         int st;
+        *ok = false;
         DBuf Rk, Dk, tk, tk2, nr;
         double *R = r.as<double>(), *Dp = d.as<double>(), *t = t4.as<double>(), *t2 = t4b.as<double>();
         if ((st = dalloc(ctx, nr, 3 * k * sizeof(double)))) return st;
@@ -928,18 +932,16 @@ struct Solver {
                 return st;
             R = Rk.as<double>(); Dp = Dk.as<double>(); t = tk.as<double>(); t2 = tk2.as<double>();
         }
-        double *nrm = nr.as<double>();
         std::vector<double> h(3 * k);
+        const double *hu = h.data(), *hx = hu + k, *hb = hx + k;
         auto norms = [&](const double *u) -> int {   // |u|, |X|, |B| of every column
             int s2;
-            if ((s2 = fp_colnorm2(ctx, u, n, n, k, nrm)) || (s2 = fp_colnorm2(ctx, X, n, n, k, nrm + k)) ||
-                (s2 = fp_colnorm2(ctx, B, n, n, k, nrm + 2 * k)))
-                return s2;
-            FP_HIP(ctx, hipMemcpyAsync(h.data(), nrm, 3 * k * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+            if ((s2 = fp_colnorms(ctx, u, X, B, n, k, nr.as<double>()))) return s2;
+            FP_HIP(ctx, hipMemcpyAsync(h.data(), nr.p, 3 * k * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
             FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            for (double &v : h) v = std::sqrt(v);
             return FP_OK;
         };
+        auto judged = [&](int64_t c) { return !std::isnan(hb[c]); };
         if ((st = lu64_correct(B, X, k, t, t2))) return st;
         double before = 1.0;
         for (int it = 0; it < 6; ++it) {
@@ -947,21 +949,25 @@ struct Solver {
                 (st = fp_axpby(ctx, 1.0, Dp, 1.0, X, n * k)) || (st = norms(Dp)))
                 return st;
             double size = 0;
-            for (int64_t c = 0; c < k; ++c)
-                if (h[k + c] > 0 || h[c] > 0) size = worst_residual(size, h[c] / h[k + c]);
+            for (int64_t c = 0; c < k; ++c) {
+                if (!judged(c)) continue;
+                if (hb[c] != 0 && !(hb[c] > 1e-150 && hb[c] < 1e150)) return FP_OK;
+                if (hx[c] > 0 || !(hu[c] == 0)) size = worst_residual(size, hu[c] / hx[c]);
+            }
             if (!(size * std::min(1.0, size / before) > 1e-17) || !(size < 0.5 * before)) break;
             before = size;
         }
         if ((st = fp_resid_dd(ctx, a.A64, n, a.ld, X, k, B, R)) || (st = norms(R))) return st;
-        double eta = 0, worst = 0;
+        double worst = 0;
+        bool stable = true;
         for (int64_t c = 0; c < k; ++c) {
-            const double den = anorm * h[k + c] + h[2 * k + c];
-            if (den > 0 || !(h[c] == 0)) eta = worst_residual(eta, h[c] / den);
-            worst = worst_residual(worst, h[2 * k + c] > 0 ? h[c] / h[2 * k + c]
-                                                           : (h[c] == 0 && h[2 * k + c] == 0 ? 0.0 : NAN));
+            worst = worst_residual(worst, hb[c] > 0 ? hu[c] / hb[c] : (hu[c] == 0 && hb[c] == 0 ? 0.0 : NAN));
+            if (!judged(c)) continue;
+            const double den = anorm * hx[c] + hb[c];
+            stable = stable && std::isfinite(den) && hu[c] <= 1e-14 * den;   // (a NaN is not stable)
         }
         if (rel) *rel = worst;
-        *ok = !(eta > 1e-14);   // a right-hand side that is not finite shows in the result, whatever the factors
+        *ok = stable;
         return FP_OK;
     }
 

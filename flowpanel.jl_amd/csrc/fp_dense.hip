@@ -1922,6 +1922,54 @@ int fp_colnorm2(fp_ctx *ctx, const double *R, int64_t n, int64_t ld, int64_t k, 
     return FP_OK;
 }
 
+// |v| of the columns of three column-major n x k blocks (ld n) at out, out + k and out + 2 k: finite whenever it
+// is in the range of FP64, also where the squares are not (a second pass on scaled values then); NaN if an entry
+// is NaN, else infinite if one is.
+__global__ __launch_bounds__(256) void k_colnorms(const double *__restrict__ U, const double *__restrict__ X,
+                                                  const double *__restrict__ B, int64_t n, int64_t k,
+                                                  double *__restrict__ out)
+{
+    __shared__ double red[4], redm[4];
+    const int w = threadIdx.x >> 6;
+    const bool first = (threadIdx.x & 63) == 0;
+    const double *v = (blockIdx.y == 0 ? U : blockIdx.y == 1 ? X : B) + (int64_t)blockIdx.x * n;
+    double scale = 1.0, m = 0.0;
+    for (int pass = 0;; ++pass) {
+        double s = 0;
+        m = 0;
+        for (int64_t i = threadIdx.x; i < n; i += 256) {
+            const double x = v[i] * scale;
+            s += x * x;
+            m = fmax(m, fabs(x));   // (drops NaN; the sum does not)
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            s += __shfl_xor(s, o);
+            m = fmax(m, __shfl_xor(m, o));
+        }
+        if (first) { red[w] = s; redm[w] = m; }
+        __syncthreads();
+        s = red[0] + red[1] + red[2] + red[3];
+        m = fmax(fmax(redm[0], redm[1]), fmax(redm[2], redm[3]));
+        // uniform: in range, zeros, or not finite whatever the scale
+        if (pass || (s > 1e-280 && s < 1e280) || m == 0 || isinf(m) || s != s) {
+            if (threadIdx.x == 0) out[(int64_t)blockIdx.y * k + blockIdx.x] = sqrt(s) / scale;
+            return;
+        }
+        int e;
+        (void)frexp(m, &e);
+        scale = ldexp(1.0, min(max(-e, -1000), 1000));
+        __syncthreads();   // red is written again
+    }
+}
+
+int fp_colnorms(fp_ctx *ctx, const double *U, const double *X, const double *B, int64_t n, int64_t k, double *out)
+{
+    if (k <= 0) return FP_OK;
+    hipLaunchKernelGGL(k_colnorms, dim3((unsigned)k, 3), dim3(256), 0, ctx->stream, U, X, B, n, k, out);
+    FP_HIP(ctx, hipGetLastError());
+    return FP_OK;
+}
+
 // ----------------------------------------------------------------------------
 // Block-Jacobi inverses by Gauss-Jordan with partial pivoting, the block held
 // in registers (TG x TG threads, thread (tr, tc) holding rows tr + TG i and

@@ -352,6 +352,8 @@ int fp_gemv_multi(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, const double *
                   int64_t ldy);
 // out[c] = |R[:, c]|^2 (device)
 int fp_colnorm2(fp_ctx *ctx, const double *R, int64_t n, int64_t ld, int64_t k, double *out);
+// the columns' norms of three n x k blocks (ld n), 3 k of them, in range wherever the norm itself is
+int fp_colnorms(fp_ctx *ctx, const double *U, const double *X, const double *B, int64_t n, int64_t k, double *out);
 // Block-Jacobi inverses straight from A, block <= 1024: Gauss-Jordan in registers
 // up to 256 rows, above that blocked Gauss-Jordan over chunks of at most 256
 // rows (scratch of fp_bj_gj_scratch_floats floats), and their application

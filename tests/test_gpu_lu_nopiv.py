@@ -104,3 +104,95 @@ def test_refined_solution_is_accurate_to_the_data(fp, n, k):
     X = rng.integers(-9, 10, (n, k)).astype(float)
     got = fp.solve_ludiv(None, A, A @ X).reshape(n, k)
     assert np.abs(got - X).max() < 1e-14 * np.abs(X).max()
+
+
+def _butterfly(m, seed):
+    """One side of the randomization of order 4 m that the library draws from `seed` (splitmix64)."""
+    def draw(i):
+        mask = (1 << 64) - 1
+        z = (seed + (i + 1) * 0x9E3779B97F4A7C15) & mask
+        z = ((z ^ (z >> 30)) * 0xBF58476D1CE4E5B9) & mask
+        z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & mask
+        return np.exp((((z ^ (z >> 31)) >> 11) * 2.0 ** -53 - 0.5) / 10.0)
+    F, h = np.zeros((4 * m, 4 * m)), np.sqrt(0.5)
+    for q in range(m):
+        r = [draw(8 * q + j) for j in range(8)]
+        Z = h * np.array([[r[0], 0, r[1], 0], [0, r[2], 0, r[3]], [r[0], 0, -r[1], 0], [0, r[2], 0, -r[3]]])
+        Y = h * np.array([[r[4], r[5], 0, 0], [r[4], -r[5], 0, 0], [0, 0, r[6], r[7]], [0, 0, r[6], -r[7]]])
+        at = q + m * np.arange(4)
+        F[np.ix_(at, at)] = Y @ Z
+    return F
+
+
+SEED = 0x46504C5533324952
+
+
+def _passes_the_pivots_only(n=64):
+    """Condition ~200, but the randomized matrix starts with two pivots of 1e-10 of its norm one behind the other:
+    above the pivot test's 1e-11, with an element growth of 1e16 that leaves the factors no correct digit."""
+    rng = np.random.default_rng(1)
+    M = rng.standard_normal((n, n))
+    M[0, 0] = M[1, 1] = 1e-10 * np.linalg.norm(M)
+    M[1, 0] = 0.0
+    U, V = _butterfly(n // 4, SEED), _butterfly(n // 4, SEED ^ 0x5DEECE66D)
+    return np.linalg.solve(U.T, M) @ np.linalg.inv(V)
+
+
+def _counted(fp, A, B):
+    ctx = fp._native.context()
+    ctx.profile(True)
+    X = fp.solve_ludiv(None, A, B)
+    counts = {name: ctx.profile_get(name)[0] for name in ("getrs", "panel_tslu")}
+    ctx.profile(False)
+    return X, counts
+
+
+@pytest.mark.parametrize("k", [1, 3])
+def test_factors_without_a_correct_digit_fall_back_to_pivoting(fp, k):
+    A = _passes_the_pivots_only()
+    n = A.shape[0]
+    X = np.random.default_rng(2).standard_normal((n, k))
+    B = A @ X
+    got, counts = _counted(fp, A, B if k > 1 else B[:, 0])
+    assert counts["getrs"] >= 3 and counts["panel_tslu"] > 0, counts   # refined, found wanting, then pivoted
+    bound = 64 * n * EPS * np.linalg.cond(A)
+    assert np.abs(got.reshape(n, k) - X).max() <= bound * np.abs(X).max()
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("at", [0, 1, 2])
+def test_a_column_that_is_not_finite_leaves_the_others(fp, bad, at):
+    # the pivoted LU treats columns independently; so does the refined one, also where only pivoting serves
+    for A in (_matrix(200, 11)[0], _passes_the_pivots_only()):
+        n = A.shape[0]
+        X = np.random.default_rng(12).standard_normal((n, 3))
+        B = A @ X
+        B[5, at] = bad
+        got = fp.solve_ludiv(None, A, B)
+        assert not np.isfinite(got[:, at]).all()
+        rest = [c for c in range(3) if c != at]
+        bound = 64 * n * EPS * np.linalg.cond(A)
+        assert np.abs(got[:, rest] - X[:, rest]).max() <= bound * np.abs(X[:, rest]).max()
+
+
+@pytest.mark.parametrize("scale", [1e-200, 1e200])
+def test_columns_beyond_the_range_of_their_squares(fp, scale):
+    # |b|^2 over- or underflows: the acceptance test cannot see such a column, and a right-hand side of zeros is one
+    # with nothing to see
+    A = _passes_the_pivots_only()
+    n = A.shape[0]
+    X = np.random.default_rng(13).standard_normal((n, 3))
+    X[:, 1] = 0.0
+    B = A @ X
+    B[:, 0] *= scale
+    got = fp.solve_ludiv(None, A, B)
+    got[:, 0] /= scale
+    bound = 64 * n * EPS * np.linalg.cond(A)
+    assert np.abs(got - X).max() <= bound * np.abs(X).max()
+    assert not got[:, 1].any()
+    # zeros alone are no reason to pivot
+    A, rng = _matrix(130, 14)
+    X = rng.standard_normal((130, 3))
+    X[:, 1] = 0.0
+    got, counts = _counted(fp, A, A @ X)
+    assert counts["panel_tslu"] == 0 and not got[:, 1].any()
