@@ -78,6 +78,22 @@ int dalloc(fp_ctx *ctx, DBuf &b, size_t bytes)
     return FP_OK;
 }
 
+// Host to device and back on the context's stream, done on return.  (A blocking hipMemcpy runs on the null stream,
+// which does not wait for the context's: it could write a buffer from the pool under the late work of a call that
+// ended with an error.)
+int h2d(fp_ctx *ctx, void *d, const void *h, size_t bytes)
+{
+    FP_HIP(ctx, hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, ctx->stream));
+    FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return FP_OK;
+}
+int d2h(fp_ctx *ctx, void *h, const void *d, size_t bytes)
+{
+    FP_HIP(ctx, hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return FP_OK;
+}
+
 int64_t round_ld(int64_t n) { return std::max<int64_t>(64, (n + 63) / 64 * 64); }
 
 struct Timer {
@@ -1352,7 +1368,7 @@ int upload_soa3(fp_ctx *ctx, const double *h, int64_t n, double *d)
     std::vector<double> tmp(3 * n);
     for (int64_t i = 0; i < n; ++i)
         for (int c = 0; c < 3; ++c) tmp[c * n + i] = h[3 * i + c];
-    FP_HIP(ctx, hipMemcpy(d, tmp.data(), 3 * n * sizeof(double), hipMemcpyHostToDevice));
+    if (int st = h2d(ctx, d, tmp.data(), 3 * n * sizeof(double))) return st;
     return FP_OK;
 }
 
@@ -1402,8 +1418,8 @@ int build_horseshoes(fp_ctx *ctx, fp_body *b)
     tab.insert(tab.end(), gptr.begin(), gptr.end());
     FP_HIP(ctx, hipMalloc((void **)&b->d_hh, soa.size() * sizeof(double)));
     FP_HIP(ctx, hipMalloc((void **)&b->d_hcol, tab.size() * sizeof(int)));
-    FP_HIP(ctx, hipMemcpy(b->d_hh, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice));
-    FP_HIP(ctx, hipMemcpy(b->d_hcol, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice));
+    if (int st = h2d(ctx, b->d_hh, soa.data(), soa.size() * sizeof(double))) return st;
+    if (int st = h2d(ctx, b->d_hcol, tab.data(), tab.size() * sizeof(int))) return st;
     b->nh = nh;
     b->nhg = ng;
     return FP_OK;
@@ -1615,7 +1631,7 @@ struct BatchImpl {
         }
         int st = dalloc(ctx, items, it.size() * sizeof(AssemblyItem));
         if (st) return st;
-        FP_HIP(ctx, hipMemcpy(items.p, it.data(), it.size() * sizeof(AssemblyItem), hipMemcpyHostToDevice));
+        if ((st = h2d(ctx, items.p, it.data(), it.size() * sizeof(AssemblyItem)))) return st;
         return FP_OK;
     }
 
@@ -1760,7 +1776,7 @@ struct BatchImpl {
             lu_tab.reset();
             if ((st = dalloc(ctx, lu_tab, t.size() * sizeof(fp_lu_desc)))) return st;
         }
-        FP_HIP(ctx, hipMemcpy(lu_tab.p, t.data(), t.size() * sizeof(fp_lu_desc), hipMemcpyHostToDevice));
+        if ((st = h2d(ctx, lu_tab.p, t.data(), t.size() * sizeof(fp_lu_desc)))) return st;
         return FP_OK;
     }
 
@@ -1926,7 +1942,7 @@ void fp_pool::put(void *p, size_t size)
         std::lock_guard<std::mutex> g(mu);
         const bool sm = size < FP_POOL_SMALL;
         bool keep = ctx != nullptr;
-        if (keep && sm)
+        if (keep)
             for (hipStream_t s : {ctx->side, ctx->side2, ctx->side3}) {
                 if (!s) continue;
                 const hipError_t e = hipStreamQuery(s);
@@ -2203,9 +2219,9 @@ int fp_body_create(fp_ctx *ctx, const double *nodes, int64_t nnodes, const int64
     FP_HIP(ctx, hipMalloc((void **)&b->d_geo, (size_t)FP_GEO_STRIDE * N * sizeof(double)));
     FP_HIP(ctx, hipMalloc((void **)&b->d_uinf, (size_t)3 * N * sizeof(double)));
     FP_HIP(ctx, hipMalloc((void **)&b->d_strength, N * sizeof(double)));
-    FP_HIP(ctx, hipMemcpy(b->d_pv, pv.data(), pv.size() * sizeof(double), hipMemcpyHostToDevice));
-    FP_HIP(ctx, hipMemcpy(b->d_nv, nvv.data(), N * sizeof(int), hipMemcpyHostToDevice));
-    FP_HIP(ctx, hipMemset(b->d_strength, 0, N * sizeof(double)));
+    if (int st = h2d(ctx, b->d_pv, pv.data(), pv.size() * sizeof(double))) return st;
+    if (int st = h2d(ctx, b->d_nv, nvv.data(), N * sizeof(int))) return st;
+    FP_HIP(ctx, hipMemsetAsync(b->d_strength, 0, N * sizeof(double), ctx->stream));
     int st = fp_launch_geometry(ctx, b.get());
     if (st) return st;
     if ((st = fp_body_build_edge_blocks(ctx, b.get()))) return st;
@@ -2270,7 +2286,7 @@ int fp_body_set_strength(fp_ctx *ctx, fp_body *b, const double *s)
 {
     if (!ctx || !b || b->ctx != ctx || !s) return FP_ERR_ARG;
     if (b->ns > 0 && !b->has_wake) return fp_fail(ctx, FP_ERR_ARG, "set the wake directions first");
-    FP_HIP(ctx, hipMemcpy(b->d_strength, s, b->N * sizeof(double), hipMemcpyHostToDevice));
+    if (int st = h2d(ctx, b->d_strength, s, b->N * sizeof(double))) return st;
     b->solved = true;
     return FP_OK;
 }
@@ -2769,7 +2785,7 @@ int fp_mat_upload(fp_ctx *ctx, int64_t n, const double *Ah, fp_mat **out)
     DBuf tmp;
     int st = dalloc(ctx, tmp, (size_t)n * n * sizeof(double));
     if (st) return st;
-    FP_HIP(ctx, hipMemcpy(tmp.p, Ah, (size_t)n * n * sizeof(double), hipMemcpyHostToDevice));
+    if ((st = h2d(ctx, tmp.p, Ah, (size_t)n * n * sizeof(double)))) return st;
     FP_HIP(ctx, hipMalloc(&m->A, (size_t)n * m->ld * sizeof(double)));
     if ((st = fp_mat_convert(ctx, tmp.as<double>(), n, n, m->A, m->ld, FP_F64, 1))) { (void)hipFree(m->A); return st; }
     FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -2902,7 +2918,7 @@ int fp_solve_mat(fp_ctx *ctx, fp_mat *m, const double *bh, int64_t k, double *xh
     DBuf b, x, W;
     if ((st = dalloc(ctx, b, (size_t)n * k * sizeof(double)))) return st;
     if ((st = dalloc(ctx, x, (size_t)n * k * sizeof(double)))) return st;
-    FP_HIP(ctx, hipMemcpy(b.p, bh, (size_t)n * k * sizeof(double), hipMemcpyHostToDevice));
+    if ((st = h2d(ctx, b.p, bh, (size_t)n * k * sizeof(double)))) return st;
     // FP64 residual operator: stored FP64 matrix, else matrix-free from the bodies
     std::unique_ptr<Operator> resid;
     std::unique_ptr<MatrixFreeOp> mf;
@@ -2952,7 +2968,7 @@ int fp_solve_mat(fp_ctx *ctx, fp_mat *m, const double *bh, int64_t k, double *xh
     st = solver.setup(s);
     if (!st) st = solver.solve_multi(b.as<double>(), x.as<double>(), k, s);
     if (st) { if (stats) *stats = s; return st; }
-    FP_HIP(ctx, hipMemcpy(xh, x.p, (size_t)n * k * sizeof(double), hipMemcpyDeviceToHost));
+    if ((st = d2h(ctx, xh, x.p, (size_t)n * k * sizeof(double)))) return st;
     if (stats) *stats = s;
     return FP_OK;
 }
@@ -3081,7 +3097,7 @@ static int ensure_shedding_on_device(fp_ctx *ctx, fp_body *b)
 {
     if (b->ns > 0 && !b->d_sh) {
         FP_HIP(ctx, hipMalloc((void **)&b->d_sh, 6 * b->ns * sizeof(int64_t)));
-        FP_HIP(ctx, hipMemcpy(b->d_sh, b->shedding.data(), 6 * b->ns * sizeof(int64_t), hipMemcpyHostToDevice));
+        if (int st = h2d(ctx, b->d_sh, b->shedding.data(), 6 * b->ns * sizeof(int64_t))) return st;
     }
     return FP_OK;
 }
@@ -3795,7 +3811,7 @@ int fp_batch_solve(fp_ctx *ctx, fp_batch *h, fp_batch_stats *stats)
     bool refall = false;
     for (auto &bb : B.bodies) {
         int info = 0;
-        FP_HIP(ctx, hipMemcpy(&info, bb->info.p, sizeof(int), hipMemcpyDeviceToHost));
+        if ((st = d2h(ctx, &info, bb->info.p, sizeof(int)))) return st;
         if (info && B.lu32() && !bb->pivoted) {
             // the randomized no-pivot LU met a bad pivot: this body switches to the pivoted LU
             if ((st = B.fallback(*bb))) return st;
@@ -3901,7 +3917,7 @@ static int body_neighbors(fp_ctx *ctx, fp_body *b)
         }
     }
     FP_HIP(ctx, hipMalloc((void **)&b->d_nbr, nb.size() * sizeof(int)));
-    FP_HIP(ctx, hipMemcpy(b->d_nbr, nb.data(), nb.size() * sizeof(int), hipMemcpyHostToDevice));
+    if (int st = h2d(ctx, b->d_nbr, nb.data(), nb.size() * sizeof(int))) return st;
     return FP_OK;
 }
 
@@ -3928,7 +3944,7 @@ int fp_calcfield_ugradmu(fp_ctx *ctx, fp_body *const *bodies, int nb, int te_cor
         if ((st = body_neighbors(ctx, b))) return st;
         if (b->ns > 0 && !b->d_sh) {
             FP_HIP(ctx, hipMalloc((void **)&b->d_sh, 6 * b->ns * sizeof(int64_t)));
-            FP_HIP(ctx, hipMemcpy(b->d_sh, b->shedding.data(), 6 * b->ns * sizeof(int64_t), hipMemcpyHostToDevice));
+            if ((st = h2d(ctx, b->d_sh, b->shedding.data(), 6 * b->ns * sizeof(int64_t)))) return st;
         }
         if ((st = fp_launch_ugradmu(ctx, b, b->d_nbr, b->d_sh, te_correction, o.as<double>() + 3 * off))) return st;
         off += b->N;
@@ -4099,7 +4115,7 @@ int fp_calcfield_ugradmu_combined(fp_ctx *ctx, fp_body *const *bodies, int nb, i
         if ((st = body_neighbors(ctx, b))) return st;
         if (b->ns > 0 && !b->d_sh) {
             FP_HIP(ctx, hipMalloc((void **)&b->d_sh, 6 * b->ns * sizeof(int64_t)));
-            FP_HIP(ctx, hipMemcpy(b->d_sh, b->shedding.data(), 6 * b->ns * sizeof(int64_t), hipMemcpyHostToDevice));
+            if ((st = h2d(ctx, b->d_sh, b->shedding.data(), 6 * b->ns * sizeof(int64_t)))) return st;
         }
         if ((st = dalloc(ctx, cellv, 3 * std::max<int64_t>(1, N) * sizeof(double)))) return st;
         if ((st = dalloc(ctx, nodev, 3 * std::max<int64_t>(1, N) * sizeof(double)))) return st;

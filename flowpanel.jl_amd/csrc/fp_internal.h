@@ -38,9 +38,12 @@ struct fp_prof_rec {
 // Device buffers are kept when the call that used them ends, for the next request of the same size (repeated
 // solves re-use their storage without hipMalloc / hipFree, which take 5 to 700 us each and wait for the device):
 // at most FP_POOL_MAX bytes, and of buffers below FP_POOL_SMALL at most FP_POOL_SMALL_MAX, oldest released
-// first.  A buffer outlives neither its device work nor the pool: the next user is on the same stream, small
-// buffers are only kept while the context's other streams are idle, and the pool closes with the context
-// (buffers released later are freed).
+// first.  A kept buffer may still be in use by work queued on the context's stream (a call that ends with an error
+// does not wait for what it queued), so whatever touches a buffer next does so on that stream or on one that was
+// made to wait for it afterwards: host copies go through h2d / d2h of fp_abi.hip, never through the null
+// stream.  The context's other streams are not waited for: while one of them is busy a released buffer is
+// freed (hipFree waits for the device), not kept.  The pool closes with the context (buffers released later
+// are freed).
 struct fp_ctx;
 constexpr size_t FP_POOL_SMALL = (size_t)16 << 20;
 constexpr size_t FP_POOL_SMALL_MAX = 256;

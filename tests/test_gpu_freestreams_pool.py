@@ -29,7 +29,7 @@ def test_freestreams_match_single_solves(fp, geo, k, nc, ns):
 
 
 def test_small_buffers_survive_many_sizes_and_a_closed_context(fp):
-    # more sizes than the pool keeps, then a trim, then matrices that outlive nothing of it
+    # more sizes than the pool keeps, then a trim, then another context closed with buffers in its pool
     rng = np.random.Generator(np.random.PCG64(5))
     for n in list(range(3, 90)) + [40, 40]:
         A = rng.standard_normal((n, n)) + n * np.eye(n)
@@ -43,6 +43,23 @@ def test_small_buffers_survive_many_sizes_and_a_closed_context(fp):
     del other
     gc.collect()
     assert np.allclose(fp.solve_ludiv(None, A, A @ np.ones(50)), 1.0)
+
+
+def test_a_failed_call_leaves_nothing_behind_in_the_pool(fp, geo):
+    # the call is refused by the preconditioner's set-up while its assembly is still queued; the matrix uploaded next
+    # has the assembly's size (n = 4,800 is a multiple of 64, so that n x n and n x ld are the same)
+    grid, sh = geo.loft_wing(n_chord=60, n_span=80, span=10.0, taper=0.5, sweep_deg=30.0)
+    b = fp.RigidWakeBody(grid, sh)
+    V = fp.direction(4.0, 0.0)
+    U, D = np.tile(V[:, None], (1, b.ncells)), np.tile(V[:, None], (1, b.nsheddings))
+    rng = np.random.Generator(np.random.PCG64(6))
+    n = b.ncells
+    A = rng.standard_normal((n, n)) + n * np.eye(n)
+    for _ in range(3):
+        with pytest.raises(fp.FPError, match="4096"):
+            fp.solve(b, U, D, D, solver=fp.solve_gmres, solver_optargs={"precond_block": 60, "coarse_block": 1})
+        got = fp.solve_ludiv(None, A, A @ np.ones(n))
+        assert np.abs(got - 1.0).max() < 1e-12
 
 
 @pytest.mark.parametrize("k", [8, 9, 16, 17, 32, 33, 64, 65])

@@ -221,3 +221,12 @@ def test_revolution_liftbody_is_closed_and_outward(fp, orc):
     for pi, nia, nib, pj, nja, njb in tsh.T:
         ci, cj = tg.cell(pi), tg.cell(pj)
         assert np.allclose(X[:, ci[nia]], X[:, cj[njb]]) and np.allclose(X[:, ci[nib]], X[:, cj[nja]])
+
+
+def test_host_copies_wait_for_the_context_stream():
+    # buffers are re-used while work of the context's (non-blocking) stream may still be queued on them: a copy on
+    # the null stream would not wait for it
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flowpanel.jl_amd", "csrc")
+    with open(os.path.join(csrc, "fp_abi.hip")) as f:
+        code = re.sub(r"//[^\n]*", "", f.read())
+    assert re.findall(r"\bhip(?:Memcpy|Memset)\s*\(", code) == []
