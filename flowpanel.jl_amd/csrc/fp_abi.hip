@@ -67,15 +67,25 @@ int dalloc(fp_ctx *ctx, DBuf &b, size_t bytes)
     b.pool = ctx->pool;
     b.bytes = bytes;
     if ((b.p = ctx->pool->get(bytes))) return FP_OK;
-    hipError_t e = hipMalloc(&b.p, bytes);
+    hipError_t e = ctx->pool->room(bytes) ? hipMalloc(&b.p, bytes) : hipErrorOutOfMemory;
     if (e != hipSuccess) {
         // out of memory: release what is held for re-use and try once more
         b.p = nullptr;
         (void)hipGetLastError();
-        if (ctx->pool->trim()) e = hipMalloc(&b.p, bytes);
+        if (ctx->pool->trim() && ctx->pool->room(bytes)) e = hipMalloc(&b.p, bytes);
     }
     if (e != hipSuccess) { b.p = nullptr; return fp_hip_fail(ctx, e, "hipMalloc"); }
+    ctx->pool->taken(bytes);
     return FP_OK;
+}
+
+// A step that can do without: true (and the error forgotten) if `st` says that there was no room for it.
+bool no_room(fp_ctx *ctx, int st)
+{
+    if (st != FP_ERR_NOMEM) return false;
+    (void)hipGetLastError();
+    ctx->err.clear();
+    return true;
 }
 
 // Host to device and back on the context's stream, done on return.  (A blocking hipMemcpy runs on the null stream,
@@ -776,13 +786,34 @@ struct Solver {
     const void *diag_ready = nullptr;
     Solver(fp_ctx *c, const SolveArgs &args, const fp_solve_opts &opts) : ctx(c), a(args), o(opts) {}
 
-    // Randomize and factor without pivoting; false (and nothing kept) when a
-    // diagonal block meets a zero or non-finite pivot: the caller then pivots.
+    // gives back what the randomized path holds
+    void rbt_release()
+    {
+        rbt = rbt64 = inv = false;
+        for (DBuf *b : {&Ar, &Wrbt, &fwork, &t4, &t4b, &YL, &YU, &w4}) b->reset();
+        if (a.solver == FP_SOLVER_LU) {
+            r.reset();
+            d.reset();
+        }
+    }
+
+    // Randomize and factor without pivoting; false (and nothing kept) when a diagonal block meets a zero or
+    // non-finite pivot, or where there is no room for it: the caller then pivots in place.
     int rbt_setup(bool *ok)
+    {
+        *ok = false;
+        const int st = rbt_factor(ok);
+        if (*ok) {
+            rbt = true;
+            return st;
+        }
+        rbt_release();
+        return no_room(ctx, st) ? FP_OK : st;
+    }
+    int rbt_factor(bool *ok)
     {
         const int64_t n = a.n;
         int st;
-        *ok = false;
         diag_ready = nullptr;
         n4 = fp_rbt_size(n);
         ld4 = round_ld(n4);
@@ -813,13 +844,7 @@ struct Solver {
         int hinfo = 0;
         FP_HIP(ctx, hipMemcpyAsync(&hinfo, info.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (hinfo) {
-            Ar.reset();
-            YL.reset();
-            YU.reset();
-            inv = false;
-            return FP_OK;
-        }
+        if (hinfo) return FP_OK;
         if (inv) {
             // the triangular inverses take Ar's place; the scratch T reuses Ar after them
             DBuf T;
@@ -829,29 +854,33 @@ struct Solver {
             Ar.reset();
         }
         *ok = true;
-        rbt = true;
         return FP_OK;
     }
 
-    // FP64 LU of the randomized matrix without pivoting (FP_SOLVER_LU), with refinement; the matrix
-    // itself stays as it is.  *ok = false, and nothing kept, where it does not serve: no room for the copy, a zero or non-finite pivot, or a pivot below 1e-11 |A|_F (a matrix
-    // singular to rounding, or near it): those take the pivoted LU in place, with its results and errors.
+    // FP64 LU of the randomized matrix without pivoting (FP_SOLVER_LU), with refinement; the matrix itself stays as it
+    // is.  *ok = false, and nothing kept, where it does not serve: no room for the copy, the block inverses or
+    // the vectors, a zero or non-finite pivot, or a pivot below 1e-11 |A|_F (a matrix singular to rounding, or near
+    // it): those take the pivoted LU in place, with its results and errors.
     int rbt64_setup(bool *ok)
+    {
+        *ok = false;
+        const int st = rbt64_factor(ok);
+        if (*ok) {
+            rbt64 = true;
+            return st;
+        }
+        rbt_release();
+        return no_room(ctx, st) ? FP_OK : st;
+    }
+    int rbt64_factor(bool *ok)
     {
         const int64_t n = a.n;
         int st;
-        *ok = false;
         n4 = fp_rbt_size(n);
         ld4 = round_ld(n4);
         DBuf np, chk;
-        if ((st = dalloc(ctx, Ar, (size_t)n4 * ld4 * sizeof(double)))) {
-            if (st != FP_ERR_NOMEM) return st;
-            (void)hipGetLastError();
-            ctx->err.clear();
-            return FP_OK;
-        }
         const int64_t parts = fp_rbt_norm_parts(n);
-        if ((st = dalloc(ctx, Wrbt, fp_rbt_weights_bytes(n))) ||
+        if ((st = dalloc(ctx, Ar, (size_t)n4 * ld4 * sizeof(double))) || (st = dalloc(ctx, Wrbt, fp_rbt_weights_bytes(n))) ||
             (st = dalloc(ctx, t4, n4 * sizeof(double))) || (st = dalloc(ctx, t4b, n4 * sizeof(double))) ||
             (st = dalloc(ctx, fwork, fp_getrf_nopiv_work_bytes(n4, sizeof(double)))) || (st = dalloc(ctx, info, sizeof(int))) ||
             (st = dalloc(ctx, np, parts * sizeof(double))) || (st = dalloc(ctx, chk, 2 * sizeof(double))) ||
@@ -871,11 +900,7 @@ struct Solver {
         FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
         anorm = std::sqrt(hc[0]);
         // (the norm's square has to be in range for the tests on it to mean anything)
-        if (hinfo || !(anorm > 1e-140 && anorm < 1e140) || !(hc[1] > 1e-11 * anorm)) {
-            Ar.reset();
-            return FP_OK;
-        }
-        *ok = rbt64 = true;
+        *ok = !hinfo && anorm > 1e-140 && anorm < 1e140 && hc[1] > 1e-11 * anorm;
         return FP_OK;
     }
 
@@ -898,12 +923,8 @@ struct Solver {
             (st = dalloc(ctx, Wrbt, 2 * half)) || (st = dalloc(ctx, t4, n4 * sizeof(double))) ||
             (st = dalloc(ctx, t4b, n4 * sizeof(double))) || (st = dalloc(ctx, info, sizeof(int))) ||
             (st = dalloc(ctx, r, a.n * sizeof(double))) || (st = dalloc(ctx, d, a.n * sizeof(double)))) {
-            if (st != FP_ERR_NOMEM) return st;
-            (void)hipGetLastError();
-            ctx->err.clear();
-            Ar.reset();
-            fwork.reset();
-            return FP_OK;
+            rbt_release();
+            return no_room(ctx, st) ? FP_OK : st;
         }
         if ((st = fp_mat_transpose(ctx, f.Ar.as<double>(), n4, ld4, Ar.p, FP_F64)) ||
             (st = fp_tri_inverse_transposed<double>(ctx, n4, f.fwork.p, fwork.p)))
@@ -941,13 +962,14 @@ struct Solver {
         *ok = false;
         DBuf Rk, Dk, tk, tk2, nr;
         double *R = r.as<double>(), *Dp = d.as<double>(), *t = t4.as<double>(), *t2 = t4b.as<double>();
-        if ((st = dalloc(ctx, nr, 3 * k * sizeof(double)))) return st;
-        if (k > 1) {
-            if ((st = dalloc(ctx, Rk, (size_t)n * k * sizeof(double))) || (st = dalloc(ctx, Dk, (size_t)n * k * sizeof(double))) ||
-                (st = dalloc(ctx, tk, (size_t)n4 * k * sizeof(double))) || (st = dalloc(ctx, tk2, (size_t)n4 * k * sizeof(double))))
-                return st;
+        st = dalloc(ctx, nr, 3 * k * sizeof(double));
+        if (k > 1 && !st) {
+            if (!(st = dalloc(ctx, Rk, (size_t)n * k * sizeof(double))) && !(st = dalloc(ctx, Dk, (size_t)n * k * sizeof(double))) &&
+                !(st = dalloc(ctx, tk, (size_t)n4 * k * sizeof(double))))
+                st = dalloc(ctx, tk2, (size_t)n4 * k * sizeof(double));
             R = Rk.as<double>(); Dp = Dk.as<double>(); t = tk.as<double>(); t2 = tk2.as<double>();
         }
+        if (st) return no_room(ctx, st) ? FP_OK : st;   // (not ok: the pivoted LU needs none of them)
         std::vector<double> h(3 * k);
         const double *hu = h.data(), *hx = hu + k, *hb = hx + k;
         auto norms = [&](const double *u) -> int {   // |u|, |X|, |B| of every column
@@ -991,8 +1013,7 @@ struct Solver {
     int lu64_pivoted(fp_solve_stats &stats)
     {
         int st;
-        rbt64 = false;
-        Ar.reset();
+        rbt_release();
         if ((st = dalloc(ctx, perm, a.n * sizeof(int)))) return st;
         if ((st = factor<double>(ctx, a.A64, a.n, a.ld, perm.as<int>(), &stats.info))) return st;
         return dalloc(ctx, work, fp_getrs_work_bytes(a.n, 1));
@@ -1002,12 +1023,8 @@ struct Solver {
     int lu32_pivoted(fp_solve_stats &stats)
     {
         int st;
-        rbt = false;
-        inv = false;
+        rbt_release();
         diag_ready = nullptr;
-        Ar.reset();
-        YL.reset();
-        YU.reset();
         if ((st = dalloc(ctx, perm, a.n * sizeof(int)))) return st;
         if ((st = factor<float>(ctx, a.A32, a.n, a.ld, perm.as<int>(), &stats.info))) return st;
         return dalloc(ctx, work, fp_getrs_work_bytes(a.n, 1));
@@ -1145,6 +1162,8 @@ struct Solver {
             }
         } else if (a.solver == FP_SOLVER_LU32_IR || a.solver == FP_SOLVER_GMRES_IR) {
             if (!a.A32) return fp_fail(ctx, FP_ERR_ARG, "internal: no FP32 matrix");
+            // (first: what the randomized factors leave of the memory is theirs to lose)
+            if ((st = dalloc(ctx, r, n * sizeof(double))) || (st = dalloc(ctx, d, n * sizeof(double)))) return st;
             if (a.solver == FP_SOLVER_LU32_IR) {
                 bool ok = false;
                 const char *pv = getenv("FLOWPANEL_LU32_PIVOTED");
@@ -1157,8 +1176,6 @@ struct Solver {
                 g.reset(new Gmres());
                 if ((st = g->init(ctx, n, std::max(1, o.restart)))) return st;
             }
-            if ((st = dalloc(ctx, r, n * sizeof(double)))) return st;
-            if ((st = dalloc(ctx, d, n * sizeof(double)))) return st;
         } else {
             return fp_fail(ctx, FP_ERR_ARG, "unknown solver");
         }
@@ -1298,9 +1315,9 @@ struct Solver {
             }
             if ((st = lu64_pivoted(stats))) return st;
         }
-        DBuf wk;
+        DBuf wk;   // of the pivoted factors
         const size_t wbytes = fp_getrs_work_bytes(n, k);
-        if ((st = dalloc(ctx, wk, wbytes))) return st;
+        if (!rbt && (st = dalloc(ctx, wk, wbytes))) return st;
         FP_HIP(ctx, hipMemcpyAsync(X, B, (size_t)n * k * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
         if (a.solver == FP_SOLVER_LU) {
             if ((st = fp_getrs<double>(ctx, a.A64, n, a.ld, perm.as<int>(), X, k, n, wk.p, wbytes))) return st;
@@ -1327,8 +1344,12 @@ struct Solver {
         for (;;) {
         while (!converged(rel, o.tol) && std::isfinite(rel) && it - it0 < o.max_refine && !stalled) {
             const double before = rel;
-            if ((st = lu32_correct(R.as<double>(), D.as<double>(), k, wk.p, wbytes)))
-                return st;
+            st = lu32_correct(R.as<double>(), D.as<double>(), k, wk.p, wbytes);
+            if (rbt && no_room(ctx, st)) {   // for the randomized factors' vectors: the pivoted ones take over
+                stalled = true;
+                continue;
+            }
+            if (st) return st;
             if ((st = fp_axpby(ctx, 1.0, D.as<double>(), 1.0, X, n * k))) return st;
             if ((st = fp_gemv_multi<double>(ctx, a.R64, n, a.ld, X, n, k, R.as<double>(), n))) return st;
             if ((st = fp_residual_update(ctx, B, R.as<double>(), n * k))) return st;
@@ -1343,7 +1364,7 @@ struct Solver {
         }
         // the randomized no-pivot factors failed to converge: start over with the pivoted LU
         if (rbt && !converged(rel, o.tol) && std::isfinite(rel0)) {
-            if ((st = lu32_pivoted(stats))) return st;
+            if ((st = lu32_pivoted(stats)) || (st = dalloc(ctx, wk, wbytes))) return st;
             it0 = it;
             stalled = false;
             FP_HIP(ctx, hipMemsetAsync(X, 0, (size_t)n * k * sizeof(double), ctx->stream));
@@ -1923,9 +1944,22 @@ void *fp_pool::get(size_t want)
         if (blks[i].bytes == want) {
             void *p = blks[i].p;
             drop(i);
+            live += want;
             return p;
         }
     return nullptr;
+}
+
+bool fp_pool::room(size_t want)
+{
+    std::lock_guard<std::mutex> g(mu);
+    return want <= limit && live + bytes <= limit - want;
+}
+
+void fp_pool::taken(size_t size)
+{
+    std::lock_guard<std::mutex> g(mu);
+    live += size;
 }
 
 void fp_pool::drop(size_t i)
@@ -1941,6 +1975,7 @@ void fp_pool::put(void *p, size_t size)
     {
         std::lock_guard<std::mutex> g(mu);
         const bool sm = size < FP_POOL_SMALL;
+        live -= size;
         bool keep = ctx != nullptr;
         if (keep)
             for (hipStream_t s : {ctx->side, ctx->side2, ctx->side3}) {
@@ -1996,6 +2031,12 @@ void fp_pool::close()
 fp_ctx::~fp_ctx() { pool->close(); }
 
 extern "C" {
+
+void fp_test_limit_bytes(fp_ctx *ctx, int64_t bytes)
+{
+    std::lock_guard<std::mutex> g(ctx->pool->mu);
+    ctx->pool->limit = bytes < 0 ? SIZE_MAX : (size_t)bytes;
+}
 
 void fp_solve_opts_default(fp_solve_opts *o, int solver)
 {

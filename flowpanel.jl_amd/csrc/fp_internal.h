@@ -57,8 +57,12 @@ struct fp_pool {
     fp_ctx *ctx;   // null once the context is gone
     std::vector<Blk> blks;
     size_t bytes = 0, small = 0;
+    // bytes handed out, and the most that may be handed out and kept (fp_test_limit_bytes)
+    size_t live = 0, limit = SIZE_MAX;
     explicit fp_pool(fp_ctx *c) : ctx(c) {}
     void *get(size_t want);            // null if there is none of this size
+    bool room(size_t want);            // whether `want` bytes more stay within the limit
+    void taken(size_t size);           // a buffer allocated for the context
     void put(void *p, size_t size);    // keeps it or frees it
     bool trim();                       // frees all; whether there were any
     void close();                      // the context ends
@@ -96,6 +100,10 @@ struct fp_ctx {
     std::shared_ptr<fp_pool> pool = std::make_shared<fp_pool>(this);
     ~fp_ctx();
 };
+
+// For tests of a full device, without filling one: an allocation that would take the context's buffers beyond `bytes`
+// (negative: no limit) fails as hipMalloc does when the memory is used up.  Not part of the public interface.
+extern "C" void fp_test_limit_bytes(fp_ctx *ctx, int64_t bytes);
 
 // Brackets the launches of one kernel with events on the context stream when
 // profiling is on (fp_ctx_profile); the elapsed times are folded in on query.

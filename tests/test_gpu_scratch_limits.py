@@ -1,0 +1,86 @@
+"""Solves where the device memory is nearly used up: what the randomized factors need beyond the matrix may be
+missing, never the answer.
+
+The context is given a byte limit (a request beyond it fails as hipMalloc does on a full device), in steps from less
+than the pivoted LU in place needs to more than every path needs.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+NOMEM = 9
+
+
+@pytest.fixture
+def limit(fp):
+    ctx = fp._native.context()
+    f = fp._native.lib().fp_test_limit_bytes
+    f.argtypes, f.restype = [ctypes.c_void_p, ctypes.c_int64], None
+
+    def set_limit(nbytes):
+        ctx.trim()
+        f(ctx.handle, int(nbytes))
+    yield set_limit
+    f(ctx.handle, -1)
+
+
+def _attempt(fp, call):
+    try:
+        return call()
+    except fp.FPError as e:
+        assert e.code == NOMEM, e
+        return None
+
+
+def _matrix(n):
+    rng = np.random.default_rng(n)
+    return rng.standard_normal((n, n)) + 2 * np.sqrt(n) * np.eye(n), rng
+
+
+@pytest.mark.parametrize("k", [1, 3, 40])
+def test_fp64_lu_serves_wherever_the_pivoted_one_does(fp, limit, monkeypatch, k):
+    n = 700   # the copy takes 3.9 MB, its block inverses 10.5 MB
+    A, rng = _matrix(n)
+    X = rng.standard_normal((n, k))
+    B = A @ X
+    ctx, paths = fp._native.context(), set()
+    for mb in np.arange(3.5, 40.0, 0.7):
+        got = []
+        for pivoted in ("1", "0"):
+            monkeypatch.setenv("FLOWPANEL_LU64_PIVOTED", pivoted)
+            limit(mb * 1e6)
+            ctx.profile(True)
+            got.append(_attempt(fp, lambda: fp.solve_ludiv(None, A, B)))
+            tslu = ctx.profile_get("panel_tslu")[0]
+            ctx.profile(False)
+        if got[0] is not None:
+            assert got[1] is not None, mb
+        if got[1] is not None:
+            assert np.abs(got[1] - X).max() < 1e-11 * np.abs(X).max(), mb
+            paths.add(tslu > 0)
+    assert paths == {True, False}
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 40])
+def test_fp32_lu_serves_wherever_its_matrix_and_a_copy_fit(fp, limit, k):
+    # the explicit inverses (from four columns on) take three more FP32 matrices, the block inverses 5.2 MB
+    n, ld = 700, 704
+    A, rng = _matrix(n)
+    X = rng.standard_normal((n, k))
+    B = A @ X
+    need = 2 * 4 * n * ld + 9 * 8 * n * max(k, 4) + 2 * 8 * 128 * 128 * 6
+    for nbytes in [need] + [need + x * 1e6 for x in np.arange(0.4, 18.0, 1.1)]:
+        limit(nbytes)
+        got = fp.solve_lu32_ir(None, A, B)
+        assert np.abs(got - X).max() < 1e-9 * np.abs(X).max(), nbytes
+
+
+def test_a_released_limit_gives_the_randomized_path_back(fp, limit):
+    A, rng = _matrix(300)
+    limit(1000)
+    assert _attempt(fp, lambda: fp.solve_ludiv(None, A, A[:, 0])) is None
+    limit(-1)
+    x = fp.solve_ludiv(None, A, A[:, 0])
+    assert abs(x[0] - 1) < 1e-12 and np.abs(x[1:]).max() < 1e-12
