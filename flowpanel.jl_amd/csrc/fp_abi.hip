@@ -2568,7 +2568,7 @@ static int lsq_bordered(fp_ctx *ctx, fp_body *const *bodies, int nb, const std::
     FP_HIP(ctx, hipStreamSynchronize(ctx->stream));   // the host vectors go out of scope
     s.ms_assemble = tm.stop();
     // solve B^T Z = E_P, then B y = b_red - Z (Z^T Z)^-1 Z^T b_red, with the chosen solver
-    std::unique_ptr<Solver> first;   // of B^T: its LU serves B as well
+    std::unique_ptr<Solver> first;   // of B^T, where its LU serves B as well
     auto square_solve = [&](DBuf &M, const double *rhs_d, int64_t k, double *out) -> int {
         SolveArgs a;
         a.solver = o.solver;
@@ -2581,7 +2581,12 @@ static int lsq_bordered(fp_ctx *ctx, fp_body *const *bodies, int nb, const std::
         a.R64 = M.as<double>();
         int s2;
         if (o.solver == FP_SOLVER_LU) {
-            if ((s2 = dalloc(ctx, W, (size_t)n * ld * sizeof(double)))) return s2;
+            s2 = dalloc(ctx, W, (size_t)n * ld * sizeof(double));
+            if (first && no_room(ctx, s2)) {   // without the first matrix's factors there may be
+                first.reset();
+                s2 = dalloc(ctx, W, (size_t)n * ld * sizeof(double));
+            }
+            if (s2) return s2;
             FP_HIP(ctx, hipMemcpyAsync(W.p, M.p, (size_t)n * ld * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
             a.A64 = W.as<double>();
         } else if (o.solver == FP_SOLVER_GMRES) {
@@ -2598,7 +2603,13 @@ static int lsq_bordered(fp_ctx *ctx, fp_body *const *bodies, int nb, const std::
         first.reset();
         if (!ok && (s2 = solver->setup(s))) return s2;
         if ((s2 = solver->solve_multi(rhs_d, out, k, s))) return s2;
-        if (&M == &Bt) first = std::move(solver);
+        if (&M == &Bt && solver->rbt64) {
+            // its factors alone: the matrices and the operator end here
+            solver->a.A64 = nullptr;
+            solver->a.R64 = nullptr;
+            solver->a.resid = nullptr;
+            first = std::move(solver);
+        }
         return FP_OK;
     };
     if (np) {

@@ -84,3 +84,28 @@ def test_a_released_limit_gives_the_randomized_path_back(fp, limit):
     limit(-1)
     x = fp.solve_ludiv(None, A, A[:, 0])
     assert abs(x[0] - 1) < 1e-12 and np.abs(x[1:]).max() < 1e-12
+
+
+def test_least_squares_serves_wherever_the_pivoted_one_does(fp, geo, limit, monkeypatch):
+    # the factors of the first matrix stay for the second, unless its copy needs their room
+    body = fp.RigidWakeBody(geo.sphere(n_meridional=23, n_azimuthal=24), None, formulation=2)
+    U = np.tile([[1.0], [0.2], [0.0]], (1, body.ncells))
+    ctx, factored = fp._native.context(), set()
+    ref = None
+    for mb in list(np.arange(45.0, 6.0, -0.5)):
+        got = []
+        for pivoted in ("1", "0"):
+            monkeypatch.setenv("FLOWPANEL_LU64_PIVOTED", pivoted)
+            limit(mb * 1e6)
+            ctx.profile(True)
+            ok = _attempt(fp, lambda: fp.solve(body, U, solver=fp.solve_ludiv) or True)
+            counts = tuple(ctx.profile_get(c)[0] > 0 for c in ("lu_nopiv_diag", "panel_tslu"))
+            ctx.profile(False)
+            got.append(body.strength.copy() if ok else None)
+        if got[0] is not None:
+            ref = got[0] if ref is None else ref
+            assert got[1] is not None, mb
+        if got[1] is not None:
+            assert np.abs(got[1] - ref).max() < 1e-9 * np.abs(ref).max(), mb
+            factored.add(counts)
+    assert {(True, False), (False, True)} <= factored
