@@ -1611,22 +1611,33 @@ struct BatchImpl {
             const int64_t n = bb->n, ld = bb->ld;
             if (stored() && (st = dalloc(ctx, bb->A64, (size_t)n * ld * sizeof(double)))) return st;
             if (lu32() && (st = dalloc(ctx, bb->A32, (size_t)n * ld * sizeof(float)))) return st;
-            if (lu32()) {
-                bb->n4 = fp_rbt_size(n);
-                bb->ld4 = round_ld(bb->n4);
-                if ((st = dalloc(ctx, bb->Ar, (size_t)bb->n4 * bb->ld4 * sizeof(float))) ||
-                    (st = dalloc(ctx, bb->W, fp_rbt_weights_bytes(n))) ||
-                    (st = dalloc(ctx, bb->nwork, fp_getrf_nopiv_work_bytes(bb->n4, sizeof(float)))) ||
-                    (st = dalloc(ctx, bb->t4, bb->n4 * sizeof(double))) || (st = dalloc(ctx, bb->t4b, bb->n4 * sizeof(double))))
-                    return st;
-                if ((st = fp_rbt_weights(ctx, n, RBT_SEED, bb->W.as<double>()))) return st;
-            }
             if ((st = dalloc(ctx, bb->rhs, n * sizeof(double))) || (st = dalloc(ctx, bb->x, n * sizeof(double))) ||
                 (st = dalloc(ctx, bb->r, n * sizeof(double))) || (st = dalloc(ctx, bb->d, n * sizeof(double))) ||
                 (st = dalloc(ctx, bb->perm, n * sizeof(int))) || (st = dalloc(ctx, bb->info, sizeof(int))) ||
                 (st = dalloc(ctx, bb->fwork, fp_getrf_work_bytes(n, lu32() ? sizeof(float) : sizeof(double)))) ||
                 (st = dalloc(ctx, bb->swork, fp_getrs_work_bytes(n, 1))))
                 return st;
+        }
+        // the randomized copies come last: a body without room for its own takes the pivoted LU of A32
+        if ((st = dalloc(ctx, items, bodies.size() * sizeof(AssemblyItem))) ||
+            (lu32() && (st = dalloc(ctx, lu_tab, bodies.size() * sizeof(fp_lu_desc)))))
+            return st;
+        for (auto &bb : bodies) {
+            if (!lu32()) break;
+            const int64_t n = bb->n;
+            bb->n4 = fp_rbt_size(n);
+            bb->ld4 = round_ld(bb->n4);
+            if (!(st = dalloc(ctx, bb->Ar, (size_t)bb->n4 * bb->ld4 * sizeof(float))) &&
+                !(st = dalloc(ctx, bb->W, fp_rbt_weights_bytes(n))) &&
+                !(st = dalloc(ctx, bb->nwork, fp_getrf_nopiv_work_bytes(bb->n4, sizeof(float)))) &&
+                !(st = dalloc(ctx, bb->t4, bb->n4 * sizeof(double))) && !(st = dalloc(ctx, bb->t4b, bb->n4 * sizeof(double))))
+                st = fp_rbt_weights(ctx, n, RBT_SEED, bb->W.as<double>());
+            if (no_room(ctx, st)) {
+                bb->pivoted = true;
+                for (DBuf *b : {&bb->Ar, &bb->W, &bb->nwork, &bb->t4, &bb->t4b}) b->reset();
+            } else if (st) {
+                return st;
+            }
         }
         return FP_OK;
     }

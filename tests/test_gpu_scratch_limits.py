@@ -109,3 +109,35 @@ def test_least_squares_serves_wherever_the_pivoted_one_does(fp, geo, limit, monk
             assert np.abs(got[1] - ref).max() < 1e-9 * np.abs(ref).max(), mb
             factored.add(counts)
     assert {(True, False), (False, True)} <= factored
+
+
+def test_batch_bodies_without_room_for_a_randomized_copy_are_pivoted(fp, geo, limit):
+    # 800, 1,008 and 384 panels, whose block inverses take 5.2, 5.2 and 2.6 MB
+    V = fp.direction(4.0, 0.0)
+    bodies, ref = [], []
+    for nc, ns in ((40, 20), (42, 24), (16, 24)):
+        b = fp.RigidWakeBody(*geo.loft_wing(n_chord=nc, n_span=ns, span=8.0, taper=0.5, sweep_deg=20.0))
+        U, D = np.tile(V[:, None], (1, b.ncells)), np.tile(V[:, None], (1, b.nsheddings))
+        fp.solve(b, U, D, D, solver=fp.solve_ludiv)
+        ref.append(b.strength.copy())
+        bodies.append(b)
+
+    def solve():
+        batch = fp.BodyBatch(bodies, solver=fp.solve_lu32_ir)
+        for _ in range(3):   # replays of one graph
+            batch.solve()
+        return [b.strength.copy() for b in bodies]
+
+    # FP64 and FP32 matrices, their copies, and the workspaces of two substitutions and a pivoted panel
+    sizes = [(b.ncells, (b.ncells + 63) // 64 * 64) for b in bodies]
+    need = sum(16 * n * ld + 2 * 8 * (2 * n + 2 * 16384 * ((n + 127) // 128)) + 1200000 + 200 * n for n, ld in sizes)
+    served = 0
+    for nbytes in [need] + [need + x * 1e6 for x in np.arange(-22.0, 14.0, 1.5)]:
+        limit(nbytes)
+        got = _attempt(fp, solve)
+        assert got is not None or nbytes < need
+        if got is not None:
+            served += 1
+            for g, r in zip(got, ref):
+                assert np.abs(g - r).max() < 1e-8 * np.abs(r).max(), nbytes
+    assert served >= 10
