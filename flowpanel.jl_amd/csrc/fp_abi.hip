@@ -88,6 +88,16 @@ bool no_room(fp_ctx *ctx, int st)
     return true;
 }
 
+// Scratch for the partial sums of split field launches, `bytes` of it; none (and bytes = 0) where there is no room:
+// the launches then run with as many splits as they are given scratch for, one if there is none.
+int field_scratch(fp_ctx *ctx, DBuf &part, size_t &bytes)
+{
+    const int st = bytes ? dalloc(ctx, part, bytes) : FP_OK;
+    if (!no_room(ctx, st)) return st;
+    bytes = 0;
+    return FP_OK;
+}
+
 // Host to device and back on the context's stream, done on return.  (A blocking hipMemcpy runs on the null stream,
 // which does not wait for the context's: it could write a buffer from the pool under the late work of a call that
 // ended with an error.)
@@ -225,7 +235,7 @@ struct MatrixFreeOp : Operator {
     int init()
     {
         for (auto *b : bodies) part_bytes = std::max(part_bytes, fp_field_partial_bytes(tv.M, b->N));
-        return part_bytes ? dalloc(ctx, part, part_bytes) : FP_OK;
+        return field_scratch(ctx, part, part_bytes);
     }
     int apply(const double *x, double *y) override
     {
@@ -3057,7 +3067,7 @@ static int field_eval(fp_ctx *ctx, fp_body *const *bodies, int nb, const double 
     tv.x = tg.as<double>(); tv.y = tv.x + nt; tv.z = tv.x + 2 * nt; tv.M = nt;
     size_t pb = 0;
     for (int k = 0; k < nb; ++k) pb = std::max(pb, fp_field_partial_bytes(nt, bodies[k]->N));
-    if (pb && (st = dalloc(ctx, part, pb))) return st;
+    if ((st = field_scratch(ctx, part, pb))) return st;
     for (int k = 0; k < nb; ++k)
         if ((st = fp_launch_field(ctx, bodies[k], bodies[k]->d_strength, tv, mode, o.as<double>(), part.as<double>(), pb)))
             return st;
@@ -3103,7 +3113,7 @@ int fp_calcfield_U(fp_ctx *ctx, fp_body *const *bodies, int nb, double *out)
     }
     size_t pb = 0;
     for (int k = 0; k < nb; ++k) pb = std::max(pb, fp_field_partial_bytes(M, bodies[k]->N));
-    if (pb && (st = dalloc(ctx, part, pb))) return st;
+    if ((st = field_scratch(ctx, part, pb))) return st;
     for (int k = 0; k < nb; ++k)
         if ((st = fp_launch_field(ctx, bodies[k], bodies[k]->d_strength, t.tv, 0, o.as<double>(), part.as<double>(), pb)))
             return st;
@@ -3521,7 +3531,7 @@ static int liftdrag_run(fp_ctx *ctx, fp_body *const *bodies, int nb, const doubl
     tp.M = M;
     size_t fpb = 0;
     for (int k = 0; k < nb; ++k) fpb = std::max(fpb, fp_field_partial_bytes(M, bodies[k]->N));
-    if (fpb && (st = dalloc(ctx, fpart, fpb))) return st;
+    if ((st = field_scratch(ctx, fpart, fpb))) return st;
     FP_HIP(ctx, hipMemsetAsync(V.p, 0, 3 * M * sizeof(double), ctx->stream));
     for (int k = 0; k < nb; ++k)
         if ((st = fp_launch_field(ctx, bodies[k], bodies[k]->d_strength, tp, 0, V.as<double>(), fpart.as<double>(), fpb)))

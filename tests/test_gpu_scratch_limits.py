@@ -141,3 +141,20 @@ def test_batch_bodies_without_room_for_a_randomized_copy_are_pivoted(fp, geo, li
             for g, r in zip(got, ref):
                 assert np.abs(g - r).max() < 1e-8 * np.abs(r).max(), nbytes
     assert served >= 10
+
+
+@pytest.mark.parametrize("what", ["Uind", "phi"])
+def test_field_without_room_for_partial_sums(fp, geo, limit, what):
+    # 530,000 targets and what is returned there fit, the partial sums of the splits do not
+    b = fp.RigidWakeBody(*geo.loft_wing(n_chord=24, n_span=40, span=8.0, sweep_deg=20.0))
+    V = fp.direction(4.0, 0.0)
+    U, D = np.tile(V[:, None], (1, b.ncells)), np.tile(V[:, None], (1, b.nsheddings))
+    fp.solve(b, U, D, D)
+    nt = 530000
+    T = np.asfortranarray(np.random.default_rng(7).uniform([[-1.0], [-4.0], [-1.0]], [[3.0], [4.0], [1.0]], (3, nt)))
+    out = [np.zeros((3, nt) if what == "Uind" else nt, order="F") for _ in range(2)]
+    getattr(fp, what)(b, T, out[0])
+    limit(24 * nt + out[0].nbytes + 4096)
+    getattr(fp, what)(b, T, out[1])
+    # the same terms in one sum instead of several
+    assert np.abs(out[0] - out[1]).max() < 2000 * np.finfo(float).eps * np.abs(out[0]).max()
