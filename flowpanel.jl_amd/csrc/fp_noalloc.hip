@@ -9,7 +9,6 @@
 // stream capture, in tight time-stepping loops).
 #include "fp_internal.h"
 
-#include <algorithm>
 #include <cstdio>
 #include <mutex>
 
@@ -105,16 +104,11 @@ extern "C" int fp_uind_noalloc(fp_ctx *ctx, fp_body *const *bodies, int nb, cons
     }
     if (!device_array(d_targets, d) || !device_array(d_out, d))
         return fp_fail(ctx, FP_ERR_ARG, "fp_uind_noalloc: targets and out must be device memory of the context's GPU");
-    // scratch layout: [targets SoA | partial sums]
+    // scratch layout: [targets SoA | partial sums]; the launches split the panels as far as the rest of the
+    // scratch holds partial sums (2^20 targets leave 40 MiB for splits of 24 bytes a target: one)
     const size_t stage = ((size_t)3 * nt * sizeof(double) + NOALLOC_ALIGN - 1) / NOALLOC_ALIGN * NOALLOC_ALIGN;
-    size_t need = 0;
-    for (int k = 0; k < nb; ++k) need = std::max(need, fp_field_partial_bytes(nt, bodies[k]->N));
-    if (stage + need > NOALLOC_SCRATCH_BYTES) {
-        char buf[160];
-        snprintf(buf, sizeof buf, "fp_uind_noalloc: %zu scratch bytes needed, %zu available", stage + need,
-                 NOALLOC_SCRATCH_BYTES);
-        return fp_fail(ctx, FP_ERR_ARG, buf);
-    }
+    static_assert((size_t)3 * FP_UIND_NOALLOC_MAX_TARGETS * sizeof(double) + NOALLOC_ALIGN <= NOALLOC_SCRATCH_BYTES,
+                  "the scratch holds the targets of every call that is taken");
     double *soa = (double *)base;
     double *partial = (double *)((char *)base + stage);
     hipLaunchKernelGGL(k_aos_to_soa3, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, ctx->stream, d_targets, nt, soa);

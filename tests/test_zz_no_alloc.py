@@ -79,6 +79,28 @@ def test_uind_noalloc_matches_uind(fp, geo, hip):
         assert np.array_equal(out, ref), (nt, np.abs(out - ref).max())
 
 
+@pytest.mark.parametrize("nt", [700001, 1 << 20])
+def test_uind_noalloc_takes_every_count_up_to_its_limit(fp, geo, hip, nt):
+    # the partial sums of the splits fp_uind would choose here do not fit behind the staged targets: fewer splits do
+    g, sh = geo.loft_wing(n_chord=24, n_span=16, span=6.0, sweep_deg=20.0)
+    body = fp.RigidWakeBody(g, sh)
+    V = fp.direction(4.0)
+    D = np.tile(V[:, None], (1, body.nsheddings))
+    fp.solve(body, np.tile(V[:, None], (1, body.ncells)), D, D)
+    T = np.asfortranarray(np.random.default_rng(22).uniform([-1, -4, -1], [3, 4, 1], size=(nt, 3)).T)
+    ref = np.zeros((3, nt), order="F")
+    fp.Uind(body, T, ref)
+    dt, do = DeviceArray(hip, T), DeviceArray(hip, np.zeros((3, nt)))
+    try:
+        _noalloc(fp, body, dt.ptr, nt, do.ptr)
+        out = do.download()
+    finally:
+        dt.free()
+        do.free()
+    # the same terms in other partial sums: rounding of a sum over 384 panels
+    assert np.abs(out - ref).max() < 400 * np.finfo(float).eps * np.abs(ref).max()
+
+
 def test_uind_noalloc_rejects_what_it_cannot_take(fp, geo, hip):
     body = fp.NonLiftingBody(geo.sphere(n_meridional=6, n_azimuthal=8))
     fp.solve(body, np.tile([[1.0], [0.0], [0.0]], (1, body.ncells)))
