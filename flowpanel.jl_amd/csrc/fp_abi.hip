@@ -40,6 +40,18 @@ int fp_hip_fail(fp_ctx *ctx, hipError_t e, const char *what)
     return fp_fail(ctx, e == hipErrorOutOfMemory ? FP_ERR_NOMEM : FP_ERR_DEVICE, buf);
 }
 
+int fp_dev_malloc(fp_ctx *ctx, void **p, size_t bytes)
+{
+    *p = nullptr;
+    hipError_t e = ctx->pool->room(bytes) ? hipMalloc(p, bytes) : hipErrorOutOfMemory;
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();
+        if (ctx->pool->trim() && ctx->pool->room(bytes) && (e = hipMalloc(p, bytes)) != hipSuccess) *p = nullptr;
+    }
+    return e == hipSuccess ? FP_OK : fp_hip_fail(ctx, e, "hipMalloc");
+}
+
 namespace {
 
 // device buffer owned by a host scope; goes back to its context's pool when released
@@ -67,14 +79,7 @@ int dalloc(fp_ctx *ctx, DBuf &b, size_t bytes)
     b.pool = ctx->pool;
     b.bytes = bytes;
     if ((b.p = ctx->pool->get(bytes))) return FP_OK;
-    hipError_t e = ctx->pool->room(bytes) ? hipMalloc(&b.p, bytes) : hipErrorOutOfMemory;
-    if (e != hipSuccess) {
-        // out of memory: release what is held for re-use and try once more
-        b.p = nullptr;
-        (void)hipGetLastError();
-        if (ctx->pool->trim() && ctx->pool->room(bytes)) e = hipMalloc(&b.p, bytes);
-    }
-    if (e != hipSuccess) { b.p = nullptr; return fp_hip_fail(ctx, e, "hipMalloc"); }
+    if (int st = fp_dev_malloc(ctx, &b.p, bytes)) return st;
     ctx->pool->taken(bytes);
     return FP_OK;
 }
@@ -1447,8 +1452,8 @@ int build_horseshoes(fp_ctx *ctx, fp_body *b)
     gptr.push_back(nh);
     tab.insert(tab.end(), ord.begin(), ord.end());
     tab.insert(tab.end(), gptr.begin(), gptr.end());
-    FP_HIP(ctx, hipMalloc((void **)&b->d_hh, soa.size() * sizeof(double)));
-    FP_HIP(ctx, hipMalloc((void **)&b->d_hcol, tab.size() * sizeof(int)));
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_hh, soa.size() * sizeof(double))) return st;
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_hcol, tab.size() * sizeof(int))) return st;
     if (int st = h2d(ctx, b->d_hh, soa.data(), soa.size() * sizeof(double))) return st;
     if (int st = h2d(ctx, b->d_hcol, tab.data(), tab.size() * sizeof(int))) return st;
     b->nh = nh;
@@ -2275,12 +2280,12 @@ int fp_body_create(fp_ctx *ctx, const double *nodes, int64_t nnodes, const int64
             for (int d = 0; d < 3; ++d) pv[(size_t)(3 * k + d) * N + j] = b->nodes[3 * v + d];
         }
     }
-    FP_HIP(ctx, hipMalloc((void **)&b->d_pv, pv.size() * sizeof(double)));
-    FP_HIP(ctx, hipMalloc((void **)&b->d_nv, N * sizeof(int)));
-    FP_HIP(ctx, hipMalloc((void **)&b->d_hs, (size_t)FP_HS_STRIDE(nvp) * N * sizeof(double)));
-    FP_HIP(ctx, hipMalloc((void **)&b->d_geo, (size_t)FP_GEO_STRIDE * N * sizeof(double)));
-    FP_HIP(ctx, hipMalloc((void **)&b->d_uinf, (size_t)3 * N * sizeof(double)));
-    FP_HIP(ctx, hipMalloc((void **)&b->d_strength, N * sizeof(double)));
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_pv, pv.size() * sizeof(double))) return st;
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_nv, N * sizeof(int))) return st;
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_hs, (size_t)FP_HS_STRIDE(nvp) * N * sizeof(double))) return st;
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_geo, (size_t)FP_GEO_STRIDE * N * sizeof(double))) return st;
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_uinf, (size_t)3 * N * sizeof(double))) return st;
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_strength, N * sizeof(double))) return st;
     if (int st = h2d(ctx, b->d_pv, pv.data(), pv.size() * sizeof(double))) return st;
     if (int st = h2d(ctx, b->d_nv, nvv.data(), N * sizeof(int))) return st;
     FP_HIP(ctx, hipMemsetAsync(b->d_strength, 0, N * sizeof(double), ctx->stream));
@@ -2838,7 +2843,7 @@ int fp_assemble(fp_ctx *ctx, fp_body *const *bodies, int nb, int precision, fp_m
     m->ld = round_ld(t.M);
     m->precision = precision;
     const size_t es = precision == FP_F64 ? sizeof(double) : sizeof(float);
-    FP_HIP(ctx, hipMalloc(&m->A, (size_t)m->n * m->ld * es));
+    if (int st = fp_dev_malloc(ctx, &m->A, (size_t)m->n * m->ld * es)) return st;
     if ((st = assemble_into(ctx, bodies, nb, t.tv, precision, m->A, m->ld))) { (void)hipFree(m->A); return st; }
     m->bodies.assign(bodies, bodies + nb);
     FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -2859,7 +2864,7 @@ int fp_mat_upload(fp_ctx *ctx, int64_t n, const double *Ah, fp_mat **out)
     int st = dalloc(ctx, tmp, (size_t)n * n * sizeof(double));
     if (st) return st;
     if ((st = h2d(ctx, tmp.p, Ah, (size_t)n * n * sizeof(double)))) return st;
-    FP_HIP(ctx, hipMalloc(&m->A, (size_t)n * m->ld * sizeof(double)));
+    if (int st = fp_dev_malloc(ctx, &m->A, (size_t)n * m->ld * sizeof(double))) return st;
     if ((st = fp_mat_convert(ctx, tmp.as<double>(), n, n, m->A, m->ld, FP_F64, 1))) { (void)hipFree(m->A); return st; }
     FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     *out = m.release();
@@ -3169,7 +3174,7 @@ int fp_calcfield_cp(fp_ctx *ctx, const double *Us, int64_t n, double uref, const
 static int ensure_shedding_on_device(fp_ctx *ctx, fp_body *b)
 {
     if (b->ns > 0 && !b->d_sh) {
-        FP_HIP(ctx, hipMalloc((void **)&b->d_sh, 6 * b->ns * sizeof(int64_t)));
+        if (int st = fp_dev_malloc(ctx, (void **)&b->d_sh, 6 * b->ns * sizeof(int64_t))) return st;
         if (int st = h2d(ctx, b->d_sh, b->shedding.data(), 6 * b->ns * sizeof(int64_t))) return st;
     }
     return FP_OK;
@@ -3989,7 +3994,7 @@ static int body_neighbors(fp_ctx *ctx, fp_body *b)
                 if (o != j) { nb[(size_t)k * N + j] = (int)o; break; }
         }
     }
-    FP_HIP(ctx, hipMalloc((void **)&b->d_nbr, nb.size() * sizeof(int)));
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_nbr, nb.size() * sizeof(int))) return st;
     if (int st = h2d(ctx, b->d_nbr, nb.data(), nb.size() * sizeof(int))) return st;
     return FP_OK;
 }
@@ -4016,7 +4021,7 @@ int fp_calcfield_ugradmu(fp_ctx *ctx, fp_body *const *bodies, int nb, int te_cor
         fp_body *b = bodies[k];
         if ((st = body_neighbors(ctx, b))) return st;
         if (b->ns > 0 && !b->d_sh) {
-            FP_HIP(ctx, hipMalloc((void **)&b->d_sh, 6 * b->ns * sizeof(int64_t)));
+            if (int st = fp_dev_malloc(ctx, (void **)&b->d_sh, 6 * b->ns * sizeof(int64_t))) return st;
             if ((st = h2d(ctx, b->d_sh, b->shedding.data(), 6 * b->ns * sizeof(int64_t)))) return st;
         }
         if ((st = fp_launch_ugradmu(ctx, b, b->d_nbr, b->d_sh, te_correction, o.as<double>() + 3 * off))) return st;
@@ -4187,7 +4192,7 @@ int fp_calcfield_ugradmu_combined(fp_ctx *ctx, fp_body *const *bodies, int nb, i
         const int64_t N = b->N;
         if ((st = body_neighbors(ctx, b))) return st;
         if (b->ns > 0 && !b->d_sh) {
-            FP_HIP(ctx, hipMalloc((void **)&b->d_sh, 6 * b->ns * sizeof(int64_t)));
+            if (int st = fp_dev_malloc(ctx, (void **)&b->d_sh, 6 * b->ns * sizeof(int64_t))) return st;
             if ((st = h2d(ctx, b->d_sh, b->shedding.data(), 6 * b->ns * sizeof(int64_t)))) return st;
         }
         if ((st = dalloc(ctx, cellv, 3 * std::max<int64_t>(1, N) * sizeof(double)))) return st;

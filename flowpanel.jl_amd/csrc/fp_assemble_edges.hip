@@ -259,7 +259,7 @@ int fp_body_build_edge_blocks(fp_ctx *ctx, fp_body *b)
     int64_t sums[2];
     const int64_t nblocks = build_edge_blocks(b->nodes.data(), (int64_t)b->nodes.size() / 3, b->cell_ptr.data(),
                                               b->cell_idx.data(), b->N, tab, sums);
-    FP_HIP(ctx, hipMalloc((void **)&b->d_eb, tab.size() * sizeof(int32_t)));
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_eb, tab.size() * sizeof(int32_t))) return st;
     FP_HIP(ctx, hipMemcpy(b->d_eb, tab.data(), tab.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     b->eb_nblocks = nblocks;
     b->eb_nodes = sums[0];
@@ -275,7 +275,7 @@ static int body_build_pair_blocks(fp_ctx *ctx, fp_body *b)
     const int64_t npb = build_pair_blocks(b->nodes.data(), (int64_t)b->nodes.size() / 3, b->cell_ptr.data(),
                                           b->cell_idx.data(), b->N, pt, sums);
     if (npb <= 0) return fp_fail(ctx, FP_ERR_UNSUPPORTED, "edge-pair tables: a block does not pair into 256 lanes");
-    FP_HIP(ctx, hipMalloc((void **)&b->d_pb, pt.size() * sizeof(int32_t)));
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_pb, pt.size() * sizeof(int32_t))) return st;
     FP_HIP(ctx, hipMemcpy(b->d_pb, pt.data(), pt.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     b->pb_nblocks = npb;
     return FP_OK;

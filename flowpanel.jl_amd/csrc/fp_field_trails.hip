@@ -111,8 +111,8 @@ int fp_body_build_trails(fp_ctx *ctx, fp_body *b)
                                    cptr, cpan);
     if (S == 0) return FP_OK;
     const size_t ib = (S + (S + 1) + std::max<size_t>(1, cpan.size())) * sizeof(int32_t);
-    FP_HIP(ctx, hipMalloc((void **)&b->d_tr_tab, ib));
-    FP_HIP(ctx, hipMalloc((void **)&b->d_tr, (size_t)TR_COMP * S * sizeof(double)));
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_tr_tab, ib)) return st;
+    if (int st = fp_dev_malloc(ctx, (void **)&b->d_tr, (size_t)TR_COMP * S * sizeof(double))) return st;
     int32_t *t = b->d_tr_tab;
     FP_HIP(ctx, hipMemcpy(t, ref.data(), S * sizeof(int32_t), hipMemcpyHostToDevice));
     FP_HIP(ctx, hipMemcpy(t + S, cptr.data(), (S + 1) * sizeof(int32_t), hipMemcpyHostToDevice));

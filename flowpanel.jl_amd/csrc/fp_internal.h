@@ -101,6 +101,10 @@ struct fp_ctx {
     ~fp_ctx();
 };
 
+// hipMalloc for the context; out of memory, it releases the pool's buffers and tries once more.  FP_ERR_NOMEM if
+// that does not help (*p null).
+int fp_dev_malloc(fp_ctx *ctx, void **p, size_t bytes);
+
 // For tests of a full device, without filling one: an allocation that would take the context's buffers beyond `bytes`
 // (negative: no limit) fails as hipMalloc does when the memory is used up.  Not part of the public interface.
 extern "C" void fp_test_limit_bytes(fp_ctx *ctx, int64_t bytes);
