@@ -26,7 +26,7 @@
 //
 // A x = b becomes  A_r y = U^T b,  x = V y.  A depth-2 butterfly couples only
 // the four indices {p, p + m, p + 2m, p + 3m} (m = n4 / 4, n4 = n rounded up
-// to a multiple of 4, the pad being the identity), so U^T A V is one pass of
+// to a multiple of 4, the pad being a diagonal), so U^T A V is one pass of
 // 4 x 4 . 4 x 4 . 4 x 4 products over the (p, q) orbit blocks, and the vector
 // transforms are 4 x 4 products per orbit.  A zero or non-finite pivot is
 // reported through `info` and the caller falls back to the pivoted LU.
@@ -803,9 +803,11 @@ __global__ void k_fill_info(int *p, int v)
 }
 
 // U^T A V over the orbit blocks: thread (p, q) reads the 4 x 4 block of A at rows
-// p + i m, columns q + j m (the identity beyond n), forms U_p^T B V_q in FP64 and
+// p + i m, columns q + j m, forms U_p^T B V_q in FP64 and
 // stores it rounded to T.  W holds the 4 x 4 butterfly of every orbit,
-// row-major: U's at W[16 p], V's at W[16 (m + q)].  With part set, part[workgroup]
+// row-major: U's at W[16 p], V's at W[16 (m + q)].  Beyond n the matrix is continued by a diagonal
+// of the size of its own entries (the largest of the same orbit block): the butterflies mix the pad's rows with
+// rows of A, whose digits a 1 among entries of 1e-12 would take.  With part set, part[workgroup]
 // receives the sum of squares of the entries of A it read.
 template <typename Tin, typename T>
 __global__ __launch_bounds__(256) void k_rbt_matrix(const Tin *__restrict__ A, int64_t n, int64_t lda,
@@ -823,9 +825,20 @@ __global__ __launch_bounds__(256) void k_rbt_matrix(const Tin *__restrict__ A, i
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int64_t gc = q + j * m;
-                B[i][j] = (gr < n && gc < n) ? (double)A[gr * lda + gc] : (gr == gc ? 1.0 : 0.0);
+                B[i][j] = (gr < n && gc < n) ? (double)A[gr * lda + gc] : 0.0;
                 sq = fma(B[i][j], B[i][j], sq);
             }
+        }
+        if (p == q && p + 3 * m >= n) {   // (the last row of an orbit is in the pad if any of it is)
+            double pad = 0.0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) pad = fmax(pad, fabs(B[i][j]));
+            if (!(pad > 0.0) || isinf(pad)) pad = 1.0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (p + i * m >= n) B[i][i] = pad;
         }
         const double *U = W + 16 * p, *V = W + 16 * (m + q);
         double X[4][4];
@@ -851,7 +864,7 @@ __global__ __launch_bounds__(256) void k_rbt_matrix(const Tin *__restrict__ A, i
     if (threadIdx.x == 0) part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = sw[0] + sw[1] + sw[2] + sw[3];
 }
 
-// out[0] = sum of part[0 .. np), out[1] = smallest |A(i, i)| (NaN when one is NaN); one workgroup
+// out[0] = sum of part[0 .. np), out[1] = smallest |A(i, i)| (0 when one is NaN); one workgroup
 __global__ __launch_bounds__(1024) void k_lu_check(const double *__restrict__ part, int64_t np,
                                                    const double *__restrict__ A, int64_t n, int64_t ld,
                                                    double *__restrict__ out)

@@ -196,3 +196,20 @@ def test_columns_beyond_the_range_of_their_squares(fp, scale):
     X[:, 1] = 0.0
     got, counts = _counted(fp, A, A @ X)
     assert counts["panel_tslu"] == 0 and not got[:, 1].any()
+
+
+@pytest.mark.parametrize("n", [257, 258, 259, 260, 5])
+@pytest.mark.parametrize("scale", [1e-12, 1.0, 1e12])
+@pytest.mark.parametrize("solver", ["solve_ludiv", "solve_lu32_ir"])
+def test_units_do_not_decide_the_path(fp, n, scale, solver):
+    # the randomized matrix is padded to a multiple of 4: its pad has the matrix's own scale, and is no part of its norm
+    A, rng = _matrix(n, 300 + n)
+    A += 1.5 * np.sqrt(n) * np.eye(n)   # no eigenvalue near zero: FP32 factors refine it
+    X = rng.standard_normal(n)
+    ctx = fp._native.context()
+    ctx.profile(True)
+    x = getattr(fp, solver)(None, scale * A, scale * (A @ X))
+    pivoted = ctx.profile_get("panel_tslu")[0]
+    ctx.profile(False)
+    assert pivoted == 0
+    assert np.abs(x - X).max() <= max(64 * n * EPS, 1e-12) * np.linalg.cond(A) * np.abs(X).max()
