@@ -3884,12 +3884,15 @@ int fp_batch_solve(fp_ctx *ctx, fp_batch *h, fp_batch_stats *stats)
     S.ms_graph = t.stop();
     const size_t nb = B.bodies.size();
     std::vector<double> nr(2 * nb);
+    std::vector<int> infos(nb, 0);
     FP_HIP(ctx, hipMemcpyAsync(nr.data(), B.norms.p, nr.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    for (size_t k = 0; k < nb; ++k)
+        FP_HIP(ctx, hipMemcpyAsync(&infos[k], B.bodies[k]->info.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     FP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     bool refall = false;
-    for (auto &bb : B.bodies) {
-        int info = 0;
-        if ((st = d2h(ctx, &info, bb->info.p, sizeof(int)))) return st;
+    for (size_t k = 0; k < nb; ++k) {
+        auto &bb = B.bodies[k];
+        const int info = infos[k];
         if (info && B.lu32() && !bb->pivoted) {
             // the randomized no-pivot LU met a bad pivot: this body switches to the pivoted LU
             if ((st = B.fallback(*bb))) return st;
