@@ -1044,6 +1044,7 @@ int fp_rbt_vec(fp_ctx *ctx, const double *in, int64_t ldin, double *out, int64_t
 {
     const int64_t m = fp_rbt_size(n) / 4;
     if (m == 0 || k == 0) return FP_OK;
+    if (k > 65535) return fp_fail(ctx, FP_ERR_UNSUPPORTED, "getrs: too many right-hand sides in one call");   // as fp_getrs
     hipLaunchKernelGGL(k_rbt_vec, dim3((unsigned)((m + 255) / 256), (unsigned)k), dim3(256), 0, ctx->stream, in, ldin,
                        out, ldout, n, m, k, d_W, transpose_u);
     FP_HIP(ctx, hipGetLastError());

@@ -213,3 +213,19 @@ def test_units_do_not_decide_the_path(fp, n, scale, solver):
     ctx.profile(False)
     assert pivoted == 0
     assert np.abs(x - X).max() <= max(64 * n * EPS, 1e-12) * np.linalg.cond(A) * np.abs(X).max()
+
+
+@pytest.mark.parametrize("solver", ["solve_ludiv", "solve_lu32_ir"])
+def test_more_columns_than_a_launch_takes_are_refused_as_by_the_pivoted_lu(fp, solver, monkeypatch):
+    A, _ = _matrix(4, 15)
+    text = []
+    for pivoted in ("1", "0"):
+        monkeypatch.setenv("FLOWPANEL_LU64_PIVOTED", pivoted)
+        monkeypatch.setenv("FLOWPANEL_LU32_PIVOTED", pivoted)
+        with pytest.raises(fp.FPError) as e:
+            getattr(fp, solver)(None, A, np.ones((4, 65536)))
+        assert e.value.code == 10
+        text.append(str(e.value))
+    assert text[0] == text[1]
+    X = getattr(fp, solver)(None, A, A @ np.ones((4, 65535)))
+    assert np.abs(X - 1).max() < 1e-10
