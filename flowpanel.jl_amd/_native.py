@@ -221,7 +221,7 @@ class Context:
         self.check(lib().fp_ctx_synchronize(self.handle))
 
     def trim(self):
-        """Free the large device buffers the context keeps for re-use by the next call of the same size."""
+        """Free the device buffers the context keeps for re-use by the next call of the same size."""
         self.check(lib().fp_ctx_trim(self.handle))
 
     def profile(self, enable=True, only=None):

@@ -2914,6 +2914,7 @@ int fp_coarse_setup(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, int cs, floa
         hipLaunchKernelGGL(k_probe_check, gv, dim3(256), 0, ctx->stream, (const double *)v, (const double *)z, nc,
                            0.5 * COARSE_LU_TOL, info_dev);
     } else {
+        ProfScope ps(ctx, "coarse_inverse_gj");
         // larger coarse spaces: FP32 blocked Gauss-Jordan of E (it only feeds the
         // preconditioner), widened back in place; work (2 nc^2 doubles) holds the
         // FP32 inverse and the Gauss-Jordan scratch

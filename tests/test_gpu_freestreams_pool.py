@@ -1,4 +1,5 @@
 """Many freestreams in one call, and the context's pool of small buffers."""
+import ctypes
 import gc
 
 import numpy as np
@@ -39,8 +40,16 @@ def test_small_buffers_survive_many_sizes_and_a_closed_context(fp):
     fp.context().trim()
     A = rng.standard_normal((50, 50)) + 50 * np.eye(50)
     assert np.allclose(fp.solve_ludiv(None, A, A @ np.ones(50)), 1.0)
-    other = fp._native.Context(0)
-    del other
+    nat = fp._native
+    L, other = nat.lib(), nat.Context(0)
+    h, Af, x = ctypes.c_void_p(), nat.f64(A), np.zeros((50, 1), order="F")
+    other.check(L.fp_mat_upload(other.handle, 50, nat.dptr(Af), ctypes.byref(h)))
+    o = nat.opts(nat.FP_SOLVER_LU)
+    other.check(L.fp_solve_mat(other.handle, h, nat.dptr(nat.f64((A @ np.ones(50)).reshape(50, 1))), 1, nat.dptr(x),
+                               ctypes.byref(o), None))
+    L.fp_mat_destroy(h)
+    assert np.allclose(x, 1.0)
+    del other   # with the solve's buffers in its pool
     gc.collect()
     assert np.allclose(fp.solve_ludiv(None, A, A @ np.ones(50)), 1.0)
 

@@ -16,6 +16,15 @@ def _matrix(n, seed):
     return rng.standard_normal((n, n)) + 0.5 * np.sqrt(n) * np.eye(n), rng
 
 
+def _counted(fp, A, B):
+    ctx = fp._native.context()
+    ctx.profile(True)
+    X = fp.solve_ludiv(None, A, B)
+    counts = {name: ctx.profile_get(name)[0] for name in ("getrs", "panel_tslu")}
+    ctx.profile(False)
+    return X, counts
+
+
 @pytest.mark.parametrize("n", [1, 2, 5, 15, 17, 63, 64, 65, 129, 255, 256, 257, 288, 290, 321, 513, 771])
 @pytest.mark.parametrize("k", [1, 3])
 @pytest.mark.parametrize("pivoted", ["0", "1"])
@@ -24,7 +33,9 @@ def test_fp64_lu_matches_lapack(fp, n, k, pivoted, monkeypatch):
     A, rng = _matrix(n, 100 + n)
     X = rng.standard_normal((n, k))
     B = A @ X
-    got = fp.solve_ludiv(None, A, B if k > 1 else B[:, 0]).reshape(n, k)
+    got, counts = _counted(fp, A, B if k > 1 else B[:, 0])
+    assert (counts["panel_tslu"] > 0) == (pivoted == "1"), counts   # the path asked for, and no other
+    got = got.reshape(n, k)
     ref = np.linalg.solve(A, B)
     bound = 64 * n * EPS * np.linalg.cond(A)
     assert np.abs(got - ref).max() <= bound * np.abs(ref).max()
@@ -136,15 +147,6 @@ def _passes_the_pivots_only(n=64):
     M[1, 0] = 0.0
     U, V = _butterfly(n // 4, SEED), _butterfly(n // 4, SEED ^ 0x5DEECE66D)
     return np.linalg.solve(U.T, M) @ np.linalg.inv(V)
-
-
-def _counted(fp, A, B):
-    ctx = fp._native.context()
-    ctx.profile(True)
-    X = fp.solve_ludiv(None, A, B)
-    counts = {name: ctx.profile_get(name)[0] for name in ("getrs", "panel_tslu")}
-    ctx.profile(False)
-    return X, counts
 
 
 @pytest.mark.parametrize("k", [1, 3])
