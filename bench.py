@@ -388,7 +388,7 @@ def adjoint_leg(fp, ctx, fd_coords=64, reps=3, block=400):
     r64 = fp.lift_drag_gradient(body, U, **kw)
     g_m = np.concatenate([r["dCL_dnodes"][0].ravel(), r["dCDi_dnodes"][0].ravel()])
     g_64 = np.concatenate([r64["dCL_dnodes"][0].ravel(), r64["dCDi_dnodes"][0].ravel()])
-    kernels = {k: {"launches": v[0], "total_ms": round(v[1] / reps, 3)} for k, v in prof.items()}
+    kernels = {k: {"launches": v[0] // reps, "total_ms": round(v[1] / reps, 3)} for k, v in prof.items()}
     rec = {
         "workload": "wing NACA 2412, AR 8, twist 0 -> -3 deg, 100 x 100 vortex-ring quads + rigid wake, AoA 4.0",
         "panels": body.ncells, "nodes": body.grid.nnodes,
