@@ -841,8 +841,12 @@ struct Solver {
         st = a.R64 ? fp_rbt_matrix<double, float>(ctx, a.R64, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>())
                    : fp_rbt_matrix<float, float>(ctx, a.A32, n, a.ld, Ar.as<float>(), ld4, Wrbt.as<double>());
         if (st) return st;
-        // the inverses cost about twice the factorisation ((4/3) n^3 against (2/3) n^3 on MFMA) and
-        // pay off when many right-hand sides are corrected together; FLOWPANEL_LU32_INVERSE=1/0 forces them
+        // explicit inverses cost about twice the factorisation ((4/3) n^3 against (2/3) n^3 on MFMA) and save part
+        // of every correction.  The line of four columns dates from sweeps of one 128-row block at a time; beside
+        // those through 512-row block inverses it lies too low.  Factors, three corrections included, sweeps against
+        // inverses, ms: 480 panels 0.53 and 0.84 at 4 columns, 0.56 and 0.87 at 64; 2,000 1.50 and 2.43, 1.91 and
+        // 2.75; 4,800 3.77 and 5.71, 5.84 and 7.44; 9,000 11.7 and 19.5, 18.9 and 26.7 (four corrections).
+        // FLOWPANEL_LU32_INVERSE=1/0 forces them
         const char *gi = getenv("FLOWPANEL_LU32_INVERSE");
         inv = gi && (gi[0] == '0' || gi[0] == '1') ? gi[0] == '1' : a.nrhs >= 4;
         if (inv) {
@@ -875,7 +879,8 @@ struct Solver {
     // FP64 LU of the randomized matrix without pivoting (FP_SOLVER_LU), with refinement; the matrix itself stays as it
     // is.  *ok = false, and nothing kept, where it does not serve: no room for the copy, the block inverses or
     // the vectors, a zero or non-finite pivot, or a pivot below 1e-11 |A|_F (a matrix singular to rounding, or near
-    // it): those take the pivoted LU in place, with its results and errors.
+    // it): those take the pivoted LU in place, with its results and errors, and cost both factorisations (a matrix
+    // singular to rounding: 500 unknowns 2.66 ms against 2.20 for the pivoted LU alone, 4,800 31.4 against 26.6).
     int rbt64_setup(bool *ok)
     {
         *ok = false;
@@ -1486,12 +1491,6 @@ __global__ void k_cp(const double *__restrict__ U, int64_t n, double uref, doubl
     if (i >= n) return;
     const double u = sqrt(U[3 * i] * U[3 * i] + U[3 * i + 1] * U[3 * i + 1] + U[3 * i + 2] * U[3 * i + 2]) / uref;
     out[i] += 1 - u * u;
-}
-
-__device__ __forceinline__ int64_t lane_value(int64_t v, int l)   // v of lane l (the same l in every lane)
-{
-    const uint32_t lo = __builtin_amdgcn_readlane((int)v, l), hi = __builtin_amdgcn_readlane((int)(v >> 32), l);
-    return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
 // One wave, 64 edges at a time: a lane per edge where no panel belongs to two of the 64 (compared lane by

@@ -138,12 +138,6 @@ __device__ __forceinline__ double wave_sum6(const double (&v)[6], int lane)
     return s;
 }
 
-__device__ __forceinline__ int64_t lane_value(int64_t v, int l)   // v of lane l (the same l in every lane)
-{
-    const uint32_t lo = __builtin_amdgcn_readlane((int)v, l), hi = __builtin_amdgcn_readlane((int)(v >> 32), l);
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
 // Kutta averaging (forward) of c0 in list order, or its reverse on c0 and c1 in reverse order.  One wave, 64
 // edges at a time: a lane per edge where no panel belongs to two of the 64, else one lane in order.  100 edges
 // by one lane: 194 us for the reverse (dependent loads).

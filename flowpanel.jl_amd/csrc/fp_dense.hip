@@ -623,25 +623,6 @@ static int trsm_llu(fp_ctx *ctx, int nb, int64_t ncols, const T *L, int64_t ldl,
 }
 
 // ----------------------------------------------------------------------------
-// Row interchanges: rows i in [k1, k2) swapped with ipiv[i] (sequentially), for
-// every column; one lane per column (row-major rows are contiguous).
-template <typename T>
-__global__ void k_laswp(T *__restrict__ A, int64_t ld, int64_t ncols, int64_t ld_rows, const int *__restrict__ ipiv,
-                        int k1, int k2)
-{
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncols) return;
-    for (int i = k1; i < k2; ++i) {
-        const int p = ipiv[i];
-        if (p != i && p >= 0 && (int64_t)p < ld_rows) {
-            const T a = A[(int64_t)i * ld + c];
-            A[(int64_t)i * ld + c] = A[(int64_t)p * ld + c];
-            A[(int64_t)p * ld + c] = a;
-        }
-    }
-}
-
-// ----------------------------------------------------------------------------
 // Tournament pivoting.
 constexpr int PW = 32;      // sub-panel width
 constexpr int CH = 256;     // rows per candidate chunk
@@ -1759,7 +1740,12 @@ int fp_gemv_multi(fp_ctx *ctx, const T *A, int64_t n, int64_t ld, const double *
     if (ld % 4 || ((uintptr_t)A & 15)) return fp_fail(ctx, FP_ERR_ARG, "gemv needs an aligned matrix");
     ProfScope ps(ctx, sizeof(T) == 8 ? "gemv_multi_f64" : "gemv_multi_f32");
     if constexpr (sizeof(T) == 4) {
-        if (k > GEMVM_NV) {   // up to one group of columns the vector form reads A once and wastes no products
+        // up to one group of eight columns the vector form reads A once and wastes no products.  Vector form and this
+        // one, us: 480 rows 18.4 and 9.4 at 9 columns, 18.0 and 10.9 at 17, 18.1 and 17.4 at 64; 9,000 rows (A beyond
+        // the last-level cache) 277 and 221, 391 and 279, 1,192 and 508; 4,800 rows, whose 92 MB a second pass finds in
+        // that cache, 94 and 95, 104 and 123, 179 and 155 at 32, 328 and 220 at 64: there 10 to 17 columns lose
+        // up to a fifth.
+        if (k > GEMVM_NV) {
             const int nx = k > 32 ? 4 : k > 16 ? 2 : 1;
             const dim3 g((unsigned)((n + MM_R - 1) / MM_R), (unsigned)((k + 16 * nx - 1) / (16 * nx)));
             auto kern = nx == 4 ? k_gemm_multi<4> : nx == 2 ? k_gemm_multi<2> : k_gemm_multi<1>;
@@ -2839,6 +2825,9 @@ __global__ __launch_bounds__(256) void k_widen_f32(const float *__restrict__ x, 
 // no-pivot FP32 LU and the inverses of its factors (about 4 nc^3 flop of MFMA products),
 // smaller ones by the blocked Gauss-Jordan (2 nc^3, but a chain of nc / 64 passes).  3,000
 // vectors (30,000 panels), whole preconditioner set-up: Gauss-Jordan 8.6 ms, LU 6.5 ms (6.2 with the row sums below).
+// Set-up just above the line and further on, Gauss-Jordan and LU, ms: 4,800 panels 534 vectors 1.02 and 0.78, 1,200
+// 1.83 and 1.47; 10,000 panels 527 1.48 and 1.00, 2,000 3.49 and 2.60; 18,000 panels 530 2.26 and 1.50, 3,000 5.97
+// and 4.60, at the same iteration counts.
 // The inverse has to return a probe vector from its product with E to COARSE_LU_TOL of the
 // vector's size; a zero pivot or a worse inverse sets info, and the caller repeats the
 // set-up with the Gauss-Jordan, whose verdict is final.  FLOWPANEL_COARSE_INV=gj: always

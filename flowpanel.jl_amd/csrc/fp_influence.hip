@@ -600,7 +600,10 @@ __global__ void k_field_reduce(const double *__restrict__ partial, int splits, i
 // Splits of the panel range over grid.y.  Up to 512 workgroups of targets: 2,048 workgroups, one
 // round of the chip.  Above that the last, partly filled round costs (2,344 workgroups of 600,000
 // targets are 9.2 a compute unit, of which the last 1.2 run nearly alone), so the work is cut to
-// 8,192 and more; the partial sums are 24 bytes a target and split.
+// 8,192 and more; the partial sums are 24 bytes a target and split.  Kernel ms cut to 2,048 and to 8,192: 10,000
+// panels, 131,073 targets 5.71 and 5.19, 300,000 12.95 and 11.62, 520,000 20.04 and 19.98, 600,001 25.7 and 23.2,
+// 2,000,000 (one split both) 74.0 and 74.2; 2,000 panels 1.30 and 1.26, 2.98 and 2.75, 4.86 and 4.73, 6.09 and 5.51;
+// 400 panels 0.31 and 0.31, 0.70 and 0.66, 1.13 and 1.13, 1.41 and 1.30.
 static int field_splits(int64_t M, int64_t N)
 {
     const int64_t bx = (M + 255) / 256;

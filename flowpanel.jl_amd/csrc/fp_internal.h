@@ -109,6 +109,13 @@ int fp_dev_malloc(fp_ctx *ctx, void **p, size_t bytes);
 // (negative: no limit) fails as hipMalloc does when the memory is used up.  Not part of the public interface.
 extern "C" void fp_test_limit_bytes(fp_ctx *ctx, int64_t bytes);
 
+// v of lane l (the same l in every lane)
+__device__ __forceinline__ int64_t lane_value(int64_t v, int l)
+{
+    const uint32_t lo = __builtin_amdgcn_readlane((int)v, l), hi = __builtin_amdgcn_readlane((int)(v >> 32), l);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
 // Brackets the launches of one kernel with events on the context stream when
 // profiling is on (fp_ctx_profile); the elapsed times are folded in on query.
 struct ProfScope {
@@ -395,8 +402,6 @@ int fp_mat_convert(fp_ctx *ctx, const double *src, int64_t n, int64_t lds, void 
 int fp_mat_narrow(fp_ctx *ctx, const double *src, float *dst, int64_t n, int64_t ld);
 int fp_rhs_kernel(fp_ctx *ctx, const fp_body *b, double *rhs);   // rhs_i = -Uinf_i . n_i
 int fp_residual_update(fp_ctx *ctx, const double *b, double *r, int64_t n);   // r = b - r
-int fp_dot(fp_ctx *ctx, const double *x, const double *y, int64_t n, double *d_out);
-int fp_axpy(fp_ctx *ctx, double a, const double *x, double *y, int64_t n);
 // R = B - A X (n x k, column-major, ld n), accumulated in twice FP64
 int fp_resid_dd(fp_ctx *ctx, const double *A, int64_t n, int64_t ld, const double *X, int64_t k, const double *B, double *R);
 int fp_fill(fp_ctx *ctx, double *x, int64_t n, double v);   // x[:] = v (a kernel: safe inside graphs)

@@ -421,10 +421,12 @@ template <typename T> __device__ __forceinline__ void lu_first_dev(const LuMat<T
 // not wait for U12, which lu_urow_dev forms when the outer block is done).  Workgroup 0 owns the next
 // diagonal block: it goes on to factor it, so that a step is one launch and the other strips run beside
 // the next block's pivot chain.  All products are 64 x 64 x 64 from LDS, the next tile loaded into
-// registers meanwhile.  Workgroup 0 bounds it.  With the three U12 tiles in that workgroup and four waves
-// (cycles of the diagonal block, FP32 and FP64: pivots 14,700 and 20,700, 16-row substitutions 7,500 and
-// 8,900, inverses 8,000 and 12,500, U12 19,100 and 36,200, of 61,500 and 94,800) the first block took 26 and
-// 39 us and 4,800 unknowns 3.2 and 6.3 ms; with eight waves and U12 elsewhere 14 and 22 us, 2.8 and 5.2 ms.
+// registers meanwhile.  Workgroup 0 bounds it.  Cycles of its parts at 4,800 unknowns, FP32 and FP64 (a clock
+// read at each, on the average over the steps): L tile 6,200 and 9,200, W 4,200 and 11,400, the columns' update
+// 11,500 and 21,000 (two tiles), then the diagonal block's pivots 16,300 and 22,600, 16-row substitutions 7,200
+// and 7,100, trailing tiles 3,700 and 5,800, inverses 7,700 and 13,500, stores 900 and 1,600; a launch takes 20.4
+// and 31.9 us.  With the three U12 tiles in that workgroup and four waves the first block took 26 and 39 us and
+// 4,800 unknowns 3.2 and 6.3 ms; with eight waves and U12 elsewhere 16 and 23 us, 2.8 and 5.2 ms.
 template <typename T>
 __device__ __forceinline__ void lu_step_dev(const LuMat<T> &m, int64_t k, int t, int64_t kend, int b, StepLds<T> &s)
 {
@@ -1088,14 +1090,14 @@ static int64_t lu_tiles(int64_t x, int64_t w) { return x > 0 ? (x + w - 1) / w :
 // That update's columns of the next outer block are brought up to date in the launch that also factors the
 // next diagonal block (k_lu_update); as much of the rest as the chain of launches has room for goes into
 // these launches as further workgroups (lu_rest_dev), which need nothing of the chain and are not needed by
-// it before the U rows; only what is left is a launch of its own (fp_gemm_sub).  SLOTS: workgroups that the
-// chip holds (two FP32, one FP64 per compute unit); FIRST, STEP: tiles per slot that the launch of a diagonal
+// it before the U rows; only what is left is a launch of its own (fp_gemm_sub).  PER_CU: workgroups that a
+// compute unit holds, a slot each; FIRST, STEP: tiles per slot that the launch of a diagonal
 // block and a step take before the chain waits for them, by measurement.  4,800 (8,000) unknowns, ms, FP32:
 // nothing carried 2.80 (6.66), 1/1 2.54 (6.18), 1/2 2.37 (5.85), 2/2 2.35 (5.79), 2/3 2.36 (5.80); FP64: nothing
 // 5.23 (13.1), 1/1 4.86 (12.5), 1/2 4.50 (11.95), 2/2 4.52 (12.06), 2/4 4.77 (12.5).
 template <typename T> struct LuRoom;
-template <> struct LuRoom<float> { static constexpr int SLOTS = 512, FIRST = 2, STEP = 2; };
-template <> struct LuRoom<double> { static constexpr int SLOTS = 256, FIRST = 1, STEP = 2; };
+template <> struct LuRoom<float> { static constexpr int PER_CU = 2, FIRST = 2, STEP = 2; };
+template <> struct LuRoom<double> { static constexpr int PER_CU = 1, FIRST = 1, STEP = 2; };
 
 template <typename T>
 int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void *work, T *YL, T *YU)
@@ -1105,6 +1107,7 @@ int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void
     hipLaunchKernelGGL(k_fill_info, dim3(1), dim3(64), 0, ctx->stream, info_dev, 0);
     const LuMat<T> m{A, ld, n, (T *)work, (T *)work + lu_dsize(n), info_dev, YL, YU};
     int st;
+    const int64_t slots = (int64_t)LuRoom<T>::PER_CU * ctx->num_cu;
     int64_t rest_j = n;   // columns from here on still miss the previous outer block's update
     for (int64_t k = 0; k < n; k += NOB) {
         const int64_t kend = std::min<int64_t>(k + NOB, n), rows = lu_tiles(n - k, NPB);
@@ -1119,7 +1122,7 @@ int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void
             ProfScope ps(ctx, "lu_nopiv_diag");
             hipLaunchKernelGGL(k_lu_first<T>, dim3(1), dim3(LT), 0, ctx->stream, m, k);
         } else {
-            const int64_t pc = lu_tiles(kend - k, NPB), x = take(LuRoom<T>::SLOTS * LuRoom<T>::FIRST - pc * rows, rows == 1);
+            const int64_t pc = lu_tiles(kend - k, NPB), x = take(slots * LuRoom<T>::FIRST - pc * rows, rows == 1);
             ProfScope ps(ctx, "lu_nopiv_update");
             hipLaunchKernelGGL(k_lu_update<T>, dim3((unsigned)(pc * rows + x)), dim3(LT), 0, ctx->stream, m, k, (int)pc,
                                (int)(pc * rows), r);
@@ -1128,7 +1131,7 @@ int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void
         for (int t = 0; t < NIN; ++t) {
             const int64_t strips = rows - 1 - t;
             if (strips <= 0) break;
-            const int64_t x = take((LuRoom<T>::SLOTS - strips) * LuRoom<T>::STEP, t + 2 >= NIN || strips == 1);
+            const int64_t x = take((slots - strips) * LuRoom<T>::STEP, t + 2 >= NIN || strips == 1);
             ProfScope ps(ctx, "lu_nopiv_step");
             hipLaunchKernelGGL(k_lu_step<T>, dim3((unsigned)(strips + x)), dim3(LT), 0, ctx->stream, m, k, t, kend, (int)strips,
                                r);
@@ -1144,9 +1147,9 @@ int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void
         if (right <= 0) break;
         // tile columns of the update right of the next outer block, as many as its launches have room for
         const int64_t rt = lu_tiles(right, NPB), pt = std::min<int64_t>(NIN, rt);
-        int64_t room = std::max<int64_t>((int64_t)LuRoom<T>::SLOTS * LuRoom<T>::FIRST - pt * rt, 0);
+        int64_t room = std::max<int64_t>(slots * LuRoom<T>::FIRST - pt * rt, 0);
         for (int t = 0; t < std::min<int64_t>(NIN - 1, rt - 1); ++t)
-            room += std::max<int64_t>(LuRoom<T>::SLOTS - (rt - 1 - t), 0) * LuRoom<T>::STEP;
+            room += std::max<int64_t>(slots - (rt - 1 - t), 0) * LuRoom<T>::STEP;
         const int64_t now = rt - pt - std::min(room / rt, rt - pt);   // the others, at once
         const int64_t j0 = kend + pt * NPB;
         rest_j = std::min(j0 + now * NPB, n);

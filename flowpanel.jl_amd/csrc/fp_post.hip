@@ -78,8 +78,7 @@ __global__ __launch_bounds__(64) void k_ugradmu_te(const double *__restrict__ pv
         const int64_t own = q0 + threadIdx.x < 2 * ns ? sh[3 * (q0 + threadIdx.x)] : -1;
         const int m = (int)(2 * ns - q0 < 64 ? 2 * ns - q0 : 64);
         for (int l = 0; l < m; ++l) {
-            const uint32_t lo = __builtin_amdgcn_readlane((int)own, l), hi = __builtin_amdgcn_readlane((int)(own >> 32), l);
-            const bool same = (int64_t)(((uint64_t)hi << 32) | lo) == c;
+            const bool same = lane_value(own, l) == c;
             first = first && !(same && q0 + l < i);
             times += same && q0 + l > i;
         }
