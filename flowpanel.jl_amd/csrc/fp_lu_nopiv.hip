@@ -640,9 +640,11 @@ __device__ __forceinline__ void lu_urow_dev(const LuMat<T> &m, int64_t k, int64_
     }
 }
 
+// (the first launch of a factorisation: it also clears the info word)
 template <typename T> __global__ __launch_bounds__(LT) void k_lu_first(LuMat<T> m, int64_t k)
 {
     __shared__ StepLds<T> s;
+    if (threadIdx.x == 0) atomicExch(m.info, 0);
     lu_first_dev<T>(m, k, s);
 }
 // The previous outer block's update of the columns [k, k + 64 pc), one 64 x 64 tile per workgroup (np of them),
@@ -799,11 +801,6 @@ __global__ __launch_bounds__(256) void k_tri_gemv(const T *__restrict__ M, int64
         }
 }
 
-__global__ void k_fill_info(int *p, int v)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
-}
-
 // U^T A V over the orbit blocks: thread (p, q) reads the 4 x 4 block of A at rows
 // p + i m, columns q + j m (zeros beyond n), forms U_p^T B V_q in FP64 and
 // stores it rounded to T.  W holds the 4 x 4 butterfly of every orbit,
@@ -875,7 +872,9 @@ __global__ __launch_bounds__(256) void k_rbt_matrix(const Tin *__restrict__ A, i
 }
 
 // The blocks with a pad once more, now with it (three at most, the last ones of the diagonal).  In the kernel above the
-// same lines took its registers from 76 to 102, and the batch's launches, which share the chip, from 450 to 725 us.
+// same lines took its registers from 76 to 102, and the batch's launches, which share the chip, from 450 to 725 us;
+// with selects from the three other diagonal entries and 76 registers they took 560 (its loads of rows then wait
+// for each other).
 template <typename Tin, typename T>
 __global__ __launch_bounds__(64) void k_rbt_pad(const Tin *__restrict__ A, int64_t n, int64_t lda, T *__restrict__ Ar,
                                                 int64_t m, int64_t ldr, const double *__restrict__ W)
@@ -1104,7 +1103,6 @@ int fp_getrf_nopiv(fp_ctx *ctx, T *A, int64_t n, int64_t ld, int *info_dev, void
 {
     if (n <= 0) return FP_OK;
     if (ld % 4) return fp_fail(ctx, FP_ERR_ARG, "internal: no-pivot LU needs a leading dimension divisible by 4");
-    hipLaunchKernelGGL(k_fill_info, dim3(1), dim3(64), 0, ctx->stream, info_dev, 0);
     const LuMat<T> m{A, ld, n, (T *)work, (T *)work + lu_dsize(n), info_dev, YL, YU};
     int st;
     const int64_t slots = (int64_t)LuRoom<T>::PER_CU * ctx->num_cu;
